@@ -225,7 +225,10 @@ int u1_tune_enable(int32_t on);
  * results are bit-identical to two launches.  mode 0: never; 1 (default):
  * where the tuner measures the fused launch faster (needs tuning on); 2:
  * always.  The tune cache keeps the decision as "MetropolisPair" /
- * "OverRelaxationPair" entries (block.x 0 = two launches). */
+ * "OverRelaxationPair" entries (block.x 0 = two launches).  In mode 1 the
+ * phases (parity, 2) and (parity, 3) can likewise run as one launch, by
+ * wavefronts walking along the diagonals e_t - e_z, bit-identical too; entries
+ * "MetropolisWalk" / "OverRelaxationWalk" (block.x 0 = two launches). */
 int u1_set_pair_fusion(int32_t mode);
 /* Fused parity passes (no reference counterpart): on a single lattice without
  * multilevel mask whose (z, t) planes tile 2 x 4 (Nz even, Nt a multiple of
@@ -265,7 +268,8 @@ int u1_tune_entries(int32_t* n);
  * a scratch copy of the lattice (the chain is not advanced): per launch class
  * c of the sweep -- 0 Metropolis phase, 1 overrelaxation phase, 2 measuring
  * overrelaxation phase, 3 fused Metropolis pair, 4 fused overrelaxation pair,
- * 5 measuring fused overrelaxation pair (u1_set_pair_fusion), 6 fused
+ * 5 measuring fused overrelaxation pair (u1_set_pair_fusion; the walks over
+ * (parity, 2) + (parity, 3) count as pairs), 6 fused
  * Metropolis pass, 7 fused overrelaxation pass, 8 measuring fused
  * overrelaxation pass (u1_set_pass_fusion) -- 32 back-to-back launches in the
  * sweep's shapes between one event pair;

@@ -39,6 +39,8 @@ constexpr int kChainMaxMargin = 1024;  // fused-pass schedule margin accepted fr
 // binary32 Metropolis pass chosen at 5 % ahead ran no faster in full sweeps).
 constexpr float kChainMinGainOR = 0.97f;
 constexpr float kChainMinGainMetropolis = 0.90f;
+// A walk must take under this fraction of the two phases' time.
+constexpr float kWalkMinGain = 0.97f;
 double* g_scratch_dev[kMaxDevices] = {};
 
 // Launch shape of an update phase kernel: workgroup size, even/odd sites per
@@ -502,6 +504,171 @@ int pair_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseA
   return U1_OK;
 }
 
+// Launch shapes of one kernel class on one geometry (block 0: not fused).
+// walk: spt segments per wavefront (64 / width), tile the strip groups.
+struct Shapes {
+  Cfg phase = kDefaultCfg, pair{0, 1, 0, 0}, walk{0, 1, 0, 0}, chain{0, 1, 0, 0};
+};
+bool walk_cfg_ok(const RepDesc& r, int prec, const Cfg& c) {
+  return c.spt >= 1 && 64 % c.spt == 0 &&
+         u1d::walk_shape_ok(r, (int)elem_size(prec), c.block, 64 / c.spt, c.xcd ? 1 << c.tile : 0);
+}
+
+// The phases (a0.parity, mu0) and (a0.parity, mu0 + 1), mu0 = 0 or 2, in as many
+// launches as sh has them.  rows(mu): measurement rows of the launch that starts
+// with phase mu (null: not measuring).
+template <typename Rows>
+int launch_two_phases(int prec, int kind, void* lat, const PhaseArgs& a0, const Shapes& sh, int mu0, Rows rows) {
+  PhaseArgs a = a0;
+  if (mu0 == 2 && sh.walk.block != 0) {
+    const Cfg& w = sh.walk;
+    a.meas = rows(mu0);
+    HIPCHK(u1d::launch_walk(prec, kind, lat, a, w.block, 64 / w.spt, w.xcd ? 1 << w.tile : 0, G.st));
+    return U1_OK;
+  }
+  if (mu0 == 0 && sh.pair.block != 0) {
+    a.xcd = (uint32_t)sh.pair.xcd;
+    a.meas = rows(mu0);
+    set_pair_blocks(a.single, sh.pair);
+    HIPCHK(u1d::launch_pair(prec, kind, lat, a, a.single.nblk, sh.pair.block, sh.pair.spt,
+                            a.single.nxh * a.single.N[1], G.st));
+    return U1_OK;
+  }
+  a.xcd = (uint32_t)sh.phase.xcd;
+  set_update_blocks(a.single, sh.phase);
+  for (int mu = mu0; mu < mu0 + 2; ++mu) {
+    a.meas = mu > 0 ? rows(mu) : nullptr;
+    HIPCHK(u1d::launch_phase(prec, kind, mu, lat, a, a.single.nblk, sh.phase.block, sh.phase.spt, G.st));
+  }
+  return U1_OK;
+}
+const auto no_rows = [](int) -> double* { return nullptr; };
+
+template <typename Rows>
+int launch_parity(int prec, int kind, void* lat, const PhaseArgs& a, const Shapes& sh, Rows rows) {
+  RET(launch_two_phases(prec, kind, lat, a, sh, 0, rows));
+  return launch_two_phases(prec, kind, lat, a, sh, 2, rows);
+}
+
+// Shapes of the (parity, 2) + (parity, 3) walk: wavefronts and segments per
+// wavefront in strip-grouped order (first tuning stage), then the orders of
+// the best of them (second stage).
+std::vector<Cfg> walk_shapes(const RepDesc& r, int prec) {
+  std::vector<Cfg> v;
+  for (int spt : {1, 2, 4})
+    for (int w : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16}) {
+      const Cfg c{64 * w, spt, 1, 1};
+      if (walk_cfg_ok(r, prec, c)) v.push_back(c);
+    }
+  return v;
+}
+std::vector<Cfg> walk_orders(const std::vector<Cfg>& shapes, const std::vector<float>& t) {
+  std::vector<size_t> by(shapes.size());
+  for (size_t i = 0; i < by.size(); ++i) by[i] = i;
+  std::sort(by.begin(), by.end(), [&](size_t a, size_t b) { return t[a] < t[b]; });
+  std::vector<Cfg> v;
+  for (size_t i = 0; i < by.size() && i < 3; ++i)
+    for (int x = -1; x < 4; ++x) {
+      Cfg c = shapes[by[i]];
+      c.xcd = x >= 0;
+      c.tile = std::max(x, 0);
+      v.push_back(c);
+    }
+  return v;
+}
+
+// Shape of the walk for kernel class `kind`, or block = 0 for the two phases (sh:
+// the shapes it would replace): where the tuner measures it faster, as pair_cfg;
+// only with fused pairs left to the tuner (forced fusion means the plane pairs).
+int walk_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseArgs& proto, const Shapes& sh,
+             Cfg* cfg) {
+  *cfg = Cfg{0, 1, 0, 0};
+  if (G.pair != 1) return U1_OK;
+  const char* name = kind == u1d::KIND_METROPOLIS ? "MetropolisWalk" : "OverRelaxationWalk";
+  const std::string key = tune_key(name, g, prec);
+  const std::vector<Cfg> shapes = walk_shapes(proto.single, prec);
+  if (shapes.empty()) return U1_OK;
+  auto it = G.tunecache.find(key);
+  if (it != G.tunecache.end()) {  // block 0: the tuner measured the two phases faster
+    if (it->second.block != 0 && walk_cfg_ok(proto.single, prec, it->second)) *cfg = it->second;
+    return U1_OK;
+  }
+  if (!G.tune) return U1_OK;
+  const int64_t bytes = 4 * (int64_t)proto.single.V * (int64_t)elem_size(prec);
+  DevBuf scratch;
+  HIPCHK(scratch.alloc(bytes));
+  HIPCHK(hipMemcpyAsync(scratch.p, lat, bytes, hipMemcpyDeviceToDevice, G.st));
+  EventSet es;
+  hipEvent_t e0, e1;
+  HIPCHK(es.create(&e0));
+  HIPCHK(es.create(&e1));
+  PhaseArgs a = proto;
+  a.accepts = nullptr;
+  a.meas = nullptr;
+  Shapes s = sh;
+  auto timed = [&](const Cfg& c, float* best) -> int {
+    s.walk = c;
+    RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));  // warm-up
+    HIPCHK(hipEventRecord(e0, G.st));
+    for (int rep = 0; rep < 4; ++rep) RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));
+    HIPCHK(hipEventRecord(e1, G.st));
+    HIPCHK(hipEventSynchronize(e1));
+    float ms = 0;
+    HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+    *best = std::min(*best, ms);
+    return U1_OK;
+  };
+  auto shape = [](const Cfg& c) {
+    std::ostringstream o;
+    o << c.block / 64 << " wavefronts of " << c.spt << " segment(s), ";
+    if (c.xcd) o << (1 << c.tile) << " strip group(s)";
+    else o << "plain order";
+    return o.str();
+  };
+  auto search = [&](const std::vector<Cfg>& cands, std::vector<float>& tbest) -> int {
+    tbest.assign(cands.size(), 1e30f);
+    for (int round = 0; round < 3; ++round)
+      for (size_t i = 0; i < cands.size(); ++i) RET(timed(cands[i], &tbest[i]));
+    if (G.verbosity >= 2)
+      for (size_t i = 0; i < cands.size(); ++i)
+        std::fprintf(stderr, "tune %s: %s: %.2f us per walk\n", key.c_str(), shape(cands[i]).c_str(),
+                     1e3 * tbest[i] / 4.0);
+    return U1_OK;
+  };
+  std::vector<float> t1, t2;
+  RET(search(shapes, t1));
+  const std::vector<Cfg> orders = walk_orders(shapes, t1);
+  RET(search(orders, t2));
+  const Cfg best = orders[(size_t)(std::min_element(t2.begin(), t2.end()) - t2.begin())];
+  // both sides timed afresh, alternating (chain_cfg), and a clear win asked for
+  float tb = 1e30f, tsep = 1e30f;
+  for (int round = 0; round < 5; ++round) {
+    RET(timed(best, &tb));
+    RET(timed(Cfg{0, 1, 0, 0}, &tsep));
+  }
+  const bool use = tb < kWalkMinGain * tsep;
+  if (G.verbosity >= 1)
+    std::fprintf(stderr, "tune %s: walk %.2f us (%s) vs two launches %.2f us: %s\n", key.c_str(), 1e3 * tb / 4.0,
+                 shape(best).c_str(), 1e3 * tsep / 4.0, use ? "walk" : "separate");
+  *cfg = use ? best : Cfg{0, 1, 0, 0};
+  G.tunecache[key] = *cfg;
+  return U1_OK;
+}
+
+// Measurement rows of the phases (1, 1..3) of a pass launched by launch_parity:
+// first row of the launch covering phase mu, and (mu = 4) their total.
+int parity_row(const RepDesc& single, const Shapes& sh, int mu) {
+  RepDesc r = single;
+  set_update_blocks(r, sh.phase);
+  const int n = r.nblk;
+  set_pair_blocks(r, sh.pair);
+  int row = 0;
+  if (mu > 1) row += sh.pair.block != 0 ? r.nblk : n;
+  if (mu > 2) row += sh.walk.block != 0 ? u1d::walk_rows(single, 64 / sh.walk.spt) : n;
+  if (mu > 3 && sh.walk.block == 0) row += n;
+  return row;
+}
+
 // ------------------------------------------------------------ fused passes
 // Reports, and clears, a wait timeout of a fused pass (k_chain) since the
 // last check; called after the library stream has been synchronised.
@@ -627,36 +794,14 @@ int chain_launch(int prec, int kind, void* lat, const PhaseArgs& a0, const Cfg& 
   return U1_OK;
 }
 
-// The four phases of one parity as the unfused path launches them: the
-// fused (parity, 0) + (parity, 1) pair if pc says so, then the phases.
-int unfused_parity_pass(int prec, int kind, void* lat, const PhaseArgs& a0, const Cfg& c, const Cfg& pc) {
-  PhaseArgs a = a0;
-  for (int mu = 0; mu < 4; ++mu) {
-    if (mu == 0 && pc.block != 0) {
-      a.single = a0.single;
-      a.xcd = (uint32_t)pc.xcd;
-      set_pair_blocks(a.single, pc);
-      HIPCHK(u1d::launch_pair(prec, kind, lat, a, a.single.nblk, pc.block, pc.spt, a.single.nxh * a.single.N[1], G.st));
-      ++mu;
-    } else {
-      a.single = a0.single;
-      a.xcd = (uint32_t)c.xcd;
-      set_update_blocks(a.single, c);
-      HIPCHK(u1d::launch_phase(prec, kind, mu, lat, a, a.single.nblk, c.block, c.spt, G.st));
-    }
-  }
-  return U1_OK;
-}
-
 // Shape of the fused parity pass for kernel class `kind` on this geometry, or
 // block = 0 for the unfused launches.  With tuning, every fused shape is timed
-// against the unfused pass (tuned phase and pair shapes c, pc) on a scratch
-// copy: four passes each (parities 0, 1, 0, 1); the decision is cached
+// against the unfused pass (tuned shapes sh) on a scratch copy: four passes each (parities 0, 1, 0, 1); the decision is cached
 // (MetropolisChain / OverRelaxationChain, block.x 0 = unfused).  Only for an
 // unmasked single lattice whose (z, t) planes tile 2 x 4 (Nz even, Nt % 4 ==
 // 0), and never during stream capture (the counter targets are per launch).
-int chain_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseArgs& proto, const Cfg& c,
-              const Cfg& pc, Cfg* cfg) {
+int chain_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseArgs& proto, const Shapes& sh,
+              Cfg* cfg) {
   *cfg = Cfg{0, 1, 0, 0};
   if (G.chain == 0 || proto.ml != 0) return U1_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -696,7 +841,7 @@ int chain_cfg(int prec, int kind, const u1_geom* g, const void* lat, const Phase
     auto one = [&](int i) -> int {
       a.parity = i & 1;
       if (fused) return chain_launch(prec, kind, scratch.p, a, cc);
-      return unfused_parity_pass(prec, kind, scratch.p, a, c, pc);
+      return launch_parity(prec, kind, scratch.p, a, sh, no_rows);
     };
     RET(one(0));  // warm-up
     HIPCHK(hipEventRecord(e0, G.st));
@@ -773,22 +918,28 @@ int chain_cfg(int prec, int kind, const u1_geom* g, const void* lat, const Phase
   return U1_OK;
 }
 
+// Launch shapes of kernel class `kind` (tuned, if enabled).
+int kind_shapes(int prec, int kind, const u1_geom* g, const void* lat, const PhaseArgs& proto, Shapes* sh) {
+  RET(phase_cfg(prec, kind, g, lat, proto, &sh->phase));
+  RET(pair_cfg(prec, kind, g, lat, proto, sh->phase, &sh->pair));
+  RET(walk_cfg(prec, kind, g, lat, proto, *sh, &sh->walk));
+  return chain_cfg(prec, kind, g, lat, proto, *sh, &sh->chain);
+}
+
 // Settles (tunes, if enabled) every launch shape a sweep of this geometry
 // uses, and the fused passes' schedules and counters, so that a later sweep
 // allocates and synchronises nothing (graph capture, timed regions).
 int settle_update_cfgs(int prec, const u1_geom* g, const void* lat, const PhaseArgs& proto, int metrop, int ovrn) {
-  Cfg c, pc, cc;
+  Shapes sh;
   for (int kind = 0; kind < 2; ++kind) {
     if ((kind == u1d::KIND_METROPOLIS ? metrop : ovrn) <= 0) continue;
-    RET(phase_cfg(prec, kind, g, lat, proto, &c));
-    RET(pair_cfg(prec, kind, g, lat, proto, c, &pc));
-    RET(chain_cfg(prec, kind, g, lat, proto, c, pc, &cc));
-    if (cc.block != 0) {
+    RET(kind_shapes(prec, kind, g, lat, proto, &sh));
+    if (sh.chain.block != 0) {
       RepDesc r = proto.single;
-      set_chain_blocks(r, cc);
+      set_chain_blocks(r, sh.chain);
       u1d::ChainArgs ca{};
       int nb = 0;
-      RET(chain_prepare(r, cc, &ca, &nb));
+      RET(chain_prepare(r, sh.chain, &ca, &nb));
     }
   }
   return U1_OK;
@@ -819,70 +970,42 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
   a.sweep_dev = sweep_dev;
   a.sweep_mul = sweep_mul;
   a.accepts = acc_dev;
-  Cfg cm = kDefaultCfg, co = kDefaultCfg, pm{0, 1, 0, 0}, po{0, 1, 0, 0}, chm{0, 1, 0, 0}, cho{0, 1, 0, 0};
-  if (metrop > 0) RET(phase_cfg(prec, u1d::KIND_METROPOLIS, g, lat, a, &cm));
-  if (ovrn > 0) RET(phase_cfg(prec, u1d::KIND_OVERRELAX, g, lat, a, &co));
-  if (metrop > 0) RET(pair_cfg(prec, u1d::KIND_METROPOLIS, g, lat, a, cm, &pm));
-  if (ovrn > 0) RET(pair_cfg(prec, u1d::KIND_OVERRELAX, g, lat, a, co, &po));
-  if (metrop > 0) RET(chain_cfg(prec, u1d::KIND_METROPOLIS, g, lat, a, cm, pm, &chm));
-  if (ovrn > 0) RET(chain_cfg(prec, u1d::KIND_OVERRELAX, g, lat, a, co, po, &cho));
-  RepDesc rm = a.single, ro = a.single, rpm = a.single, rpo = a.single;
-  set_update_blocks(rm, cm);
-  set_update_blocks(ro, co);
-  set_pair_blocks(rpm, pm);
-  set_pair_blocks(rpo, po);
+  Shapes sm, so;
+  if (metrop > 0) RET(kind_shapes(prec, u1d::KIND_METROPOLIS, g, lat, a, &sm));
+  if (ovrn > 0) RET(kind_shapes(prec, u1d::KIND_OVERRELAX, g, lat, a, &so));
   if (meas_dst && (ml != 0 || metrop + ovrn == 0)) return fail(U1_ERR_ARG, "no measuring pass");
-  // measuring phases: parity 1, mu >= 1 of the last pass; rows of phase 1 (in
-  // a fused pair: one per plane), then of phases 2 and 3 (a fused pass: its
-  // own rows for phases 1-3, launch_chain)
-  const bool meas_or = ovrn > 0;
-  const Cfg& meas_chain = meas_or ? cho : chm;
-  const int meas_nblk = meas_or ? ro.nblk : rm.nblk;
-  const int meas_nblk1 = (meas_or ? po.block : pm.block) != 0 ? (meas_or ? rpo.nblk : rpm.nblk) : meas_nblk;
-  int meas_rows_total = meas_nblk1 + 2 * meas_nblk;
-  if (meas_chain.block != 0) {
+  // measuring phases: parity 1, mu >= 1 of the last pass; one row per
+  // workgroup of each launch that covers them, in launch order (a fused pass:
+  // its own rows for phases 1-3, launch_chain)
+  const Shapes& smeas = ovrn > 0 ? so : sm;
+  int meas_rows_total = parity_row(a.single, smeas, 4);
+  if (smeas.chain.block != 0) {
     RepDesc rc = a.single;
-    set_chain_blocks(rc, meas_chain);
+    set_chain_blocks(rc, smeas.chain);
     meas_rows_total = 3 * rc.N[2] * rc.N[3] * rc.bpp;
   }
   if (meas_dst) RET(ensure_fold(meas_rows_total, 4));
-  auto meas_rows = [&](bool last_pass, int parity, int mu) -> double* {
-    if (!meas_dst || !last_pass || parity != 1 || mu < 1) return nullptr;
-    return G.partials + 4 * (mu == 1 ? 0 : (size_t)meas_nblk1 + (size_t)meas_nblk * (size_t)(mu - 2));
-  };
-  // one pass of kind `kind`: per parity, one fused pass (chc), or (parity, 0)
-  // + (parity, 1) fused or not, then (parity, 2) and (parity, 3)
-  auto pass = [&](int kind, uint32_t p, bool last, const Cfg& c, const RepDesc& r, const Cfg& pc,
-                  const RepDesc& rp, const Cfg& chc) -> int {
+  // one pass of kind `kind`: per parity, one fused pass, or launch_parity
+  auto pass = [&](int kind, uint32_t p, bool last, const Shapes& sh) -> int {
     a.pass = p;
     for (int parity = 0; parity < 2; ++parity) {
-      if (chc.block != 0) {
-        a.parity = parity;
-        a.meas = meas_rows(last, parity, 1);  // rows from 0: phases 1-3 of the fused pass
-        RET(chain_launch(prec, kind, lat, a, chc));
+      const bool meas = meas_dst && last && parity == 1;
+      a.parity = parity;
+      if (sh.chain.block != 0) {
+        PhaseArgs b = a;
+        b.meas = meas ? G.partials : nullptr;
+        RET(chain_launch(prec, kind, lat, b, sh.chain));
         continue;
       }
-      for (int mu = 0; mu < 4; ++mu) {
-        const bool pair = mu == 0 && pc.block != 0;
-        a.parity = parity;
-        a.meas = meas_rows(last, parity, pair ? 1 : mu);
-        if (pair) {
-          a.single = rp;
-          a.xcd = (uint32_t)pc.xcd;
-          HIPCHK(u1d::launch_pair(prec, kind, lat, a, rp.nblk, pc.block, pc.spt, rp.nxh * rp.N[1], G.st));
-          ++mu;
-        } else {
-          a.single = r;
-          a.xcd = (uint32_t)c.xcd;
-          HIPCHK(u1d::launch_phase(prec, kind, mu, lat, a, r.nblk, c.block, c.spt, G.st));
-        }
-      }
+      RET(launch_parity(prec, kind, lat, a, sh, [&](int mu) -> double* {
+        return meas ? G.partials + 4 * (size_t)parity_row(a.single, sh, std::max(mu, 1)) : nullptr;
+      }));
     }
     return U1_OK;
   };
   for (int p = 0; p < metrop; ++p)
-    RET(pass(u1d::KIND_METROPOLIS, (uint32_t)p, ovrn == 0 && p == metrop - 1, cm, rm, pm, rpm, chm));
-  for (int o = 0; o < ovrn; ++o) RET(pass(u1d::KIND_OVERRELAX, (uint32_t)o, o == ovrn - 1, co, ro, po, rpo, cho));
+    RET(pass(u1d::KIND_METROPOLIS, (uint32_t)p, ovrn == 0 && p == metrop - 1, sm));
+  for (int o = 0; o < ovrn; ++o) RET(pass(u1d::KIND_OVERRELAX, (uint32_t)o, o == ovrn - 1, so));
   if (meas_dst)
     HIPCHK(u1d::launch_finish_sums(G.partials, meas_rows_total, 4, 1.0 / (3.0 * (double)a.single.V), meas_dst,
                                    fold_scratch_ptr(meas_rows_total, 4), G.st));
@@ -2129,11 +2252,15 @@ int u1_tune_load(const char* path) {
       parsed.push_back({vol + "\t" + name, Cfg{bx, by, 1, bz, bx == 0 ? 0 : gx}});
       continue;
     }
-    if (name.find("Pair_") != std::string::npos)  // fused pair: block 0 = two launches
+    const bool walk = name.find("Walk_") != std::string::npos;
+    if (walk)  // block 0 = two launches; block.y segments per wavefront
+      known = (bx == 0 && by == 1) || (bx >= 64 && bx <= 64 * u1d::walk_max_waves(f32 ? 4 : 8) && bx % 64 == 0 &&
+                                       (by == 1 || by == 2 || by == 4));
+    else if (name.find("Pair_") != std::string::npos)  // fused pair: block 0 = two launches
       known = (bx == 0 && by == 1) || pair_shape_ok(f32 ? U1_F32 : U1_F64, Cfg{bx, by, 0, 0});
     else
       for (const Cfg& c : kShapes) known = known || (c.block == bx && c.spt == by);
-    if (!known || (by == 4 && !f32) || bz < 1 || bz > 4)
+    if (!known || (by == 4 && !f32 && !walk) || bz < 1 || bz > (walk ? 8 : 4))
       return fail(U1_ERR_IO, std::string("Bad launch shape in ") + path + ": " + line);
     parsed.push_back({vol + "\t" + name, Cfg{bx, by, (bz - 1) & 1, (bz - 1) >> 1}});
   }
@@ -2156,7 +2283,9 @@ int u1_tune_save(const char* path) {
     f << vol << "\t" << name << "\tthreads=halfvolume\t" << kv.second.block << "\t" << kv.second.spt << "\t"
       << (chain ? kv.second.tile : 1 + kv.second.xcd + 2 * kv.second.tile) << "\t" << (chain ? kv.second.margin : 0)
       << "\t1\t1\t0\t# block.x = workgroup size, block.y = sites per thread, block.z - 1 = XCD-aware order (1) + "
-         "tiled planes (2); Pair: fused (parity, 0) + (parity, 1) launch, block.x 0 = two launches; Chain: fused "
+         "tiled planes (2); Pair: fused (parity, 0) + (parity, 1) launch, block.x 0 = two launches; "
+         "Walk: (parity, 2) + (parity, 3) in one launch along their diagonals, block.x 0 = two launches, block.y = "
+         "segments per wavefront, block.z - 1 = XCD order (1) + 2 log2 strip groups; Chain: fused "
          "parity pass (phases 0-3) in one launch, block.x 0 = unfused, block.z = tiles along z, grid.x = schedule "
          "margin\n";
   }
@@ -2185,15 +2314,10 @@ int time_launch_classes(const u1_geom* g, int prec, const void* lat, int metrop,
   a.step = m->step;
   a.stream = U1_STREAM_UPDATE;
   a.sweep = sweep;
-  Cfg cfg[2] = {kDefaultCfg, kDefaultCfg}, pcfg[2] = {{0, 1, 0, 0}, {0, 1, 0, 0}},
-      ccfg[2] = {{0, 1, 0, 0}, {0, 1, 0, 0}};
+  Shapes shapes[2];
   const int passes[2] = {metrop, ovrn};
   for (int kind = 0; kind < 2; ++kind)
-    if (passes[kind] > 0) {
-      RET(phase_cfg(prec, kind, g, lat, a, &cfg[kind]));
-      RET(pair_cfg(prec, kind, g, lat, a, cfg[kind], &pcfg[kind]));
-      RET(chain_cfg(prec, kind, g, lat, a, cfg[kind], pcfg[kind], &ccfg[kind]));
-    }
+    if (passes[kind] > 0) RET(kind_shapes(prec, kind, g, lat, a, &shapes[kind]));
   const int64_t bytes = 4 * (int64_t)a.single.V * (int64_t)elem_size(prec);
   DevBuf scratch;
   HIPCHK(scratch.alloc(bytes));
@@ -2212,16 +2336,15 @@ int time_launch_classes(const u1_geom* g, int prec, const void* lat, int metrop,
     const int kind = (c == LC_METRO || c == LC_METRO_PAIR || c == LC_METRO_CHAIN) ? u1d::KIND_METROPOLIS
                                                                                   : u1d::KIND_OVERRELAX;
     const bool cmeas = c == LC_OR_MEAS || c == LC_OR_PAIR_MEAS || c == LC_OR_CHAIN_MEAS;
-    const Cfg& pc = pcfg[kind];
-    const bool fused = pc.block != 0;
-    const bool chained = ccfg[kind].block != 0;
+    const Shapes& sh = shapes[kind];
+    const bool chained = sh.chain.block != 0;
     if (passes[kind] == 0 || (cmeas && !meas_or) || chain != chained) continue;
     if (chain) {
       // one launch per parity and pass; the parity-1 launch of the last pass measures
       per_sweep[c] = cmeas ? 1.0 : 2.0 * passes[kind] - (meas_or && kind == u1d::KIND_OVERRELAX ? 1 : 0);
       if (cmeas) {
         RepDesc rc = a.single;
-        set_chain_blocks(rc, ccfg[kind]);
+        set_chain_blocks(rc, sh.chain);
         RET(ensure_fold(3 * rc.N[2] * rc.N[3] * rc.bpp, 4));
       }
       PhaseArgs b = a;
@@ -2229,7 +2352,7 @@ int time_launch_classes(const u1_geom* g, int prec, const void* lat, int metrop,
         b.parity = cmeas ? 1 : i & 1;
         b.pass = (uint32_t)(i >> 1);
         b.meas = cmeas ? G.partials : nullptr;
-        return chain_launch(prec, kind, scratch.p, b, ccfg[kind]);
+        return chain_launch(prec, kind, scratch.p, b, sh.chain);
       };
       RET(launch(0));  // warm-up
       HIPCHK(hipEventRecord(e0, G.st));
@@ -2242,38 +2365,34 @@ int time_launch_classes(const u1_geom* g, int prec, const void* lat, int metrop,
       ms[c] = t / kTimingLaunches;
       continue;
     }
-    if (pair && !fused) continue;
-    // the (parity, mu) launches of one pass in this class (a pair is listed by mu 0)
+    // the (parity, mu) launches of one pass in this class (a fused pair is
+    // listed by its first mu); launches per sweep without and with measurement
     std::vector<std::pair<int, int>> ph;
+    int n_meas = 0;
     for (int parity = 0; parity < 2; ++parity)
       for (int mu = 0; mu < 4; ++mu) {
-        if (pair ? mu != 0 : (fused && mu < 2)) continue;
+        const bool fused = (mu < 2 ? sh.pair : sh.walk).block != 0;
+        if (fused != pair || (fused && mu % 2 != 0)) continue;
         const bool is_meas = parity == 1 && (pair || mu >= 1);
+        n_meas += is_meas;
         if (!cmeas || is_meas) ph.push_back({parity, mu});
       }
+    if (ph.empty()) continue;
     if (cmeas)
       per_sweep[c] = (double)ph.size();
-    else {
-      const int n_meas = meas_or && kind == u1d::KIND_OVERRELAX ? (pair ? 1 : (fused ? 2 : 3)) : 0;
-      per_sweep[c] = (double)ph.size() * passes[kind] - n_meas;
-    }
-    PhaseArgs b = a;
-    b.xcd = (uint32_t)(pair ? pc.xcd : cfg[kind].xcd);
-    if (pair)
-      set_pair_blocks(b.single, pc);
     else
-      set_update_blocks(b.single, cfg[kind]);
-    if (cmeas) RET(ensure_fold(b.single.nblk, 4));
+      per_sweep[c] = (double)ph.size() * passes[kind] - (meas_or && kind == u1d::KIND_OVERRELAX ? n_meas : 0);
+    if (cmeas) RET(ensure_fold(parity_row(a.single, sh, 4), 4));
     auto launch = [&](int i) -> int {
+      PhaseArgs b = a;
+      const int mu = ph[(size_t)i % ph.size()].second;
       b.parity = ph[(size_t)i % ph.size()].first;
       b.pass = (uint32_t)(i / (int)ph.size());
       b.meas = cmeas ? G.partials : nullptr;
-      if (pair)
-        HIPCHK(u1d::launch_pair(prec, kind, scratch.p, b, b.single.nblk, pc.block, pc.spt, b.single.nxh * b.single.N[1],
-                                G.st));
-      else
-        HIPCHK(u1d::launch_phase(prec, kind, ph[(size_t)i % ph.size()].second, scratch.p, b, b.single.nblk,
-                                 cfg[kind].block, cfg[kind].spt, G.st));
+      if (pair) return launch_two_phases(prec, kind, scratch.p, b, sh, mu, [&](int) { return b.meas; });
+      b.xcd = (uint32_t)sh.phase.xcd;
+      set_update_blocks(b.single, sh.phase);
+      HIPCHK(u1d::launch_phase(prec, kind, mu, scratch.p, b, b.single.nblk, sh.phase.block, sh.phase.spt, G.st));
       return U1_OK;
     };
     RET(launch(0));  // warm-up

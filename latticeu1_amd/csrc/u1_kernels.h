@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "u1_device.h"
+#include "u1_walk.h"
 
 namespace u1d {
 
@@ -73,6 +74,17 @@ struct ChainArgs {
 };
 hipError_t launch_chain(int prec, int kind, void* lat_base, const PhaseArgs& a, const ChainArgs& c, int nblocks,
                         int block, int spt, hipStream_t st);
+
+// The phases (parity, 2) and (parity, 3) in one launch, by walks along
+// diagonals (k_walk, u1_walk.h).  A single lattice; any extents, multilevel
+// masks included; block, width and strip groups sg of walk_shape_ok.  a.meas:
+// walk_rows rows of 4 doubles with the plaquette sums of both phases.
+hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, int block, int width, int sg,
+                       hipStream_t st);
+
+// binary32 proposal constants: a (2 wu 2^-32 - 1) with a = pi (independent
+// angle) or step (theta + delta); a 2^-31 is exact
+PhaseArgs with_f32_constants(const PhaseArgs& a);
 
 hipError_t launch_hotstart(int prec, void* lat, const RepDesc& r, int block, hipStream_t st);
 

@@ -1,0 +1,184 @@
+// u1_walk.hip -- kernels of the diagonal walks (u1_walk.h): two checkerboard
+// phases of a pass in one launch.  Every update is the phases' own arithmetic
+// on the same angles (u1_link.h), so the results are those of two launches bit
+// for bit.
+#include "u1_walk.h"
+
+#include "u1_link.h"
+
+namespace u1d {
+
+namespace {
+
+typedef __attribute__((ext_vector_type(2))) uint32_t U32x2;
+
+// The four directions' angles as raw buffers: an access is a uniform byte
+// offset (a scalar register) plus a lane byte offset, with no 64-bit vector
+// address to form.  Each buffer spans one direction's V angles (< 4 GiB).
+template <typename Real>
+struct WalkMem {
+  __amdgpu_buffer_rsrc_t dir[4];
+  __device__ __forceinline__ WalkMem(Real* lat, const RepDesc& r) {
+#pragma unroll
+    for (int mu = 0; mu < 4; ++mu)
+      dir[mu] = __builtin_amdgcn_make_buffer_rsrc(lat + (size_t)mu * r.V, 0, (int)((uint32_t)r.V * (uint32_t)sizeof(Real)),
+                                                  0x00027000);
+  }
+  __device__ __forceinline__ Real operator()(int mu, uint32_t base, uint32_t off) const {
+    if constexpr (sizeof(Real) == 4)
+      return __builtin_bit_cast(Real, __builtin_amdgcn_raw_buffer_load_b32(dir[mu], (int)off, (int)base, 0));
+    else
+      return __builtin_bit_cast(Real, __builtin_amdgcn_raw_buffer_load_b64(dir[mu], (int)off, (int)base, 0));
+  }
+  __device__ __forceinline__ void store(int mu, const WalkPos& p, Real v) const {
+    const int base = __builtin_amdgcn_readfirstlane((int)p.base);  // uniform, which the compiler does not always see
+    if constexpr (sizeof(Real) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), dir[mu], (int)p.off, base, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U32x2, v), dir[mu], (int)p.off, base, 0);
+  }
+};
+
+// The six angles of direction DIR in the staple of a MU link (StapleIn).
+template <typename Real, int MU, int DIR>
+__device__ __forceinline__ void staple_dir(StapleIn<Real>& in, Real a, Real b, Real c, Real d, Real e, Real f) {
+  constexpr int j = DIR < MU ? DIR : DIR - 1;
+  in.a[j] = a;
+  in.b[j] = b;
+  in.c[j] = c;
+  in.d[j] = d;
+  in.e[j] = e;
+  in.f[j] = f;
+}
+
+// One link update of a walk; returns the new angle.
+template <typename Real, int MU, int KIND, bool MEAS>
+__device__ __forceinline__ Real walk_update(const WalkMem<Real>& mem, const PhaseArgs& a, const RepDesc& r,
+                                            const StapleIn<Real>& in, Real th_old, const WalkPos& p, bool valid,
+                                            uint64_t vmask, double& re_sum, double& im_sum, uint32_t& acc) {
+  const Real xi = sizeof(Real) == sizeof(float) ? (Real)r.aniso_f : (Real)r.aniso;
+  PlaqPieces<Real> pp = {0, 0, 0, 0};
+  const Staple<Real> S[1] = {staple_sum<Real, MU, MEAS>(in, xi, (Real)r.inv_aniso_f, r.aniso != 1.0, &pp)};
+  Real th[1] = {th_old};
+  const uint32_t l[1] = {p.off / (uint32_t)sizeof(Real) + (p.base / (uint32_t)sizeof(Real) + MU * (uint32_t)r.V)};
+  const uint64_t vm[1] = {vmask};
+  update_angles<Real, KIND, 1>(a, r, S, th, l, vm, acc);
+  if (valid) mem.store(MU, p, th[0]);
+  if (MEAS) add_plaquettes<Real, MU>(pp, th[0], valid, re_sum, im_sum);
+  return th[0];
+}
+
+// Measured, binary32 overrelaxation, per launch against the two phase launches
+// it replaces: 23.5 us against 31.2 us at 48^4 (lattice in the MALL), 407 us
+// against 630 us at 96^4 (from HBM: 1.70 GB compulsory, 4.2 TB/s), 6.7 us
+// against 8.5 us at 24^3 x 48, 5.1 us against 7.4 us at 24^4.  78 vector
+// instructions per link (uniform form) where a phase issues 108-120: offsets
+// instead of per-load addresses.  At 48^4 the vector units are 70 % busy and
+// 108 workgroups per XCD of 64 sites each leave 12 of its 32 CUs with a fourth
+// workgroup; segments of 32 sites halve that unit, which is why narrow strips
+// win there in spite of their extra instructions.  Metropolis is bound by its
+// arithmetic: level with two launches in the caches, 548 us against 659 us at
+// 96^4.  Binary64 is arithmetic-bound throughout and seldom gains.
+enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
+
+// The two phases (parity, 2) and (parity, 3) of one lattice (walk_args).  MODE
+// WALK_MEAS: also the plaquette sums of both, one row of a.meas per strip and
+// diagonal; WALK_MASK: with the multilevel mask a.ml (frozen slices keep
+// theta_2).  Every wavefront leaves the first new theta_2 of its segments in
+// LDS, meets the barrier, and takes the last one it needs from there.
+template <typename Real, int KIND, int MODE, bool UNIFORM>
+__global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real* __restrict__ lat_base, PhaseArgs a,
+                                                                           WalkArgs wa) {
+  using Walk = WalkZT<sizeof(Real), UNIFORM>;
+  constexpr int A = Walk::A, B = Walk::B, C = Walk::C, D = Walk::D;
+  constexpr bool MEAS = MODE == WALK_MEAS;
+  __shared__ Real first[64 * walk_max_waves(sizeof(Real))];
+  uint32_t strip, orbit;
+  if (!walk_place(wa, blockIdx.x, &strip, &orbit)) return;
+  const RepDesc& r = a.single;
+  // segment of this lane, and its place in the strip
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t seg = UNIFORM ? wave : threadIdx.x / (uint32_t)wa.width;
+  const uint32_t lane = UNIFORM ? threadIdx.x & 63u : threadIdx.x & (uint32_t)(wa.width - 1);
+  const int32_t j0 = (int32_t)seg * wa.seg, j1 = min(j0 + wa.seg, wa.len);
+  const int32_t steps = UNIFORM ? j1 - j0 : wa.seg;  // uniform over the wavefront
+  const uint32_t P = (uint32_t)r.sz, site = strip * (uint32_t)wa.width + lane;
+  const bool valid = site < P;
+  Walk wk;
+  // lanes past the end of the plane walk its last site and store nothing
+  wk.init(r, a.parity, valid ? site : P - 1, (int32_t)orbit, j0);
+  const WalkMem<Real> mem(lat_base + r.lat_off, r);
+  const uint32_t ml1 = (uint32_t)a.ml - 1u;
+  const uint64_t vmask = KIND == KIND_METROPOLIS ? wave_mask(valid) : 0;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  uint32_t acc = 0;
+  auto update_a = [&](const RungSite<Real>& q, const WalkPos& p, const Rung<Real>& r0, const Rung<Real>& r1,
+                      Real before) -> Real {
+    const bool moves = MODE != WALK_MASK || ((uint32_t)p.t & ml1) != 0;
+    if (MODE == WALK_MASK && UNIFORM && !moves) return q.x[0];  // uniform
+    StapleIn<Real> in;
+    staple_dir<Real, A, B>(in, r0.u[1], r1.u[0], q.x[1], before, r0.va, r0.vb);
+    staple_dir<Real, A, C>(in, r0.u[2], q.ap[0], q.x[2], r0.w[0], q.am[0], q.f[0]);
+    staple_dir<Real, A, D>(in, r0.u[3], q.ap[1], q.x[3], r0.w[1], q.am[1], q.f[1]);
+    const uint64_t vm = MODE == WALK_MASK && KIND == KIND_METROPOLIS ? wave_mask(valid && moves) : vmask;
+    const Real n = walk_update<Real, A, KIND, MEAS>(mem, a, r, in, q.x[0], p, valid && moves, vm, v[0], v[1], acc);
+    return moves ? n : q.x[0];
+  };
+  auto update_b = [&](const RungSite<Real>& q, const WalkPos& p, Real ub, const Rung<Real>& r1, Real n0, Real n1) {
+    StapleIn<Real> in;
+    staple_dir<Real, B, A>(in, r1.u[0], ub, n0, n1, r1.vb, r1.va);
+    staple_dir<Real, B, C>(in, r1.u[2], q.bp[0], q.x[2], r1.w[0], q.bm[0], q.f[0]);
+    staple_dir<Real, B, D>(in, r1.u[3], q.bp[1], q.x[3], r1.w[1], q.bm[1], q.f[1]);
+    walk_update<Real, B, KIND, MEAS>(mem, a, r, in, q.x[1], p, valid, vmask, v[2], v[3], acc);
+  };
+  WalkSegment<Real, Walk, WalkMem<Real>, decltype(update_a), decltype(update_b)> sg{wk, mem, update_a, update_b};
+  if (steps > 0) first[threadIdx.x] = sg.first();
+  __syncthreads();
+  if (steps > 0)
+    sg.template rest<KIND == KIND_OVERRELAX>(
+        steps, [&] { return first[j1 == wa.len ? lane : threadIdx.x + (uint32_t)wa.width]; });
+  if (MEAS) {
+    double o[4];
+    block_sum<4>(v, o);
+    if (threadIdx.x == 0)
+      for (int k = 0; k < 4; ++k) a.meas[4 * ((size_t)orbit * (uint32_t)wa.strips + strip) + k] = o[k];
+  }
+  if (KIND == KIND_METROPOLIS && a.accepts && (threadIdx.x & 63) == 0 && acc)
+    atomicAdd(a.accepts, (unsigned long long)acc);
+}
+
+template <typename Real, int KIND, int MODE>
+hipError_t launch_walk_width(Real* lat, const PhaseArgs& a, const WalkArgs& w, int block, hipStream_t s) {
+  if (w.width == 64)
+    k_walk<Real, KIND, MODE, true><<<walk_blocks(w), block, 0, s>>>(lat, a, w);
+  else
+    k_walk<Real, KIND, MODE, false><<<walk_blocks(w), block, 0, s>>>(lat, a, w);
+  return hipGetLastError();
+}
+
+template <typename Real, int KIND>
+hipError_t launch_walk_mode(Real* lat, const PhaseArgs& a, const WalkArgs& w, int block, hipStream_t s) {
+  if (a.meas != nullptr) return launch_walk_width<Real, KIND, WALK_MEAS>(lat, a, w, block, s);
+  if (a.ml != 0) return launch_walk_width<Real, KIND, WALK_MASK>(lat, a, w, block, s);
+  return launch_walk_width<Real, KIND, WALK_PLAIN>(lat, a, w, block, s);
+}
+
+template <typename Real>
+hipError_t launch_walk_prec(int kind, Real* lat, const PhaseArgs& a, const WalkArgs& w, int block, hipStream_t s) {
+  return kind == KIND_METROPOLIS ? launch_walk_mode<Real, KIND_METROPOLIS>(lat, a, w, block, s)
+                                 : launch_walk_mode<Real, KIND_OVERRELAX>(lat, a, w, block, s);
+}
+
+}  // namespace
+
+hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, int block, int width, int sg,
+                       hipStream_t s) {
+  if (!walk_shape_ok(a.single, prec == PREC_F64 ? 8 : 4, block, width, sg) || a.reps != nullptr ||
+      (a.meas != nullptr && a.ml != 0))
+    return hipErrorInvalidValue;
+  const WalkArgs w = walk_args(a.single, block / 64, width, sg);
+  if (prec == PREC_F64) return launch_walk_prec<double>(kind, (double*)lat_base, a, w, block, s);
+  return launch_walk_prec<float>(kind, (float*)lat_base, with_f32_constants(a), w, block, s);
+}
+
+}  // namespace u1d
