@@ -197,7 +197,11 @@ __device__ __forceinline__ void update_angles(const PhaseArgs& a, const RepDesc&
     const Real beta = (Real)r.beta;
     // binary32 hit constants (metro_hit_f32), rounded on the host
     const float bl2e = r.bl2e_f;
-    const float pscale = a.pscale_f, poff = a.poff_f, thm = a.thm_f;
+    const float pscale = a.pscale_f, thm = a.thm_f;
+    // kept in a vector register: the proposal FMA reads pscale and poff, and
+    // one scalar register only (else a vector move per hit)
+    float poff = a.poff_f;
+    if constexpr (sizeof(Real) == sizeof(float)) asm("" : "+v"(poff));
     // hits in blocks of up to four (two Philox draws of four words each)
     for (int h4 = 0; h4 < a.nhit; h4 += 4) {
 #pragma unroll
