@@ -7,7 +7,8 @@ module at 100 significant digits and rounded once to binary64 / binary32:
 * pi from Machin's formula  pi = 16 atan(1/5) - 4 atan(1/239);
 * ln 2 from the series      ln 2 = 2 atanh(1/3);
 * Taylor coefficients 1/n! and 1/(2k+1) exactly as rationals (binary32
-  sin/cos/atan of the measurement kernels);
+  sin/cos/atan of the measurement kernels), and those of the Bessel series
+  1/(k!)^2 and 1/(k!(k+1)!);
 * minimax tables from Remez exchanges, kept as literals: binary32 atan on
   [0, 1] for the FP32 update kernels (remez_atan01), and the binary64 sin,
   cos, exp and atan polynomials shared by the oracle and the FP64 kernels
@@ -156,6 +157,9 @@ def coeff_tables():
     # atan t = t + t^3 A(t^2) through t^23
     for name in MM64:
         t[name] = [float.fromhex(h) for h in MM64_HEX[name]]
+    # power series in q = x^2/4 of I0(x) and of I1(x) / (x/2), through q^26
+    t["BESI0_64"] = [to_f64(inv_fact(k) ** 2) for k in range(26, -1, -1)]
+    t["BESI1_64"] = [to_f64(inv_fact(k) * inv_fact(k + 1)) for k in range(26, -1, -1)]
     # float tables
     t["SIN32"] = [to_f32(inv_fact(2 * k + 3) * (-1) ** (k + 1)) for k in range(3, -1, -1)]  # through r^9
     t["COS32"] = [to_f32(inv_fact(2 * k + 2) * (-1) ** (k + 1)) for k in range(4, -1, -1)]  # through r^10

@@ -1033,7 +1033,7 @@ int plaquette_async(const u1_geom* g, int prec, const void* lat, double* dst) {
 int poly_volume_async(int prec, const void* lat, const RepDesc& r, int mode, const u1_metro* mh, uint32_t stream,
                       uint32_t c1, uint32_t c3, double* P, double* tl) {
   if (mode == U1_POLY_PLAIN) {
-    HIPCHK(u1d::launch_poly_volume(prec, lat, r, mode, 0, 0, 0.0, stream, c1, c3, P, 256, G.st));
+    HIPCHK(u1d::launch_poly_volume(prec, lat, r, P, G.st));
     return U1_OK;
   }
   HIPCHK(u1d::launch_temporal_links(prec, lat, r, mode, mh ? mh->proposal : 0, mh ? mh->nhit : 0,

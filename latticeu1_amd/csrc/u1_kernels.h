@@ -104,9 +104,7 @@ inline int fold_groups(int nblk) { return (nblk + kFoldRows - 1) / kFoldRows; }
 inline size_t fold_scratch(int nblk, int nv) { return (size_t)nv * (size_t)fold_groups(nblk); }
 hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double scale, double* out, double* scratch,
                               hipStream_t st);
-hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
-                              double step, uint32_t stream, uint32_t c1, uint32_t c3, double* P, int block,
-                              hipStream_t st);
+hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st);
 // c1_dev (nullable): Philox counter word c1 read from device memory (graph replays)
 hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
                                  double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block,

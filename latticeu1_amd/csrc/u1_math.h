@@ -213,6 +213,34 @@ U1_HD void bessel_i0i1_d(double x, double* i0, double* i1) {
   *i1 = 0.5 * x * s1;
 }
 
+// The same two series at q = x^2/4 without the (x/2): I1(x) / ((x/2) I0(x)),
+// for the analytic multihit, which needs only this ratio.  Both as Horner
+// polynomials in q with the correctly rounded coefficients 1/(k!)^2 and
+// 1/(k!(k+1)!) -- two FMAs per term where the running terms above take two
+// divisions -- cut where the next term falls below 2^-54 of the sum: 19 terms
+// for q <= 9 (x <= 6), 27 for q <= 36 (x <= 12).  Beyond, bessel_i0i1_d.
+// All terms are positive, so the rounding error of the polynomials stays near
+// one unit (the running sums carry two roundings per term).
+template <int N>
+U1_HD double bessel_ratio_poly(double q) {
+  const double c0[N_BESI0_64] = {U1M_BESI0_64_COEFFS}, c1[N_BESI1_64] = {U1M_BESI1_64_COEFFS};
+  double s0 = c0[N_BESI0_64 - N], s1 = c1[N_BESI1_64 - N];
+#pragma unroll
+  for (int k = N_BESI0_64 - N + 1; k < N_BESI0_64; ++k) {
+    s0 = fmad(s0, q, c0[k]);
+    s1 = fmad(s1, q, c1[k]);
+  }
+  return s1 / s0;
+}
+U1_HD double bessel_ratio_d(double q) {
+  if (q <= 9.0) return bessel_ratio_poly<19>(q);
+  if (q <= 36.0) return bessel_ratio_poly<27>(q);
+  double i0, i1;
+  const double x = 2.0 * __builtin_sqrt(q);
+  bessel_i0i1_d(x, &i0, &i1);
+  return i1 / (i0 * (0.5 * x));
+}
+
 // ---------------------------------------------------------------- FP32 sincos
 // Same construction in binary32 (Taylor through r^9 / r^10); used by the
 // FP32-bulk path, whose parity bar is a tolerance, not bit identity.
@@ -235,8 +263,9 @@ U1_HD void sincos_f(float x, float* sp, float* cp) {
   const float cn = fmaf_(z, pc, 1.0f);
   const float a = (q & 1) ? cn : sn;
   const float b = (q & 1) ? sn : cn;
-  *sp = (q & 2) ? -a : a;
-  *cp = ((q + 1) & 2) ? -b : b;
+  // quadrant signs as a flip of the sign bit (exact), as in sincos_d
+  *sp = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, a) ^ ((uint32_t)(q & 2) << 30));
+  *cp = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, b) ^ ((uint32_t)((q + 1) & 2) << 30));
 }
 
 U1_HD float atan01_f(float z) {

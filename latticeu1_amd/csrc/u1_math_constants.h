@@ -40,6 +40,10 @@ static constexpr int N_EXP64 = 11;
 #define U1M_EXP64_COEFFS 0x1.1e3d557e25f52p-29, 0x1.af6bad920703bp-26, 0x1.27e5b3f37a4fbp-22, 0x1.71ddf0419bf66p-19, 0x1.a01a0136d60b9p-16, 0x1.a01a01b3715f4p-13, 0x1.6c16c16c30321p-10, 0x1.111111110ec7ep-7, 0x1.5555555555503p-5, 0x1.555555555555bp-3, 0x1.0000000000000p-1
 static constexpr int N_ATAN64 = 11;
 #define U1M_ATAN64_COEFFS -0x1.2565a607b5743p-6, 0x1.37d2c7d80af0ap-5, -0x1.9cd14a1039218p-5, 0x1.df0ee3b60d900p-5, -0x1.10ebaf736a466p-4, 0x1.3b11182728061p-4, -0x1.745cf8cb68c93p-4, 0x1.c71c70e552a3ap-4, -0x1.24924922aaf63p-3, 0x1.99999999957e7p-3, -0x1.555555555553dp-2
+static constexpr int N_BESI0_64 = 27;
+#define U1M_BESI0_64_COEFFS 0x1.2d843c1f0a6f9p-177, 0x1.8e189760fbc74p-168, 0x1.e5f504c9e358cp-159, 0x1.1159d2b18fe1fp-149, 0x1.1a6d4e307528fp-140, 0x1.0afb53e9cec0bp-131, 0x1.cbeaf38dc529fp-123, 0x1.674f8e46c208cp-114, 0x1.faaf2fa1c79e5p-106, 0x1.40a2dc2460523p-97, 0x1.69f7da8510bcdp-89, 0x1.69f7da8510bcdp-81, 0x1.3e22d70ef3b5fp-73, 0x1.e725594ee52e9p-66, 0x1.4197a7f5154bcp-58, 0x1.69ca9cf3b7f54p-51, 0x1.5601885e63e5dp-44, 0x1.0b313289be0b9p-37, 0x1.522a43f65486ap-31, 0x1.522a43f65486ap-25, 0x1.02e85c0898b71p-19, 0x1.23456789abcdfp-14, 0x1.c71c71c71c71cp-10, 0x1.c71c71c71c71cp-6, 0x1.0000000000000p-2, 0x1.0000000000000p+0, 0x1.0000000000000p+0
+static constexpr int N_BESI1_64 = 27;
+#define U1M_BESI1_64_COEFFS 0x1.655a5a37c0843p-182, 0x1.e9f6e1b270f54p-173, 0x1.37033643c4b3bp-163, 0x1.6c77c3976a829p-154, 0x1.88f11edf3ed4cp-145, 0x1.84564b82a1184p-136, 0x1.5e69de22df5cep-127, 0x1.1f72d8389b3a3p-118, 0x1.aaae78f4066a6p-110, 0x1.1d028acb00491p-101, 0x1.54ad09e6a6575p-93, 0x1.69f7da8510bcdp-85, 0x1.53585cdcbfb10p-77, 0x1.165e7c2d153f3p-69, 0x1.8bce58901a35ep-62, 0x1.e2637bef9ff1ap-55, 0x1.f17697cf1cf13p-48, 0x1.ab81ea75fcdf4p-41, 0x1.2c9758daf5cd0p-34, 0x1.522a43f65486ap-28, 0x1.27e4fb7789f5cp-22, 0x1.845c8a0ce5129p-17, 0x1.6c16c16c16c17p-12, 0x1.c71c71c71c71cp-8, 0x1.5555555555555p-4, 0x1.0000000000000p-1, 0x1.0000000000000p+0
 static constexpr int N_SIN32 = 4;
 #define U1M_SIN32_COEFFS 0x1.71de3a0000000p-19f, -0x1.a01a020000000p-13f, 0x1.1111120000000p-7f, -0x1.5555560000000p-3f
 static constexpr int N_COS32 = 5;

@@ -27,70 +27,85 @@ __device__ __forceinline__ C64 exp_i(Real a) {
   return {(double)c, (double)s};
 }
 
+// sin and cos of the measurement kernels: Prec's bits; binary64 with the
+// small-argument case behind a wavefront vote (UMath<double>).
+template <typename Real>
+__device__ __forceinline__ void msincos(Real x, Real* s, Real* c) {
+  if constexpr (sizeof(Real) == 8)
+    UMath<double>::sincos(x, s, c);
+  else
+    Prec<Real>::sincos(x, s, c);
+}
+
 // Temporal-link staple (staple.h:79-102 with mu = TDir): all six staples are
-// space-time, weight xi.  Same operation order as the update kernels.
+// space-time, weight xi.  Same operation order as the update kernels (their
+// space-space term is 0 / xi = 0).
 template <typename Real>
 __device__ __forceinline__ void staple_t(const Real* __restrict__ lat, const RepDesc& r, const Site& s, int32_t id,
                                          int32_t parity, Real& Sre, Real& Sim) {
   const int32_t same = parity * r.HV + id;
   const int32_t opp = (1 - parity) * r.HV + id;
   const Real* pm = lat + 3 * (int64_t)r.V;
-  Real ssr = 0, ssi = 0, str = 0, sti = 0;
+  Real str = 0, sti = 0;
 #pragma unroll
   for (int nu = 0; nu < 3; ++nu) {
     const Real* pn = lat + (int64_t)nu * r.V;
-    const Real a = pn[opp + s.fwd[3]];
-    const Real b = pm[opp + s.fwd[nu]];
-    const Real c = pn[same];
-    const Real d = pn[same + s.fwd[3] + s.bwd[nu]];
-    const Real e = pm[opp + s.bwd[nu]];
-    const Real f = pn[opp + s.bwd[nu]];
+    const Real a = ld(pn, opp + s.fwd[3]);
+    const Real b = ld(pm, opp + s.fwd[nu]);
+    const Real c = ld(pn, same);
+    const Real d = ld(pn, same + s.fwd[3] + s.bwd[nu]);
+    const Real e = ld(pm, opp + s.bwd[nu]);
+    const Real f = ld(pn, opp + s.bwd[nu]);
     const Real up = (a - b) - c;
     const Real lo = ((-d) - e) + f;
     Real su, cu, sl, cl;
-    Prec<Real>::sincos(up, &su, &cu);
-    Prec<Real>::sincos(lo, &sl, &cl);
+    msincos<Real>(up, &su, &cu);
+    msincos<Real>(lo, &sl, &cl);
     str += cu + cl;
     sti += su + sl;
   }
   const Real xi = (Real)r.aniso;
-  Sre = ssr / xi + str * xi;
-  Sim = ssi / xi + sti * xi;
+  Sre = (Real)0 + str * xi;
+  Sim = (Real)0 + sti * xi;
 }
 
-// Temporal link value at even/odd site (id, parity): e^{i theta_t}, the analytic
-// multihit mean (lattice_functions.h:92-105) or the stochastic nhit mean.
-template <typename Real>
-__device__ C64 temporal_value(const Real* __restrict__ lat, const RepDesc& r, int32_t id, int32_t parity, int mode,
-                              int proposal, int nhit, double step, uint32_t stream, uint32_t c1, uint32_t c3) {
-  const int32_t l = id + parity * r.HV + 3 * r.V;
-  if (mode == 0) return exp_i<Real>(lat[l]);
-  Site s;
-  site_of(r, id, parity, s);
-  Real Sre, Sim;
-  staple_t<Real>(lat, r, s, id, parity, Sre, Sim);
-  if (mode == 1) {
-    const double sr = (double)Sre, si = (double)Sim;
-    const double alpha = __builtin_sqrt(sr * sr + si * si);
-    if (alpha == 0.0) return {0.0, 0.0};
-    double i0, i1;
-    u1m::bessel_i0i1_d(r.beta * alpha, &i0, &i1);
-    const double temp = i1 / (i0 * alpha);
-    return {temp * sr, -temp * si};
-  }
-  // stochastic: nhit Metropolis hits with the staple fixed, mean of e^{i theta}
-  Real th = lat[l], s0, c0;
-  Prec<Real>::sincos(th, &s0, &c0);
+// nhit Metropolis hits of a temporal link with its staple fixed; returns the
+// sums of cos and sin of the angle after each hit.  The proposals are those of
+// the update kernels (one FMA for a (2u - 1): the same bits as the two-step
+// form).  NEAR: every lane's angle starts in [-pi, pi], so theta + delta needs
+// one wrap step each way (|delta| <= pi); otherwise wrap_d's four.  Bound by
+// its vector instructions: a binary32 hit takes 62 of them (80 before the FMA
+// proposal, the single wrap steps and the sign flips of u1m::sincos_f) and half
+// a Philox draw.  The 100-hit correlator at 24^3 x 48 takes 150 us, 200 us
+// before (about 30 us of that from the hits).
+template <typename Real, bool NEAR>
+__device__ __forceinline__ C64 multihit_sum(const RepDesc& r, Real th, Real Sre, Real Sim, uint32_t l, int proposal,
+                                            int nhit, double step, uint32_t stream, uint32_t c1, uint32_t c3) {
+  Real s0, c0;
+  msincos<Real>(th, &s0, &c0);
   Real re_old = Sre * c0 - Sim * s0;
   const Real beta = (Real)r.beta;
   double ac = 0.0, as = 0.0;
   auto hit = [&](uint32_t wu, uint32_t wb) {
-    const double u = u1r::u01_d(wu);
-    const Real tn = (Real)(proposal == 0 ? u1m::K_PI * (2.0 * u - 1.0) : u1m::wrap_d((double)th + step * (2.0 * u - 1.0)));
-    Real sn, cn;
-    Prec<Real>::sincos(tn, &sn, &cn);
+    double x;
+    if (proposal == 0) {
+      x = __builtin_fma((double)wu, u1m::K_PI * 0x1p-31, -u1m::K_PI);
+    } else {
+      x = (double)th + __builtin_fma((double)wu, step * 0x1p-31, -step);
+      if (NEAR) {
+        if (x >= u1m::K_PI) x -= u1m::K_TWO_PI;
+        if (x < -u1m::K_PI) x += u1m::K_TWO_PI;
+      } else {
+        x = u1m::wrap_d(x);
+      }
+    }
+    const Real tn = (Real)x;
+    Real sn, cn, dS;
+    if constexpr (sizeof(Real) == 8) UMath<double>::sincos_in_loop(tn, &sn, &cn);
+    else Prec<Real>::sincos(tn, &sn, &cn);
     const Real re_new = Sre * cn - Sim * sn;
-    const Real dS = Prec<Real>::exp(beta * (re_new - re_old));
+    if constexpr (sizeof(Real) == 8) dS = UMath<double>::exp_in_loop(beta * (re_new - re_old));
+    else dS = Prec<Real>::exp(beta * (re_new - re_old));
     if (dS > Prec<Real>::u01(wb)) {
       th = tn;
       re_old = re_new;
@@ -102,11 +117,40 @@ __device__ C64 temporal_value(const Real* __restrict__ lat, const RepDesc& r, in
   };
   // hits 2j and 2j + 1 read words (0, 1) and (2, 3) of one Philox call
   for (int h = 0; h < nhit; h += 2) {
-    const u1r::U32x4 w = u1r::draw(r.seed, (uint32_t)l, c1, u1r::ctr2(stream, 0, (uint32_t)(h >> 1)), c3);
+    const u1r::U32x4 w = u1r::draw(r.seed, l, c1, u1r::ctr2(stream, 0, (uint32_t)(h >> 1)), c3);
     hit(w.v[0], w.v[1]);
     if (h + 1 < nhit) hit(w.v[2], w.v[3]);
   }
-  return {ac / (double)nhit, as / (double)nhit};
+  return {ac, as};
+}
+
+// Temporal link value at even/odd site (id, parity) = s: e^{i theta_t}, the
+// analytic multihit mean (lattice_functions.h:92-105) or the stochastic nhit
+// mean.  MODE 0, 1, 2.
+template <typename Real, int MODE>
+__device__ __forceinline__ C64 temporal_value(const Real* __restrict__ lat, const RepDesc& r, const Site& s, int32_t id,
+                                              int32_t parity, int proposal, int nhit, double step, uint32_t stream,
+                                              uint32_t c1, uint32_t c3) {
+  const int32_t l = id + parity * r.HV + 3 * r.V;
+  if (MODE == 0) return exp_i<Real>(lat[l]);
+  Real Sre, Sim;
+  staple_t<Real>(lat, r, s, id, parity, Sre, Sim);
+  if (MODE == 1) {
+    // (binary64 at 32^3 x 16: 22.6 us per field with two divisions per series
+    // term, 13.4 us with the polynomials)
+    // conj(S) I1(x) / (I0(x) |S|), x = beta |S|: (beta / 2) conj(S) times a
+    // function of x^2, so that no square root and one division are left
+    const double sr = (double)Sre, si = (double)Sim, a2 = sr * sr + si * si;
+    if (a2 == 0.0) return {0.0, 0.0};
+    const double temp = 0.5 * r.beta * u1m::bessel_ratio_d(0.25 * (r.beta * r.beta) * a2);
+    return {temp * sr, -temp * si};
+  }
+  const Real th = lat[l];
+  // (the negated test also sends NaN the general way)
+  const bool near = __all(!((double)th > 3.1415927410125733 || (double)th < -3.1415927410125733) && th == th);
+  const C64 sum = near ? multihit_sum<Real, true>(r, th, Sre, Sim, (uint32_t)l, proposal, nhit, step, stream, c1, c3)
+                       : multihit_sum<Real, false>(r, th, Sre, Sim, (uint32_t)l, proposal, nhit, step, stream, c1, c3);
+  return {sum.re / (double)nhit, sum.im / (double)nhit};
 }
 
 // plaquette.cu:93-118: per site, sum over mu < nu of 1 - e^{iP}, split into
@@ -188,7 +232,16 @@ __global__ __launch_bounds__(256) void k_polyakov(const Real* __restrict__ lat, 
     const int32_t id = idx - parity * half;  // eo-id of (x, t = 0)
     const Real* pt = lat + 3 * (int64_t)r.V;
     double tmp = 0.0;
-    for (int t = 0; t < r.N[3]; ++t) tmp += (double)pt[((parity + t) & 1) * r.HV + id + t * half];
+    // (loads in groups of eight: one after the other they were the whole time)
+    int t = 0;
+    for (; t + 8 <= r.N[3]; t += 8) {
+      Real q[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = pt[((parity + t + k) & 1) * r.HV + id + (t + k) * half];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) tmp += (double)q[k];
+    }
+    for (; t < r.N[3]; ++t) tmp += (double)pt[((parity + t) & 1) * r.HV + id + t * half];
     double s, c;
     u1m::sincos_d(tmp, &s, &c);
     v[0] = c;
@@ -226,21 +279,27 @@ __global__ __launch_bounds__(256) void k_fold_rows(const double* __restrict__ pa
   if (threadIdx.x == 0) l1[(int64_t)g * nv + k] = o[0];
 }
 
-// polyakov.cu:415-440: P(x) = prod_t T(x, t), stored at the lexicographic
-// spatial index (indexIdS).
+// polyakov.cu:415-440 without multihit: P(x) = prod_t e^{i theta_t(x, t)},
+// stored at the lexicographic spatial index (indexIdS).  The angles are loaded
+// in groups of eight; the product keeps its order.
 template <typename Real>
-__global__ __launch_bounds__(256) void k_poly_volume(const Real* __restrict__ lat, RepDesc r, int mode, int proposal,
-                                                     int nhit, double step, uint32_t stream, uint32_t c1, uint32_t c3,
-                                                     double* __restrict__ P) {
+__global__ __launch_bounds__(256) void k_poly_volume(const Real* __restrict__ lat, RepDesc r, double* __restrict__ P) {
   const int32_t idx = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
   if (idx >= r.SV) return;
   const int32_t half = r.SV / 2;
   const int32_t parity = idx >= half ? 1 : 0;
   const int32_t id = idx - parity * half;
+  const Real* pt = lat + 3 * (int64_t)r.V;
   C64 res = {1.0, 0.0};
-  for (int t = 0; t < r.N[3]; ++t)
-    res = cmul(res, temporal_value<Real>(lat, r, id + t * half, (parity + t) & 1, mode, proposal, nhit, step, stream,
-                                         c1, c3));
+  int t = 0;
+  for (; t + 8 <= r.N[3]; t += 8) {
+    Real q[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) q[k] = pt[((parity + t + k) & 1) * r.HV + id + (t + k) * half];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) res = cmul(res, exp_i<Real>(q[k]));
+  }
+  for (; t < r.N[3]; ++t) res = cmul(res, exp_i<Real>(pt[((parity + t) & 1) * r.HV + id + t * half]));
   Site s;
   site_of(r, id, parity, s);
   const int32_t j = s.x[0] + r.N[0] * (s.x[1] + r.N[1] * s.x[2]);
@@ -249,73 +308,81 @@ __global__ __launch_bounds__(256) void k_poly_volume(const Real* __restrict__ la
 }
 
 // multilevel.cu:239-258: per-site temporal link at the lexicographic 4D index.
-template <typename Real>
-__global__ __launch_bounds__(256) void k_temporal_links(const Real* __restrict__ lat, RepDesc r, int mode,
-                                                        int proposal, int nhit, double step, uint32_t stream,
-                                                        uint32_t c1, uint32_t c3, double* __restrict__ out,
-                                                        const uint32_t* c1_dev) {
+template <typename Real, int MODE>
+__global__ __launch_bounds__(256) void k_temporal_links(const Real* __restrict__ lat, RepDesc r, int proposal, int nhit,
+                                                        double step, uint32_t stream, uint32_t c1, uint32_t c3,
+                                                        double* __restrict__ out, const uint32_t* c1_dev) {
   const int32_t idx = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
   if (idx >= r.V) return;
   if (c1_dev) c1 = *c1_dev;
   const int32_t parity = idx >= r.HV ? 1 : 0;
   const int32_t id = idx - parity * r.HV;
-  const C64 v = temporal_value<Real>(lat, r, id, parity, mode, proposal, nhit, step, stream, c1, c3);
-  // lex = 2*id + (x0 & 1); x0 parity = (y + z + t + parity) & 1
   Site s;
   site_of(r, id, parity, s);
-  const int64_t j = s.x[0] + (int64_t)r.N[0] * (s.x[1] + (int64_t)r.N[1] * (s.x[2] + (int64_t)r.N[2] * s.x[3]));
+  const C64 v = temporal_value<Real, MODE>(lat, r, s, id, parity, proposal, nhit, step, stream, c1, c3);
+  // lex = 2*id + (x0 & 1); x0 parity = (y + z + t + parity) & 1
+  const int64_t j = 2 * (int64_t)id + (s.x[0] & 1);
   out[2 * j] = v.re;
   out[2 * j + 1] = v.im;
 }
 
 // Product over t of a per-site temporal-link field (lexicographic 4D index),
-// in t order as polyakov.cu:430-437: P(x) = prod_t T(x, t).
-__global__ __launch_bounds__(256) void k_tprod(const double* __restrict__ tl, RepDesc r, double* __restrict__ P) {
+// in t order as polyakov.cu:430-437: P(x) = prod_t T(x, t).  Loads in groups of
+// eight (one after the other, with a wavefront per CU, they were the whole
+// time: 14 us at 24^3 x 48), one wavefront per workgroup to spread the few of
+// them over the CUs.
+__global__ __launch_bounds__(64) void k_tprod(const double* __restrict__ tl, RepDesc r, double* __restrict__ P) {
   const int32_t j = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
   if (j >= r.SV) return;
   C64 res = {1.0, 0.0};
-  for (int t = 0; t < r.N[3]; ++t) {
-    const int64_t k = j + (int64_t)t * r.SV;
-    res = cmul(res, C64{tl[2 * k], tl[2 * k + 1]});
+  int t = 0;
+  for (; t + 8 <= r.N[3]; t += 8) {
+    C64 q[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t m = j + (int64_t)(t + k) * r.SV;
+      q[k] = {tl[2 * m], tl[2 * m + 1]};
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) res = cmul(res, q[k]);
+  }
+  for (; t < r.N[3]; ++t) {
+    const int64_t m = j + (int64_t)t * r.SV;
+    res = cmul(res, C64{tl[2 * m], tl[2 * m + 1]});
   }
   P[2 * (int64_t)j] = res.re;
   P[2 * (int64_t)j + 1] = res.im;
 }
 
 // polyakov.cu:514-535: sum over x and the three spatial axes of
-// P(x) conj(P(x + R e_dir)), R = 1..rmax; one partial row of 2*rmax per workgroup.
+// P(x) conj(P(x + R e_dir)), R = 1..rmax; one partial row of 2*rmax per 256
+// sites.  One R per workgroup (blockIdx.y): 15.6 us at 24^3 when a workgroup
+// took all R in turn, two barriers each.
 __global__ __launch_bounds__(256) void k_pp(const double* __restrict__ P, RepDesc r, int rmax,
                                             double* __restrict__ partials) {
   const int32_t id = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-  const bool act = id < r.SV;
-  int32_t x[3] = {0, 0, 0};
-  C64 p0 = {0.0, 0.0};
-  if (act) {
-    x[0] = id % r.N[0];
-    x[1] = (id / r.N[0]) % r.N[1];
-    x[2] = id / (r.N[0] * r.N[1]);
-    p0 = {P[2 * (int64_t)id], P[2 * (int64_t)id + 1]};
-  }
-  for (int R = 1; R <= rmax; ++R) {
-    double v[2] = {0.0, 0.0};
-    if (act) {
+  const int32_t R = (int32_t)blockIdx.y + 1;
+  double v[2] = {0.0, 0.0};
+  if (id < r.SV) {
+    const int32_t row = (int32_t)((uint32_t)id / (uint32_t)r.N[0]), x2 = (int32_t)((uint32_t)row / (uint32_t)r.N[1]);
+    const int32_t x[3] = {id - row * r.N[0], row - x2 * r.N[1], x2};
+    const int32_t stride[3] = {1, r.N[0], r.N[0] * r.N[1]};
+    const C64 p0 = {P[2 * (int64_t)id], P[2 * (int64_t)id + 1]};
 #pragma unroll
-      for (int dir = 0; dir < 3; ++dir) {
-        int32_t y[3] = {x[0], x[1], x[2]};
-        y[dir] = (y[dir] + R) % r.N[dir];
-        const int64_t j = y[0] + (int64_t)r.N[0] * (y[1] + (int64_t)r.N[1] * y[2]);
-        const C64 q = {P[2 * j], -P[2 * j + 1]};
-        const C64 t = cmul(p0, q);
-        v[0] += t.re;
-        v[1] += t.im;
-      }
+    for (int dir = 0; dir < 3; ++dir) {
+      const int32_t y = (int32_t)((uint32_t)(x[dir] + R) % (uint32_t)r.N[dir]);
+      const int64_t j = id + (int64_t)(y - x[dir]) * stride[dir];
+      const C64 q = {P[2 * j], -P[2 * j + 1]};
+      const C64 t = cmul(p0, q);
+      v[0] += t.re;
+      v[1] += t.im;
     }
-    double o[2];
-    block_sum<2>(v, o);
-    if (threadIdx.x == 0) {
-      partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2] = o[0];
-      partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2 + 1] = o[1];
-    }
+  }
+  double o[2];
+  block_sum<2>(v, o);
+  if (threadIdx.x == 0) {
+    partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2] = o[0];
+    partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2 + 1] = o[1];
   }
 }
 
@@ -572,38 +639,54 @@ hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double s
   return hipGetLastError();
 }
 
-hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
-                              double step, uint32_t stream, uint32_t c1, uint32_t c3, double* P, int block,
-                              hipStream_t st) {
-  const int nb = nblocks(r.SV, block);
+hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st) {
+  const int block = 64, nb = nblocks(r.SV, block);
   if (prec == PREC_F64)
-    k_poly_volume<double><<<nb, block, 0, st>>>((const double*)lat, r, mode, proposal, nhit, step, stream, c1, c3, P);
+    k_poly_volume<double><<<nb, block, 0, st>>>((const double*)lat, r, P);
   else
-    k_poly_volume<float><<<nb, block, 0, st>>>((const float*)lat, r, mode, proposal, nhit, step, stream, c1, c3, P);
+    k_poly_volume<float><<<nb, block, 0, st>>>((const float*)lat, r, P);
   return hipGetLastError();
 }
 
 hipError_t launch_tprod(const double* tl, const RepDesc& r, double* P, hipStream_t st) {
-  k_tprod<<<nblocks(r.SV, 256), 256, 0, st>>>(tl, r, P);
+  k_tprod<<<nblocks(r.SV, 64), 64, 0, st>>>(tl, r, P);
   return hipGetLastError();
 }
+
+namespace {
+template <typename Real>
+hipError_t temporal_links_mode(const Real* lat, const RepDesc& r, int mode, int proposal, int nhit, double step,
+                               uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block, hipStream_t st,
+                               const uint32_t* c1_dev) {
+  const int nb = nblocks(r.V, block);
+  switch (mode) {
+    case 0:
+      k_temporal_links<Real, 0><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
+      break;
+    case 1:
+      k_temporal_links<Real, 1><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
+      break;
+    default:
+      k_temporal_links<Real, 2><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
+      break;
+  }
+  return hipGetLastError();
+}
+}  // namespace
 
 hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
                                  double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block,
                                  hipStream_t st, const uint32_t* c1_dev) {
-  const int nb = nblocks(r.V, block);
   if (prec == PREC_F64)
-    k_temporal_links<double><<<nb, block, 0, st>>>((const double*)lat, r, mode, proposal, nhit, step, stream, c1, c3,
-                                                   out, c1_dev);
-  else
-    k_temporal_links<float><<<nb, block, 0, st>>>((const float*)lat, r, mode, proposal, nhit, step, stream, c1, c3,
-                                                  out, c1_dev);
-  return hipGetLastError();
+    return temporal_links_mode<double>((const double*)lat, r, mode, proposal, nhit, step, stream, c1, c3, out, block,
+                                       st, c1_dev);
+  return temporal_links_mode<float>((const float*)lat, r, mode, proposal, nhit, step, stream, c1, c3, out, block, st,
+                                    c1_dev);
 }
 
 hipError_t launch_pp(const double* P, const RepDesc& r, int rmax, double* partials, int nblk, int block,
                      hipStream_t st) {
-  k_pp<<<nblk, block, 0, st>>>(P, r, rmax, partials);
+  k_pp<<<dim3(nblk, rmax), block, 0, st>>>(P, r, rmax, partials);
   return hipGetLastError();
 }
 
