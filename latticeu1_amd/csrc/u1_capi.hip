@@ -39,6 +39,10 @@ constexpr int kChainMaxMargin = 1024;  // fused-pass schedule margin accepted fr
 // binary32 Metropolis pass chosen at 5 % ahead ran no faster in full sweeps).
 constexpr float kChainMinGainOR = 0.97f;
 constexpr float kChainMinGainMetropolis = 0.90f;
+// Multilevel: device memory for the two-slice products of level-2 steps that are
+// accumulated together, and the largest workspace kept between calls.
+constexpr size_t kMlSlotBytes = (size_t)256 << 20;
+constexpr size_t kMlKeepBytes = (size_t)1 << 30;
 // A walk must take under this fraction of the two phases' time.
 constexpr float kWalkMinGain = 0.97f;
 double* g_scratch_dev[kMaxDevices] = {};
@@ -58,6 +62,8 @@ struct Ctx {
   size_t partials_cap = 0;     // in doubles
   double* work = nullptr;      // Polyakov-volume and temporal-link scratch of u1_poly_volume / u1_poly2
   size_t work_cap = 0;         // in doubles
+  void* ml = nullptr;          // multilevel workspace, kept between calls up to kMlKeepBytes
+  size_t ml_cap = 0;           // in bytes
   unsigned long long* counter = nullptr;
   double* dres = nullptr;  // small device result buffer (64 doubles)
   bool tune = true;
@@ -232,6 +238,17 @@ int ensure_work(size_t n) {
   G.work_cap = 0;
   HIPCHK(hipMalloc((void**)&G.work, n * sizeof(double)));
   G.work_cap = n;
+  return U1_OK;
+}
+
+int ensure_ml(size_t bytes) {
+  if (bytes <= G.ml_cap) return U1_OK;
+  HIPCHK(hipStreamSynchronize(G.st));
+  if (G.ml) HIPCHK(hipFree(G.ml));
+  G.ml = nullptr;
+  G.ml_cap = 0;
+  HIPCHK(hipMalloc(&G.ml, bytes));
+  G.ml_cap = bytes;
   return U1_OK;
 }
 
@@ -1037,7 +1054,7 @@ int poly_volume_async(int prec, const void* lat, const RepDesc& r, int mode, con
     return U1_OK;
   }
   HIPCHK(u1d::launch_temporal_links(prec, lat, r, mode, mh ? mh->proposal : 0, mh ? mh->nhit : 0,
-                                    mh ? mh->step : 0.0, stream, c1, c3, tl, 256, G.st));
+                                    mh ? mh->step : 0.0, stream, c1, c3, tl, G.st));
   HIPCHK(u1d::launch_tprod(tl, r, P, G.st));
   return U1_OK;
 }
@@ -1482,6 +1499,9 @@ int u1_finalize(void) {
   if (G.work) HIPCHK(hipFree(G.work));
   G.work = nullptr;
   G.work_cap = 0;
+  if (G.ml) HIPCHK(hipFree(G.ml));
+  G.ml = nullptr;
+  G.ml_cap = 0;
   if (G.counter) HIPCHK(hipFree(G.counter));
   if (G.dres) HIPCHK(hipFree(G.dres));
   for (auto& kv : G.chain_sched) HIPCHK(hipFree(kv.second));
@@ -1714,7 +1734,7 @@ int u1_temporal_links(const u1_geom* g, int prec, const void* lat, int32_t mode,
   if (mode == U1_POLY_MULTIHIT_STOCHASTIC) RET(check_metro(mh));
   const RepDesc r = make_rep(g, seed, c3);
   HIPCHK(u1d::launch_temporal_links(prec, lat, r, mode, mh ? mh->proposal : 0, mh ? mh->nhit : 0,
-                                    mh ? mh->step : 0.0, stream, c1, c3, (double*)out_dev, 256, G.st));
+                                    mh ? mh->step : 0.0, stream, c1, c3, (double*)out_dev, G.st));
   return U1_OK;
 }
 
@@ -1772,8 +1792,20 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
   const int64_t nl2 = r.N[3] / 2, nl4 = r.N[3] / 4;
   if (sz * nl2 >= ((int64_t)1 << 31)) return fail(U1_ERR_ARG, "lattice too large for the multilevel T2 tensor");
   const size_t latb = 4 * (size_t)r.V * elem_size(prec);
-  void *wl = nullptr, *tl = nullptr, *pq = nullptr, *l2 = nullptr, *l4 = nullptr;
-  uint32_t* ctr = nullptr;  // level-2 step counter i * n2 + k, advanced by the graph
+  // Workspace: the working lattice, the step counter, the two-slice products of
+  // as many level-2 steps as fit kMlSlotBytes, the T4 tensor and, if the steps
+  // of a level-4 step need more than one chunk of slots, the T2 tensor.
+  const size_t slot = 16 * (size_t)r.SV * (size_t)nl2;
+  const int slots = (int)std::min<size_t>((size_t)n2, std::max<size_t>(1, kMlSlotBytes / slot));
+  const bool chunked = slots < n2;
+  auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t o_ctr = pad(latb), o_p2 = o_ctr + 256, o_l4 = o_p2 + pad(slot * slots),
+               o_l2 = o_l4 + pad(16 * (size_t)sz * nl4), total = o_l2 + (chunked ? pad(16 * (size_t)sz * nl2) : 0);
+  RET(ensure_ml(total));
+  char* ws = (char*)G.ml;
+  void* wl = ws;
+  uint32_t* ctr = (uint32_t*)(ws + o_ctr);  // level-2 step counter i * n2 + k, advanced by the device
+  double *p2 = (double*)(ws + o_p2), *l4 = (double*)(ws + o_l4), *l2 = chunked ? (double*)(ws + o_l2) : nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int rc = U1_OK;
@@ -1781,12 +1813,11 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     (void)hipStreamSynchronize(G.st);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (wl) (void)hipFree(wl);
-    if (tl) (void)hipFree(tl);
-    if (pq) (void)hipFree(pq);
-    if (l2) (void)hipFree(l2);
-    if (l4) (void)hipFree(l4);
-    if (ctr) (void)hipFree(ctr);
+    if (G.ml_cap > kMlKeepBytes) {
+      (void)hipFree(G.ml);
+      G.ml = nullptr;
+      G.ml_cap = 0;
+    }
   };
 #define MLCHK(expr)                                                                          \
   do {                                                                                       \
@@ -1796,15 +1827,8 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
       return fail(U1_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));           \
     }                                                                                        \
   } while (0)
-  MLCHK(hipMalloc(&wl, latb));
-  MLCHK(hipMalloc(&tl, 2 * (size_t)r.V * sizeof(double)));
-  MLCHK(hipMalloc(&pq, 4 * (size_t)r.SV * (size_t)nl2 * sizeof(double)));
-  MLCHK(hipMalloc(&l2, 2 * (size_t)sz * nl2 * sizeof(double)));
-  MLCHK(hipMalloc(&l4, 2 * (size_t)sz * nl4 * sizeof(double)));
   MLCHK(hipMemcpyAsync(wl, lat, latb, hipMemcpyDeviceToDevice, G.st));
-  MLCHK(u1d::launch_fill_zero(l4, 2 * sz * nl4 * (int64_t)sizeof(double), G.st));
-  MLCHK(hipMalloc((void**)&ctr, sizeof(uint32_t)));
-  MLCHK(u1d::launch_fill_zero(ctr, sizeof(uint32_t), G.st));
+  MLCHK(u1d::launch_fill_zero(ctr, 2 * sizeof(uint32_t), G.st));
   const double l2norm = 1.0 / (double)n2, l4norm = 1.0 / (double)n4;
   const int mp = mh ? mh->proposal : 0, mn = mh ? mh->nhit : 0;
   const double ms = mh ? mh->step : 0.0;
@@ -1820,8 +1844,8 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
       return rc;
     }
   }
-  // One level-2 step -- k2 masked sweeps (Philox sweep index ctr * k2 + l),
-  // the temporal-link field (c1 = ctr), the T2 accumulation and ctr += 1 --
+  // One level-2 step -- k2 masked sweeps (Philox sweep index ctr * k2 + l) and
+  // the two-slice products of the temporal links (c1 = ctr, then ctr += 1) --
   // captured once and replayed n4 * n2 times (multilevel.cu:680-700 order;
   // sweep and c1 indices equal to ((i n2 + k) k2 + l) and (i n2 + k)), or
   // enqueued eagerly with the same device counter when graphs are off.
@@ -1829,11 +1853,8 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     for (int l = 0; l < k2; ++l)
       RET(run_update(g, prec, wl, metrop, ovrn, m, seed, u1r::STREAM_ML_L2, (uint32_t)l, call_id, 2, nullptr,
                      nullptr, ctr, (uint32_t)k2));
-    hipError_t e = u1d::launch_temporal_links(prec, wl, r, mh_mode, mp, mn, ms, u1r::STREAM_ML_MULTIHIT, 0, call_id,
-                                              (double*)tl, 256, G.st, ctr);
-    if (e == hipSuccess) e = u1d::launch_ml_l2((const double*)tl, (double*)pq, (double*)l2, r, rmax, 256, G.st);
-    if (e == hipSuccess) e = u1d::launch_increment(ctr, G.st);
-    if (e != hipSuccess) return fail(U1_ERR_HIP, std::string("multilevel level-2 step: ") + hipGetErrorString(e));
+    HIPCHK(u1d::launch_temporal_pairs(prec, wl, r, mh_mode, mp, mn, ms, u1r::STREAM_ML_MULTIHIT, call_id, p2, ctr,
+                                      (uint32_t)n2, (uint32_t)slots, G.st));
     return U1_OK;
   };
   if (G.graphs) {
@@ -1851,23 +1872,21 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     for (int j = 0; j < k4 && rc == U1_OK; ++j)
       rc = run_update(g, prec, wl, metrop, ovrn, m, seed, u1r::STREAM_ML_L4, (uint32_t)(i * k4 + j), call_id, 4,
                       nullptr);
-    if (rc != U1_OK) break;
-    MLCHK(u1d::launch_fill_zero(l2, 2 * sz * nl2 * (int64_t)sizeof(double), G.st));
     for (int k = 0; k < n2 && rc == U1_OK; ++k) {
       if (exec)
         MLCHK(hipGraphLaunch(exec, G.st));
       else
         rc = level2_step();
+      const bool last = k + 1 == n2;
+      if (rc == U1_OK && (last || (k + 1) % slots == 0))
+        MLCHK(u1d::launch_ml_accum(p2, k % slots + 1, l2, k >= slots, !last, l4, r, rmax, l2norm, i == 0, G.st));
     }
-    if (rc != U1_OK) break;
-    MLCHK(u1d::launch_ml_l4((const double*)l2, (double*)l4, r, rmax, l2norm, 256, G.st));
   }
   if (rc == U1_OK) {
     const int block = 256, nblk = (r.SV + block - 1) / block;
     rc = ensure_fold(nblk, 2 * rmax);
     if (rc == U1_OK) {
-      MLCHK(u1d::launch_ml_final((const double*)l4, (double*)ppspace_dev, r, rmax, l4norm, G.partials, nblk, block,
-                                 G.st));
+      MLCHK(u1d::launch_ml_final(l4, (double*)ppspace_dev, r, rmax, l4norm, G.partials, nblk, block, G.st));
       MLCHK(u1d::launch_finish_sums(G.partials, nblk, 2 * rmax, 1.0 / (3.0 * (double)r.SV), G.dres,
                                     fold_scratch_ptr(nblk, 2 * rmax), G.st));
       rc = copy_back(out, G.dres, 2 * (size_t)rmax);

@@ -105,10 +105,14 @@ inline size_t fold_scratch(int nblk, int nv) { return (size_t)nv * (size_t)fold_
 hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double scale, double* out, double* scratch,
                               hipStream_t st);
 hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st);
-// c1_dev (nullable): Philox counter word c1 read from device memory (graph replays)
 hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
-                                 double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block,
-                                 hipStream_t st, const uint32_t* c1_dev = nullptr);
+                                 double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, hipStream_t st);
+// Multilevel: two-slice products of the temporal links of level-2 step ctr[0]
+// (2 SV Nt/2 doubles) into its slot of p2, then ctr[0] += 1 (ctr: two words,
+// the second zero between launches).
+hipError_t launch_temporal_pairs(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
+                                 double step, uint32_t stream, uint32_t c3, double* p2, uint32_t* ctr, uint32_t n2,
+                                 uint32_t slots, hipStream_t st);
 // P(x) = prod_t T(x, t) from a temporal-link field (2*V doubles, lexicographic 4D)
 hipError_t launch_tprod(const double* tl, const RepDesc& r, double* P, hipStream_t st);
 hipError_t launch_pp(const double* P, const RepDesc& r, int rmax, double* partials /*2*rmax*nblk*/, int nblk,
@@ -123,12 +127,11 @@ hipError_t launch_plaquette_fields(int prec, const void* lat, const RepDesc& r, 
 hipError_t launch_fill_zero(void* p, int64_t bytes, hipStream_t st);
 
 // multilevel (u1_multilevel.hip)
-// T2 accumulation of one level-2 step; pq: scratch of 4 SV (Nt/2) doubles for
-// the two-slice products.
-hipError_t launch_ml_l2(const double* tl, double* pq, double* l2, const RepDesc& r, int rmax, int block,
-                        hipStream_t st);
-hipError_t launch_ml_l4(const double* l2, double* l4, const RepDesc& r, int rmax, double l2norm, int block,
-                        hipStream_t st);
+// Level-2 sums of nslots steps (slots of two-slice products p2) and, unless
+// store, the level-4 accumulation (first: l4 is written, not added to).  load,
+// store: the sums come from, go to the T2 tensor l2, for more steps than slots.
+hipError_t launch_ml_accum(const double* p2, int nslots, double* l2, bool load, bool store, double* l4,
+                           const RepDesc& r, int rmax, double l2norm, bool first, hipStream_t st);
 hipError_t launch_ml_final(const double* l4, double* ppspace, const RepDesc& r, int rmax, double l4norm,
                            double* partials /*2*rmax*nblk*/, int nblk, int block, hipStream_t st);
 

@@ -8,6 +8,8 @@
 // shared-memory fold plus one FP64 atomicAdd per block (reduce_block_1d.h:41-64,
 // cudaAtomic.h:147-177), whose summation order is nondeterministic.  All sums
 // are FP64 for both lattice precisions.
+#include <type_traits>
+
 #include "u1_kernels.h"
 
 namespace u1d {
@@ -311,10 +313,9 @@ __global__ __launch_bounds__(256) void k_poly_volume(const Real* __restrict__ la
 template <typename Real, int MODE>
 __global__ __launch_bounds__(256) void k_temporal_links(const Real* __restrict__ lat, RepDesc r, int proposal, int nhit,
                                                         double step, uint32_t stream, uint32_t c1, uint32_t c3,
-                                                        double* __restrict__ out, const uint32_t* c1_dev) {
+                                                        double* __restrict__ out) {
   const int32_t idx = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
   if (idx >= r.V) return;
-  if (c1_dev) c1 = *c1_dev;
   const int32_t parity = idx >= r.HV ? 1 : 0;
   const int32_t id = idx - parity * r.HV;
   Site s;
@@ -324,6 +325,45 @@ __global__ __launch_bounds__(256) void k_temporal_links(const Real* __restrict__
   const int64_t j = 2 * (int64_t)id + (s.x[0] & 1);
   out[2 * j] = v.re;
   out[2 * j + 1] = v.im;
+}
+
+// Multilevel, level-2 step c = *ctr: the products of the temporal links of two
+// slices, p2[l SV + x] = T(x, 2l) T(x, 2l + 1) (from 1, in the order of
+// multilevel.cu:342-347; the product of the conjugates is its conjugate), into
+// slot (c % n2) % slots of p2.  Philox counter word c1 = c.  The workgroup that
+// finishes last advances the step counter, which the sweeps of the next step
+// read: ctr[1] counts workgroups that have used ctr[0], so no launch of its
+// own is needed for it (3.9 us per step).
+template <typename Real, int MODE>
+__global__ __launch_bounds__(256) void k_temporal_pairs(const Real* __restrict__ lat, RepDesc r, int proposal, int nhit,
+                                                        double step, uint32_t stream, uint32_t c3,
+                                                        double* __restrict__ p2, uint32_t* ctr, uint32_t n2,
+                                                        uint32_t slots) {
+  const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x, half = (uint32_t)r.SV / 2u;
+  const uint32_t n = (uint32_t)r.SV * (uint32_t)(r.N[3] / 2), c = *(const volatile uint32_t*)ctr;
+  if (idx < n) {
+    const uint32_t l = idx / (uint32_t)r.SV, q = idx - l * (uint32_t)r.SV;
+    const int32_t parity = q >= half ? 1 : 0;
+    const int32_t i = (int32_t)(q - (parity ? half : 0u));  // eo-id of (x, t = 0)
+    C64 p = {1.0, 0.0};
+    int32_t odd = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int32_t id = i + (int32_t)((2 * l + h) * half), par = parity ^ h;
+      Site s;
+      site_of(r, id, par, s);
+      odd = s.x[0] & 1;
+      p = cmul(p, temporal_value<Real, MODE>(lat, r, s, id, par, proposal, nhit, step, stream, c, c3));
+    }
+    double* out = p2 + 2 * ((size_t)(c % n2 % slots) * n + (size_t)l * (uint32_t)r.SV + 2u * (uint32_t)i + (uint32_t)odd);
+    out[0] = p.re;
+    out[1] = p.im;
+  }
+  __syncthreads();  // every thread of the workgroup has used c
+  if (threadIdx.x == 0 && atomicAdd(ctr + 1, 1u) == gridDim.x - 1) {
+    ctr[1] = 0;
+    ctr[0] = c + 1;
+  }
 }
 
 // Product over t of a per-site temporal-link field (lexicographic 4D index),
@@ -653,35 +693,31 @@ hipError_t launch_tprod(const double* tl, const RepDesc& r, double* P, hipStream
   return hipGetLastError();
 }
 
-namespace {
-template <typename Real>
-hipError_t temporal_links_mode(const Real* lat, const RepDesc& r, int mode, int proposal, int nhit, double step,
-                               uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block, hipStream_t st,
-                               const uint32_t* c1_dev) {
-  const int nb = nblocks(r.V, block);
-  switch (mode) {
-    case 0:
-      k_temporal_links<Real, 0><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
-      break;
-    case 1:
-      k_temporal_links<Real, 1><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
-      break;
-    default:
-      k_temporal_links<Real, 2><<<nb, block, 0, st>>>(lat, r, proposal, nhit, step, stream, c1, c3, out, c1_dev);
-      break;
-  }
+hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
+                                 double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, hipStream_t st) {
+  const int block = 256, nb = nblocks(r.V, block);
+  auto go = [&](auto* l) {
+    typedef std::remove_cv_t<std::remove_pointer_t<decltype(l)>> Real;
+    auto* k = mode == 0 ? k_temporal_links<Real, 0> : mode == 1 ? k_temporal_links<Real, 1> : k_temporal_links<Real, 2>;
+    k<<<nb, block, 0, st>>>(l, r, proposal, nhit, step, stream, c1, c3, out);
+  };
+  if (prec == PREC_F64) go((const double*)lat);
+  else go((const float*)lat);
   return hipGetLastError();
 }
-}  // namespace
 
-hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
-                                 double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, int block,
-                                 hipStream_t st, const uint32_t* c1_dev) {
-  if (prec == PREC_F64)
-    return temporal_links_mode<double>((const double*)lat, r, mode, proposal, nhit, step, stream, c1, c3, out, block,
-                                       st, c1_dev);
-  return temporal_links_mode<float>((const float*)lat, r, mode, proposal, nhit, step, stream, c1, c3, out, block, st,
-                                    c1_dev);
+hipError_t launch_temporal_pairs(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
+                                 double step, uint32_t stream, uint32_t c3, double* p2, uint32_t* ctr, uint32_t n2,
+                                 uint32_t slots, hipStream_t st) {
+  const int block = 256, nb = nblocks((int64_t)r.SV * (r.N[3] / 2), block);
+  auto go = [&](auto* l) {
+    typedef std::remove_cv_t<std::remove_pointer_t<decltype(l)>> Real;
+    auto* k = mode == 0 ? k_temporal_pairs<Real, 0> : mode == 1 ? k_temporal_pairs<Real, 1> : k_temporal_pairs<Real, 2>;
+    k<<<nb, block, 0, st>>>(l, r, proposal, nhit, step, stream, c3, p2, ctr, n2, slots);
+  };
+  if (prec == PREC_F64) go((const double*)lat);
+  else go((const float*)lat);
+  return hipGetLastError();
 }
 
 hipError_t launch_pp(const double* P, const RepDesc& r, int rmax, double* partials, int nblk, int block,
