@@ -65,7 +65,10 @@ struct Ctx {
   void* ml = nullptr;          // multilevel workspace, kept between calls up to kMlKeepBytes
   size_t ml_cap = 0;           // in bytes
   unsigned long long* counter = nullptr;
-  double* dres = nullptr;  // small device result buffer (64 doubles)
+  // results of a measurement (64 doubles): pinned host memory that the last
+  // kernel of the fold writes through its device address (no copy afterwards)
+  double* dres = nullptr;
+  double* dres_dev = nullptr;
   bool tune = true;
   // fused (parity, 0) + (parity, 1) update launches on single lattices:
   // 0 never, 1 where the tuner measures them faster, 2 always
@@ -1059,6 +1062,13 @@ int poly_volume_async(int prec, const void* lat, const RepDesc& r, int mode, con
   return U1_OK;
 }
 
+// The n results the queued work leaves in G.dres, once it is done.
+int take_results(double* host, size_t n) {
+  HIPCHK(hipStreamSynchronize(G.st));
+  std::memcpy(host, G.dres, n * sizeof(double));
+  return chain_check();
+}
+
 int copy_back(double* host, const double* dev, size_t n) {
   HIPCHK(hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, G.st));
   HIPCHK(hipStreamSynchronize(G.st));
@@ -1480,7 +1490,8 @@ int u1_init(int device) {
   // nor lands inside one of its stream captures
   HIPCHK(hipStreamCreateWithFlags(&G.st, hipStreamNonBlocking));
   HIPCHK(hipMalloc((void**)&G.counter, sizeof(unsigned long long)));
-  HIPCHK(hipMalloc((void**)&G.dres, 64 * sizeof(double)));
+  HIPCHK(hipHostMalloc((void**)&G.dres, 64 * sizeof(double), hipHostMallocMapped));
+  HIPCHK(hipHostGetDevicePointer((void**)&G.dres_dev, G.dres, 0));
   if (device < kMaxDevices && !g_scratch_dev[device]) {
     void* p = nullptr;
     HIPCHK(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
@@ -1503,7 +1514,7 @@ int u1_finalize(void) {
   G.ml = nullptr;
   G.ml_cap = 0;
   if (G.counter) HIPCHK(hipFree(G.counter));
-  if (G.dres) HIPCHK(hipFree(G.dres));
+  if (G.dres) HIPCHK(hipHostFree(G.dres));
   for (auto& kv : G.chain_sched) HIPCHK(hipFree(kv.second));
   G.chain_sched.clear();
   G.chain_sched_len.clear();
@@ -1517,7 +1528,7 @@ int u1_finalize(void) {
   G.partials = nullptr;
   G.partials_cap = 0;
   G.counter = nullptr;
-  G.dres = nullptr;
+  G.dres = G.dres_dev = nullptr;
   G.st = nullptr;
   G.init = false;
   return U1_OK;
@@ -1628,8 +1639,8 @@ int u1_update_plaquette(const u1_geom* g, int prec, void* lat, int32_t metrop, i
   RET(check_metro(m));
   if (!lat || !out) return fail(U1_ERR_ARG, "null argument");
   if (metrop < 0 || ovrn < 0 || metrop > 4095 || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
-  RET(run_update(g, prec, lat, metrop, ovrn, m, seed, stream, sweep, c3, 0, nullptr, G.dres));
-  return copy_back(out, G.dres, 4);
+  RET(run_update(g, prec, lat, metrop, ovrn, m, seed, stream, sweep, c3, 0, nullptr, G.dres_dev));
+  return take_results(out, 4);
 }
 
 int u1_phase(const u1_geom* g, int prec, void* lat, int32_t kind, int32_t parity, int32_t mu, const u1_metro* m,
@@ -1667,8 +1678,8 @@ int u1_plaquette(const u1_geom* g, int prec, const void* lat, double out[4]) {
   REQ_PTR(out);
   RET(check_geom(g));
   RET(check_prec(prec));
-  RET(plaquette_async(g, prec, lat, G.dres));
-  return copy_back(out, G.dres, 4);
+  RET(plaquette_async(g, prec, lat, G.dres_dev));
+  return take_results(out, 4);
 }
 
 int u1_plaquette_noalloc(const u1_geom* g, int prec, const void* lat, double* out_dev) {
@@ -1705,8 +1716,8 @@ int u1_polyakov(const u1_geom* g, int prec, const void* lat, double out[2]) {
   const int block = 256, nblk = (r.SV + block - 1) / block;
   RET(ensure_fold(nblk, 2));
   HIPCHK(u1d::launch_polyakov(prec, lat, r, G.partials, nblk, block, G.st));
-  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 2, 1.0 / (double)r.SV, G.dres, fold_scratch_ptr(nblk, 2), G.st));
-  return copy_back(out, G.dres, 2);
+  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 2, 1.0 / (double)r.SV, G.dres_dev, fold_scratch_ptr(nblk, 2), G.st));
+  return take_results(out, 2);
 }
 
 int u1_poly_volume(const u1_geom* g, int prec, const void* lat, int32_t mode, const u1_metro* mh, uint64_t seed,
@@ -1748,9 +1759,9 @@ int u1_pp(const u1_geom* g, const void* P_dev, int32_t rmax, double* out) {
   const int block = 256, nblk = (r.SV + block - 1) / block;
   RET(ensure_fold(nblk, 2 * rmax));
   HIPCHK(u1d::launch_pp((const double*)P_dev, r, rmax, G.partials, nblk, block, G.st));
-  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 2 * rmax, 1.0 / (3.0 * (double)r.SV), G.dres,
+  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 2 * rmax, 1.0 / (3.0 * (double)r.SV), G.dres_dev,
                                  fold_scratch_ptr(nblk, 2 * rmax), G.st));
-  return copy_back(out, G.dres, 2 * (size_t)rmax);
+  return take_results(out, 2 * (size_t)rmax);
 }
 
 int u1_poly2(const u1_geom* g, int prec, const void* lat, int32_t mode, const u1_metro* mh, uint64_t seed,
@@ -1887,9 +1898,9 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     rc = ensure_fold(nblk, 2 * rmax);
     if (rc == U1_OK) {
       MLCHK(u1d::launch_ml_final(l4, (double*)ppspace_dev, r, rmax, l4norm, G.partials, nblk, block, G.st));
-      MLCHK(u1d::launch_finish_sums(G.partials, nblk, 2 * rmax, 1.0 / (3.0 * (double)r.SV), G.dres,
+      MLCHK(u1d::launch_finish_sums(G.partials, nblk, 2 * rmax, 1.0 / (3.0 * (double)r.SV), G.dres_dev,
                                     fold_scratch_ptr(nblk, 2 * rmax), G.st));
-      rc = copy_back(out, G.dres, 2 * (size_t)rmax);
+      rc = take_results(out, 2 * (size_t)rmax);
     }
   }
 #undef MLCHK
@@ -1923,9 +1934,9 @@ int u1_plaquette_fields(const u1_geom* g, int prec, const void* lat, int32_t spa
   RET(ensure_fold(nblk, 12));
   HIPCHK(u1d::launch_plaquette_fields(prec, lat, r, spacetime, eo_order, (double*)field_dev, G.partials, nblk, block,
                                       G.st));
-  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 12, 1.0 / (double)size, G.dres, fold_scratch_ptr(nblk, 12),
+  HIPCHK(u1d::launch_finish_sums(G.partials, nblk, 12, 1.0 / (double)size, G.dres_dev, fold_scratch_ptr(nblk, 12),
                                  G.st));
-  return copy_back(means, G.dres, 12);
+  return take_results(means, 12);
 }
 
 // ---------------------------------------------------------------- checkpoint
