@@ -67,6 +67,43 @@ U1_HD float absf_(float x) { return __builtin_fabsf(x); }
 U1_HD bool signbitd(double x) { return __builtin_signbit(x); }
 U1_HD bool signbitf_(float x) { return __builtin_signbit(x); }
 
+// x with its sign flipped if bit 1 of q is set (exact, zeros included).  On
+// gfx950 one shift and one three-input operation on the high word, x ^ (y & m)
+// (truth table 0x78).
+U1_HD double flip_sign_q(double x, uint32_t q) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(u >> 32), q << 30, 0x80000000u, 0x78);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | (uint32_t)u);
+#else
+  return __builtin_bit_cast(double, u ^ ((uint64_t)(q & 2) << 62));
+#endif
+}
+
+U1_HD float flip_sign_q(float x, uint32_t q) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(float, __builtin_amdgcn_bitop3_b32(u, q << 30, 0x80000000u, 0x78));
+#else
+  return __builtin_bit_cast(float, u ^ ((q & 2) << 30));
+#endif
+}
+
+// (q odd) ? x : y.  On gfx950 a mask from bit 0 of q and two bit selects
+// instead of a test, a comparison and two conditional moves.
+U1_HD double select_odd(uint32_t q, double x, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)q, 0, 1);  // all ones if q is odd
+  const uint64_t u = __builtin_bit_cast(uint64_t, x), v = __builtin_bit_cast(uint64_t, y);
+  // (m & x) | (~m & y): truth table 0xCA
+  const uint32_t lo = __builtin_amdgcn_bitop3_b32(m, (uint32_t)u, (uint32_t)v, 0xCA);
+  const uint32_t hi = __builtin_amdgcn_bitop3_b32(m, (uint32_t)(u >> 32), (uint32_t)(v >> 32), 0xCA);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+#else
+  return (q & 1u) ? x : y;
+#endif
+}
+
 // ---------------------------------------------------------------- FP64 sincos
 // sincos_d_main: sincos_d without its case |x| < 2^-27, where sincos_d
 // returns sin x = x itself.  PIN: see kc (the same results either way).
@@ -76,7 +113,7 @@ U1_HD void sincos_d_main(double x, double* sp, double* cp) {
   double r = fmad(-k, K_PIO2_1, x);
   r = fmad(-k, K_PIO2_2, r);
   r = fmad(-k, K_PIO2_3, r);
-  const int q = (int)k & 3;
+  const uint32_t q = (uint32_t)(int)k;
   const double z = r * r;
   const double cs_[N_SIN64] = {U1M_SIN64_COEFFS};
   const double cc_[N_COS64] = {U1M_COS64_COEFFS};
@@ -88,14 +125,8 @@ U1_HD void sincos_d_main(double x, double* sp, double* cp) {
   for (int i = 1; i < N_COS64; ++i) pc = fmad(pc, z, kc<PIN>(cc_[i]));
   const double sn = fmad(r * z, ps, r);  // r + r^3 P(r^2)
   const double cn = fmad(z, pc, 1.0);    // 1 + r^2 Q(r^2)
-  const double a = (q & 1) ? cn : sn;
-  const double b = (q & 1) ? sn : cn;
-  // quadrant signs as a flip of the sign bit (exact, zeros included): one
-  // integer op on the high word instead of a negation and a 64-bit select
-  const double sa = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, a) ^ ((uint64_t)(q & 2) << 62));
-  const double sb = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, b) ^ ((uint64_t)((q + 1) & 2) << 62));
-  *sp = sa;
-  *cp = sb;
+  *sp = flip_sign_q(select_odd(q, cn, sn), q);
+  *cp = flip_sign_q(select_odd(q, sn, cn), q + 1);
 }
 
 template <bool PIN = false>
@@ -249,7 +280,7 @@ U1_HD void sincos_f(float x, float* sp, float* cp) {
   float r = fmaf_(-k, KF_PIO2_1, x);
   r = fmaf_(-k, KF_PIO2_2, r);
   r = fmaf_(-k, KF_PIO2_3, r);
-  const int q = (int)k & 3;
+  const uint32_t q = (uint32_t)(int)k;
   const float z = r * r;
   const float cs_[N_SIN32] = {U1M_SIN32_COEFFS};
   const float cc_[N_COS32] = {U1M_COS32_COEFFS};
@@ -263,9 +294,9 @@ U1_HD void sincos_f(float x, float* sp, float* cp) {
   const float cn = fmaf_(z, pc, 1.0f);
   const float a = (q & 1) ? cn : sn;
   const float b = (q & 1) ? sn : cn;
-  // quadrant signs as a flip of the sign bit (exact), as in sincos_d
-  *sp = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, a) ^ ((uint32_t)(q & 2) << 30));
-  *cp = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, b) ^ ((uint32_t)((q + 1) & 2) << 30));
+  // quadrant signs as flips of the sign bit (exact), as in sincos_d
+  *sp = flip_sign_q(a, q);
+  *cp = flip_sign_q(b, q + 1);
 }
 
 U1_HD float atan01_f(float z) {
