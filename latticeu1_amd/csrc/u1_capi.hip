@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
@@ -205,6 +206,10 @@ RepDesc make_rep(const u1_geom* g, uint64_t seed, uint32_t c3) {
   r.inv_aniso_f = (float)(1.0 / g->aniso);
   r.aniso_f = (float)g->aniso;
   r.bl2e_f = (float)(g->beta * 1.4426950408889634);  // beta log2(e)
+  // |S| <= 6 xi (temporal links) or 4 / xi + 2 xi, so a weight's exponent
+  // beta (Re' - Re) is at most 2 |beta| |S|
+  const double smax = std::max(6.0 * g->aniso, 4.0 / g->aniso + 2.0 * g->aniso);
+  r.exp_small = 2.0 * std::fabs(g->beta) * smax < 650.0 ? 1u : 0u;
   r.seed = seed;
   r.lat_off = 0;
   return r;

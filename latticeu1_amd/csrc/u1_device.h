@@ -49,6 +49,8 @@ struct RepDesc {
   // binary32 update constants, rounded once on the host: aniso, and
   // beta log2(e) for the exp2 form of the Metropolis weight
   float aniso_f, bl2e_f;
+  // the couplings bound every Metropolis weight's exponent by 650 in modulus
+  uint32_t exp_small;
 };
 
 // Round-up magic division (Granlund & Montgomery 1994): for 1 <= d < 2^31 and
@@ -251,26 +253,17 @@ template <typename Real>
 struct UMath;
 template <>
 struct UMath<double> {
-  // sincos_d's bits: sincos_d_main, then its small-argument case only in a
-  // wavefront where some lane has |x| < 2^-27 (one vote instead of a test
-  // and a 64-bit select per call)
-  template <bool PIN = false>
-  static __device__ __forceinline__ void sincos_voted(double x, double* s, double* c) {
-    u1m::sincos_d_main<PIN>(x, s, c);
-    if (!__all(__builtin_fabs(x) >= 0x1p-27))
-      if (__builtin_fabs(x) < 0x1p-27) *s = x;
-  }
-  static __device__ __forceinline__ void sincos(double x, double* s, double* c) { sincos_voted<false>(x, s, c); }
-  static __device__ __forceinline__ double exp(double x) { return u1m::exp_d(x); }
-  // the same functions for calls inside a loop (coefficients pinned to
-  // scalar registers, u1m::kc; identical results)
+  // sincos_d's values (sincos_d_main: sin(-0) is +0, and the sign of a zero
+  // changes no sum it enters here: they start from +0)
+  static __device__ __forceinline__ void sincos(double x, double* s, double* c) { u1m::sincos_d_main<false>(x, s, c); }
+  // the same for calls inside a loop (coefficients pinned to scalar registers,
+  // u1m::kc; identical results)
   static __device__ __forceinline__ void sincos_in_loop(double x, double* s, double* c) {
-    sincos_voted<true>(x, s, c);
+    u1m::sincos_d_main<true>(x, s, c);
   }
   // exp_d's bits for every x: exp_d_inrange, then exp_d's three special
   // cases only in a wavefront where some lane's argument is outside
-  // |x| < 708 (one vote per hit instead of three tests; the Metropolis
-  // weights stay far inside at any usual coupling)
+  // |x| < 708 (one vote per hit instead of three tests)
   static __device__ __forceinline__ double exp_in_loop(double x) {
     double y = u1m::exp_d_inrange<true>(x);
     if (!__all(__builtin_fabs(x) < 708.0)) {
@@ -280,7 +273,33 @@ struct UMath<double> {
     }
     return y;
   }
-  static __device__ __forceinline__ double atan2(double y, double x) { return u1m::atan2_d(y, x); }
+  // Metropolis accept test exp(x) > w 2^-32.  small: the couplings keep every
+  // |x| below 650 (RepDesc::exp_small; NaN stays NaN), so that e^x 2^32 > w is
+  // the same test, without the vote and the scaling of w.
+  static __device__ __forceinline__ bool accept(double x, uint32_t w, bool small) {
+    if (small) return u1m::exp_d_inrange<true, 32>(x) > (double)w;
+    return exp_in_loop(x) > u1r::u01_d(w);
+  }
+  // atan2_d's bits (of a NaN: some NaN); its special cases only in a wavefront
+  // with a zero, infinite or NaN argument sum (0x180: positive normal or
+  // denormal)
+  static __device__ __forceinline__ double atan2(double y, double x) {
+    const double ax = __builtin_fabs(x), ay = __builtin_fabs(y);
+    double a = u1m::atan_ratio_d(__builtin_fmin(ax, ay), __builtin_fmax(ax, ay));
+    if (!__all(__builtin_amdgcn_class(ax + ay, 0x180))) {
+      if (ax + ay == 0.0) a = 0.0;
+      else if (ax == ay) a = u1m::K_PIO4;  // |x| + |y| overflows, or both infinite
+      else if (x != x || y != y) a = x + y;
+    }
+    return u1m::atan2_place_d(y, x, a);
+  }
+  // wrap_d's bits: its second steps only in a wavefront where some lane may
+  // need one
+  static __device__ __forceinline__ double wrap(double x) {
+    double y = u1m::wrap_step_d(x);
+    if (!__all(__builtin_fabs(y) < u1m::K_PI)) y = u1m::wrap_d(x);
+    return y;
+  }
 };
 template <>
 struct UMath<float> {

@@ -120,27 +120,20 @@ struct MetroState {
 // Re(S e^{i theta}) form), binary64: the oracle's operations in its order.
 // wu: proposal word, wb: accept-test word.  For theta + delta one wrap step
 // each way suffices because |delta| <= step <= pi.
-template <typename Real>
-__device__ __forceinline__ bool metro_hit(MetroState<Real>& m, Staple<Real> S, Real beta, int proposal, double step,
-                                          uint32_t wu, uint32_t wb) {
+__device__ __forceinline__ bool metro_hit_f64(MetroState<double>& m, Staple<double> S, double beta, bool exp_small,
+                                              int proposal, double step, uint32_t wu, uint32_t wb) {
   // a * (2u - 1) with u = wu 2^-32 as one FMA: 2u - 1 is exact in binary64,
   // so fma(wu, a 2^-31, -a) is the same correctly rounded product as the
   // oracle's two-step form (a 2^-31 is exact).
-  double tnd;
-  if (proposal == 0) {
-    tnd = __builtin_fma((double)wu, u1m::K_PI * 0x1p-31, -u1m::K_PI);
-  } else {
-    tnd = (double)m.th + __builtin_fma((double)wu, step * 0x1p-31, -step);
-    if (tnd >= u1m::K_PI) tnd -= u1m::K_TWO_PI;
-    if (tnd < -u1m::K_PI) tnd += u1m::K_TWO_PI;
-  }
-  const Real tn = (Real)tnd;
-  Real sn, cn;
-  UMath<Real>::sincos_in_loop(tn, &sn, &cn);
-  const Real re_new = S.re * cn - S.im * sn;
-  const Real dS = UMath<Real>::exp_in_loop(beta * (re_new - m.re_old));
-  const Real b = Prec<Real>::u01(wb);
-  const bool ok = dS > b;
+  double tn;
+  if (proposal == 0)
+    tn = __builtin_fma((double)wu, u1m::K_PI * 0x1p-31, -u1m::K_PI);
+  else
+    tn = u1m::wrap_step_d(m.th + __builtin_fma((double)wu, step * 0x1p-31, -step));
+  double sn, cn;
+  UMath<double>::sincos_in_loop(tn, &sn, &cn);
+  const double re_new = S.re * cn - S.im * sn;
+  const bool ok = UMath<double>::accept(beta * (re_new - m.re_old), wb, exp_small);
   if (ok) {
     m.th = tn;
     m.re_old = re_new;
@@ -195,6 +188,7 @@ __device__ __forceinline__ void update_angles(const PhaseArgs& a, const RepDesc&
     }
     const uint32_t sweep = a.sweep_dev ? *a.sweep_dev * a.sweep_mul + a.sweep : a.sweep;
     const Real beta = (Real)r.beta;
+    const bool exp_small = r.exp_small != 0;
     // binary32 hit constants (metro_hit_f32), rounded on the host
     const float bl2e = r.bl2e_f;
     const float pscale = a.pscale_f, thm = a.thm_f;
@@ -220,10 +214,10 @@ __device__ __forceinline__ void update_angles(const PhaseArgs& a, const RepDesc&
               acc_wave += count_wave(ok1, vmask[k]);
             }
           } else {
-            const bool ok0 = metro_hit<Real>(m[k], S[k], beta, a.proposal, a.step, w.v[0], w.v[1]);
+            const bool ok0 = metro_hit_f64(m[k], S[k], beta, exp_small, a.proposal, a.step, w.v[0], w.v[1]);
             acc_wave += count_wave(ok0, vmask[k]);
             if (h + 1 < a.nhit) {
-              const bool ok1 = metro_hit<Real>(m[k], S[k], beta, a.proposal, a.step, w.v[2], w.v[3]);
+              const bool ok1 = metro_hit_f64(m[k], S[k], beta, exp_small, a.proposal, a.step, w.v[2], w.v[3]);
               acc_wave += count_wave(ok1, vmask[k]);
             }
           }
@@ -247,7 +241,7 @@ __device__ __forceinline__ void update_angles(const PhaseArgs& a, const RepDesc&
       if constexpr (sizeof(Real) == sizeof(float))  // -theta - 2 t2 and the wrap in binary64
         th[k] = (float)u1m::wrap_near_d(__builtin_fma(-2.0, (double)t2, -(double)th[k]));
       else
-        th[k] = u1m::wrap_d(-th[k] - 2.0 * t2);
+        th[k] = UMath<double>::wrap(-th[k] - 2.0 * t2);
     }
   }
 }

@@ -64,6 +64,18 @@ U1_HD double rintd(double x) { return __builtin_rint(x); }
 U1_HD float rintf_(float x) { return __builtin_rintf(x); }
 U1_HD double absd(double x) { return __builtin_fabs(x); }
 U1_HD float absf_(float x) { return __builtin_fabsf(x); }
+// Nearest integer of y (ties to even) and, in q, its low 32 bits plus ADD: adding
+// 1.5 2^52 rounds y to an integer and leaves it in the low bits of the sum, so
+// no separate rounding and conversion are needed.  |y| < 2^51; a zero result is
+// +0 for every sign of y, where rint keeps the sign -- the callers' products
+// with it are zeros that vanish in their sums.
+template <int ADD = 0>
+U1_HD double rint_q(double y, uint32_t* q) {
+  constexpr double magic = 0x1.8p52 + ADD;
+  const double t = y + magic;
+  *q = (uint32_t)__builtin_bit_cast(uint64_t, t);
+  return t - magic;
+}
 U1_HD bool signbitd(double x) { return __builtin_signbit(x); }
 U1_HD bool signbitf_(float x) { return __builtin_signbit(x); }
 
@@ -106,14 +118,16 @@ U1_HD double select_odd(uint32_t q, double x, double y) {
 
 // ---------------------------------------------------------------- FP64 sincos
 // sincos_d_main: sincos_d without its case |x| < 2^-27, where sincos_d
-// returns sin x = x itself.  PIN: see kc (the same results either way).
+// returns sin x = x itself.  The two differ at x = -0 only (sin +0 here): for
+// other tiny x, k = 0, r = x and the polynomial adds less than half a unit.
+// PIN: see kc (the same results either way).
 template <bool PIN = false>
 U1_HD void sincos_d_main(double x, double* sp, double* cp) {
-  const double k = rintd(x * K_TWO_OVER_PI);
+  uint32_t q;
+  const double k = rint_q(x * K_TWO_OVER_PI, &q);
   double r = fmad(-k, K_PIO2_1, x);
   r = fmad(-k, K_PIO2_2, r);
   r = fmad(-k, K_PIO2_3, r);
-  const uint32_t q = (uint32_t)(int)k;
   const double z = r * r;
   const double cs_[N_SIN64] = {U1M_SIN64_COEFFS};
   const double cc_[N_COS64] = {U1M_COS64_COEFFS};
@@ -146,9 +160,11 @@ U1_HD double cos_d(double x) { double s, c; sincos_d(x, &s, &c); return c; }
 // exp_d for -745.1332191019412 <= x <= 709.782712893384 (no tests): e^r
 // scaled by 2^k with ldexp, which rounds once where the result is subnormal
 // and overflows to infinity exactly where the product would.
-template <bool PIN = false>
+// E: e^x 2^E, exact scaling within the range.
+template <bool PIN = false, int E = 0>
 U1_HD double exp_d_inrange(double x) {
-  const double k = rintd(x * K_LOG2E);
+  uint32_t q;
+  const double k = rint_q<E>(x * K_LOG2E, &q);
   double r = fmad(-k, K_LN2_HI, x);
   r = fmad(-k, K_LN2_LO, r);
   const double ce[N_EXP64] = {U1M_EXP64_COEFFS};
@@ -156,7 +172,7 @@ U1_HD double exp_d_inrange(double x) {
 #pragma unroll
   for (int i = 1; i < N_EXP64; ++i) p = fmad(p, r, kc<PIN>(ce[i]));
   const double t = fmad(r * r, p, r);  // r + r^2 E(r) = e^r - 1
-  return __builtin_ldexp(1.0 + t, (int)k);
+  return __builtin_ldexp(1.0 + t, (int)q);
 }
 
 template <bool PIN = false>
@@ -183,12 +199,20 @@ U1_HD double atan_ratio_d(double num, double den) {
   return red ? (at + K_PIO4_LO) + K_PIO4 : at;
 }
 
+// atan2_d after its octant: a = atan(min / max of |x|, |y|)
+U1_HD double atan2_place_d(double y, double x, double a) {
+  if (absd(y) > absd(x)) a = (K_PIO2_HI - a) + K_PIO2_LO;
+  if (signbitd(x)) a = (K_PI - a) + K_PI_LO;
+  // the sign of y, as a flip of the sign bit (exact)
+  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, a) ^
+                                        (__builtin_bit_cast(uint64_t, y) & 0x8000000000000000ull));
+}
+
 U1_HD double atan2_d(double y, double x) {
   if (x != x || y != y) return x + y;
   const double ax = absd(x), ay = absd(y);
-  const bool swap = ay > ax;
-  const double num = swap ? ax : ay;
-  const double den = swap ? ay : ax;
+  const double num = ay > ax ? ax : ay;
+  const double den = ay > ax ? ay : ax;
   double a;
   if (den == 0.0) {
     a = 0.0;
@@ -197,11 +221,7 @@ U1_HD double atan2_d(double y, double x) {
   } else {
     a = atan_ratio_d(num, den);
   }
-  if (swap) a = (K_PIO2_HI - a) + K_PIO2_LO;
-  if (signbitd(x)) a = (K_PI - a) + K_PI_LO;
-  // the sign of y, as a flip of the sign bit (exact)
-  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, a) ^
-                                        (__builtin_bit_cast(uint64_t, y) & 0x8000000000000000ull));
+  return atan2_place_d(y, x, a);
 }
 
 // ------------------------------------------------------- wrap into [-pi, pi)
@@ -213,6 +233,15 @@ U1_HD double wrap_d(double x) {
   if (x < -K_PI) x += K_TWO_PI;
   if (x < -K_PI) x += K_TWO_PI;
   return x;
+}
+
+// One step of wrap_d either way, as one FMA: x - 2pi, x or x + 2pi.  wrap_d
+// itself wherever the result lies in (-pi, pi) (its second steps then do
+// nothing).
+U1_HD double wrap_step_d(double x) {
+  uint32_t hi = x >= K_PI ? 0x3FF00000u : 0u;  // high word of 1, -1 or 0
+  hi = x < -K_PI ? 0xBFF00000u : hi;
+  return fmad(-__builtin_bit_cast(double, (uint64_t)hi << 32), K_TWO_PI, x);
 }
 
 // Wrap of the binary32 update kernels, done in binary64: x - 2pi rint(x / 2pi)

@@ -29,8 +29,8 @@ __device__ __forceinline__ C64 exp_i(Real a) {
   return {(double)c, (double)s};
 }
 
-// sin and cos of the measurement kernels: Prec's bits; binary64 with the
-// small-argument case behind a wavefront vote (UMath<double>).
+// sin and cos of the temporal links: Prec's values (UMath<double>: but for
+// sin(-0)).
 template <typename Real>
 __device__ __forceinline__ void msincos(Real x, Real* s, Real* c) {
   if constexpr (sizeof(Real) == 8)
@@ -94,21 +94,17 @@ __device__ __forceinline__ C64 multihit_sum(const RepDesc& r, Real th, Real Sre,
       x = __builtin_fma((double)wu, u1m::K_PI * 0x1p-31, -u1m::K_PI);
     } else {
       x = (double)th + __builtin_fma((double)wu, step * 0x1p-31, -step);
-      if (NEAR) {
-        if (x >= u1m::K_PI) x -= u1m::K_TWO_PI;
-        if (x < -u1m::K_PI) x += u1m::K_TWO_PI;
-      } else {
-        x = u1m::wrap_d(x);
-      }
+      x = NEAR ? u1m::wrap_step_d(x) : u1m::wrap_d(x);
     }
     const Real tn = (Real)x;
-    Real sn, cn, dS;
+    Real sn, cn;
     if constexpr (sizeof(Real) == 8) UMath<double>::sincos_in_loop(tn, &sn, &cn);
     else Prec<Real>::sincos(tn, &sn, &cn);
     const Real re_new = Sre * cn - Sim * sn;
-    if constexpr (sizeof(Real) == 8) dS = UMath<double>::exp_in_loop(beta * (re_new - re_old));
-    else dS = Prec<Real>::exp(beta * (re_new - re_old));
-    if (dS > Prec<Real>::u01(wb)) {
+    bool ok;
+    if constexpr (sizeof(Real) == 8) ok = UMath<double>::accept(beta * (re_new - re_old), wb, r.exp_small != 0);
+    else ok = Prec<Real>::exp(beta * (re_new - re_old)) > Prec<Real>::u01(wb);
+    if (ok) {
       th = tn;
       re_old = re_new;
       s0 = sn;
