@@ -228,7 +228,9 @@ int u1_tune_enable(int32_t on);
  * "OverRelaxationPair" entries (block.x 0 = two launches).  In mode 1 the
  * phases (parity, 2) and (parity, 3) can likewise run as one launch, by
  * wavefronts walking along the diagonals e_t - e_z, bit-identical too; entries
- * "MetropolisWalk" / "OverRelaxationWalk" (block.x 0 = two launches). */
+ * "MetropolisWalk" / "OverRelaxationWalk" (block.x 0 = two launches).  An
+ * ensemble takes both kinds of launch over all its replicas, tuned over whole
+ * sweeps (mode 1) or always (mode 2), but for the measuring parity. */
 int u1_set_pair_fusion(int32_t mode);
 /* Fused parity passes (no reference counterpart): on a single lattice without
  * multilevel mask whose (z, t) planes tile 2 x 4 (Nz even, Nt a multiple of

@@ -1082,6 +1082,14 @@ int copy_back(double* host, const double* dev, size_t n) {
 
 }  // namespace
 
+// Batched walks of one kernel class (u1d::WalkBatch; block 0: none).
+struct EnsembleWalk {
+  Cfg cfg = {0, 1, 0, 0};
+  u1d::WalkArgs* args = nullptr;
+  u1d::WalkBlock* map = nullptr;
+  int blocks = 0;
+};
+
 struct u1_ensemble {
   int32_t nrep = 0;
   int prec = U1_F32;
@@ -1118,6 +1126,8 @@ struct u1_ensemble {
   uint16_t* pair_map = nullptr;
   int pair_blocks = 0;
   int pair_plane = 0;  // largest plane (Nx/2 * Ny sites) of the replicas: the pair kernel's LDS
+  // walks over (parity, 2) + (parity, 3), one shape per kernel class
+  EnsembleWalk walk[2];
 };
 
 namespace {
@@ -1151,14 +1161,17 @@ int ensemble_build_update(u1_ensemble* e, Cfg c) {
 
 int ensemble_tune(u1_ensemble* e);
 int ensemble_build_pair(u1_ensemble* e, Cfg c);
+int ensemble_build_walk(u1_ensemble* e, int kind, Cfg c);
 // Settles the ensemble's launch shapes before either graph exists (they fix
 // the launch layout): tuned, or, with tuning off and fused pairs forced
-// (u1_set_pair_fusion(2)), a default pair shape.
+// (u1_set_pair_fusion(2)), default pair and walk shapes.
 int ensemble_settle(u1_ensemble* e) {
   if (e->tuned || e->exec || e->mexec) return U1_OK;
   if (G.tune) return ensemble_tune(e);
-  if (G.pair == 2 && e->pcfg.block == 0) return ensemble_build_pair(e, Cfg{256, 1, 1, 0});
-  return U1_OK;
+  if (G.pair != 2 || e->pcfg.block != 0) return U1_OK;
+  for (const int kind : {u1d::KIND_METROPOLIS, u1d::KIND_OVERRELAX})
+    RET(ensemble_build_walk(e, kind, Cfg{128, 1, 0, 0}));  // two whole wavefronts: any extents
+  return ensemble_build_pair(e, Cfg{256, 1, 1, 0});
 }
 
 // Per-replica tables of the fused pair launches for shape c (block 0: none).
@@ -1192,10 +1205,44 @@ int ensemble_build_pair(u1_ensemble* e, Cfg c) {
   return U1_OK;
 }
 
+void ensemble_drop_walk(EnsembleWalk& w) {
+  if (w.args) (void)hipFree(w.args);
+  if (w.map) (void)hipFree(w.map);
+  w = EnsembleWalk{};
+}
+// Tables of kernel class `kind`'s walks for shape c (spt segments per
+// wavefront; block 0, or a shape some replica cannot take: none).
+int ensemble_build_walk(u1_ensemble* e, int kind, Cfg c) {
+  EnsembleWalk& w = e->walk[kind];
+  ensemble_drop_walk(w);
+  if (c.block == 0) return U1_OK;
+  std::vector<u1d::WalkArgs> args;
+  for (const RepDesc& r : e->upd_host) {
+    if (!walk_cfg_ok(r, e->prec, c)) return U1_OK;
+    args.push_back(u1d::walk_args(r, c.block / 64, 64 / c.spt, 0));
+  }
+  const std::vector<u1d::WalkBlock> map = u1d::walk_batch_order(args);
+  HIPCHK(hipMalloc((void**)&w.args, args.size() * sizeof(args[0])));
+  HIPCHK(hipMalloc((void**)&w.map, map.size() * sizeof(map[0])));
+  HIPCHK(hipMemcpyAsync(w.args, args.data(), args.size() * sizeof(args[0]), hipMemcpyHostToDevice, G.st));
+  HIPCHK(hipMemcpyAsync(w.map, map.data(), map.size() * sizeof(map[0]), hipMemcpyHostToDevice, G.st));
+  HIPCHK(hipStreamSynchronize(G.st));
+  w.blocks = (int)map.size();
+  w.cfg = c;
+  return U1_OK;
+}
+int ensemble_launch_walk(u1_ensemble* e, int kind, void* lat, const PhaseArgs& a) {
+  const EnsembleWalk& w = e->walk[kind];
+  HIPCHK(u1d::launch_walk_batched(e->prec, kind, lat, a, u1d::WalkBatch{w.args, w.map}, w.blocks, w.cfg.block,
+                                  64 / w.cfg.spt, G.st));
+  return U1_OK;
+}
+
 // mrows (nullable): plaquette rows of the measuring phases (parity 1, mu >= 1
 // of the last pass), segment mu - 1 at row offset (mu - 1) * upd_blocks.
-// With fused pairs (e->pcfg), the phases (parity, 0) + (parity, 1) of every
-// pass run as one launch, except the measuring parity 1 of the last pass.
+// With fused pairs (e->pcfg) the phases (parity, 0) + (parity, 1) of every
+// pass, and with walks (e->walk) the phases (parity, 2) + (parity, 3), run as
+// one launch, except the measuring parity 1 of the last pass.
 int ensemble_enqueue_phases(u1_ensemble* e, void* lat, double* mrows = nullptr) {
   auto meas_rows = [&](bool last_pass, int parity, int mu) -> double* {
     if (!mrows || !last_pass || parity != 1 || mu < 1) return nullptr;
@@ -1232,6 +1279,11 @@ int ensemble_enqueue_phases(u1_ensemble* e, void* lat, double* mrows = nullptr) 
           continue;
         }
         a.meas = meas_rows(last, parity, mu);
+        if (mu == 2 && e->walk[kind].cfg.block != 0 && !a.meas) {
+          RET(ensemble_launch_walk(e, kind, lat, a));
+          ++mu;
+          continue;
+        }
         HIPCHK(u1d::launch_phase(e->prec, kind, mu, lat, a, e->upd_blocks, e->cfg.block, e->cfg.spt, G.st));
       }
     return U1_OK;
@@ -1259,20 +1311,27 @@ int ensemble_tune(u1_ensemble* e) {
   hipEvent_t e0, e1;
   HIPCHK(es.create(&e0));
   HIPCHK(es.create(&e1));
-  float best = 1e30f;
-  Cfg bestc = e->cfg;
-  for (const Cfg c : candidates(false)) {  // batched launches keep lexicographic planes
-    if (c.spt == 4 && e->prec != U1_F32) continue;
-    RET(ensemble_build_update(e, c));
-    RET(ensemble_enqueue_phases(e, scratch.p));  // warm-up
+  // one sweep, after one to warm up
+  auto timed = [&](float* t) -> int {
+    RET(ensemble_enqueue_phases(e, scratch.p));
     HIPCHK(hipEventRecord(e0, G.st));
     RET(ensemble_enqueue_phases(e, scratch.p));
     HIPCHK(hipEventRecord(e1, G.st));
     HIPCHK(hipEventSynchronize(e1));
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-    if (ms < best) {
-      best = ms;
+    *t = std::min(*t, ms);
+    return U1_OK;
+  };
+  float best = 1e30f;
+  Cfg bestc = e->cfg;
+  for (const Cfg c : candidates(false)) {  // batched launches keep lexicographic planes
+    if (c.spt == 4 && e->prec != U1_F32) continue;
+    RET(ensemble_build_update(e, c));
+    float t = 1e30f;
+    RET(timed(&t));
+    if (t < best) {
+      best = t;
       bestc = c;
     }
   }
@@ -1285,15 +1344,10 @@ int ensemble_tune(u1_ensemble* e) {
     for (const Cfg pc : {Cfg{64, 1, 1, 0}, Cfg{128, 1, 1, 0}, Cfg{256, 1, 1, 0}, Cfg{512, 1, 1, 0}, Cfg{128, 2, 1, 0},
                          Cfg{256, 2, 1, 0}, Cfg{128, 1, 0, 0}, Cfg{256, 1, 0, 0}}) {
       RET(ensemble_build_pair(e, pc));
-      RET(ensemble_enqueue_phases(e, scratch.p));  // warm-up
-      HIPCHK(hipEventRecord(e0, G.st));
-      RET(ensemble_enqueue_phases(e, scratch.p));
-      HIPCHK(hipEventRecord(e1, G.st));
-      HIPCHK(hipEventSynchronize(e1));
-      float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-      if (ms < tp) {
-        tp = ms;
+      float t = 1e30f;
+      RET(timed(&t));
+      if (t < tp) {
+        tp = t;
         bestp = pc;
       }
     }
@@ -1303,6 +1357,47 @@ int ensemble_tune(u1_ensemble* e) {
                    "vs %.1f us without: %s\n", e->nrep, 1e3 * tp, bestp.block, bestp.spt, 1e3 * tnone,
                    use ? "fused" : "separate");
     RET(ensemble_build_pair(e, use ? bestp : none));
+    if (use) best = tp;
+    // walks of each class: shapes of a power of two segments per diagonal (the
+    // others have more uneven ends or fit few extents) that all replicas
+    // take, against none
+    for (const int kind : {u1d::KIND_METROPOLIS, u1d::KIND_OVERRELAX}) {
+      if ((kind == u1d::KIND_METROPOLIS ? e->metrop : e->ovrn) == 0) continue;
+      float tw = 1e30f;
+      Cfg bestw = none;
+      for (const Cfg& wc : walk_shapes(e->upd_host[0], e->prec)) {
+        const int segs = wc.block / 64 * wc.spt;
+        if (segs < 2 || (segs & (segs - 1)) != 0) continue;
+        RET(ensemble_build_walk(e, kind, wc));
+        if (e->walk[kind].cfg.block == 0) continue;
+        float t = 1e30f;
+        RET(timed(&t));
+        if (G.verbosity >= 2)
+          std::fprintf(stderr, "tune ensemble, %s: %d wavefronts of %d segment(s): %.1f us per sweep\n",
+                       kind == u1d::KIND_METROPOLIS ? "Metropolis" : "OverRelaxation", wc.block / 64, wc.spt, 1e3 * t);
+        if (t < tw) {
+          tw = t;
+          bestw = wc;
+        }
+      }
+      if (bestw.block == 0) continue;
+      // both sides afresh, alternating
+      float tsep = 1e30f;
+      tw = 1e30f;
+      for (int round = 0; round < 3; ++round) {
+        RET(ensemble_build_walk(e, kind, none));
+        RET(timed(&tsep));
+        RET(ensemble_build_walk(e, kind, bestw));
+        RET(timed(&tw));
+      }
+      const bool usew = G.pair == 2 || tw < tsep;
+      if (G.verbosity >= 1)
+        std::fprintf(stderr, "tune ensemble (%d replicas), %s: walks %.1f us per sweep (%d wavefronts of %d segment(s)) "
+                     "vs %.1f us without: %s\n", e->nrep,
+                     kind == u1d::KIND_METROPOLIS ? "Metropolis" : "OverRelaxation", 1e3 * tw, bestw.block / 64,
+                     bestw.spt, 1e3 * tsep, usew ? "walks" : "separate");
+      if (!usew) RET(ensemble_build_walk(e, kind, none));
+    }
   }
   e->tuned = true;
   return U1_OK;
@@ -1321,6 +1416,7 @@ void ensemble_release(u1_ensemble* e) {
   if (e->upd_map) (void)hipFree(e->upd_map);
   if (e->pair_dev) (void)hipFree(e->pair_dev);
   if (e->pair_map) (void)hipFree(e->pair_map);
+  for (EnsembleWalk& w : e->walk) ensemble_drop_walk(w);
   if (e->meas_map) (void)hipFree(e->meas_map);
   if (e->lat) (void)hipFree(e->lat);
   if (e->sweep_dev) (void)hipFree(e->sweep_dev);
@@ -1404,8 +1500,8 @@ constexpr int kTimingLaunches = 32;  // back-to-back launches per class
 // launches of each class over all replicas, in the sweep's launch tables, with
 // (parity, mu) cycling over the phases the class covers in a pass.  ms[c]:
 // mean launch duration; per_sweep[c]: launches per measuring sweep (the last
-// overrelaxation pass measures in its parity-1 launches of mu >= 1 and, with
-// fused pairs, leaves its parity-1 pair unfused).
+// overrelaxation pass measures in its parity-1 launches of mu >= 1 and leaves
+// its parity-1 phases unfused).
 int time_ensemble_classes(u1_ensemble* e, double* ms, double* per_sweep) {
   const size_t bytes = (size_t)e->total_links * elem_size(e->prec);
   DevBuf scratch, rows;
@@ -1425,43 +1521,49 @@ int time_ensemble_classes(u1_ensemble* e, double* ms, double* per_sweep) {
   a.stream = u1r::STREAM_UPDATE;
   a.sweep = (uint32_t)e->sweeps_done;
   a.xcd = (uint32_t)e->cfg.xcd;
-  const bool fused = e->pcfg.block != 0;
   for (int c = 0; c < LC_COUNT; ++c) ms[c] = per_sweep[c] = 0.0;
   for (int c = 0; c < LC_COUNT; ++c) {
-    if (c == LC_OR_PAIR_MEAS || c >= LC_METRO_CHAIN) continue;  // the measuring parity-1 pair stays unfused
+    if (c == LC_OR_PAIR_MEAS || c >= LC_METRO_CHAIN) continue;  // the measuring parity 1 stays unfused
     const bool pair = c == LC_METRO_PAIR || c == LC_OR_PAIR;
     const int kind = (c == LC_METRO || c == LC_METRO_PAIR) ? u1d::KIND_METROPOLIS : u1d::KIND_OVERRELAX;
     const int passes = kind == u1d::KIND_METROPOLIS ? e->metrop : e->ovrn;
-    const bool cmeas = c == LC_OR_MEAS, measured_kind = kind == u1d::KIND_OVERRELAX;
-    if (passes == 0 || (pair && !fused)) continue;
-    std::vector<std::pair<int, int>> ph;  // (parity, mu); a pair is listed by mu 0
+    const bool cmeas = c == LC_OR_MEAS;
+    const int measured = kind == u1d::KIND_OVERRELAX ? 1 : 0;  // parities with measuring launches
+    const bool fused[4] = {e->pcfg.block != 0, e->pcfg.block != 0, e->walk[kind].cfg.block != 0,
+                           e->walk[kind].cfg.block != 0};
+    const int nfused = (fused[0] ? 1 : 0) + (fused[2] ? 1 : 0);
+    if (passes == 0 || (pair && nfused == 0)) continue;
+    std::vector<std::pair<int, int>> ph;  // (parity, mu); a fused launch is listed by its first mu
     for (int parity = 0; parity < 2; ++parity)
       for (int mu = 0; mu < 4; ++mu) {
-        if (cmeas ? !(parity == 1 && mu >= 1) : (pair ? mu != 0 : (fused && mu < 2))) continue;
+        if (cmeas ? !(parity == 1 && mu >= 1) : (pair ? !(fused[mu] && mu % 2 == 0) : fused[mu])) continue;
         ph.push_back({parity, mu});
       }
     if (cmeas)
       per_sweep[c] = 3;
     else if (pair)
-      per_sweep[c] = 2.0 * passes - (measured_kind ? 1 : 0);
+      per_sweep[c] = nfused * (2.0 * passes - measured);
     else
-      per_sweep[c] = (fused ? 4.0 : 8.0) * passes - (measured_kind ? (fused ? 1 : 3) : 0);
+      per_sweep[c] = (4.0 - 2 * nfused) * (2.0 * passes - measured) + measured;
+    if (per_sweep[c] == 0.0) continue;
+    if (ph.empty()) ph.push_back({1, 0});  // the measuring parity's phase 0 only
     PhaseArgs b = a;
-    if (pair) {
-      b.reps = e->pair_dev;
-      b.blockmap = e->pair_map;
-      b.xcd = (uint32_t)e->pcfg.xcd;
-    }
     b.meas = cmeas ? rows.as<double>() : nullptr;
     auto launch = [&](int i) -> int {
+      const int mu = ph[(size_t)i % ph.size()].second;
       b.parity = ph[(size_t)i % ph.size()].first;
       b.pass = (uint32_t)(i / (int)ph.size());
-      if (pair)
-        HIPCHK(u1d::launch_pair(e->prec, kind, scratch.p, b, e->pair_blocks, e->pcfg.block, e->pcfg.spt,
+      if (pair && mu == 2) return ensemble_launch_walk(e, kind, scratch.p, b);
+      if (pair) {
+        PhaseArgs q = b;
+        q.reps = e->pair_dev;
+        q.blockmap = e->pair_map;
+        q.xcd = (uint32_t)e->pcfg.xcd;
+        HIPCHK(u1d::launch_pair(e->prec, kind, scratch.p, q, e->pair_blocks, e->pcfg.block, e->pcfg.spt,
                                 e->pair_plane, G.st));
-      else
-        HIPCHK(u1d::launch_phase(e->prec, kind, ph[(size_t)i % ph.size()].second, scratch.p, b, e->upd_blocks,
-                                 e->cfg.block, e->cfg.spt, G.st));
+      } else {
+        HIPCHK(u1d::launch_phase(e->prec, kind, mu, scratch.p, b, e->upd_blocks, e->cfg.block, e->cfg.spt, G.st));
+      }
       return U1_OK;
     };
     RET(launch(0));  // warm-up

@@ -81,6 +81,11 @@ hipError_t launch_chain(int prec, int kind, void* lat_base, const PhaseArgs& a, 
 // walk_rows rows of 4 doubles with the plaquette sums of both phases.
 hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, int block, int width, int sg,
                        hipStream_t st);
+// The same for all replicas of a batch (a.reps; w: device tables for `nblk`
+// workgroups, walk_batch_order; every replica's shape checked by the caller
+// with walk_shape_ok, sg = 0).  No measurement, no masks.
+hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBatch& w, int nblk,
+                               int block, int width, hipStream_t st);
 
 // binary32 proposal constants: a (2 wu 2^-32 - 1) with a = pi (independent
 // angle) or step (theta + delta); a 2^-31 is exact

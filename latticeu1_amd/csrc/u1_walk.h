@@ -27,6 +27,9 @@
 #pragma once
 #include <stdint.h>
 
+#include <algorithm>
+#include <vector>
+
 #include "u1_device.h"
 
 namespace u1d {
@@ -220,6 +223,16 @@ struct WalkArgs {
   int32_t gs, go;  // strips and diagonals of a group (rounded up)
   uint32_t gs_m, gs_s;
 };
+// Batched replicas: workgroup b walks block map[b].y (walk_place, plain order)
+// of replica map[b].x; map[b].x = kWalkNone: empty.
+struct WalkBlock {
+  uint32_t x, y;
+};
+constexpr uint32_t kWalkNone = 0xffffffffu;
+struct WalkBatch {
+  const WalkArgs* args;  // per replica, one width
+  const WalkBlock* map;
+};
 inline int walk_gcd(int a, int b) {
   while (b != 0) {
     const int m = a % b;
@@ -257,6 +270,34 @@ __host__ __device__ __forceinline__ bool walk_place(const WalkArgs& w, uint32_t 
   *strip = gx * (uint32_t)w.gs + s;
   *orbit = gy * (uint32_t)w.go + q;
   return *strip < (uint32_t)w.strips && *orbit < (uint32_t)w.orbits;
+}
+
+// Workgroup order of a batch: replicas with the longest segments first, cut
+// into eight lists of equal work (steps, and one for a segment's start), one
+// per XCD (workgroup index modulo 8): a replica's planes then share one L2, no
+// XCD is left with the long ones, and the short ones fill the end.
+inline std::vector<WalkBlock> walk_batch_order(const std::vector<WalkArgs>& w) {
+  std::vector<uint32_t> by(w.size());
+  uint64_t total = 0;
+  for (size_t i = 0; i < w.size(); ++i) {
+    by[i] = (uint32_t)i;
+    total += (uint64_t)walk_blocks(w[i]) * (uint64_t)(w[i].seg + 1);
+  }
+  std::stable_sort(by.begin(), by.end(), [&](uint32_t a, uint32_t b) { return w[a].seg > w[b].seg; });
+  std::vector<WalkBlock> list[8];
+  uint64_t done = 0;
+  size_t longest = 0;
+  for (const uint32_t i : by)
+    for (int b = 0; b < walk_blocks(w[i]); ++b) {
+      std::vector<WalkBlock>& l = list[8 * done / total];
+      l.push_back({i, (uint32_t)b});
+      longest = std::max(longest, l.size());
+      done += (uint64_t)(w[i].seg + 1);
+    }
+  std::vector<WalkBlock> map(8 * longest, WalkBlock{kWalkNone, 0});
+  for (int x = 0; x < 8; ++x)
+    for (size_t k = 0; k < list[x].size(); ++k) map[8 * k + (size_t)x] = list[x][k];
+  return map;
 }
 
 // Launch shapes the kernels take: whole wavefronts, none without a step.

@@ -4,6 +4,8 @@
 // for bit.
 #include "u1_walk.h"
 
+#include <type_traits>
+
 #include "u1_link.h"
 
 namespace u1d {
@@ -86,16 +88,31 @@ enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
 // diagonal; WALK_MASK: with the multilevel mask a.ml (frozen slices keep
 // theta_2).  Every wavefront leaves the first new theta_2 of its segments in
 // LDS, meets the barrier, and takes the last one it needs from there.
-template <typename Real, int KIND, int MODE, bool UNIFORM>
+// BATCHED: all replicas of an ensemble (WalkBatch), each with its own
+// descriptor, copied into registers before the first store.  64 replicas of
+// 8^4 to 24^3 x 32 (11.7 M sites), binary32: overrelaxation 44 us against
+// 63 us for the two phase launches, Metropolis 82 us against 91 us.
+template <typename Real, int KIND, int MODE, bool UNIFORM, bool BATCHED = false>
 __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real* __restrict__ lat_base, PhaseArgs a,
-                                                                           WalkArgs wa) {
+                                                                           std::conditional_t<BATCHED, WalkBatch, WalkArgs> w) {
   using Walk = WalkZT<sizeof(Real), UNIFORM>;
   constexpr int A = Walk::A, B = Walk::B, C = Walk::C, D = Walk::D;
   constexpr bool MEAS = MODE == WALK_MEAS;
   __shared__ Real first[64 * walk_max_waves(sizeof(Real))];
   uint32_t strip, orbit;
-  if (!walk_place(wa, blockIdx.x, &strip, &orbit)) return;
-  const RepDesc& r = a.single;
+  RepDesc rep;
+  WalkArgs wa;
+  if constexpr (BATCHED) {
+    const WalkBlock e = w.map[blockIdx.x];
+    if (e.x == kWalkNone) return;
+    rep = a.reps[e.x];
+    wa = w.args[e.x];
+    (void)walk_place(wa, e.y, &strip, &orbit);  // never empty in plain order
+  } else {
+    wa = w;
+    if (!walk_place(wa, blockIdx.x, &strip, &orbit)) return;
+  }
+  const RepDesc& r = BATCHED ? rep : a.single;
   // segment of this lane, and its place in the strip
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t seg = UNIFORM ? wave : threadIdx.x / (uint32_t)wa.width;
@@ -147,6 +164,22 @@ __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real
     atomicAdd(a.accepts, (unsigned long long)acc);
 }
 
+template <typename Real, int KIND>
+hipError_t launch_walk_batch(Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block, int width,
+                             hipStream_t s) {
+  if (width == 64)
+    k_walk<Real, KIND, WALK_PLAIN, true, true><<<nblk, block, 0, s>>>(lat, a, w);
+  else
+    k_walk<Real, KIND, WALK_PLAIN, false, true><<<nblk, block, 0, s>>>(lat, a, w);
+  return hipGetLastError();
+}
+template <typename Real>
+hipError_t launch_walk_batch_prec(int kind, Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block,
+                                  int width, hipStream_t s) {
+  return kind == KIND_METROPOLIS ? launch_walk_batch<Real, KIND_METROPOLIS>(lat, a, w, nblk, block, width, s)
+                                 : launch_walk_batch<Real, KIND_OVERRELAX>(lat, a, w, nblk, block, width, s);
+}
+
 template <typename Real, int KIND, int MODE>
 hipError_t launch_walk_width(Real* lat, const PhaseArgs& a, const WalkArgs& w, int block, hipStream_t s) {
   if (w.width == 64)
@@ -179,6 +212,13 @@ hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, i
   const WalkArgs w = walk_args(a.single, block / 64, width, sg);
   if (prec == PREC_F64) return launch_walk_prec<double>(kind, (double*)lat_base, a, w, block, s);
   return launch_walk_prec<float>(kind, (float*)lat_base, with_f32_constants(a), w, block, s);
+}
+
+hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBatch& w, int nblk,
+                               int block, int width, hipStream_t s) {
+  if (a.reps == nullptr || a.meas != nullptr || a.ml != 0 || nblk < 1) return hipErrorInvalidValue;
+  if (prec == PREC_F64) return launch_walk_batch_prec<double>(kind, (double*)lat_base, a, w, nblk, block, width, s);
+  return launch_walk_batch_prec<float>(kind, (float*)lat_base, with_f32_constants(a), w, nblk, block, width, s);
 }
 
 }  // namespace u1d
