@@ -1111,8 +1111,10 @@ struct u1_ensemble {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   // sweep with the plaquette summed in its last pass (u1_ensemble_sweep_plaquette)
-  double* mrows = nullptr;      // 3 segments x upd_blocks rows x 4 doubles
-  int mrows_blocks = 0;         // upd_blocks that mrows was sized for
+  double* mrows = nullptr;           // 4 doubles per row of the measuring launches
+  u1d::RowSpan* mspans = nullptr;    // rows per launch and replica
+  int mlaunches = 0;                 // measuring launches of a sweep
+  int mfirst[4] = {0, 0, 0, 0};      // first row of the one that measures phase mu >= 1
   double* series_dev = nullptr;  // kEnsSeriesCap sweeps x nrep x 4 doubles
   uint32_t* base_dev = nullptr;  // sweep index of series row 0
   hipGraph_t mgraph = nullptr;
@@ -1120,8 +1122,10 @@ struct u1_ensemble {
   Cfg cfg = {256, 1, 1, 0};  // launch shape of the update phases (tuned on first use)
   bool tuned = false;
   // fused (parity, 0) + (parity, 1) launches (block 0: none): per-replica
-  // plane tables with one workgroup per (z, t) plane
+  // plane tables with one workgroup per (z, t) plane, or, where every plane
+  // fits one (pair_packed), several planes to a workgroup
   Cfg pcfg = {0, 1, 0, 0};
+  u1d::WalkBlock* pair_packed = nullptr;
   RepDesc* pair_dev = nullptr;
   uint16_t* pair_map = nullptr;
   int pair_blocks = 0;
@@ -1160,6 +1164,7 @@ int ensemble_build_update(u1_ensemble* e, Cfg c) {
 }
 
 int ensemble_tune(u1_ensemble* e);
+bool ensemble_pair_packs(const u1_ensemble* e, int plane);
 int ensemble_build_pair(u1_ensemble* e, Cfg c);
 int ensemble_build_walk(u1_ensemble* e, int kind, Cfg c);
 // Settles the ensemble's launch shapes before either graph exists (they fix
@@ -1171,7 +1176,32 @@ int ensemble_settle(u1_ensemble* e) {
   if (G.pair != 2 || e->pcfg.block != 0) return U1_OK;
   for (const int kind : {u1d::KIND_METROPOLIS, u1d::KIND_OVERRELAX})
     RET(ensemble_build_walk(e, kind, Cfg{128, 1, 0, 0}));  // two whole wavefronts: any extents
-  return ensemble_build_pair(e, Cfg{256, 1, 1, 0});
+  int plane = 0;
+  for (const RepDesc& r : e->upd_host) plane = std::max(plane, r.nxh * r.N[1]);
+  return ensemble_build_pair(e, Cfg{ensemble_pair_packs(e, plane) ? (plane + 63) / 64 * 64 : 256, 1, 1, 0});
+}
+
+// Planes that fit a workgroup are packed (k_pair_packed): 64 replicas of 8^4 to
+// 24^3 x 32, binary32, 970 us per sweep against 1136 us with one
+// workgroup per plane.
+bool ensemble_pair_packs(const u1_ensemble* e, int plane) {
+  return (plane + 63) / 64 * 64 <= u1d::pair_max_block((int)elem_size(e->prec), 1);
+}
+// Workgroups of replica r's packed pairs (r.N, planes of 64-site chunks).
+int ensemble_pair_groups(const RepDesc& r, const Cfg& c) {
+  const int room = c.block / 64 / ((r.nxh * r.N[1] + 63) / 64);  // planes of a workgroup
+  return (r.N[2] * r.N[3] + room - 1) / room;
+}
+int ensemble_launch_pair(u1_ensemble* e, int kind, void* lat, const PhaseArgs& a0) {
+  PhaseArgs a = a0;
+  a.reps = e->pair_dev;
+  a.blockmap = e->pair_map;
+  a.xcd = (uint32_t)e->pcfg.xcd;
+  if (e->pair_packed)
+    HIPCHK(u1d::launch_pair_packed(e->prec, kind, lat, a, e->pair_packed, e->pair_blocks, e->pcfg.block, G.st));
+  else
+    HIPCHK(u1d::launch_pair(e->prec, kind, lat, a, e->pair_blocks, e->pcfg.block, e->pcfg.spt, e->pair_plane, G.st));
+  return U1_OK;
 }
 
 // Per-replica tables of the fused pair launches for shape c (block 0: none).
@@ -1184,6 +1214,27 @@ int ensemble_build_pair(u1_ensemble* e, Cfg c) {
   std::vector<RepDesc> reps(e->upd_host);
   std::vector<uint16_t> pmap;
   int nb = 0;
+  if (ensemble_pair_packs(e, plane)) {
+    if (c.block < plane || c.spt != 1) return U1_OK;
+    std::vector<u1d::WalkBlock> map;
+    for (int i = 0; i < e->nrep; ++i) {
+      RepDesc& p = reps[i];
+      u1d::set_phase_blocks(p, 64);
+      p.tile = 0;
+      const int room = c.block / 64 / p.bpp;  // planes of a workgroup
+      for (int b = 0; b < ensemble_pair_groups(p, c); ++b) map.push_back({(uint32_t)i, (uint32_t)(b * room * p.bpp)});
+    }
+    if (!e->pair_dev) HIPCHK(hipMalloc((void**)&e->pair_dev, e->nrep * sizeof(RepDesc)));
+    if (e->pair_packed) HIPCHK(hipFree(e->pair_packed));
+    e->pair_packed = nullptr;
+    HIPCHK(hipMalloc((void**)&e->pair_packed, map.size() * sizeof(map[0])));
+    HIPCHK(hipMemcpyAsync(e->pair_packed, map.data(), map.size() * sizeof(map[0]), hipMemcpyHostToDevice, G.st));
+    HIPCHK(hipMemcpyAsync(e->pair_dev, reps.data(), e->nrep * sizeof(RepDesc), hipMemcpyHostToDevice, G.st));
+    HIPCHK(hipStreamSynchronize(G.st));
+    e->pair_blocks = (int)map.size();
+    e->pcfg = c;
+    return U1_OK;
+  }
   for (int i = 0; i < e->nrep; ++i) {
     RepDesc& p = reps[i];
     u1d::set_phase_blocks(p, p.nxh * p.N[1]);  // one chunk per plane
@@ -1217,9 +1268,12 @@ int ensemble_build_walk(u1_ensemble* e, int kind, Cfg c) {
   ensemble_drop_walk(w);
   if (c.block == 0) return U1_OK;
   std::vector<u1d::WalkArgs> args;
+  int rows = 0;
   for (const RepDesc& r : e->upd_host) {
     if (!walk_cfg_ok(r, e->prec, c)) return U1_OK;
     args.push_back(u1d::walk_args(r, c.block / 64, 64 / c.spt, 0));
+    args.back().row = rows;
+    rows += u1d::walk_blocks(args.back());
   }
   const std::vector<u1d::WalkBlock> map = u1d::walk_batch_order(args);
   HIPCHK(hipMalloc((void**)&w.args, args.size() * sizeof(args[0])));
@@ -1238,16 +1292,34 @@ int ensemble_launch_walk(u1_ensemble* e, int kind, void* lat, const PhaseArgs& a
   return U1_OK;
 }
 
-// mrows (nullable): plaquette rows of the measuring phases (parity 1, mu >= 1
-// of the last pass), segment mu - 1 at row offset (mu - 1) * upd_blocks.
-// With fused pairs (e->pcfg) the phases (parity, 0) + (parity, 1) of every
-// pass, and with walks (e->walk) the phases (parity, 2) + (parity, 3), run as
-// one launch, except the measuring parity 1 of the last pass.
+// Measuring launches of a sweep -- parity 1 of its last pass: the pair (packed
+// pairs only) or phase 1, the walk or phases 2 and 3 -- and their rows: spans,
+// launch by launch, and e->mfirst.  Returns the number of rows.
+int ensemble_meas_rows(u1_ensemble* e, std::vector<u1d::RowSpan>* spans) {
+  const int kind = e->ovrn > 0 ? u1d::KIND_OVERRELAX : u1d::KIND_METROPOLIS;
+  spans->clear();
+  int rows = 0;
+  for (int mu = 1; mu < 4; ++mu) {
+    const bool pair = mu == 1 && e->pcfg.block != 0 && e->pair_packed, walk = mu >= 2 && e->walk[kind].cfg.block != 0;
+    e->mfirst[mu] = mu == 3 && walk ? e->mfirst[2] : rows;
+    if (mu == 3 && walk) continue;
+    for (const RepDesc& r : e->upd_host) {
+      int n = r.nblk;
+      if (pair) n = ensemble_pair_groups(r, e->pcfg);
+      if (walk) n = u1d::walk_rows(r, 64 / e->walk[kind].cfg.spt);
+      spans->push_back({rows, n});
+      rows += n;
+    }
+  }
+  return rows;
+}
+
+// mrows (nullable): plaquette rows of the measuring launches (parity 1 of the
+// last pass), laid out by ensemble_meas_rows.  With fused pairs (e->pcfg) the
+// phases (parity, 0) + (parity, 1) of every pass, and with walks (e->walk) the
+// phases (parity, 2) + (parity, 3), run as one launch; only a measuring pair
+// that is not packed runs as two.
 int ensemble_enqueue_phases(u1_ensemble* e, void* lat, double* mrows = nullptr) {
-  auto meas_rows = [&](bool last_pass, int parity, int mu) -> double* {
-    if (!mrows || !last_pass || parity != 1 || mu < 1) return nullptr;
-    return mrows + 4 * (size_t)e->upd_blocks * (size_t)(mu - 1);
-  };
   PhaseArgs a{};
   a.reps = e->upd_dev;
   a.blockmap = e->upd_map;
@@ -1261,31 +1333,27 @@ int ensemble_enqueue_phases(u1_ensemble* e, void* lat, double* mrows = nullptr) 
   a.sweep_mul = 1;
   a.accepts = nullptr;
   a.xcd = (uint32_t)e->cfg.xcd;
-  const bool fused = e->pcfg.block != 0;
   auto pass = [&](int kind, uint32_t p, bool last) -> int {
     a.pass = p;
-    for (int parity = 0; parity < 2; ++parity)
+    for (int parity = 0; parity < 2; ++parity) {
+      const bool measure = mrows && last && parity == 1;
+      a.parity = parity;
       for (int mu = 0; mu < 4; ++mu) {
-        a.parity = parity;
-        if (mu == 0 && fused && !meas_rows(last, parity, 1)) {
-          PhaseArgs b = a;
-          b.reps = e->pair_dev;
-          b.blockmap = e->pair_map;
-          b.meas = nullptr;
-          b.xcd = (uint32_t)e->pcfg.xcd;
-          HIPCHK(u1d::launch_pair(e->prec, kind, lat, b, e->pair_blocks, e->pcfg.block, e->pcfg.spt, e->pair_plane,
-                                  G.st));
+        if (mu == 0 && e->pcfg.block != 0 && (!measure || e->pair_packed)) {
+          a.meas = measure ? mrows + 4 * (size_t)e->mfirst[1] : nullptr;
+          RET(ensemble_launch_pair(e, kind, lat, a));
           ++mu;
           continue;
         }
-        a.meas = meas_rows(last, parity, mu);
-        if (mu == 2 && e->walk[kind].cfg.block != 0 && !a.meas) {
+        a.meas = measure && mu >= 1 ? mrows + 4 * (size_t)e->mfirst[mu] : nullptr;
+        if (mu == 2 && e->walk[kind].cfg.block != 0) {
           RET(ensemble_launch_walk(e, kind, lat, a));
           ++mu;
           continue;
         }
         HIPCHK(u1d::launch_phase(e->prec, kind, mu, lat, a, e->upd_blocks, e->cfg.block, e->cfg.spt, G.st));
       }
+    }
     return U1_OK;
   };
   for (int p = 0; p < e->metrop; ++p)
@@ -1341,8 +1409,18 @@ int ensemble_tune(u1_ensemble* e) {
     const Cfg none{0, 1, 0, 0};
     float tnone = best, tp = 1e30f;
     Cfg bestp = none;
-    for (const Cfg pc : {Cfg{64, 1, 1, 0}, Cfg{128, 1, 1, 0}, Cfg{256, 1, 1, 0}, Cfg{512, 1, 1, 0}, Cfg{128, 2, 1, 0},
-                         Cfg{256, 2, 1, 0}, Cfg{128, 1, 0, 0}, Cfg{256, 1, 0, 0}}) {
+    int plane = 0;
+    for (const RepDesc& r : e->upd_host) plane = std::max(plane, r.nxh * r.N[1]);
+    std::vector<Cfg> shapes = {{64, 1, 1, 0},  {128, 1, 1, 0}, {256, 1, 1, 0}, {512, 1, 1, 0},
+                               {128, 2, 1, 0}, {256, 2, 1, 0}, {128, 1, 0, 0}, {256, 1, 0, 0}};
+    if (ensemble_pair_packs(e, plane)) {
+      // the largest plane's wavefronts, and up to twice as many
+      shapes.clear();
+      const int w = (plane + 63) / 64, most = u1d::pair_max_block((int)elem_size(e->prec), 1) / 64;
+      for (int k = w; k <= std::min(2 * w, most); k += std::max(1, w / 4)) shapes.push_back({64 * k, 1, 1, 0});
+      shapes.push_back({64 * w, 1, 0, 0});
+    }
+    for (const Cfg& pc : shapes) {
       RET(ensemble_build_pair(e, pc));
       float t = 1e30f;
       RET(timed(&t));
@@ -1409,6 +1487,7 @@ void ensemble_release(u1_ensemble* e) {
   if (e->mexec) (void)hipGraphExecDestroy(e->mexec);
   if (e->mgraph) (void)hipGraphDestroy(e->mgraph);
   if (e->mrows) (void)hipFree(e->mrows);
+  if (e->mspans) (void)hipFree(e->mspans);
   if (e->series_dev) (void)hipFree(e->series_dev);
   if (e->base_dev) (void)hipFree(e->base_dev);
   if (e->upd_dev) (void)hipFree(e->upd_dev);
@@ -1416,6 +1495,7 @@ void ensemble_release(u1_ensemble* e) {
   if (e->upd_map) (void)hipFree(e->upd_map);
   if (e->pair_dev) (void)hipFree(e->pair_dev);
   if (e->pair_map) (void)hipFree(e->pair_map);
+  if (e->pair_packed) (void)hipFree(e->pair_packed);
   for (EnsembleWalk& w : e->walk) ensemble_drop_walk(w);
   if (e->meas_map) (void)hipFree(e->meas_map);
   if (e->lat) (void)hipFree(e->lat);
@@ -1429,24 +1509,26 @@ void ensemble_release(u1_ensemble* e) {
 // sweep, sweep index + 1.
 int ensemble_build_mgraph(u1_ensemble* e) {
   if (e->mexec) return U1_OK;
-  // (kept across a failed capture and reused by the next attempt, unless a
-  // later tuning has given the update launches more workgroups)
-  if (e->mrows && e->mrows_blocks < e->upd_blocks) {
-    HIPCHK(hipFree(e->mrows));
-    e->mrows = nullptr;
-  }
-  if (!e->mrows) {
-    HIPCHK(hipMalloc((void**)&e->mrows, 3 * 4 * (size_t)e->upd_blocks * sizeof(double)));
-    e->mrows_blocks = e->upd_blocks;
-  }
+  // (rebuilt by an attempt after a failed capture: the shapes may have changed)
+  if (e->mrows) HIPCHK(hipFree(e->mrows));
+  e->mrows = nullptr;
+  if (e->mspans) HIPCHK(hipFree(e->mspans));
+  e->mspans = nullptr;
+  std::vector<u1d::RowSpan> spans;
+  const int nrows = ensemble_meas_rows(e, &spans);
+  e->mlaunches = (int)(spans.size() / (size_t)e->nrep);
+  HIPCHK(hipMalloc((void**)&e->mrows, 4 * (size_t)nrows * sizeof(double)));
+  HIPCHK(hipMalloc((void**)&e->mspans, spans.size() * sizeof(spans[0])));
+  HIPCHK(hipMemcpyAsync(e->mspans, spans.data(), spans.size() * sizeof(spans[0]), hipMemcpyHostToDevice, G.st));
+  HIPCHK(hipStreamSynchronize(G.st));
   if (!e->series_dev)
     HIPCHK(hipMalloc((void**)&e->series_dev, (size_t)kEnsSeriesCap * e->nrep * 4 * sizeof(double)));
   if (!e->base_dev) HIPCHK(hipMalloc((void**)&e->base_dev, sizeof(uint32_t)));
   HIPCHK(hipStreamBeginCapture(G.st, hipStreamCaptureModeThreadLocal));
   int rc = ensemble_enqueue_phases(e, e->lat, e->mrows);
   if (rc == U1_OK) {
-    hipError_t f = u1d::launch_ensemble_plaquette_fold(e->mrows, 3, e->upd_blocks, e->upd_dev, e->nrep, e->sweep_dev,
-                                                       e->base_dev, kEnsSeriesCap, e->series_dev, G.st);
+    hipError_t f = u1d::launch_ensemble_plaquette_fold(e->mrows, e->mlaunches, e->mspans, e->upd_dev, e->nrep,
+                                                       e->sweep_dev, e->base_dev, kEnsSeriesCap, e->series_dev, G.st);
     if (f == hipSuccess) f = u1d::launch_increment(e->sweep_dev, G.st);
     if (f != hipSuccess) rc = fail(U1_ERR_HIP, std::string("ensemble capture: ") + hipGetErrorString(f));
   }
@@ -1500,13 +1582,15 @@ constexpr int kTimingLaunches = 32;  // back-to-back launches per class
 // launches of each class over all replicas, in the sweep's launch tables, with
 // (parity, mu) cycling over the phases the class covers in a pass.  ms[c]:
 // mean launch duration; per_sweep[c]: launches per measuring sweep (the last
-// overrelaxation pass measures in its parity-1 launches of mu >= 1 and leaves
-// its parity-1 phases unfused).
+// overrelaxation pass measures in its parity-1 launches of mu >= 1; a measuring
+// pair that is not packed runs as two phases).
 int time_ensemble_classes(u1_ensemble* e, double* ms, double* per_sweep) {
   const size_t bytes = (size_t)e->total_links * elem_size(e->prec);
+  std::vector<u1d::RowSpan> spans;
+  const int nrows = ensemble_meas_rows(e, &spans);
   DevBuf scratch, rows;
   HIPCHK(scratch.alloc(bytes));
-  HIPCHK(rows.alloc(4 * (size_t)e->upd_blocks * sizeof(double)));
+  HIPCHK(rows.alloc(4 * (size_t)nrows * sizeof(double)));
   HIPCHK(hipMemcpyAsync(scratch.p, e->lat, bytes, hipMemcpyDeviceToDevice, G.st));
   EventSet es;
   hipEvent_t e0, e1;
@@ -1521,49 +1605,43 @@ int time_ensemble_classes(u1_ensemble* e, double* ms, double* per_sweep) {
   a.stream = u1r::STREAM_UPDATE;
   a.sweep = (uint32_t)e->sweeps_done;
   a.xcd = (uint32_t)e->cfg.xcd;
-  for (int c = 0; c < LC_COUNT; ++c) ms[c] = per_sweep[c] = 0.0;
-  for (int c = 0; c < LC_COUNT; ++c) {
-    if (c == LC_OR_PAIR_MEAS || c >= LC_METRO_CHAIN) continue;  // the measuring parity 1 stays unfused
-    const bool pair = c == LC_METRO_PAIR || c == LC_OR_PAIR;
-    const int kind = (c == LC_METRO || c == LC_METRO_PAIR) ? u1d::KIND_METROPOLIS : u1d::KIND_OVERRELAX;
-    const int passes = kind == u1d::KIND_METROPOLIS ? e->metrop : e->ovrn;
-    const bool cmeas = c == LC_OR_MEAS;
-    const int measured = kind == u1d::KIND_OVERRELAX ? 1 : 0;  // parities with measuring launches
-    const bool fused[4] = {e->pcfg.block != 0, e->pcfg.block != 0, e->walk[kind].cfg.block != 0,
-                           e->walk[kind].cfg.block != 0};
-    const int nfused = (fused[0] ? 1 : 0) + (fused[2] ? 1 : 0);
-    if (passes == 0 || (pair && nfused == 0)) continue;
-    std::vector<std::pair<int, int>> ph;  // (parity, mu); a fused launch is listed by its first mu
-    for (int parity = 0; parity < 2; ++parity)
+  // launches of a class in a sweep: (parity, first mu), with repetitions
+  struct Launch {
+    int parity, mu;
+  };
+  std::vector<Launch> list[LC_COUNT];
+  auto add_pass = [&](int kind, bool measured) {
+    for (int parity = 0; parity < 2; ++parity) {
+      const bool measure = measured && parity == 1;
+      const bool pair = e->pcfg.block != 0 && (!measure || e->pair_packed), walk = e->walk[kind].cfg.block != 0;
       for (int mu = 0; mu < 4; ++mu) {
-        if (cmeas ? !(parity == 1 && mu >= 1) : (pair ? !(fused[mu] && mu % 2 == 0) : fused[mu])) continue;
-        ph.push_back({parity, mu});
+        const bool fused = mu < 2 ? pair : walk;
+        if (fused && mu % 2 == 1) continue;
+        const int c = kind == u1d::KIND_METROPOLIS ? (fused ? LC_METRO_PAIR : LC_METRO)
+                      : fused                      ? (measure ? LC_OR_PAIR_MEAS : LC_OR_PAIR)
+                                                   : (measure && mu > 0 ? LC_OR_MEAS : LC_OR);
+        list[c].push_back({parity, mu});
       }
-    if (cmeas)
-      per_sweep[c] = 3;
-    else if (pair)
-      per_sweep[c] = nfused * (2.0 * passes - measured);
-    else
-      per_sweep[c] = (4.0 - 2 * nfused) * (2.0 * passes - measured) + measured;
-    if (per_sweep[c] == 0.0) continue;
-    if (ph.empty()) ph.push_back({1, 0});  // the measuring parity's phase 0 only
+    }
+  };
+  for (int p = 0; p < e->metrop; ++p) add_pass(u1d::KIND_METROPOLIS, false);
+  for (int o = 0; o < e->ovrn; ++o) add_pass(u1d::KIND_OVERRELAX, o == e->ovrn - 1);
+  for (int c = 0; c < LC_COUNT; ++c) {
+    ms[c] = 0.0;
+    per_sweep[c] = (double)list[c].size();
+    if (list[c].empty()) continue;
+    const int kind = (c == LC_METRO || c == LC_METRO_PAIR) ? u1d::KIND_METROPOLIS : u1d::KIND_OVERRELAX;
+    const bool fused = c == LC_METRO_PAIR || c == LC_OR_PAIR || c == LC_OR_PAIR_MEAS;
+    const bool meas = c == LC_OR_MEAS || c == LC_OR_PAIR_MEAS;
     PhaseArgs b = a;
-    b.meas = cmeas ? rows.as<double>() : nullptr;
     auto launch = [&](int i) -> int {
-      const int mu = ph[(size_t)i % ph.size()].second;
-      b.parity = ph[(size_t)i % ph.size()].first;
-      b.pass = (uint32_t)(i / (int)ph.size());
-      if (pair && mu == 2) return ensemble_launch_walk(e, kind, scratch.p, b);
-      if (pair) {
-        PhaseArgs q = b;
-        q.reps = e->pair_dev;
-        q.blockmap = e->pair_map;
-        q.xcd = (uint32_t)e->pcfg.xcd;
-        HIPCHK(u1d::launch_pair(e->prec, kind, scratch.p, q, e->pair_blocks, e->pcfg.block, e->pcfg.spt,
-                                e->pair_plane, G.st));
-      } else {
-        HIPCHK(u1d::launch_phase(e->prec, kind, mu, scratch.p, b, e->upd_blocks, e->cfg.block, e->cfg.spt, G.st));
-      }
+      const int mu = list[c][(size_t)i % list[c].size()].mu;
+      b.parity = list[c][(size_t)i % list[c].size()].parity;
+      b.pass = (uint32_t)(i / (int)list[c].size());
+      b.meas = meas ? rows.as<double>() + 4 * (size_t)e->mfirst[std::max(mu, 1)] : nullptr;
+      if (fused && mu == 0) return ensemble_launch_pair(e, kind, scratch.p, b);
+      if (fused) return ensemble_launch_walk(e, kind, scratch.p, b);
+      HIPCHK(u1d::launch_phase(e->prec, kind, mu, scratch.p, b, e->upd_blocks, e->cfg.block, e->cfg.spt, G.st));
       return U1_OK;
     };
     RET(launch(0));  // warm-up

@@ -54,6 +54,13 @@ constexpr int pair_max_plane(int elem_bytes) { return 65536 / elem_bytes; }
 hipError_t launch_pair(int prec, int kind, void* lat_base, const PhaseArgs& a, int nblocks, int block, int spt,
                        int plane_sites, hipStream_t st);
 
+// The same for batched replicas whose planes all fit a workgroup (k_pair_packed):
+// descriptors with set_phase_blocks(r, 64), map[b] = replica and first chunk of
+// workgroup b, which takes floor(block / 64 / bpp) planes; no masks or accept
+// counts.  a.meas: nblocks rows, phase (parity, 1) measuring.
+hipError_t launch_pair_packed(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBlock* map, int nblocks,
+                              int block, hipStream_t st);
+
 // The four phases (parity, 0..3) of one pass in one launch (k_chain, schedule
 // and dependencies in u1_chain.h).  A single lattice without multilevel mask:
 // a.single carries set_phase_blocks(r, block * spt); sched is the list of
@@ -83,7 +90,8 @@ hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, i
                        hipStream_t st);
 // The same for all replicas of a batch (a.reps; w: device tables for `nblk`
 // workgroups, walk_batch_order; every replica's shape checked by the caller
-// with walk_shape_ok, sg = 0).  No measurement, no masks.
+// with walk_shape_ok, sg = 0).  a.meas: walk_rows rows per replica from its
+// WalkArgs::row on.  No masks.
 hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBatch& w, int nblk,
                                int block, int width, hipStream_t st);
 
@@ -146,11 +154,14 @@ hipError_t launch_plaquette_batched(int prec, const void* lat_base, const RepDes
 hipError_t launch_batched_finish(const double* partials, const RepDesc* reps, int nrep, double* out /*4*nrep*/,
                                  hipStream_t st);
 hipError_t launch_increment(uint32_t* counter, hipStream_t st);
-// Per-replica fold of the measuring phases' plaquette rows (nseg segments of
-// seg_rows rows; replica r owns rows [blk_begin, blk_begin + nblk) of each)
-// into series[(*sweep_dev - *base_dev) * nrep + r][4], skipped at or past cap.
-hipError_t launch_ensemble_plaquette_fold(const double* rows, int nseg, int seg_rows, const RepDesc* reps, int nrep,
-                                          const uint32_t* sweep_dev, const uint32_t* base_dev, int cap,
+// Per-replica fold of the measuring launches' plaquette rows (launch g, replica
+// r: spans[g * nrep + r]) into series[(*sweep_dev - *base_dev) * nrep + r][4],
+// skipped at or past cap.
+struct RowSpan {
+  int32_t begin, count;
+};
+hipError_t launch_ensemble_plaquette_fold(const double* rows, int nseg, const RowSpan* spans, const RepDesc* reps,
+                                          int nrep, const uint32_t* sweep_dev, const uint32_t* base_dev, int cap,
                                           double* series, hipStream_t st);
 
 // self test (u1_selftest.hip)

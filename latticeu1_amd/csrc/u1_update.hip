@@ -364,6 +364,51 @@ __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real
   phase_finish<1, KIND, MEAS>(a, L, v, acc0 + acc1);
 }
 
+// The same two phases for batched replicas whose planes fit one workgroup: a
+// workgroup takes as many planes of one replica as it has room for, whole
+// wavefronts each (64 sites per wavefront, map: replica and first
+// wavefront-chunk), so that replicas with small planes fill it as well as those
+// with large ones.  A replica descriptor carries set_phase_blocks(r, 64); it is
+// copied into registers, since after the first store its fields could only be
+// reloaded through the vector memory path.  Each wavefront is k_pair's one-step
+// form: all loads of both phases before phase 0 computes, two angles through
+// LDS (the plane's own part of it).  Measured, 64 replicas of 8^4 to 24^3 x 32
+// (11.7 M sites), binary32: overrelaxation 49 us, 71 us as two launches;
+// Metropolis 91 us and 94 us.  MEAS: phase (parity, 1) measures, one row per
+// workgroup.
+template <typename Real, int KIND, bool MEAS>
+__global__ __launch_bounds__(pair_max_block(sizeof(Real), 1)) void k_pair_packed(Real* __restrict__ lat_base, PhaseArgs a,
+                                                                               const WalkBlock* __restrict__ map) {
+  extern __shared__ __align__(8) unsigned char pair_lds[];
+  const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+  const WalkBlock e = map[L];
+  const RepDesc r = a.reps[e.x];
+  const uint32_t P = (uint32_t)r.sz;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t sub = mdiv(wave, r.div_bpp_m, r.div_bpp_s);  // plane of the workgroup
+  const uint32_t room = mdiv(blockDim.x >> 6, r.div_bpp_m, r.div_bpp_s);
+  const bool active = sub < room && e.y + wave < (uint32_t)r.nblk;
+  Real* th0 = reinterpret_cast<Real*>(pair_lds) + sub * P;
+  double v[2] = {0.0, 0.0};
+  uint32_t acc = 0, pbase = 0;
+  PhaseIn<Real, 1> q0, q1;
+  if (active) {
+    phase_site(r, e.y + wave, threadIdx.x & 63u, 64u, a.parity, q0.ps[0]);
+    pbase = ((uint32_t)q0.ps[0].z + (uint32_t)r.N[2] * q0.ps[0].t) * P;
+    q1.ps[0] = q0.ps[0];
+    phase_load<Real, 0, 1>(lat_base, a, r, q0);
+    pair1_load<Real, 1>(lat_base, a, r, q1);
+    phase_compute<Real, 0, KIND, 1, false>(lat_base, a, r, q0, v, acc, th0, pbase);
+    pair_take(pair_shared(q0.in[0]), q1.in[0], q1.th[0]);
+  }
+  __syncthreads();
+  if (active) {
+    phase_load_nu0_lds<Real, 1>(th0, pbase, q1);
+    phase_compute<Real, 1, KIND, 1, MEAS>(lat_base, a, r, q1, v, acc);
+  }
+  phase_finish<1, KIND, MEAS>(a, L, v, acc);
+}
+
 // Reads a completion counter at device scope (sees other XCDs' increments);
 // the value is wave-uniform.
 __device__ __forceinline__ uint32_t chain_poll(const uint32_t* p) {
@@ -562,6 +607,22 @@ hipError_t launch_pair_prec(int kind, Real* lat, const PhaseArgs& a, int nblocks
   return launch_pair_spt<Real, KIND_OVERRELAX>(spt, lat, a, nblocks, block, lds, s);
 }
 
+template <typename Real, int KIND>
+hipError_t launch_packed_meas(Real* lat, const PhaseArgs& a, const WalkBlock* map, int nblocks, int block, size_t lds,
+                              hipStream_t s) {
+  if (a.meas != nullptr)
+    k_pair_packed<Real, KIND, true><<<nblocks, block, lds, s>>>(lat, a, map);
+  else
+    k_pair_packed<Real, KIND, false><<<nblocks, block, lds, s>>>(lat, a, map);
+  return hipGetLastError();
+}
+template <typename Real>
+hipError_t launch_packed_prec(int kind, Real* lat, const PhaseArgs& a, const WalkBlock* map, int nblocks, int block,
+                              size_t lds, hipStream_t s) {
+  return kind == KIND_METROPOLIS ? launch_packed_meas<Real, KIND_METROPOLIS>(lat, a, map, nblocks, block, lds, s)
+                                 : launch_packed_meas<Real, KIND_OVERRELAX>(lat, a, map, nblocks, block, lds, s);
+}
+
 template <typename Real, int KIND, int SPT>
 hipError_t launch_chain_meas(Real* lat, const PhaseArgs& a, const ChainArgs& c, int nblocks, int block,
                              hipStream_t s) {
@@ -617,6 +678,17 @@ hipError_t launch_pair(int prec, int kind, void* lat_base, const PhaseArgs& a, i
   const size_t lds = (size_t)plane_sites * (size_t)elem;
   if (prec == PREC_F64) return launch_pair_prec<double>(kind, (double*)lat_base, a, nblocks, block, spt, lds, s);
   return launch_pair_prec<float>(kind, (float*)lat_base, with_f32_constants(a), nblocks, block, spt, lds, s);
+}
+
+hipError_t launch_pair_packed(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBlock* map, int nblocks,
+                              int block, hipStream_t s) {
+  const int elem = prec == PREC_F64 ? 8 : 4;
+  if (block < 64 || block > pair_max_block(elem, 1) || block % 64 != 0 || a.reps == nullptr || a.ml != 0 ||
+      a.accepts != nullptr || map == nullptr || nblocks < 1)
+    return hipErrorInvalidValue;
+  const size_t lds = (size_t)block * (size_t)elem;
+  if (prec == PREC_F64) return launch_packed_prec<double>(kind, (double*)lat_base, a, map, nblocks, block, lds, s);
+  return launch_packed_prec<float>(kind, (float*)lat_base, with_f32_constants(a), map, nblocks, block, lds, s);
 }
 
 hipError_t launch_chain(int prec, int kind, void* lat_base, const PhaseArgs& a, const ChainArgs& c, int nblocks,

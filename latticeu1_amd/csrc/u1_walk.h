@@ -221,6 +221,7 @@ struct WalkArgs {
   int32_t orbits, len, seg, width;
   int32_t strips, sg;
   int32_t gs, go;  // strips and diagonals of a group (rounded up)
+  int32_t row;     // first measurement row (batched replicas)
   uint32_t gs_m, gs_s;
 };
 // Batched replicas: workgroup b walks block map[b].y (walk_place, plain order)

@@ -158,20 +158,26 @@ __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real
     double o[4];
     block_sum<4>(v, o);
     if (threadIdx.x == 0)
-      for (int k = 0; k < 4; ++k) a.meas[4 * ((size_t)orbit * (uint32_t)wa.strips + strip) + k] = o[k];
+      for (int k = 0; k < 4; ++k) a.meas[4 * ((size_t)(uint32_t)wa.row + (size_t)orbit * (uint32_t)wa.strips + strip) + k] = o[k];
   }
   if (KIND == KIND_METROPOLIS && a.accepts && (threadIdx.x & 63) == 0 && acc)
     atomicAdd(a.accepts, (unsigned long long)acc);
 }
 
+template <typename Real, int KIND, int MODE>
+hipError_t launch_walk_batch_width(Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block, int width,
+                                   hipStream_t s) {
+  if (width == 64)
+    k_walk<Real, KIND, MODE, true, true><<<nblk, block, 0, s>>>(lat, a, w);
+  else
+    k_walk<Real, KIND, MODE, false, true><<<nblk, block, 0, s>>>(lat, a, w);
+  return hipGetLastError();
+}
 template <typename Real, int KIND>
 hipError_t launch_walk_batch(Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block, int width,
                              hipStream_t s) {
-  if (width == 64)
-    k_walk<Real, KIND, WALK_PLAIN, true, true><<<nblk, block, 0, s>>>(lat, a, w);
-  else
-    k_walk<Real, KIND, WALK_PLAIN, false, true><<<nblk, block, 0, s>>>(lat, a, w);
-  return hipGetLastError();
+  return a.meas != nullptr ? launch_walk_batch_width<Real, KIND, WALK_MEAS>(lat, a, w, nblk, block, width, s)
+                           : launch_walk_batch_width<Real, KIND, WALK_PLAIN>(lat, a, w, nblk, block, width, s);
 }
 template <typename Real>
 hipError_t launch_walk_batch_prec(int kind, Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block,
@@ -216,7 +222,7 @@ hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, i
 
 hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBatch& w, int nblk,
                                int block, int width, hipStream_t s) {
-  if (a.reps == nullptr || a.meas != nullptr || a.ml != 0 || nblk < 1) return hipErrorInvalidValue;
+  if (a.reps == nullptr || a.ml != 0 || nblk < 1) return hipErrorInvalidValue;
   if (prec == PREC_F64) return launch_walk_batch_prec<double>(kind, (double*)lat_base, a, w, nblk, block, width, s);
   return launch_walk_batch_prec<float>(kind, (float*)lat_base, with_f32_constants(a), w, nblk, block, width, s);
 }
