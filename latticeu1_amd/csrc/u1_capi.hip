@@ -390,12 +390,10 @@ int phase_cfg(int prec, int kind, const u1_geom* g, const void* lat, const Phase
   return U1_OK;
 }
 
-// Fused pair shapes of a geometry: whole (z, t) planes per workgroup, SPT
-// sites per thread per step, the workgroup size for one step over the plane
-// and for two, rounded up to whole wavefronts and capped at the kernel's
-// bound (larger planes take more steps).  With one site per thread, also
-// 1.25 and 1.5 times the two-step size: a full first step and a shorter
-// second one.
+// Fused pair shapes of a geometry: one step over the plane with 1, 2 or 3 sites
+// per thread, where that fits a workgroup, and skewed steps (k_pair, PAIR_SKEW)
+// of a few workgroup sizes: two, four and eight wavefronts (a barrier then joins
+// few, and several workgroups share a CU) and 2, 3 or 4 even steps.
 std::vector<Cfg> pair_candidates(int prec, const RepDesc& r) {
   const int P = r.nxh * r.N[1];
   std::vector<Cfg> v;
@@ -405,17 +403,15 @@ std::vector<Cfg> pair_candidates(int prec, const RepDesc& r) {
     for (int t = 0; t < 2; ++t)
       for (int x = 0; x < 2; ++x) v.push_back(Cfg{b, spt, x, t});
   };
-  for (int spt : {1, 2, 3, 4}) {
-    if (spt >= 3 && prec != U1_F32) continue;
-    const int maxb = u1d::pair_max_block((int)elem_size(prec), spt);
-    for (int steps = 1; steps <= 2; ++steps)
-      add(std::min(maxb, ((P + spt * steps - 1) / (spt * steps) + 63) / 64 * 64), spt);
-    if (spt == 1) {
-      const int b2 = (P + 1) / 2;
-      for (int q : {5, 6})  // b2 * q / 4
-        if (b2 * q / 4 < maxb) add((b2 * q / 4 + 63) / 64 * 64, spt);
-    }
+  auto waves = [](int n) { return (n + 63) / 64 * 64; };
+  const int maxb = u1d::pair_max_block((int)elem_size(prec), 1);
+  for (int spt = 1; spt <= (prec == U1_F32 ? 3 : 2); ++spt) {
+    const int b = waves((P + spt - 1) / spt);
+    if (b <= u1d::pair_max_block((int)elem_size(prec), spt)) add(b, spt);
   }
+  for (int b : {128, 256, 512, waves((P + 1) / 2), waves((P + 2) / 3), waves((P + 3) / 4)})
+    if (b < P && b <= maxb && b >= 2 * r.nxh) add(b, 1);
+  if (v.empty()) add(maxb, 1);  // rows of more than half a workgroup
   return v;
 }
 bool pair_shape_ok(int prec, const Cfg& c) {
@@ -459,10 +455,11 @@ int pair_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseA
   const std::string key = tune_key(name, g, prec);
   const std::vector<Cfg> cands = pair_candidates(prec, proto.single);
   // forced without a tuned pair shape: XCD order, lexicographic planes, 2
-  // (binary32) or 1 (binary64) sites per thread
+  // (binary32, one step) or 1 sites per thread
   auto forced_default = [&]() {
-    for (const Cfg& c : cands)
-      if (c.spt == (prec == U1_F32 ? 2 : 1) && c.xcd == 1 && c.tile == 0) *cfg = c;
+    for (const int spt : {1, prec == U1_F32 ? 2 : 1})
+      for (const Cfg& c : cands)
+        if (c.spt == spt && c.xcd == 1 && c.tile == 0) *cfg = c;
   };
   auto it = G.tunecache.find(key);
   if (it != G.tunecache.end()) {  // block 0: the tuner measured two launches faster

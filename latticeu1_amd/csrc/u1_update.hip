@@ -268,46 +268,58 @@ __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, Phas
 // The pair reads the lattice once (4V angles) and writes V/2 + V/2: 5V angles
 // against 9V for two launches.  MEAS applies to phase (parity, 1).  Dynamic
 // LDS: P angles (pair_lds_bytes).  Of phase 1's nineteen angles two come
-// from LDS; in the two forms below that keep a thread's sites over both
-// phases, seven more come from phase 0's loads of the same site
-// (pair_shared) and phase 1 loads ten:
-//  * one step covers the plane (P <= SPT * blockDim.x, SPT <= 3): every load
-//    of phase 1 is issued before phase 0 computes, so phase 1 waits on the
-//    barrier and two LDS reads only;
-//  * two steps (SPT = 1): the seven shared angles of both steps are kept in
-//    registers across the barrier.
-// Otherwise (more steps) phase 1 loads its seventeen angles after the
-// barrier.
-// FORM picks the form at compile time for a single lattice, whose plane
-// size the host knows (PAIR_ONE_STEP, PAIR_TWO_STEPS, PAIR_LOOP): each
-// kernel then holds the code of its own form only (in one kernel holding
-// all three, the compiler's schedule of the measuring two-step form took
-// 42 us where its own kernel takes 30 us at 48^4); PAIR_ANY (batched
-// replicas, planes of several sizes) decides per workgroup, without the
-// measuring two-step form.
-enum { PAIR_ONE_STEP = 0, PAIR_TWO_STEPS = 1, PAIR_LOOP = 2, PAIR_ANY = 3 };
+// from LDS; in the first two forms below, seven more come from phase 0's loads
+// of the same site (pair_shared), phase 1 loads ten, and both load at the same
+// time:
+//  * PAIR_ONE_STEP: one step covers the plane (P <= SPT * blockDim.x, SPT <= 3):
+//    every load of phase 1 is issued before phase 0 computes, so phase 1 waits
+//    on the barrier and two LDS reads only;
+//  * PAIR_SKEW (SPT = 1): phase 1 follows phase 0 one step behind, with a barrier
+//    after each step of phase 0, its angles kept in registers meanwhile.  Sites
+//    are in row order, and a step covers at least two rows (step >= Nx): then
+//    phase 1 of step k reads the new theta_0 of steps k and k + 1 only (and of
+//    row 0, of step 0), and phase 0 of step k + 1 reads the old theta_1 of steps
+//    k and k + 1 only (step 0: also of the last row, rewritten last).  All
+//    workgroups of an XCD go through their planes at about the same pace, so
+//    what a plane shares with its neighbours is read while it is in the L2;
+//  * PAIR_LOOP (steps of less than two rows, or more sites per thread): phase 1
+//    loads its seventeen angles after phase 0 of the whole plane, when at large
+//    planes the L2 no longer has them.
+// Binary32 overrelaxation pair, PAIR_LOOP or two steps before, PAIR_SKEW now: 563 ->
+// 466 us at 96^4 (1.70 GB compulsory), 82 -> 63 us at 64^4, 24.2 -> 23.0 us at
+// 48^4; Metropolis 651 -> 582, 120 -> 105 and 43.4 -> 39.8 us.  256 threads were
+// best (occupancy 7 at 65 to 71 registers; two sites per thread: 123 registers
+// and 5 to 30 % more time).
+// FORM picks the form at compile time for a single lattice, whose plane size
+// the host knows: each kernel then holds the code of its own form only.
+// PAIR_ANY (batched replicas with planes too large for k_pair_packed) decides
+// per workgroup between the last two; its descriptor is copied into registers
+// (see k_pair_packed).
+enum { PAIR_ONE_STEP = 0, PAIR_SKEW = 1, PAIR_LOOP = 2, PAIR_ANY = 3 };
 template <typename Real, int KIND, int SPT, bool MEAS, bool BATCHED = false, int FORM = PAIR_ANY>
 __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real* __restrict__ lat_base, PhaseArgs a) {
   extern __shared__ __align__(8) unsigned char pair_lds[];
   Real* th0 = reinterpret_cast<Real*>(pair_lds);
   const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
-  const RepDesc& r = BATCHED ? a.reps[a.blockmap[L]] : a.single;
+  RepDesc rep;
+  if constexpr (BATCHED) rep = a.reps[a.blockmap[L]];
+  const RepDesc& r = BATCHED ? rep : a.single;
   const uint32_t b = L - (uint32_t)r.blk_begin;  // the replica's plane (one chunk per plane)
   const uint32_t P = (uint32_t)r.nxh * (uint32_t)r.N[1];
   const uint32_t step = SPT * blockDim.x;
   double v0[2] = {0.0, 0.0}, v[2] = {0.0, 0.0};
   uint32_t acc0 = 0, acc1 = 0;
-  constexpr bool kOne = SPT <= 3 && (FORM == PAIR_ONE_STEP || FORM == PAIR_ANY);
-  constexpr bool kTwo = SPT == 1 && (FORM == PAIR_TWO_STEPS || (FORM == PAIR_ANY && !MEAS));
-  constexpr bool kLoop = FORM == PAIR_LOOP || FORM == PAIR_ANY;
-  if (kOne && (FORM != PAIR_ANY || P <= step)) {
-    PhaseIn<Real, SPT> q0, q1;
-    // a frozen plane (multilevel mask, uniform over the workgroup) is frozen
-    // for both phases: the whole workgroup leaves before the barrier
+  uint32_t pbase = 0;  // the plane's first id
+  // both phases' loads and phase 0 of the step at `base`; false: a frozen plane
+  // (multilevel mask, uniform over the workgroup), frozen for both phases: the
+  // whole workgroup leaves before the first barrier
+  auto phase0 = [&](uint32_t base, PhaseIn<Real, SPT>& q1) -> bool {
+    PhaseIn<Real, SPT> q0;
 #pragma unroll
-    for (int k = 0; k < SPT; ++k) phase_site(r, b, threadIdx.x + k * blockDim.x, step, a.parity, q0.ps[k]);
-    if (a.ml != 0 && (q0.ps[0].t & (uint32_t)(a.ml - 1)) == 0) return;
-    const uint32_t pbase = ((uint32_t)q0.ps[0].z + (uint32_t)r.N[2] * q0.ps[0].t) * P;  // the plane's first id
+    for (int k = 0; k < SPT; ++k)
+      phase_site(r, b, base + threadIdx.x + k * blockDim.x, step, a.parity, q0.ps[k]);
+    if (a.ml != 0 && (q0.ps[0].t & (uint32_t)(a.ml - 1)) == 0) return false;
+    pbase = ((uint32_t)q0.ps[0].z + (uint32_t)r.N[2] * q0.ps[0].t) * P;
 #pragma unroll
     for (int k = 0; k < SPT; ++k) q1.ps[k] = q0.ps[k];  // the same sites
     phase_load<Real, 0, SPT>(lat_base, a, r, q0);
@@ -315,36 +327,31 @@ __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real
     phase_compute<Real, 0, KIND, SPT, false>(lat_base, a, r, q0, v0, acc0, th0, pbase);
 #pragma unroll
     for (int k = 0; k < SPT; ++k) pair_take(pair_shared(q0.in[k]), q1.in[k], q1.th[k]);
-    __syncthreads();
+    return true;
+  };
+  auto phase1 = [&](PhaseIn<Real, SPT>& q1) {
     phase_load_nu0_lds<Real, SPT>(th0, pbase, q1);
     phase_compute<Real, 1, KIND, SPT, MEAS>(lat_base, a, r, q1, v, acc1);
-  } else if (kTwo && (FORM != PAIR_ANY || P <= 2 * step)) {
-    // two steps per phase: the angles phase 1 shares with phase 0 stay in
-    // registers across the barrier (pair_shared), one set per step
-    PhaseIn<Real, SPT> q;
-    PairShared<Real> sh[2][SPT];
-    uint32_t pbase = 0;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (phase_sites<0, SPT>(a, r, b, s * step + threadIdx.x, step, q.ps)) return;  // frozen plane
-      pbase = ((uint32_t)q.ps[0].z + (uint32_t)r.N[2] * q.ps[0].t) * P;
-      phase_load<Real, 0, SPT>(lat_base, a, r, q);
-      phase_compute<Real, 0, KIND, SPT, false>(lat_base, a, r, q, v0, acc0, th0, pbase);
-#pragma unroll
-      for (int k = 0; k < SPT; ++k) sh[s][k] = pair_shared(q.in[k]);
-    }
+  };
+  if (FORM == PAIR_ONE_STEP) {
+    PhaseIn<Real, SPT> q1;
+    if (!phase0(0, q1)) return;
     __syncthreads();
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      phase_sites<1, SPT>(a, r, b, s * step + threadIdx.x, step, q.ps);
-      pair1_load<Real, SPT>(lat_base, a, r, q);
-#pragma unroll
-      for (int k = 0; k < SPT; ++k) pair_take(sh[s][k], q.in[k], q.th[k]);
-      phase_load_nu0_lds<Real, SPT>(th0, pbase, q);
-      phase_compute<Real, 1, KIND, SPT, MEAS>(lat_base, a, r, q, v, acc1);
+    phase1(q1);
+  } else if (FORM == PAIR_SKEW || (FORM == PAIR_ANY && SPT == 1 && step >= 2 * (uint32_t)r.nxh)) {
+    PhaseIn<Real, SPT> qa, qb;  // phase 1 of alternate steps
+    if (!phase0(0, qa)) return;
+    for (uint32_t base = step;; base += 2 * step) {
+      if (base < P) phase0(base, qb);
+      __syncthreads();
+      phase1(qa);
+      if (base >= P) break;
+      if (base + step < P) phase0(base + step, qa);
+      __syncthreads();
+      phase1(qb);
+      if (base + step >= P) break;
     }
-  } else if (kLoop) {
-    uint32_t pbase = 0;
+  } else {
     for (uint32_t base = 0; base < P; base += step) {
       PhaseIn<Real, SPT> q;
       if (phase_sites<0, SPT>(a, r, b, base + threadIdx.x, step, q.ps)) return;  // frozen plane
@@ -564,8 +571,8 @@ void launch_pair_form(int form, Real* lat, const PhaseArgs& a, int nblocks, int 
       return;
     }
   if constexpr (SPT == 1)
-    if (form == PAIR_TWO_STEPS) {
-      k_pair<Real, KIND, SPT, MEAS, false, PAIR_TWO_STEPS><<<nblocks, block, lds, s>>>(lat, a);
+    if (form == PAIR_SKEW) {
+      k_pair<Real, KIND, SPT, MEAS, false, PAIR_SKEW><<<nblocks, block, lds, s>>>(lat, a);
       return;
     }
   k_pair<Real, KIND, SPT, MEAS, false, PAIR_LOOP><<<nblocks, block, lds, s>>>(lat, a);
@@ -577,12 +584,12 @@ hipError_t launch_pair_meas(Real* lat, const PhaseArgs& a, int nblocks, int bloc
     k_pair<Real, KIND, SPT, false, true><<<nblocks, block, lds, s>>>(lat, a);
     return hipGetLastError();
   }
-  // a single lattice: its plane size fixes the form (the kernel's own test)
+  // a single lattice: its plane and row size fix the form
   const int64_t P = (int64_t)a.single.nxh * a.single.N[1], step = (int64_t)SPT * block;
   const bool meas = a.meas != nullptr;
-  const int form = SPT <= 3 && P <= step ? PAIR_ONE_STEP
-                   : SPT == 1 && P <= 2 * step ? PAIR_TWO_STEPS
-                                                         : PAIR_LOOP;
+  const int form = SPT <= 3 && P <= step                   ? PAIR_ONE_STEP
+                   : SPT == 1 && step >= 2 * a.single.nxh ? PAIR_SKEW
+                                                           : PAIR_LOOP;
   if (meas)
     launch_pair_form<Real, KIND, SPT, true>(form, lat, a, nblocks, block, lds, s);
   else
