@@ -1878,7 +1878,8 @@ int u1_plaquette_noalloc(const u1_geom* g, int prec, const void* lat, double* ou
   set_blocks(r, block * spt);
   r.nblk *= 2;  // even sites, then odd sites
   const int nblk = r.nblk;
-  const size_t need = 4 * (size_t)nblk + u1d::fold_scratch(nblk, 4);
+  // rows, and a fold row for each 512 of them (more than the fold takes)
+  const size_t need = 4 * ((size_t)nblk + ((size_t)nblk + 511) / 512);
   if (need > kNoAllocScratchDoubles)
     return fail(U1_ERR_ARG, "lattice too large for u1_plaquette_noalloc: needs " + std::to_string(need) +
                                 " scratch doubles, the maximum is " + std::to_string(kNoAllocScratchDoubles));
@@ -2112,7 +2113,7 @@ int u1_plaquette_fields(const u1_geom* g, int prec, const void* lat, int32_t spa
   RET(check_prec(prec));
   const RepDesc r = make_rep(g, 0, 0);
   const int size = spacetime ? r.V : r.SV;
-  const int block = 256, nblk = (size + block - 1) / block;
+  const int block = 256, nblk = std::min((size + block - 1) / block, u1d::kFoldRows);
   RET(ensure_fold(nblk, 12));
   HIPCHK(u1d::launch_plaquette_fields(prec, lat, r, spacetime, eo_order, (double*)field_dev, G.partials, nblk, block,
                                       G.st));

@@ -112,7 +112,7 @@ hipError_t launch_polyakov(int prec, const void* lat, const RepDesc& r, double* 
 // Fold of nblk rows of nv partial sums, in row order, times scale.  Beyond
 // kFoldRows rows the fold takes two levels; scratch then holds
 // fold_groups(nblk) * nv doubles.
-constexpr int kFoldRows = 512;
+constexpr int kFoldRows = 4096;
 inline int fold_groups(int nblk) { return (nblk + kFoldRows - 1) / kFoldRows; }
 inline size_t fold_scratch(int nblk, int nv) { return (size_t)nv * (size_t)fold_groups(nblk); }
 hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double scale, double* out, double* scratch,

@@ -8,6 +8,7 @@
 // shared-memory fold plus one FP64 atomicAdd per block (reduce_block_1d.h:41-64,
 // cudaAtomic.h:147-177), whose summation order is nondeterministic.  All sums
 // are FP64 for both lattice precisions.
+#include <algorithm>
 #include <type_traits>
 
 #include "u1_kernels.h"
@@ -19,24 +20,24 @@ namespace {
 struct C64 {
   double re, im;
 };
+typedef double F64x2 __attribute__((ext_vector_type(2), aligned(8)));  // one 16-byte store, 8-byte aligned
 // complex.h:205-217 ordering
 __device__ __forceinline__ C64 cmul(C64 a, C64 b) { return {a.re * b.re - a.im * b.im, a.im * b.re + a.re * b.im}; }
 
-template <typename Real>
-__device__ __forceinline__ C64 exp_i(Real a) {
-  Real s, c;
-  Prec<Real>::sincos(a, &s, &c);
-  return {(double)c, (double)s};
-}
-
-// sin and cos of the temporal links: Prec's values (UMath<double>: but for
-// sin(-0)).
+// sin and cos of the measurement kernels: Prec's values (UMath<double>: but for
+// sin(-0), a zero of either sign here).
 template <typename Real>
 __device__ __forceinline__ void msincos(Real x, Real* s, Real* c) {
   if constexpr (sizeof(Real) == 8)
     UMath<double>::sincos(x, s, c);
   else
     Prec<Real>::sincos(x, s, c);
+}
+template <typename Real>
+__device__ __forceinline__ C64 exp_i(Real a) {
+  Real s, c;
+  msincos<Real>(a, &s, &c);
+  return {(double)c, (double)s};
 }
 
 // Temporal-link staple (staple.h:79-102 with mu = TDir): all six staples are
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(256) void k_plaquette(const Real* __restrict__ lat_
       for (int nu = mu + 1; nu < 4; ++nu) {
         const Real p = ((tm[k][mu] + tf[k][nu][mu]) - tf[k][mu][nu]) - tm[k][nu];
         Real sp, cp;
-        Prec<Real>::sincos(p, &sp, &cp);
+        msincos<Real>(p, &sp, &cp);
         const int c = nu == 3 ? 1 : 0;
         re[c] += (Real)1 - cp;
         im[c] -= sp;
@@ -254,7 +255,9 @@ __global__ __launch_bounds__(256) void k_polyakov(const Real* __restrict__ lat, 
 }
 
 // Fold nblk partial rows of nv values in workgroup order; one workgroup per value.
-__global__ __launch_bounds__(256) void k_finish(const double* __restrict__ partials, int nblk, int nv, double scale,
+// Up to kFoldRows rows it takes 2.3 to 4.5 us, a second level as much again: 2880
+// rows of 4 values 3.2 us here, 2.8 us + 2.8 us and a launch in two levels.
+__global__ __launch_bounds__(1024) void k_finish(const double* __restrict__ partials, int nblk, int nv, double scale,
                                                 double* __restrict__ out) {
   const int k = blockIdx.x;
   double v[1] = {0.0};
@@ -464,105 +467,82 @@ __global__ void k_increment(uint32_t* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) c[0] = c[0] + 1u;
 }
 
-// SixPlaquette order (lattice_functions.h:38-45): (0,3) (1,3) (2,3) (1,2) (2,0) (0,1).
-__device__ __forceinline__ void six_pair(int d, int& mu, int& nu) {
-  const int m[6] = {0, 1, 2, 1, 2, 0};
-  const int n[6] = {3, 3, 3, 2, 0, 1};
-  mu = m[d];
-  nu = n[d];
-}
-
-// Plaquette 1 - e^{iP} at the site with lexicographic coordinates x (even/odd input).
-template <typename Real>
-__device__ __forceinline__ C64 plaq_eo(const Real* __restrict__ lat, const RepDesc& r, const int32_t* x, int mu,
-                                       int nu) {
-  const int32_t lexc = x[0] + r.N[0] * (x[1] + r.N[1] * (x[2] + r.N[2] * x[3]));
-  const int32_t par = (x[0] + x[1] + x[2] + x[3]) & 1;
-  auto eo = [&](int d) {
-    int32_t y[4] = {x[0], x[1], x[2], x[3]};
-    y[d] = (y[d] + 1) % r.N[d];
-    const int32_t ly = y[0] + r.N[0] * (y[1] + r.N[1] * (y[2] + r.N[2] * y[3]));
-    return (ly >> 1) + (1 - par) * r.HV;
-  };
-  const int32_t here = (lexc >> 1) + par * r.HV;
-  Real p = lat[(int64_t)mu * r.V + here];
-  p += lat[(int64_t)nu * r.V + eo(mu)];
-  p -= lat[(int64_t)mu * r.V + eo(nu)];
-  p -= lat[(int64_t)nu * r.V + here];
-  const C64 e = exp_i<Real>(p);
-  return {1.0 - e.re, -e.im};
-}
-
-// Same with a lexicographic input lattice (lattice_functions.h:40-46).
-template <typename Real>
-__device__ __forceinline__ C64 plaq_no(const Real* __restrict__ lat, const RepDesc& r, const int32_t* x, int mu,
-                                       int nu) {
-  const int32_t here = x[0] + r.N[0] * (x[1] + r.N[1] * (x[2] + r.N[2] * x[3]));
-  auto nb = [&](int d) {
-    int32_t y[4] = {x[0], x[1], x[2], x[3]};
-    y[d] = (y[d] + 1) % r.N[d];
-    return y[0] + r.N[0] * (y[1] + r.N[1] * (y[2] + r.N[2] * y[3]));
-  };
-  Real p = lat[(int64_t)mu * r.V + here];
-  p += lat[(int64_t)nu * r.V + nb(mu)];
-  p -= lat[(int64_t)mu * r.V + nb(nu)];
-  p -= lat[(int64_t)nu * r.V + here];
-  const C64 e = exp_i<Real>(p);
-  return {1.0 - e.re, -e.im};
-}
-
 // plaquette_comps.cu:34-107: six plaquette components per site (spacetime) or
-// per spatial site averaged over t; field written at the lexicographic index,
-// component-major; partial sums of the six means per workgroup.
-template <typename Real>
-__global__ __launch_bounds__(256) void k_plaquette_fields(const Real* __restrict__ lat, RepDesc r, int spacetime,
-                                                          int eo_order, double* __restrict__ field,
-                                                          double* __restrict__ partials) {
-  const int32_t size = spacetime ? r.V : r.SV;
-  const int32_t idx = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+// per spatial site averaged over t, in SixPlaquette order
+// (lattice_functions.h:38-45): (0,3) (1,3) (2,3) (1,2) (2,0) (0,1); field written
+// at the lexicographic index, component-major; partial sums of the six means per
+// workgroup.  EO: even/odd input, else lexicographic.
+//
+// A thread takes lexicographic sites, so the field is stored in full lines, and
+// an even/odd input is read as two contiguous half rows.  A site's sixteen links
+// are loaded at once; only the loop over t keeps a second set of sums.  At most
+// kFoldRows workgroups, one row of sums each, so that the sums take one fold.
+// 24^4, binary64 (42 MB, 8 us at the copy rate): 17.8 us, 24.8 us with even/odd
+// threads, loads site by site and divisions for the coordinates.  All its
+// wavefronts are resident at once and load, compute (800 vector instructions,
+// 7 us) and store in step.
+template <typename Real, bool EO, bool SPACETIME>
+__global__ __launch_bounds__(256) void k_plaquette_fields(const Real* __restrict__ lat, RepDesc r,
+                                                         double* __restrict__ field,
+                                                         double* __restrict__ partials) {
+  const uint32_t size = (uint32_t)(SPACETIME ? r.V : r.SV);
   double v[12];
 #pragma unroll
   for (int k = 0; k < 12; ++k) v[k] = 0.0;
-  if (idx < size) {
-    int32_t x[4];
-    int32_t pos;
-    if (eo_order) {
-      const int32_t half = size / 2;
-      const int32_t parity = idx >= half ? 1 : 0;
-      const int32_t id = idx - parity * half;
-      Site s;
-      site_of(r, id, parity, s);
-      for (int k = 0; k < 4; ++k) x[k] = s.x[k];
-    } else {
-      x[0] = idx % r.N[0];
-      x[1] = (idx / r.N[0]) % r.N[1];
-      x[2] = (idx / (r.N[0] * r.N[1])) % r.N[2];
-      x[3] = spacetime ? idx / (r.N[0] * r.N[1] * r.N[2]) : 0;
-    }
-    const int nt = spacetime ? 1 : r.N[3];
+  for (uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x; idx < size; idx += gridDim.x * blockDim.x) {
+    double w[12];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) w[k] = 0.0;
+    const int nt = SPACETIME ? 1 : r.N[3];
     for (int t = 0; t < nt; ++t) {
-      if (!spacetime) x[3] = t;
+      const uint32_t n = idx + (uint32_t)(t * r.SV);  // lexicographic site
+      Site s;  // its row (of parity 0)
+      site_of(r, (int32_t)(n >> 1), 0, s);
+      const int32_t odd = (int32_t)(n & 1u), parity = (s.x[1] + s.x[2] + s.x[3] + odd) & 1;
+      const bool last = odd && (s.x[0] >> 1) == r.nxh - 1;
+      uint32_t here = n, nb[4];
+      if (EO) {
+        here = (uint32_t)(parity * r.HV) + (n >> 1);
+        const uint32_t opp = (uint32_t)((1 - parity) * r.HV) + (n >> 1);
+        nb[0] = opp + (uint32_t)(last ? 1 - r.nxh : odd);
+#pragma unroll
+        for (int mu = 1; mu < 4; ++mu) nb[mu] = opp + (uint32_t)s.fwd[mu];
+      } else {
+        nb[0] = n + (uint32_t)(last ? 1 - r.N[0] : 1);
+#pragma unroll
+        for (int mu = 1; mu < 4; ++mu) nb[mu] = n + 2u * (uint32_t)s.fwd[mu];
+      }
+      Real own[4], tf[4][4];  // tf[nu][mu] = theta_nu(x + mu)
+#pragma unroll
+      for (int mu = 0; mu < 4; ++mu) {
+        own[mu] = ld(lat + (size_t)mu * r.V, here);
+#pragma unroll
+        for (int nu = 0; nu < 4; ++nu)
+          if (nu != mu) tf[nu][mu] = ld(lat + (size_t)nu * r.V, nb[mu]);
+      }
+      constexpr int m[6] = {0, 1, 2, 1, 2, 0}, q[6] = {3, 3, 3, 2, 0, 1};
+#pragma unroll
       for (int d = 0; d < 6; ++d) {
-        int mu, nu;
-        six_pair(d, mu, nu);
-        const C64 p = eo_order ? plaq_eo<Real>(lat, r, x, mu, nu) : plaq_no<Real>(lat, r, x, mu, nu);
-        v[2 * d] += p.re;
-        v[2 * d + 1] += p.im;
+        const Real p = ((own[m[d]] + tf[q[d]][m[d]]) - tf[m[d]][q[d]]) - own[q[d]];
+        const C64 e = exp_i<Real>(p);
+        w[2 * d] += 1.0 - e.re;
+        w[2 * d + 1] += -e.im;
       }
     }
-    if (!spacetime)
-      for (int k = 0; k < 12; ++k) v[k] /= (double)r.N[3];
-    pos = spacetime ? x[0] + r.N[0] * (x[1] + r.N[1] * (x[2] + r.N[2] * x[3]))
-                    : x[0] + r.N[0] * (x[1] + r.N[1] * x[2]);
+    if (!SPACETIME)
+#pragma unroll
+      for (int k = 0; k < 12; ++k) w[k] /= (double)r.N[3];
+#pragma unroll
     for (int d = 0; d < 6; ++d) {
-      field[2 * ((int64_t)pos + (int64_t)d * size)] = v[2 * d];
-      field[2 * ((int64_t)pos + (int64_t)d * size) + 1] = v[2 * d + 1];
+      *reinterpret_cast<F64x2*>(field + 2 * ((size_t)idx + (size_t)d * size)) = F64x2{w[2 * d], w[2 * d + 1]};
+      v[2 * d] += w[2 * d];
+      v[2 * d + 1] += w[2 * d + 1];
     }
   }
   double o[12];
   block_sum<12>(v, o);
   if (threadIdx.x == 0)
-    for (int k = 0; k < 12; ++k) partials[12 * (int64_t)blockIdx.x + k] = o[k];
+    for (int k = 0; k < 12; ++k) partials[12 * (size_t)blockIdx.x + k] = o[k];
 }
 
 // Per-replica fold of batched plaquette partials, in workgroup order.
@@ -668,7 +648,7 @@ hipError_t launch_polyakov(int prec, const void* lat, const RepDesc& r, double* 
 hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double scale, double* out, double* scratch,
                               hipStream_t st) {
   if (nblk <= kFoldRows) {
-    k_finish<<<nv, 256, 0, st>>>(partials, nblk, nv, scale, out);
+    k_finish<<<nv, std::min(1024, (nblk + 63) / 64 * 64), 0, st>>>(partials, nblk, nv, scale, out);
     return hipGetLastError();
   }
   const int G = fold_groups(nblk);
@@ -750,10 +730,21 @@ hipError_t launch_convert_precision(const void* in, int in_prec, void* out, int 
 
 hipError_t launch_plaquette_fields(int prec, const void* lat, const RepDesc& r, int spacetime, int eo_order,
                                    double* field, double* partials, int nblk, int block, hipStream_t st) {
+  const auto run = [&](auto* l) {
+    using Real = std::remove_const_t<std::remove_pointer_t<decltype(l)>>;
+    if (eo_order && spacetime)
+      k_plaquette_fields<Real, true, true><<<nblk, block, 0, st>>>(l, r, field, partials);
+    else if (eo_order)
+      k_plaquette_fields<Real, true, false><<<nblk, block, 0, st>>>(l, r, field, partials);
+    else if (spacetime)
+      k_plaquette_fields<Real, false, true><<<nblk, block, 0, st>>>(l, r, field, partials);
+    else
+      k_plaquette_fields<Real, false, false><<<nblk, block, 0, st>>>(l, r, field, partials);
+  };
   if (prec == PREC_F64)
-    k_plaquette_fields<double><<<nblk, block, 0, st>>>((const double*)lat, r, spacetime, eo_order, field, partials);
+    run((const double*)lat);
   else
-    k_plaquette_fields<float><<<nblk, block, 0, st>>>((const float*)lat, r, spacetime, eo_order, field, partials);
+    run((const float*)lat);
   return hipGetLastError();
 }
 
