@@ -1376,9 +1376,15 @@ int ensemble_tune(u1_ensemble* e) {
   hipEvent_t e0, e1;
   HIPCHK(es.create(&e0));
   HIPCHK(es.create(&e1));
-  // one sweep, after one to warm up
+  // one sweep, after one pass of each kind to warm up
+  const int metrop = e->metrop, ovrn = e->ovrn;
   auto timed = [&](float* t) -> int {
-    RET(ensemble_enqueue_phases(e, scratch.p));
+    e->metrop = std::min(metrop, 1);
+    e->ovrn = std::min(ovrn, 1);
+    const int rc = ensemble_enqueue_phases(e, scratch.p);
+    e->metrop = metrop;
+    e->ovrn = ovrn;
+    RET(rc);
     HIPCHK(hipEventRecord(e0, G.st));
     RET(ensemble_enqueue_phases(e, scratch.p));
     HIPCHK(hipEventRecord(e1, G.st));
