@@ -235,6 +235,7 @@ __device__ __forceinline__ void phase_finish(const PhaseArgs& a, uint32_t L, dou
 
 template <typename Real, int MU, int KIND, bool BATCHED, int SPT, bool MEAS = false>
 __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, PhaseArgs a) {
+  fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>();
   const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
   const RepDesc& r = BATCHED ? a.reps[a.blockmap[L]] : a.single;
   const uint32_t b = L - (uint32_t)r.blk_begin;
@@ -298,6 +299,7 @@ __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, Phas
 enum { PAIR_ONE_STEP = 0, PAIR_SKEW = 1, PAIR_LOOP = 2, PAIR_ANY = 3 };
 template <typename Real, int KIND, int SPT, bool MEAS, bool BATCHED = false, int FORM = PAIR_ANY>
 __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real* __restrict__ lat_base, PhaseArgs a) {
+  fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>();
   extern __shared__ __align__(8) unsigned char pair_lds[];
   Real* th0 = reinterpret_cast<Real*>(pair_lds);
   const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
@@ -386,6 +388,7 @@ __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real
 template <typename Real, int KIND, bool MEAS>
 __global__ __launch_bounds__(pair_max_block(sizeof(Real), 1)) void k_pair_packed(Real* __restrict__ lat_base, PhaseArgs a,
                                                                                const WalkBlock* __restrict__ map) {
+  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(WalkBlock*)>();
   extern __shared__ __align__(8) unsigned char pair_lds[];
   const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
   const WalkBlock e = map[L];
@@ -498,6 +501,7 @@ __device__ __forceinline__ void chain_phase(Real* __restrict__ lat_base, const P
 // makes phases 1-3 measuring.
 template <typename Real, int KIND, int SPT, bool MEAS>
 __global__ __launch_bounds__(512) void k_chain(Real* __restrict__ lat_base, PhaseArgs a, ChainArgs c) {
+  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(ChainArgs)>();
   const uint32_t x = blockIdx.x & 7u;
   const uint32_t e = c.sched[blockIdx.x >> 3];
   const uint32_t w = e >> 10, chunk = (e >> 2) & 0xFFu;

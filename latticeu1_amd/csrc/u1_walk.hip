@@ -95,6 +95,7 @@ enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
 template <typename Real, int KIND, int MODE, bool UNIFORM, bool BATCHED = false>
 __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real* __restrict__ lat_base, PhaseArgs a,
                                                                            std::conditional_t<BATCHED, WalkBatch, WalkArgs> w) {
+  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(w)>();
   using Walk = WalkZT<sizeof(Real), UNIFORM>;
   constexpr int A = Walk::A, B = Walk::B, C = Walk::C, D = Walk::D;
   constexpr bool MEAS = MODE == WALK_MEAS;
