@@ -107,8 +107,12 @@ __host__ __device__ __forceinline__ void site_of(const RepDesc& r, int32_t id, i
 // round; the rest are hits.  Worth 0.15 to 0.25 us per launch: a binary32 sweep
 // of 16 launches takes 94 us instead of 98 at 24^4, 126 instead of 130 at 24^3 x
 // 48; no difference at 48^4.
+// Returns block, which the asm seems to need the lines for: not volatile, since a
+// volatile one counts as a write to memory and turns every later load of a
+// descriptor from global memory into vector loads (an ensemble sweep of 64
+// replicas: 1.19 ms instead of 0.87).
 template <int BYTES>
-__device__ __forceinline__ void fetch_args() {
+__device__ __forceinline__ uint32_t fetch_args(uint32_t block) {
   typedef const __attribute__((address_space(4))) uint32_t* Words;
   const Words k = (Words)__builtin_amdgcn_kernarg_segment_ptr();
   const Words m = (Words)__builtin_amdgcn_implicitarg_ptr();
@@ -117,8 +121,9 @@ __device__ __forceinline__ void fetch_args() {
   uint32_t t[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) t[i] = k[i < N ? 16 * i : 0];
-  asm volatile("" ::"s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]),
-               "s"(m[0]));
+  asm("" : "+s"(block) : "s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]),
+      "s"(m[0]));
+  return block;
 }
 
 // Loads and stores at a uniform base plus a 32-bit element index: the byte

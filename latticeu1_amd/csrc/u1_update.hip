@@ -235,8 +235,8 @@ __device__ __forceinline__ void phase_finish(const PhaseArgs& a, uint32_t L, dou
 
 template <typename Real, int MU, int KIND, bool BATCHED, int SPT, bool MEAS = false>
 __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, PhaseArgs a) {
-  fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>();
-  const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>(blockIdx.x);
+  const uint32_t L = a.xcd ? xcd_remap(block, gridDim.x) : block;
   const RepDesc& r = BATCHED ? a.reps[a.blockmap[L]] : a.single;
   const uint32_t b = L - (uint32_t)r.blk_begin;
   double v[2] = {0.0, 0.0};
@@ -299,10 +299,10 @@ __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, Phas
 enum { PAIR_ONE_STEP = 0, PAIR_SKEW = 1, PAIR_LOOP = 2, PAIR_ANY = 3 };
 template <typename Real, int KIND, int SPT, bool MEAS, bool BATCHED = false, int FORM = PAIR_ANY>
 __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real* __restrict__ lat_base, PhaseArgs a) {
-  fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>();
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>(blockIdx.x);
   extern __shared__ __align__(8) unsigned char pair_lds[];
   Real* th0 = reinterpret_cast<Real*>(pair_lds);
-  const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t L = a.xcd ? xcd_remap(block, gridDim.x) : block;
   RepDesc rep;
   if constexpr (BATCHED) rep = a.reps[a.blockmap[L]];
   const RepDesc& r = BATCHED ? rep : a.single;
@@ -388,9 +388,9 @@ __global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real
 template <typename Real, int KIND, bool MEAS>
 __global__ __launch_bounds__(pair_max_block(sizeof(Real), 1)) void k_pair_packed(Real* __restrict__ lat_base, PhaseArgs a,
                                                                                const WalkBlock* __restrict__ map) {
-  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(WalkBlock*)>();
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(WalkBlock*)>(blockIdx.x);
   extern __shared__ __align__(8) unsigned char pair_lds[];
-  const uint32_t L = a.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t L = a.xcd ? xcd_remap(block, gridDim.x) : block;
   const WalkBlock e = map[L];
   const RepDesc r = a.reps[e.x];
   const uint32_t P = (uint32_t)r.sz;
@@ -501,9 +501,9 @@ __device__ __forceinline__ void chain_phase(Real* __restrict__ lat_base, const P
 // makes phases 1-3 measuring.
 template <typename Real, int KIND, int SPT, bool MEAS>
 __global__ __launch_bounds__(512) void k_chain(Real* __restrict__ lat_base, PhaseArgs a, ChainArgs c) {
-  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(ChainArgs)>();
-  const uint32_t x = blockIdx.x & 7u;
-  const uint32_t e = c.sched[blockIdx.x >> 3];
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(ChainArgs)>(blockIdx.x);
+  const uint32_t x = block & 7u;
+  const uint32_t e = c.sched[block >> 3];
   const uint32_t w = e >> 10, chunk = (e >> 2) & 0xFFu;
   const uint32_t wt = mdiv(w, c.bz_m, c.bz_s);
   const uint32_t t = (x >> c.tz_log2) * c.bt + wt;

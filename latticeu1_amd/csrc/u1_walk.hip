@@ -95,7 +95,7 @@ enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
 template <typename Real, int KIND, int MODE, bool UNIFORM, bool BATCHED = false>
 __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real* __restrict__ lat_base, PhaseArgs a,
                                                                            std::conditional_t<BATCHED, WalkBatch, WalkArgs> w) {
-  fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(w)>();
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(w)>(blockIdx.x);
   using Walk = WalkZT<sizeof(Real), UNIFORM>;
   constexpr int A = Walk::A, B = Walk::B, C = Walk::C, D = Walk::D;
   constexpr bool MEAS = MODE == WALK_MEAS;
@@ -104,14 +104,14 @@ __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real
   RepDesc rep;
   WalkArgs wa;
   if constexpr (BATCHED) {
-    const WalkBlock e = w.map[blockIdx.x];
+    const WalkBlock e = w.map[block];
     if (e.x == kWalkNone) return;
     rep = a.reps[e.x];
     wa = w.args[e.x];
     (void)walk_place(wa, e.y, &strip, &orbit);  // never empty in plain order
   } else {
     wa = w;
-    if (!walk_place(wa, blockIdx.x, &strip, &orbit)) return;
+    if (!walk_place(wa, block, &strip, &orbit)) return;
   }
   const RepDesc& r = BATCHED ? rep : a.single;
   // segment of this lane, and its place in the strip
