@@ -88,6 +88,7 @@ struct Ctx {
   uint32_t chain_inc[4] = {};                     // launches that counted into each row since the last clear
   std::map<std::string, uint32_t*> chain_sched;   // "Nz Nt bpp" -> schedule list (device)
   std::map<std::string, int> chain_sched_len;
+  uint32_t* die_ctl = nullptr;    // counters of one-launch sweeps (DIE_CTL words, zero between launches)
   std::map<std::string, Cfg> tunecache;  // key -> launch shape
   int tune_loaded = 0;
 };
@@ -702,6 +703,13 @@ int chain_check() {
   return U1_OK;
 }
 
+int ensure_chain_err() {
+  if (G.chain_err) return U1_OK;
+  HIPCHK(hipHostMalloc((void**)&G.chain_err, sizeof(uint32_t), hipHostMallocMapped));
+  *G.chain_err = 0;
+  return U1_OK;
+}
+
 // Shapes of a fused pass: Cfg{block, spt, 1, tz, margin}, planes cut into
 // chunks of block * spt sites, the (z, t) planes in tz x (8 / tz) tiles (one
 // per XCD), dependencies at least margin + 1 schedule steps back.
@@ -775,10 +783,7 @@ int chain_prepare(const RepDesc& r, const Cfg& cc, u1d::ChainArgs* c, int* nbloc
     G.chain_cnt_cap = need;
     clear = true;
   }
-  if (!G.chain_err) {
-    HIPCHK(hipHostMalloc((void**)&G.chain_err, sizeof(uint32_t), hipHostMallocMapped));
-    *G.chain_err = 0;
-  }
+  RET(ensure_chain_err());
   if (clear) {
     HIPCHK(u1d::launch_fill_zero(G.chain_cnt, (int64_t)(need * sizeof(uint32_t)), G.st));
     G.chain_nz = nz;
@@ -967,16 +972,127 @@ int settle_update_cfgs(int prec, const u1_geom* g, const void* lat, const PhaseA
   return U1_OK;
 }
 
+// ------------------------------------------------------- one-launch sweeps
+// Lattices that one XCD's share of the card may still run faster than the whole
+// card does with a launch per one or two phases.  The tuner compares the two up
+// to here: in binary32 16^3 x 8 (2^14 sites per phase) takes 52 us per sweep
+// against 55, 16^4 84 against 56; in binary64 the two meet near 2^13.
+constexpr int kDieMaxHalfVolume = 1 << 14;
+// A one-launch sweep must take under this fraction of the launches' time.
+constexpr float kDieMinGain = 0.97f;
+
+int die_groups(const RepDesc& r, const Cfg& c) { return std::min(u1d::kDieGroups, (r.HV + c.block - 1) / c.block); }
+
+int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, const Cfg& c, double* meas_dst) {
+  RET(ensure_chain_err());
+  if (!G.die_ctl) {
+    HIPCHK(hipMalloc((void**)&G.die_ctl, u1d::DIE_CTL * sizeof(uint32_t)));
+    HIPCHK(u1d::launch_fill_zero(G.die_ctl, u1d::DIE_CTL * sizeof(uint32_t), G.st));
+  }
+  u1d::DieArgs d{};
+  void* err_dev = nullptr;
+  HIPCHK(hipHostGetDevicePointer(&err_dev, G.chain_err, 0));
+  d.ctl = G.die_ctl;
+  d.err = (uint32_t*)err_dev;
+  d.metrop = metrop;
+  d.ovrn = ovrn;
+  PhaseArgs b = a;
+  b.meas = nullptr;
+  if (meas_dst) {
+    RET(ensure_partials(4 * u1d::kDieGroups));
+    b.meas = G.partials;
+    d.out = meas_dst;
+    d.scale = 1.0 / (3.0 * (double)a.single.V);
+  }
+  HIPCHK(u1d::launch_die(prec, lat, b, d, die_groups(a.single, c), c.block, G.st));
+  return U1_OK;
+}
+
+int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, const u1_metro* m, uint64_t seed,
+               uint32_t stream, uint32_t sweep, uint32_t c3, int ml, unsigned long long* acc_dev,
+               double* meas_dst = nullptr, const uint32_t* sweep_dev = nullptr, uint32_t sweep_mul = 0,
+               bool one_launch = true);
+
+// Workgroup size of the one-launch sweep of these passes, or block = 0: not
+// with forced or forbidden fusion, masks, large lattices, or where the tuner
+// (on a scratch copy; cached per geometry and pass counts, block.x 0 =
+// launches per phase) measures the launches faster.
+int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int metrop, int ovrn, const u1_metro* m,
+            Cfg* cfg) {
+  *cfg = Cfg{0, 1, 0, 0};
+  if (G.chain != 1 || G.pair != 1 || a.ml != 0 || a.single.HV > kDieMaxHalfVolume || metrop + ovrn == 0) return U1_OK;
+  const std::string key = tune_key(("Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn)).c_str(), g, prec);
+  const auto it = G.tunecache.find(key);
+  if (it != G.tunecache.end()) {
+    *cfg = it->second;
+    return U1_OK;
+  }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(G.st, &cs));
+  if (!G.tune || cs != hipStreamCaptureStatusNone) return U1_OK;
+  const int64_t bytes = 4 * (int64_t)a.single.V * (int64_t)elem_size(prec);
+  DevBuf scratch;
+  HIPCHK(scratch.alloc(bytes));
+  HIPCHK(hipMemcpyAsync(scratch.p, lat, bytes, hipMemcpyDeviceToDevice, G.st));
+  EventSet es;
+  hipEvent_t e0, e1;
+  HIPCHK(es.create(&e0));
+  HIPCHK(es.create(&e1));
+  PhaseArgs p = a;
+  p.accepts = nullptr;
+  auto one = [&](const Cfg& c) -> int {
+    if (c.block != 0) return die_launch(prec, scratch.p, p, metrop, ovrn, c, nullptr);
+    return run_update(g, prec, scratch.p, metrop, ovrn, m, a.single.seed, a.stream, a.sweep, a.single.c3, 0, nullptr,
+                      nullptr, nullptr, 0, false);
+  };
+  auto timed = [&](const Cfg& c, float* best) -> int {
+    RET(one(c));  // warm-up
+    HIPCHK(hipEventRecord(e0, G.st));
+    for (int i = 0; i < 2; ++i) RET(one(c));
+    HIPCHK(hipEventRecord(e1, G.st));
+    HIPCHK(hipEventSynchronize(e1));
+    float ms = 0;
+    HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+    *best = std::min(*best, ms);
+    return chain_check();
+  };
+  const Cfg none{0, 1, 0, 0};
+  float tb = 1e30f, tsep = 1e30f;
+  Cfg best = none;
+  for (int b : {64, 128, 256, 512}) {
+    if (b > 64 && b / 2 >= a.single.HV) break;
+    float t = 1e30f;
+    for (int round = 0; round < 2; ++round) RET(timed(Cfg{b, 1, 0, 0}, &t));
+    if (t < tb) {
+      tb = t;
+      best = Cfg{b, 1, 0, 0};
+    }
+  }
+  // both sides afresh, alternating
+  tb = 1e30f;
+  for (int round = 0; round < 3; ++round) {
+    RET(timed(none, &tsep));
+    RET(timed(best, &tb));
+  }
+  const bool use = tb < kDieMinGain * tsep;
+  if (G.verbosity >= 1)
+    std::fprintf(stderr, "tune %s: one launch %.2f us per sweep (block %d) vs %.2f us: %s\n", key.c_str(), 1e3 * tb / 2.0,
+                 best.block, 1e3 * tsep / 2.0, use ? "one launch" : "separate");
+  G.tunecache[key] = use ? best : none;
+  *cfg = G.tunecache[key];
+  return U1_OK;
+}
+
 // One UpdateLattice on a single lattice (update.cu:449-456 loop order).
 // meas_dst (device, 4 doubles, nullable): the plaquette of the updated
 // lattice, in u1_plaquette's normalisation, from the measuring variants of
 // phases (parity 1, mu = 1, 2, 3) of the sweep's last pass.
 // sweep_dev (nullable): the Philox sweep index is *sweep_dev * sweep_mul +
 // sweep, read by the kernels (for graph capture; phase_cfg must have run).
+// one_launch: the whole sweep may run as one launch (die_cfg).
 int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, const u1_metro* m, uint64_t seed,
                uint32_t stream, uint32_t sweep, uint32_t c3, int ml, unsigned long long* acc_dev,
-               double* meas_dst = nullptr, const uint32_t* sweep_dev = nullptr,
-               uint32_t sweep_mul = 0) {
+               double* meas_dst, const uint32_t* sweep_dev, uint32_t sweep_mul, bool one_launch) {
   // the Metropolis pass index takes 12 bits of Philox counter word 2
   if (metrop < 0 || ovrn < 0 || metrop > 4095) return fail(U1_ERR_ARG, "bad pass counts");
   PhaseArgs a{};
@@ -992,6 +1108,11 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
   a.sweep_dev = sweep_dev;
   a.sweep_mul = sweep_mul;
   a.accepts = acc_dev;
+  if (one_launch) {
+    Cfg die;
+    RET(die_cfg(g, prec, lat, a, metrop, ovrn, m, &die));
+    if (die.block != 0) return die_launch(prec, lat, a, metrop, ovrn, die, meas_dst);
+  }
   Shapes sm, so;
   if (metrop > 0) RET(kind_shapes(prec, u1d::KIND_METROPOLIS, g, lat, a, &sm));
   if (ovrn > 0) RET(kind_shapes(prec, u1d::KIND_OVERRELAX, g, lat, a, &so));
@@ -1708,6 +1829,8 @@ int u1_finalize(void) {
   G.chain_sched_len.clear();
   if (G.chain_cnt) HIPCHK(hipFree(G.chain_cnt));
   if (G.chain_err) HIPCHK(hipHostFree(G.chain_err));
+  if (G.die_ctl) HIPCHK(hipFree(G.die_ctl));
+  G.die_ctl = nullptr;
   G.chain_cnt = nullptr;
   G.chain_cnt_cap = 0;
   G.chain_err = nullptr;
@@ -2463,6 +2586,12 @@ int u1_tune_load(const char* path) {
     // whole wavefronts, at most 512 threads and 4 sites per thread (binary32)
     const bool f32 = name.size() > 4 && name.compare(name.size() - 4, 4, "_f32") == 0;
     bool known = false;
+    if (name.compare(0, 5, "Sweep") == 0) {  // one-launch sweep: block 0 = launches per phase
+      if (by != 1 || !(bx == 0 || (bx >= 64 && bx <= u1d::kDieBlock && bx % 64 == 0)))
+        return fail(U1_ERR_IO, std::string("Bad launch shape in ") + path + ": " + line);
+      parsed.push_back({vol + "\t" + name, Cfg{bx, 1, 0, 0}});
+      continue;
+    }
     if (name.find("Chain_") != std::string::npos) {
       // fused pass: block 0 = unfused, block.z = tiles along z, grid.x = schedule margin
       if (!((bx == 0 && by == 1) || ((by == 1 || by == 2) && bx >= 64 && bx <= 512 && bx % 64 == 0 &&
@@ -2506,7 +2635,7 @@ int u1_tune_save(const char* path) {
          "Walk: (parity, 2) + (parity, 3) in one launch along their diagonals, block.x 0 = two launches, block.y = "
          "segments per wavefront, block.z - 1 = XCD order (1) + 2 log2 strip groups; Chain: fused "
          "parity pass (phases 0-3) in one launch, block.x 0 = unfused, block.z = tiles along z, grid.x = schedule "
-         "margin\n";
+         "margin; Sweep: whole sweep in one launch, block.x 0 = launches per phase\n";
   }
   return f ? U1_OK : fail(U1_ERR_IO, "write failed");
 }
@@ -2657,8 +2786,9 @@ int u1_bench_updates(const u1_geom* g, int prec, void* lat, int32_t metrop, int3
   HIPCHK(hipStreamSynchronize(G.st));
   HIPCHK(hipEventRecord(e0, G.st));
   for (int s = 0; s < nsweeps; ++s) {
+    // the launch classes of a sweep, which kernel_ms reports, at any size
     RET(run_update(g, prec, lat, metrop, ovrn, m, seed, U1_STREAM_UPDATE, sweep0 + (uint32_t)s, 0, 0, nullptr,
-                   measure_plaq == 1 ? series + 4 * s : nullptr));
+                   measure_plaq == 1 ? series + 4 * s : nullptr, nullptr, 0, false));
     if (measure_plaq == 2) RET(plaquette_async(g, prec, lat, series + 4 * s));
   }
   HIPCHK(hipEventRecord(e1, G.st));

@@ -1,0 +1,266 @@
+// u1_die.hip -- a whole sweep of a small lattice in one launch, on one die.
+//
+// A sweep of a lattice of a few ten thousand sites is a chain of 8 phases per
+// pass that are each over in a microsecond; a launch per one or two phases, or
+// a fused parity pass with completion counters at device scope, costs two to
+// three microseconds per phase whatever the phase does.  Here one workgroup per
+// CU of one XCD runs all passes, with a barrier between phases whose counter
+// and data live in that XCD's L2 (measured, barrier and exchange: 0.6 to 0.9 us
+// with 8 to 32 workgroups; 2.6 to 6.2 us at device scope with 32 to 256).
+//
+// The dispatcher hands workgroup b to XCD (b + const) % 8, so the launch has
+// eight times the workgroups that work and all but every eighth leave at once.
+// Nothing depends on that: before the first store every workgroup reports its
+// XCD, and unless all report the same one, stores and counters go to device
+// scope.
+//
+// Barrier and order.  A phase's workgroup first waits for its stores, then
+// counts itself; the next phase's loads of angles that the phase before wrote
+// come after the counter is complete.  All angle loads pass the L1 (device
+// scope; on one XCD the L2 serves them).  Of its eighteen staple angles a phase
+// (parity, mu) reads two that the phase before it wrote -- theta_{mu-1} at x and
+// x + mu - (mu-1), or for mu = 0 theta_3 at x + e0 and x - e3 -- so the loads and
+// four of the six staple terms of a thread's first site run while the barrier
+// completes.  Write after read: a phase overwrites theta_mu(parity), which the
+// phase before reads, and every workgroup has consumed its loads before it
+// counts itself.
+//
+// All workgroups must be resident at once: at most 32 of at most 512 threads,
+// one per CU of the XCD.  The waits are bounded all the same, and a timeout is
+// reported, not hung on.
+//
+// Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
+// overrelaxation passes, against the tuned launches: binary64 8^4 75 us against
+// 82, 12^3 x 8 86 against 95; binary32 8^4 39 us against 51, 12^3 x 16 52
+// against 67, 16^3 x 8 52 against 55.  With more sites one XCD's arithmetic
+// takes over (binary64 12^3 x 16: 113 us against 97; binary32 16^4: 84 against
+// 56).
+#include "u1_kernels.h"
+#include "u1_link.h"
+
+namespace u1d {
+
+namespace {
+
+// Polls before a wait gives up: with the poll's round trip about a second.
+constexpr uint32_t kDieSpin = 1u << 22;
+
+struct DieSync {
+  uint32_t* ctl;  // DIE_WORDS
+  uint32_t* err;
+  uint32_t n;       // workgroups
+  uint32_t target;  // arrivals that complete the last barrier
+  bool one;         // all on one XCD
+  bool dead;        // a wait timed out: no more waiting
+
+  __device__ __forceinline__ uint32_t poll(int word) const {
+    return __hip_atomic_load(ctl + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ void until(int word, uint32_t want) {
+    if (threadIdx.x == 0)
+      for (uint32_t k = 0; !dead && poll(word) < want; ++k) {
+        if (k == kDieSpin) {
+          dead = true;
+          __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    __syncthreads();
+    asm volatile("" ::: "memory");
+  }
+  __device__ __forceinline__ void start() {
+    if (threadIdx.x == 0) {
+      const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11));  // XCC_ID
+      __hip_atomic_fetch_or(ctl + DIE_XCDS, 1u << xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __hip_atomic_fetch_add(ctl + DIE_HERE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    target = 0;
+    one = false;
+    dead = false;
+  }
+  // before the first store
+  __device__ __forceinline__ void started() {
+    until(DIE_HERE, n);
+    const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)poll(DIE_XCDS));
+    one = (m & (m - 1)) == 0;
+  }
+  // this workgroup's stores are visible to the others
+  __device__ __forceinline__ void arrive() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    target += n;
+    if (threadIdx.x == 0) {
+      if (one)
+        __hip_atomic_fetch_add(ctl + DIE_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      else
+        __hip_atomic_fetch_add(ctl + DIE_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  __device__ __forceinline__ void wait() { until(DIE_DONE, target); }
+  // the last workgroup to leave clears the words for the next launch
+  __device__ __forceinline__ void leave() {
+    if (threadIdx.x != 0) return;
+    if (__hip_atomic_fetch_add(ctl + DIE_LEFT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != n) return;
+    for (int w : {DIE_HERE, DIE_XCDS, DIE_DONE, DIE_LEFT})
+      __hip_atomic_store(ctl + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+
+// Angles of direction j (not MU) of the staple; the two of the direction that
+// the phase before wrote only with DEP.
+template <typename Real, int MU>
+struct DieLoad {
+  static constexpr int LATE = MU == 0 ? 2 : MU - 1;  // j of the direction with late angles
+  const Real* lat;
+  const RepDesc& r;
+  uint32_t same, opp;
+  const int32_t (&fwd)[4];
+  const int32_t (&bwd)[4];
+  template <bool EARLY, bool DEP>
+  __device__ __forceinline__ void dir(StapleIn<Real>& in, int j) const {
+    const int nu = j < MU ? j : j + 1;
+    const Real* pm = lat + (size_t)MU * r.V;
+    const Real* pn = lat + (size_t)nu * r.V;
+    const bool late = j == LATE;
+    if (EARLY) {
+      in.b[j] = ldc(pm, opp + fwd[nu]);
+      in.e[j] = ldc(pm, opp + bwd[nu]);
+    }
+    if (late && MU == 0 ? DEP : EARLY) {
+      in.a[j] = ldc(pn, opp + fwd[MU]);
+      in.f[j] = ldc(pn, opp + bwd[nu]);
+    }
+    if (late && MU != 0 ? DEP : EARLY) {
+      in.c[j] = ldc(pn, same);
+      in.d[j] = ldc(pn, same + (uint32_t)(fwd[MU] + bwd[nu]));
+    }
+  }
+};
+
+// What changes from phase to phase, apart from MU.
+struct DieStep {
+  int kind;
+  bool begin;  // the sweep's first phase
+  bool meas;   // the last pass's parity 1
+};
+
+// One body per MU for all passes and sites: the kernel runs each of them a few
+// times only, and its instructions are cold in every cache when it begins.
+template <typename Real, int MU, bool MEAS>
+__device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArgs& a, const RepDesc& r, DieSync& sync,
+                                          uint32_t first, uint32_t stride, uint32_t& acc, double (&v)[4],
+                                          const DieStep& step) {
+  constexpr int LATE = DieLoad<Real, MU>::LATE;
+  const bool aniso = r.aniso != 1.0;
+  const Real xi = sizeof(Real) == sizeof(float) ? (Real)r.aniso_f : (Real)r.aniso;
+#pragma nounroll
+  for (uint32_t i = first; i == first || i - (threadIdx.x & 63u) < (uint32_t)r.HV; i += stride) {
+    const bool valid = i < (uint32_t)r.HV;  // others: the last site, nothing stored
+    const uint32_t id = valid ? i : (uint32_t)r.HV - 1u;
+    Site s;
+    site_of(r, (int32_t)id, a.parity, s);
+    const uint32_t same = (uint32_t)(a.parity * r.HV) + id, opp = (uint32_t)((1 - a.parity) * r.HV) + id;
+    const DieLoad<Real, MU> load{lat, r, same, opp, s.fwd, s.bwd};
+    StapleIn<Real> in;
+    StapleTerm<Real> term[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) load.template dir<true, false>(in, j);
+    Real th[1] = {ldc(lat + (size_t)MU * r.V, same)};
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (j != LATE) term[j] = staple_term(in, j);
+    if (i == first) {
+      if (step.begin)
+        sync.started();
+      else
+        sync.wait();
+    }
+    load.template dir<false, true>(in, LATE);
+    term[LATE] = staple_term(in, LATE);
+    PlaqPieces<Real> pp = {0, 0, 0, 0};
+    const Staple<Real> S[1] = {staple_of<Real, MU, MEAS>(term, xi, (Real)r.inv_aniso_f, aniso, &pp)};
+    const uint32_t l[1] = {same + (uint32_t)MU * (uint32_t)r.V};
+    const uint64_t vm[1] = {wave_mask(valid)};
+    if (step.kind == KIND_METROPOLIS)
+      update_angles<Real, KIND_METROPOLIS, 1>(a, r, S, th, l, vm, acc);
+    else
+      update_angles<Real, KIND_OVERRELAX, 1>(a, r, S, th, l, vm, acc);
+    if (valid) {
+      if (sync.one)
+        st(lat + (size_t)MU * r.V, same, th[0]);
+      else
+        stc(lat + (size_t)MU * r.V, same, th[0]);
+    }
+    if (MEAS && MU > 0)
+      if (step.meas) add_plaquettes<Real, MU>(pp, th[0], valid, v[MU == 3 ? 2 : 0], v[MU == 3 ? 3 : 1]);
+  }
+  sync.arrive();
+}
+
+template <typename Real, bool MEAS>
+__global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseArgs a, DieArgs d) {
+  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(DieArgs)>(blockIdx.x);
+  if (block & 7u) return;
+  const RepDesc& r = a.single;
+  Real* lat = lat_base + r.lat_off;
+  DieSync sync{d.ctl, d.err, gridDim.x >> 3, 0, false, false};
+  sync.start();
+  const uint32_t first = (block >> 3) * blockDim.x + threadIdx.x, stride = sync.n * blockDim.x;
+  uint32_t acc = 0;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  // (pass, parity) by (pass, parity)
+  const int halves = 2 * (d.metrop + d.ovrn);
+#pragma nounroll
+  for (int h = 0; h < halves; ++h) {
+    const bool metro = h < 2 * d.metrop;
+    a.pass = (uint32_t)((metro ? h : h - 2 * d.metrop) >> 1);
+    a.parity = h & 1;
+    DieStep step = {metro ? KIND_METROPOLIS : KIND_OVERRELAX, h == 0, h == halves - 1};
+    die_phase<Real, 0, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+    step.begin = false;
+    die_phase<Real, 1, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+    die_phase<Real, 2, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+    die_phase<Real, 3, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+  }
+  if (a.accepts && (threadIdx.x & 63) == 0 && acc) atomicAdd(a.accepts, (unsigned long long)acc);
+  if (MEAS) {
+    // one row per workgroup, folded in their order by the first
+    double o[4];
+    block_sum<4>(v, o);
+    if (threadIdx.x == 0)
+      for (uint32_t c = 0; c < 4; ++c) stc(a.meas, 4 * (block >> 3) + c, o[c]);
+    sync.arrive();
+    if (block == 0) {
+      sync.wait();
+      if (threadIdx.x < 4) {
+        double s = 0.0;
+        for (uint32_t g = 0; g < sync.n; ++g) s += ldc(a.meas, 4 * g + threadIdx.x);
+        d.out[threadIdx.x] = s * d.scale;
+      }
+    }
+  }
+  sync.leave();
+}
+
+template <typename Real>
+hipError_t launch_die_prec(Real* lat, const PhaseArgs& a, const DieArgs& d, int groups, int block, hipStream_t s) {
+  if (a.meas)
+    k_die<Real, true><<<8 * groups, block, 0, s>>>(lat, a, d);
+  else
+    k_die<Real, false><<<8 * groups, block, 0, s>>>(lat, a, d);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int groups, int block,
+                      hipStream_t s) {
+  if (block < 64 || block > kDieBlock || block % 64 != 0 || groups < 1 || groups > kDieGroups || a.reps || a.ml != 0 ||
+      d.metrop < 0 || d.ovrn < 0 || d.metrop + d.ovrn == 0 || !d.ctl || !d.err || (a.meas && !d.out))
+    return hipErrorInvalidValue;
+  if (prec == PREC_F64) return launch_die_prec<double>((double*)lat, a, d, groups, block, s);
+  return launch_die_prec<float>((float*)lat, with_f32_constants(a), d, groups, block, s);
+}
+
+}  // namespace u1d

@@ -65,28 +65,38 @@ __device__ __forceinline__ void staple_load(const Real* __restrict__ lat, const 
     in.f[j] = ld(pn, opp + bwd[nu]);
   }
 }
-// Staple of link (x, MU) (staple.h:79-102) from its angles, with the operation
-// order of the oracle.  With MEAS the plaquette pieces are collected on the
-// side (the staple is unchanged).
+// e^{i up} and e^{i lo} of one direction: cosines and sines.
+template <typename Real>
+struct StapleTerm {
+  Real cu, su, cl, sl;
+};
+template <typename Real>
+__device__ __forceinline__ StapleTerm<Real> staple_term(const StapleIn<Real>& in, int j) {
+  const Real up = (in.a[j] - in.b[j]) - in.c[j];
+  const Real lo = ((-in.d[j]) - in.e[j]) + in.f[j];
+  StapleTerm<Real> t;
+  UMath<Real>::sincos(up, &t.su, &t.cu);
+  UMath<Real>::sincos(lo, &t.sl, &t.cl);
+  return t;
+}
+
+// Staple of link (x, MU) (staple.h:79-102) from its terms (the j-th direction
+// nu != MU), with the operation order of the oracle.  With MEAS the plaquette
+// pieces are collected on the side (the staple is unchanged).
 template <typename Real, int MU, bool MEAS = false>
-__device__ __forceinline__ Staple<Real> staple_sum(const StapleIn<Real>& in, Real xi, Real inv_xi, bool aniso,
-                                                   PlaqPieces<Real>* pp = nullptr) {
+__device__ __forceinline__ Staple<Real> staple_of(const StapleTerm<Real> (&term)[3], Real xi, Real inv_xi, bool aniso,
+                                                  PlaqPieces<Real>* pp = nullptr) {
   Real ssr = 0, ssi = 0, str = 0, sti = 0;
 #pragma unroll
   for (int nu = 0; nu < 4; ++nu) {
     if (nu == MU) continue;
-    const int j = nu < MU ? nu : nu - 1;
-    const Real up = (in.a[j] - in.b[j]) - in.c[j];
-    const Real lo = ((-in.d[j]) - in.e[j]) + in.f[j];
-    Real su, cu, sl, cl;
-    UMath<Real>::sincos(up, &su, &cu);
-    UMath<Real>::sincos(lo, &sl, &cl);
-    const Real ar = cu + cl, ai = su + sl;
+    const StapleTerm<Real>& t = term[nu < MU ? nu : nu - 1];
+    const Real ar = t.cu + t.cl, ai = t.su + t.sl;
     if (MEAS && nu < MU) {
-      pp->ur += cu;
-      pp->ui += su;
-      pp->lr += cl;
-      pp->li += sl;
+      pp->ur += t.cu;
+      pp->ui += t.su;
+      pp->lr += t.cl;
+      pp->li += t.sl;
     }
     // binary32: the first term of each class initialises its sum (the oracle's
     // 0 + x is kept in binary64, where the kernels match it bit for bit)
@@ -109,6 +119,12 @@ __device__ __forceinline__ Staple<Real> staple_sum(const StapleIn<Real>& in, Rea
     if (!aniso) return {ssr + str, ssi + sti};  // xi == 1: identical to ss/1 + st*1
     return {ssr / xi + str * xi, ssi / xi + sti * xi};
   }
+}
+template <typename Real, int MU, bool MEAS = false>
+__device__ __forceinline__ Staple<Real> staple_sum(const StapleIn<Real>& in, Real xi, Real inv_xi, bool aniso,
+                                                   PlaqPieces<Real>* pp = nullptr) {
+  const StapleTerm<Real> t[3] = {staple_term(in, 0), staple_term(in, 1), staple_term(in, 2)};
+  return staple_of<Real, MU, MEAS>(t, xi, inv_xi, aniso, pp);
 }
 
 template <typename Real>
