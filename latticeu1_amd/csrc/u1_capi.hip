@@ -978,22 +978,44 @@ int settle_update_cfgs(int prec, const u1_geom* g, const void* lat, const PhaseA
 // to here: in binary32 16^3 x 8 (2^14 sites per phase) takes 52 us per sweep
 // against 55, 16^4 84 against 56; in binary64 the two meet near 2^13.
 constexpr int kDieMaxHalfVolume = 1 << 14;
+// With a multilevel mask every slab runs on an XCD by itself: sites of an XCD's
+// slabs up to which the two are compared.
+constexpr int kDieMaxSlabSites = 1 << 16;
 // A one-launch sweep must take under this fraction of the launches' time.
 constexpr float kDieMinGain = 0.97f;
 
-int die_groups(const RepDesc& r, const Cfg& c) { return std::min(u1d::kDieGroups, (r.HV + c.block - 1) / c.block); }
+bool die_possible(const RepDesc& r, int ml) {
+  if (ml == 0) return r.HV <= kDieMaxHalfVolume;
+  const int64_t rows = u1d::die_rows(u1d::die_slabs(ml, r.N[3]));
+  return rows <= u1d::kDieGroups && rows * ml * r.st <= kDieMaxSlabSites;
+}
+// Workgroups of a slab.
+uint32_t die_groups(const RepDesc& r, int ml, const Cfg& c) {
+  const uint32_t rows = u1d::die_rows(u1d::die_slabs(ml, r.N[3]));
+  const int sites = ml ? ml * r.st : r.HV;
+  return std::min<uint32_t>((uint32_t)u1d::kDieGroups / rows, (uint32_t)((sites + c.block - 1) / c.block));
+}
+
+// What one-launch sweeps need allocated (counters for as many slabs as there can
+// be).
+int die_prepare() {
+  RET(ensure_chain_err());
+  if (G.die_ctl) return U1_OK;
+  const size_t n = (size_t)u1d::DIE_CTL * 8 * u1d::kDieGroups;
+  HIPCHK(hipMalloc((void**)&G.die_ctl, n * sizeof(uint32_t)));
+  HIPCHK(u1d::launch_fill_zero(G.die_ctl, (int64_t)(n * sizeof(uint32_t)), G.st));
+  return U1_OK;
+}
 
 int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, const Cfg& c, double* meas_dst) {
-  RET(ensure_chain_err());
-  if (!G.die_ctl) {
-    HIPCHK(hipMalloc((void**)&G.die_ctl, u1d::DIE_CTL * sizeof(uint32_t)));
-    HIPCHK(u1d::launch_fill_zero(G.die_ctl, u1d::DIE_CTL * sizeof(uint32_t), G.st));
-  }
+  RET(die_prepare());
   u1d::DieArgs d{};
   void* err_dev = nullptr;
   HIPCHK(hipHostGetDevicePointer(&err_dev, G.chain_err, 0));
   d.ctl = G.die_ctl;
   d.err = (uint32_t*)err_dev;
+  d.slabs = u1d::die_slabs(a.ml, a.single.N[3]);
+  d.groups = die_groups(a.single, a.ml, c);
   d.metrop = metrop;
   d.ovrn = ovrn;
   PhaseArgs b = a;
@@ -1004,7 +1026,7 @@ int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, co
     d.out = meas_dst;
     d.scale = 1.0 / (3.0 * (double)a.single.V);
   }
-  HIPCHK(u1d::launch_die(prec, lat, b, d, die_groups(a.single, c), c.block, G.st));
+  HIPCHK(u1d::launch_die(prec, lat, b, d, c.block, G.st));
   return U1_OK;
 }
 
@@ -1014,14 +1036,16 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
                bool one_launch = true);
 
 // Workgroup size of the one-launch sweep of these passes, or block = 0: not
-// with forced or forbidden fusion, masks, large lattices, or where the tuner
+// with forced or forbidden fusion, large lattices or slabs, or where the tuner
 // (on a scratch copy; cached per geometry and pass counts, block.x 0 =
 // launches per phase) measures the launches faster.
 int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int metrop, int ovrn, const u1_metro* m,
             Cfg* cfg) {
   *cfg = Cfg{0, 1, 0, 0};
-  if (G.chain != 1 || G.pair != 1 || a.ml != 0 || a.single.HV > kDieMaxHalfVolume || metrop + ovrn == 0) return U1_OK;
-  const std::string key = tune_key(("Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn)).c_str(), g, prec);
+  if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml) || metrop + ovrn == 0) return U1_OK;
+  const std::string name = "Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn) +
+                           (a.ml ? "Mask" + std::to_string(a.ml) : "");
+  const std::string key = tune_key(name.c_str(), g, prec);
   const auto it = G.tunecache.find(key);
   if (it != G.tunecache.end()) {
     *cfg = it->second;
@@ -1040,10 +1064,11 @@ int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int
   HIPCHK(es.create(&e1));
   PhaseArgs p = a;
   p.accepts = nullptr;
+  p.sweep_dev = nullptr;
   auto one = [&](const Cfg& c) -> int {
     if (c.block != 0) return die_launch(prec, scratch.p, p, metrop, ovrn, c, nullptr);
-    return run_update(g, prec, scratch.p, metrop, ovrn, m, a.single.seed, a.stream, a.sweep, a.single.c3, 0, nullptr,
-                      nullptr, nullptr, 0, false);
+    return run_update(g, prec, scratch.p, metrop, ovrn, m, a.single.seed, a.stream, a.sweep, a.single.c3, a.ml,
+                      nullptr, nullptr, nullptr, 0, false);
   };
   auto timed = [&](const Cfg& c, float* best) -> int {
     RET(one(c));  // warm-up
@@ -1060,7 +1085,7 @@ int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int
   float tb = 1e30f, tsep = 1e30f;
   Cfg best = none;
   for (int b : {64, 128, 256, 512}) {
-    if (b > 64 && b / 2 >= a.single.HV) break;
+    if (b > 64 && b / 2 >= (a.ml ? a.ml * a.single.st : a.single.HV)) break;
     float t = 1e30f;
     for (int round = 0; round < 2; ++round) RET(timed(Cfg{b, 1, 0, 0}, &t));
     if (t < tb) {
@@ -2155,6 +2180,7 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
   const double l2norm = 1.0 / (double)n2, l4norm = 1.0 / (double)n4;
   const int mp = mh ? mh->proposal : 0, mn = mh ? mh->nhit : 0;
   const double ms = mh ? mh->step : 0.0;
+  Cfg die{0, 1, 0, 0};
   {  // launch shapes are settled before capture (the tuner allocates and synchronises)
     PhaseArgs a{};
     a.single = r;
@@ -2162,6 +2188,9 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     a.proposal = m->proposal;
     a.step = m->step;
     rc = settle_update_cfgs(prec, g, wl, a, metrop, ovrn);
+    a.ml = 2;
+    if (rc == U1_OK) rc = die_cfg(g, prec, wl, a, metrop, ovrn, m, &die);
+    if (rc == U1_OK && die.block != 0) rc = die_prepare();
     if (rc != U1_OK) {
       cleanup();
       return rc;
@@ -2180,7 +2209,8 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
                                       (uint32_t)n2, (uint32_t)slots, G.st));
     return U1_OK;
   };
-  if (G.graphs) {
+  // (nothing to gain from a graph where a sweep is one launch)
+  if (G.graphs && die.block == 0) {
     MLCHK(hipStreamBeginCapture(G.st, hipStreamCaptureModeThreadLocal));
     rc = level2_step();
     const hipError_t ce = hipStreamEndCapture(G.st, &graph);

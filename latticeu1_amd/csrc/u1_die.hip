@@ -25,8 +25,13 @@
 // phase before reads, and every workgroup has consumed its loads before it
 // counts itself.
 //
-// All workgroups must be resident at once: at most 32 of at most 512 threads,
-// one per CU of the XCD.  The waits are bounded all the same, and a timeout is
+// Multilevel masks (a.ml): between two frozen slices t % ml == 0 the links of a
+// slab -- spatial on its other slices, temporal on all -- depend on each other
+// and on frozen links only.  Each slab is a sweep of its own, on the XCD of its
+// number, and slabs on one XCD share its CUs.
+//
+// All workgroups of a barrier must be resident at once: an XCD is given at most
+// 32 of at most 512 threads, one per CU.  The waits are bounded all the same, and a timeout is
 // reported, not hung on.
 //
 // Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
@@ -145,19 +150,26 @@ struct DieStep {
   bool meas;   // the last pass's parity 1
 };
 
+// The even/odd sites of a workgroup's slab, spatial and temporal phases: n of
+// them from base on, this thread's first + k stride of those.
+struct DieSites {
+  uint32_t base, n, base3, n3, first, stride;
+};
+
 // One body per MU for all passes and sites: the kernel runs each of them a few
 // times only, and its instructions are cold in every cache when it begins.
 template <typename Real, int MU, bool MEAS>
 __device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArgs& a, const RepDesc& r, DieSync& sync,
-                                          uint32_t first, uint32_t stride, uint32_t& acc, double (&v)[4],
-                                          const DieStep& step) {
+                                          const DieSites& own, uint32_t& acc, double (&v)[4], const DieStep& step) {
+  const uint32_t first = own.first, stride = own.stride;
+  const uint32_t n = MU == 3 ? own.n3 : own.n, base = MU == 3 ? own.base3 : own.base;
   constexpr int LATE = DieLoad<Real, MU>::LATE;
   const bool aniso = r.aniso != 1.0;
   const Real xi = sizeof(Real) == sizeof(float) ? (Real)r.aniso_f : (Real)r.aniso;
 #pragma nounroll
-  for (uint32_t i = first; i == first || i - (threadIdx.x & 63u) < (uint32_t)r.HV; i += stride) {
-    const bool valid = i < (uint32_t)r.HV;  // others: the last site, nothing stored
-    const uint32_t id = valid ? i : (uint32_t)r.HV - 1u;
+  for (uint32_t i = first; i == first || i - (threadIdx.x & 63u) < n; i += stride) {
+    const bool valid = i < n;  // others: the last site, nothing stored
+    const uint32_t id = base + (valid ? i : n - 1u);
     Site s;
     site_of(r, (int32_t)id, a.parity, s);
     const uint32_t same = (uint32_t)(a.parity * r.HV) + id, opp = (uint32_t)((1 - a.parity) * r.HV) + id;
@@ -201,12 +213,18 @@ __device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArg
 template <typename Real, bool MEAS>
 __global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseArgs a, DieArgs d) {
   const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(DieArgs)>(blockIdx.x);
-  if (block & 7u) return;
   const RepDesc& r = a.single;
+  const uint32_t row = (block >> 3) / d.groups, wg = (block >> 3) - row * d.groups;  // slab row, place in the slab
+  const uint32_t slab = 8u * row + (block & 7u);
+  if (slab >= d.slabs) return;
   Real* lat = lat_base + r.lat_off;
-  DieSync sync{d.ctl, d.err, gridDim.x >> 3, 0, false, false};
+  DieSync sync{d.ctl + slab * DIE_CTL, d.err, d.groups, 0, false, false};
   sync.start();
-  const uint32_t first = (block >> 3) * blockDim.x + threadIdx.x, stride = sync.n * blockDim.x;
+  const uint32_t half = (uint32_t)r.st;  // even/odd sites of a slice
+  const uint32_t t0 = slab * (uint32_t)a.ml, nt = a.ml ? min((uint32_t)a.ml, (uint32_t)r.N[3] - t0) : (uint32_t)r.N[3];
+  const uint32_t frozen = a.ml ? 1u : 0u;
+  const DieSites own = {(t0 + frozen) * half,          (nt - frozen) * half, t0 * half, nt * half,
+                        wg * blockDim.x + threadIdx.x, d.groups * blockDim.x};
   uint32_t acc = 0;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   // (pass, parity) by (pass, parity)
@@ -217,11 +235,11 @@ __global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseA
     a.pass = (uint32_t)((metro ? h : h - 2 * d.metrop) >> 1);
     a.parity = h & 1;
     DieStep step = {metro ? KIND_METROPOLIS : KIND_OVERRELAX, h == 0, h == halves - 1};
-    die_phase<Real, 0, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+    die_phase<Real, 0, MEAS>(lat, a, r, sync, own, acc, v, step);
     step.begin = false;
-    die_phase<Real, 1, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
-    die_phase<Real, 2, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
-    die_phase<Real, 3, MEAS>(lat, a, r, sync, first, stride, acc, v, step);
+    die_phase<Real, 1, MEAS>(lat, a, r, sync, own, acc, v, step);
+    die_phase<Real, 2, MEAS>(lat, a, r, sync, own, acc, v, step);
+    die_phase<Real, 3, MEAS>(lat, a, r, sync, own, acc, v, step);
   }
   if (a.accepts && (threadIdx.x & 63) == 0 && acc) atomicAdd(a.accepts, (unsigned long long)acc);
   if (MEAS) {
@@ -229,9 +247,9 @@ __global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseA
     double o[4];
     block_sum<4>(v, o);
     if (threadIdx.x == 0)
-      for (uint32_t c = 0; c < 4; ++c) stc(a.meas, 4 * (block >> 3) + c, o[c]);
+      for (uint32_t c = 0; c < 4; ++c) stc(a.meas, 4 * wg + c, o[c]);
     sync.arrive();
-    if (block == 0) {
+    if (wg == 0) {
       sync.wait();
       if (threadIdx.x < 4) {
         double s = 0.0;
@@ -244,23 +262,25 @@ __global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseA
 }
 
 template <typename Real>
-hipError_t launch_die_prec(Real* lat, const PhaseArgs& a, const DieArgs& d, int groups, int block, hipStream_t s) {
+hipError_t launch_die_prec(Real* lat, const PhaseArgs& a, const DieArgs& d, int block, hipStream_t s) {
+  const uint32_t grid = 8u * die_rows(d.slabs) * d.groups;
   if (a.meas)
-    k_die<Real, true><<<8 * groups, block, 0, s>>>(lat, a, d);
+    k_die<Real, true><<<grid, block, 0, s>>>(lat, a, d);
   else
-    k_die<Real, false><<<8 * groups, block, 0, s>>>(lat, a, d);
+    k_die<Real, false><<<grid, block, 0, s>>>(lat, a, d);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int groups, int block,
-                      hipStream_t s) {
-  if (block < 64 || block > kDieBlock || block % 64 != 0 || groups < 1 || groups > kDieGroups || a.reps || a.ml != 0 ||
-      d.metrop < 0 || d.ovrn < 0 || d.metrop + d.ovrn == 0 || !d.ctl || !d.err || (a.meas && !d.out))
+hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int block, hipStream_t s) {
+  const uint32_t ml = (uint32_t)a.ml, nt = (uint32_t)a.single.N[3];
+  if (block < 64 || block > kDieBlock || block % 64 != 0 || !(ml == 0 || ml == 2 || ml == 4) || nt % 2 != 0 ||
+      d.slabs != die_slabs(a.ml, a.single.N[3]) || d.groups < 1 || die_rows(d.slabs) * d.groups > kDieGroups || a.reps ||
+      d.metrop < 0 || d.ovrn < 0 || d.metrop + d.ovrn == 0 || !d.ctl || !d.err || (a.meas && (!d.out || ml != 0)))
     return hipErrorInvalidValue;
-  if (prec == PREC_F64) return launch_die_prec<double>((double*)lat, a, d, groups, block, s);
-  return launch_die_prec<float>((float*)lat, with_f32_constants(a), d, groups, block, s);
+  if (prec == PREC_F64) return launch_die_prec<double>((double*)lat, a, d, block, s);
+  return launch_die_prec<float>((float*)lat, with_f32_constants(a), d, block, s);
 }
 
 }  // namespace u1d

@@ -95,10 +95,12 @@ hipError_t launch_walk(int prec, int kind, void* lat_base, const PhaseArgs& a, i
 hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseArgs& a, const WalkBatch& w, int nblk,
                                int block, int width, hipStream_t st);
 
-// All passes of a sweep of a small lattice in one launch (k_die): `groups`
-// workgroups of `block` threads on one XCD, any extents, no mask.  ctl: DIE_CTL
-// words, zero between launches.  A wait that times out sets *err (host-visible
-// memory).  a.meas: the plaquette of the updated lattice, times scale, to
+// All passes of a sweep of a small lattice in one launch (k_die), or with a mask
+// a.ml of every slab between two frozen slices: `groups` workgroups of `block`
+// threads per slab (die_slabs; 1 without mask), slab s on XCD s % 8 and at most
+// kDieGroups workgroups on an XCD; any extents.  ctl: DIE_CTL words per slab,
+// zero between launches.  A wait that times out sets *err (host-visible memory).
+// a.meas (no mask): the plaquette of the updated lattice, times scale, to
 // out[4]; a.meas holds 4 doubles per workgroup.
 enum { DIE_HERE = 0, DIE_XCDS = 32, DIE_DONE = 64, DIE_LEFT = 96, DIE_CTL = 128 };
 constexpr int kDieGroups = 32, kDieBlock = 512;
@@ -108,8 +110,11 @@ struct DieArgs {
   double* out;
   double scale;
   int32_t metrop, ovrn;
+  uint32_t slabs, groups;
 };
-hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int groups, int block, hipStream_t s);
+inline uint32_t die_slabs(int ml, int nt) { return ml ? (uint32_t)((nt + ml - 1) / ml) : 1u; }
+inline uint32_t die_rows(uint32_t slabs) { return (slabs + 7u) / 8u; }  // slabs on an XCD
+hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int block, hipStream_t s);
 
 // binary32 proposal constants: a (2 wu 2^-32 - 1) with a = pi (independent
 // angle) or step (theta + delta); a 2^-31 is exact
