@@ -151,7 +151,9 @@ struct DieStep {
 };
 
 // The even/odd sites of a workgroup's slab, spatial and temporal phases: n of
-// them from base on, this thread's first + k stride of those.
+// them from base on, this thread's first + k stride of those.  Wavefronts are
+// dealt to the workgroups in turn, so that a phase with half the sites still
+// uses every CU (binary32 level-2 sweep at 24^4: 70 -> 64 us, level 4 110 -> 86).
 struct DieSites {
   uint32_t base, n, base3, n3, first, stride;
 };
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseA
   const uint32_t t0 = slab * (uint32_t)a.ml, nt = a.ml ? min((uint32_t)a.ml, (uint32_t)r.N[3] - t0) : (uint32_t)r.N[3];
   const uint32_t frozen = a.ml ? 1u : 0u;
   const DieSites own = {(t0 + frozen) * half,          (nt - frozen) * half, t0 * half, nt * half,
-                        wg * blockDim.x + threadIdx.x, d.groups * blockDim.x};
+                        ((threadIdx.x >> 6) * d.groups + wg) * 64u + (threadIdx.x & 63u), d.groups * blockDim.x};
   uint32_t acc = 0;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   // (pass, parity) by (pass, parity)
