@@ -1084,7 +1084,8 @@ int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int
   const Cfg none{0, 1, 0, 0};
   float tb = 1e30f, tsep = 1e30f;
   Cfg best = none;
-  for (int b : {64, 128, 256, 512}) {
+  for (int b : {64, 128, 256, 512, 1024}) {
+    if (b > u1d::die_max_block((int)elem_size(prec))) break;
     if (b > 64 && b / 2 >= (a.ml ? a.ml * a.single.st : a.single.HV)) break;
     float t = 1e30f;
     for (int round = 0; round < 2; ++round) RET(timed(Cfg{b, 1, 0, 0}, &t));
@@ -2617,7 +2618,7 @@ int u1_tune_load(const char* path) {
     const bool f32 = name.size() > 4 && name.compare(name.size() - 4, 4, "_f32") == 0;
     bool known = false;
     if (name.compare(0, 5, "Sweep") == 0) {  // one-launch sweep: block 0 = launches per phase
-      if (by != 1 || !(bx == 0 || (bx >= 64 && bx <= u1d::kDieBlock && bx % 64 == 0)))
+      if (by != 1 || !(bx == 0 || (bx >= 64 && bx <= u1d::die_max_block(f32 ? 4 : 8) && bx % 64 == 0)))
         return fail(U1_ERR_IO, std::string("Bad launch shape in ") + path + ": " + line);
       parsed.push_back({vol + "\t" + name, Cfg{bx, 1, 0, 0}});
       continue;

@@ -31,7 +31,7 @@
 // number, and slabs on one XCD share its CUs.
 //
 // All workgroups of a barrier must be resident at once: an XCD is given at most
-// 32 of at most 512 threads, one per CU.  The waits are bounded all the same, and a timeout is
+// 32, one per CU.  The waits are bounded all the same, and a timeout is
 // reported, not hung on.
 //
 // Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
@@ -213,7 +213,7 @@ __device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArg
 }
 
 template <typename Real, bool MEAS>
-__global__ __launch_bounds__(512) void k_die(Real* __restrict__ lat_base, PhaseArgs a, DieArgs d) {
+__global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __restrict__ lat_base, PhaseArgs a, DieArgs d) {
   const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(DieArgs)>(blockIdx.x);
   const RepDesc& r = a.single;
   const uint32_t row = (block >> 3) / d.groups, wg = (block >> 3) - row * d.groups;  // slab row, place in the slab
@@ -277,7 +277,7 @@ hipError_t launch_die_prec(Real* lat, const PhaseArgs& a, const DieArgs& d, int 
 
 hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int block, hipStream_t s) {
   const uint32_t ml = (uint32_t)a.ml, nt = (uint32_t)a.single.N[3];
-  if (block < 64 || block > kDieBlock || block % 64 != 0 || !(ml == 0 || ml == 2 || ml == 4) || nt % 2 != 0 ||
+  if (block < 64 || block > die_max_block(prec == PREC_F64 ? 8 : 4) || block % 64 != 0 || !(ml == 0 || ml == 2 || ml == 4) || nt % 2 != 0 ||
       d.slabs != die_slabs(a.ml, a.single.N[3]) || d.groups < 1 || die_rows(d.slabs) * d.groups > kDieGroups || a.reps ||
       d.metrop < 0 || d.ovrn < 0 || d.metrop + d.ovrn == 0 || !d.ctl || !d.err || (a.meas && (!d.out || ml != 0)))
     return hipErrorInvalidValue;

@@ -103,7 +103,8 @@ hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseAr
 // a.meas (no mask): the plaquette of the updated lattice, times scale, to
 // out[4]; a.meas holds 4 doubles per workgroup.
 enum { DIE_HERE = 0, DIE_XCDS = 32, DIE_DONE = 64, DIE_LEFT = 96, DIE_CTL = 128 };
-constexpr int kDieGroups = 32, kDieBlock = 512;
+constexpr int kDieGroups = 32;
+constexpr int die_max_block(int elem_bytes) { return elem_bytes == 8 ? 512 : 1024; }
 struct DieArgs {
   uint32_t* ctl;
   uint32_t* err;

@@ -94,7 +94,7 @@ def test_fp64_one_launch_masked_sweep_parity(u1, orc, forced, dims, block, ml):
         assert np.array_equal(bits(lat.to_host()), bits(ref)), s
 
 
-@pytest.mark.parametrize("dims,block,ml", MASKED + [((24, 24, 24, 8), 512, 2)])
+@pytest.mark.parametrize("dims,block,ml", MASKED + [((24, 24, 24, 8), 512, 2), ((24, 24, 24, 8), 1024, 2)])
 def test_fp32_one_launch_masked_sweep_matches_phases(u1, forced, dims, block, ml):
     forced(dims, block, "f32")
     g = u1.geom(dims, 1.0, 1.2)
