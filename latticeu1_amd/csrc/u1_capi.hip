@@ -1196,13 +1196,23 @@ int plaquette_async(const u1_geom* g, int prec, const void* lat, double* dst) {
   return U1_OK;
 }
 
+// Doubles of the temporal-link field between links and product: the stochastic
+// multihit, whose hits keep the card busy only with every link on its own, and the
+// analytic one of more slices than k_poly_links takes.
+size_t poly_field(const RepDesc& r, int mode) {
+  const bool direct = mode == U1_POLY_PLAIN || (mode == U1_POLY_MULTIHIT && r.N[3] <= u1d::kPolyRows);
+  return direct ? 0 : 2 * (size_t)r.V;
+}
 // Polyakov-loop volume P (polyakov.cu:415-508) into P (2 SV doubles, device);
-// the multihit modes first write the temporal-link field into tl (2 V
-// doubles), then take the product along t.
+// tl: poly_field doubles, if any.
 int poly_volume_async(int prec, const void* lat, const RepDesc& r, int mode, const u1_metro* mh, uint32_t stream,
                       uint32_t c1, uint32_t c3, double* P, double* tl) {
   if (mode == U1_POLY_PLAIN) {
     HIPCHK(u1d::launch_poly_volume(prec, lat, r, P, G.st));
+    return U1_OK;
+  }
+  if (poly_field(r, mode) == 0) {
+    HIPCHK(u1d::launch_poly_links(prec, lat, r, P, G.st));
     return U1_OK;
   }
   HIPCHK(u1d::launch_temporal_links(prec, lat, r, mode, mh ? mh->proposal : 0, mh ? mh->nhit : 0,
@@ -2068,7 +2078,7 @@ int u1_poly_volume(const u1_geom* g, int prec, const void* lat, int32_t mode, co
   if (mode < 0 || mode > 2) return fail(U1_ERR_ARG, "bad Polyakov mode");
   if (mode == U1_POLY_MULTIHIT_STOCHASTIC) RET(check_metro(mh));
   const RepDesc r = make_rep(g, seed, c3);
-  if (mode != U1_POLY_PLAIN) RET(ensure_work(2 * (size_t)r.V));
+  RET(ensure_work(poly_field(r, mode)));
   return poly_volume_async(prec, lat, r, mode, mh, stream, c1, c3, (double*)P_dev, G.work);
 }
 
@@ -2112,8 +2122,8 @@ int u1_poly2(const u1_geom* g, int prec, const void* lat, int32_t mode, const u1
   if (mode < 0 || mode > 2) return fail(U1_ERR_ARG, "bad Polyakov mode");
   if (mode == U1_POLY_MULTIHIT_STOCHASTIC) RET(check_metro(mh));
   const RepDesc r = make_rep(g, seed, c3);
-  // work: P (2 SV doubles), then the temporal links (2 V doubles, multihit)
-  RET(ensure_work(2 * (size_t)r.SV + (mode != U1_POLY_PLAIN ? 2 * (size_t)r.V : 0)));
+  // work: P (2 SV doubles), then the temporal links (2 V doubles, poly_field)
+  RET(ensure_work(2 * (size_t)r.SV + poly_field(r, mode)));
   double* P = G.work;
   RET(poly_volume_async(prec, lat, r, mode, mh, U1_STREAM_MULTIHIT, c1, c3, P, G.work + 2 * (size_t)r.SV));
   return u1_pp(g, P, g->dims[0] / 2, out);

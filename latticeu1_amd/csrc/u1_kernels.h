@@ -140,6 +140,9 @@ inline size_t fold_scratch(int nblk, int nv) { return (size_t)nv * (size_t)fold_
 hipError_t launch_finish_sums(const double* partials, int nblk, int nv, double scale, double* out, double* scratch,
                               hipStream_t st);
 hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st);
+// the same of the analytic multihit links, Nt <= kPolyRows
+constexpr int kPolyRows = 32;
+hipError_t launch_poly_links(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st);
 hipError_t launch_temporal_links(int prec, const void* lat, const RepDesc& r, int mode, int proposal, int nhit,
                                  double step, uint32_t stream, uint32_t c1, uint32_t c3, double* out, hipStream_t st);
 // Multilevel: two-slice products of the temporal links of level-2 step ctr[0]

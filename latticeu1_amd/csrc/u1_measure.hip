@@ -393,6 +393,36 @@ __global__ __launch_bounds__(64) void k_tprod(const double* __restrict__ tl, Rep
   P[2 * (int64_t)j + 1] = res.im;
 }
 
+// Polyakov loops of the analytic multihit links, without the field between:
+// P(x) = prod_t T(x, t), a workgroup for kPolySites spatial sites with one thread
+// per link; the first row multiplies what the rows left in LDS, in t order as
+// k_tprod.  A loop over t, for more slices than a workgroup has rows, made the
+// compiler keep the constants of the special functions in registers (158, or
+// spills): 14 us and more.  Calls with the correlator, two kernels before: 35.3 ->
+// 31.2 us at 32^3 x 16 and 42.4 -> 34.1 us at 32^3 x 24, binary64, 32.3 -> 27.8 us
+// at 24^3 x 32 and 90.9 -> 68.6 us at 48^3 x 32, binary32.
+constexpr int kPolySites = 32;
+template <typename Real>
+__global__ __launch_bounds__(kPolySites * kPolyRows) void k_poly_links(const Real* __restrict__ lat, RepDesc r,
+                                                                       double* __restrict__ P) {
+  __shared__ C64 link[kPolyRows][kPolySites];
+  const int32_t lane = (int32_t)threadIdx.x % kPolySites, t = (int32_t)threadIdx.x / kPolySites, half = r.SV / 2;
+  const int32_t i = (int32_t)blockIdx.x * kPolySites + lane, idx = min(i, r.SV - 1);
+  const int32_t parity = idx >= half ? 1 : 0, id = idx - parity * half;  // at t = 0
+  Site s;
+  site_of(r, id + t * half, (parity + t) & 1, s);
+  link[t][lane] = temporal_value<Real, 1>(lat, r, s, id + t * half, (parity + t) & 1, 0, 0, 0.0, 0, 0, 0);
+  __syncthreads();
+  if (t == 0 && i < r.SV) {
+    C64 res = {1.0, 0.0};
+#pragma unroll 2
+    for (int32_t k = 0; k < r.N[3]; ++k) res = cmul(res, link[k][lane]);
+    const int32_t j = s.x[0] + r.N[0] * (s.x[1] + r.N[1] * s.x[2]);
+    P[2 * (int64_t)j] = res.re;
+    P[2 * (int64_t)j + 1] = res.im;
+  }
+}
+
 // polyakov.cu:514-535: sum over x and the three spatial axes of
 // P(x) conj(P(x + R e_dir)), R = 1..rmax; one partial row of 2*rmax per 256
 // sites.  One R per workgroup (blockIdx.y): 15.6 us at 24^3 when a workgroup
@@ -669,6 +699,16 @@ hipError_t launch_poly_volume(int prec, const void* lat, const RepDesc& r, doubl
 
 hipError_t launch_tprod(const double* tl, const RepDesc& r, double* P, hipStream_t st) {
   k_tprod<<<nblocks(r.SV, 64), 64, 0, st>>>(tl, r, P);
+  return hipGetLastError();
+}
+
+hipError_t launch_poly_links(int prec, const void* lat, const RepDesc& r, double* P, hipStream_t st) {
+  const int nb = nblocks(r.SV, kPolySites), block = kPolySites * r.N[3];
+  if (r.N[3] > kPolyRows) return hipErrorInvalidValue;
+  if (prec == PREC_F64)
+    k_poly_links<double><<<nb, block, 0, st>>>((const double*)lat, r, P);
+  else
+    k_poly_links<float><<<nb, block, 0, st>>>((const float*)lat, r, P);
   return hipGetLastError();
 }
 

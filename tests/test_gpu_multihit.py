@@ -37,3 +37,21 @@ def test_polyakov_loads_in_groups(u1, orc, mode, nt):
     c_orc = orc.poly2(og, ref, mode, orc.metro(1, 5, 3.0), 23)
     assert np.allclose(c_gpu, c_orc, rtol=1e-12, atol=1e-15)
     assert abs(lat.polyakov() - orc.polyakov(og, ref)) <= 1e-14
+
+
+@pytest.mark.parametrize("prec,tol", [("F64", 1e-12), ("F32", 1e-12)])
+@pytest.mark.parametrize("dims", [(2, 2, 2, 2), (4, 6, 2, 16), (6, 2, 10, 18), (4, 4, 4, 32), (4, 4, 4, 34)])
+def test_analytic_loops_are_the_products_of_the_links(u1, orc, prec, tol, dims):
+    """Loops formed in one workgroup per 32 spatial sites (8, 48, 120 and 64 sites,
+    one to 32 rows of time slices; 34: through the field) against the product of
+    the links themselves, a chain of at most 34 complex products."""
+    g, og = u1.geom(dims, 1.1, 1.2), orc.geom(dims, 1.1, 1.2)
+    ref = orc.hotstart(og, 31)
+    lat = u1.Lattice.from_host(g, ref)
+    if prec == "F32":
+        lat = lat.astype(u1.F32)
+    links = lat.temporal_links(u1.POLY_MULTIHIT).reshape(dims[3], -1)
+    P = lat.poly_volume(u1.POLY_MULTIHIT)
+    assert np.allclose(P.reshape(-1), np.prod(links, axis=0), rtol=tol, atol=1e-15)
+    if prec == "F64":
+        assert np.allclose(P, orc.poly_volume(og, ref, 1), rtol=tol, atol=1e-15)
