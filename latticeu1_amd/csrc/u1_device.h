@@ -395,10 +395,12 @@ __device__ __forceinline__ uint32_t count_wave(bool p, uint64_t m) {
   return (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(p) & m);
 }
 
-// Block sum of NV doubles per thread into out[0..NV) (valid in thread 0).
-// Partial sums of the waves go through LDS and are added in wave order.
+// Block sum of NV doubles per thread; thread k < NV returns the k-th (NV <= 64).
+// Partial sums of the waves go through LDS and are added in wave order, every
+// value by a thread of its own and four reads at a time (one thread for all of
+// them, one read after the other: 2 us of the plaquette fields' 17.7 at 24^4).
 template <int NV, int MAXW = 16>
-__device__ __forceinline__ void block_sum(double (&v)[NV], double (&out)[NV]) {
+__device__ __forceinline__ double block_sum(double (&v)[NV]) {
   __shared__ double red[MAXW][NV];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int nw = (blockDim.x + 63) >> 6;
@@ -408,15 +410,18 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double (&out)[NV]) {
     if (lane == 0) red[w][k] = s;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  double s = 0.0;
+  if (threadIdx.x < NV)
+    for (int i = 0; i < nw; i += 4) {
+      double t[4];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      double s = 0.0;
-      for (int i = 0; i < nw; ++i) s += red[i][k];
-      out[k] = s;
+      for (int j = 0; j < 4; ++j) t[j] = red[min(i + j, nw - 1)][threadIdx.x];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j < nw) s += t[j];
     }
-  }
   __syncthreads();
+  return s;
 }
 
 }  // namespace u1d

@@ -246,10 +246,8 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
   if (a.accepts && (threadIdx.x & 63) == 0 && acc) atomicAdd(a.accepts, (unsigned long long)acc);
   if (MEAS) {
     // one row per workgroup, folded in their order by the first
-    double o[4];
-    block_sum<4>(v, o);
-    if (threadIdx.x == 0)
-      for (uint32_t c = 0; c < 4; ++c) stc(a.meas, 4 * wg + c, o[c]);
+    const double o = block_sum<4>(v);
+    if (threadIdx.x < 4) stc(a.meas, 4 * wg + threadIdx.x, o);
     sync.arrive();
     if (wg == 0) {
       sync.wait();

@@ -211,12 +211,10 @@ __global__ __launch_bounds__(256) void k_plaquette(const Real* __restrict__ lat_
       v[3] += (double)im[1];
     }
   }
-  double out[4];
-  block_sum<4>(v, out);
+  const double out = block_sum<4>(v);
   // row L (the logical workgroup): a batched fold reads each replica's rows
   // [blk_begin, blk_begin + nblk)
-  if (threadIdx.x == 0)
-    for (int k = 0; k < 4; ++k) partials[4 * (int64_t)L + k] = out[k];
+  if (threadIdx.x < 4) partials[4 * (int64_t)L + threadIdx.x] = out;
 }
 
 // polyakov.cu:60-77: sum of the temporal angles along t (in FP64), then e^{i.}.
@@ -246,12 +244,8 @@ __global__ __launch_bounds__(256) void k_polyakov(const Real* __restrict__ lat, 
     v[0] = c;
     v[1] = s;
   }
-  double out[2];
-  block_sum<2>(v, out);
-  if (threadIdx.x == 0) {
-    partials[2 * (int64_t)blockIdx.x] = out[0];
-    partials[2 * (int64_t)blockIdx.x + 1] = out[1];
-  }
+  const double out = block_sum<2>(v);
+  if (threadIdx.x < 2) partials[2 * (int64_t)blockIdx.x + threadIdx.x] = out;
 }
 
 // Fold nblk partial rows of nv values in workgroup order; one workgroup per value.
@@ -262,9 +256,8 @@ __global__ __launch_bounds__(1024) void k_finish(const double* __restrict__ part
   const int k = blockIdx.x;
   double v[1] = {0.0};
   for (int i = threadIdx.x; i < nblk; i += blockDim.x) v[0] += partials[(int64_t)i * nv + k];
-  double o[1];
-  block_sum<1>(v, o);
-  if (threadIdx.x == 0) out[k] = o[0] * scale;
+  const double o = block_sum<1>(v);
+  if (threadIdx.x == 0) out[k] = o * scale;
 }
 
 // First level of a long fold: workgroup (g, k) adds rows [g R, g R + R) of
@@ -275,9 +268,8 @@ __global__ __launch_bounds__(256) void k_fold_rows(const double* __restrict__ pa
   const int r0 = g * R, r1 = min(nrows, r0 + R);
   double v[1] = {0.0};
   for (int i = r0 + (int)threadIdx.x; i < r1; i += blockDim.x) v[0] += partials[(int64_t)i * nv + k];
-  double o[1];
-  block_sum<1>(v, o);
-  if (threadIdx.x == 0) l1[(int64_t)g * nv + k] = o[0];
+  const double o = block_sum<1>(v);
+  if (threadIdx.x == 0) l1[(int64_t)g * nv + k] = o;
 }
 
 // polyakov.cu:415-440 without multihit: P(x) = prod_t e^{i theta_t(x, t)},
@@ -447,12 +439,8 @@ __global__ __launch_bounds__(256) void k_pp(const double* __restrict__ P, RepDes
       v[1] += t.im;
     }
   }
-  double o[2];
-  block_sum<2>(v, o);
-  if (threadIdx.x == 0) {
-    partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2] = o[0];
-    partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2 + 1] = o[1];
-  }
+  const double o = block_sum<2>(v);
+  if (threadIdx.x < 2) partials[((int64_t)blockIdx.x * rmax + (R - 1)) * 2 + threadIdx.x] = o;
 }
 
 // convertOrder.cu:32-63: even/odd <-> lexicographic, all four planes.  A thread
@@ -570,10 +558,8 @@ __global__ __launch_bounds__(256) void k_plaquette_fields(const Real* __restrict
       v[2 * d + 1] += w[2 * d + 1];
     }
   }
-  double o[12];
-  block_sum<12>(v, o);
-  if (threadIdx.x == 0)
-    for (int k = 0; k < 12; ++k) partials[12 * (size_t)blockIdx.x + k] = o[k];
+  const double o = block_sum<12>(v);
+  if (threadIdx.x < 12) partials[12 * (size_t)blockIdx.x + threadIdx.x] = o;
 }
 
 // Per-replica fold of batched plaquette partials, in workgroup order.
@@ -583,12 +569,8 @@ __global__ __launch_bounds__(256) void k_batched_finish(const double* __restrict
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   for (int i = threadIdx.x; i < r.nblk; i += blockDim.x)
     for (int k = 0; k < 4; ++k) v[k] += partials[4 * (int64_t)(r.blk_begin + i) + k];
-  double o[4];
-  block_sum<4>(v, o);
-  if (threadIdx.x == 0) {
-    const double n = 1.0 / (3.0 * (double)r.V);
-    for (int k = 0; k < 4; ++k) out[4 * blockIdx.x + k] = o[k] * n;
-  }
+  const double o = block_sum<4>(v);
+  if (threadIdx.x < 4) out[4 * blockIdx.x + threadIdx.x] = o * (1.0 / (3.0 * (double)r.V));
 }
 
 // Per-replica fold of the plaquette rows written by the measuring update
@@ -608,14 +590,11 @@ __global__ __launch_bounds__(256) void k_ensemble_plaquette_fold(const double* _
       for (int k = 0; k < 4; ++k) v[k] += row[k];
     }
   }
-  double o[4];
-  block_sum<4>(v, o);
-  if (threadIdx.x == 0) {
+  const double o = block_sum<4>(v);
+  if (threadIdx.x < 4) {
     const uint32_t idx = *sweep_dev - *base_dev;
-    if (idx < (uint32_t)cap) {
-      const double n = 1.0 / (3.0 * (double)r.V);
-      for (int k = 0; k < 4; ++k) series[4 * ((int64_t)idx * nrep + blockIdx.x) + k] = o[k] * n;
-    }
+    if (idx < (uint32_t)cap)
+      series[4 * ((int64_t)idx * nrep + blockIdx.x) + threadIdx.x] = o * (1.0 / (3.0 * (double)r.V));
   }
 }
 

@@ -127,12 +127,8 @@ __global__ __launch_bounds__(256) void k_ml_final(const double* __restrict__ l4,
       }
     }
   }
-  double o[2];
-  block_sum<2>(v, o);
-  if (threadIdx.x == 0) {
-    partials[((int64_t)blockIdx.x * rmax + R) * 2] = o[0];
-    partials[((int64_t)blockIdx.x * rmax + R) * 2 + 1] = o[1];
-  }
+  const double o = block_sum<2>(v);
+  if (threadIdx.x < 2) partials[((int64_t)blockIdx.x * rmax + R) * 2 + threadIdx.x] = o;
 }
 
 }  // namespace

@@ -218,15 +218,12 @@ __device__ __forceinline__ void phase_compute(Real* __restrict__ lat_base, const
 template <int MU, int KIND, bool MEAS>
 __device__ __forceinline__ void phase_finish(const PhaseArgs& a, uint32_t L, double (&v)[2], uint32_t acc_wave) {
   if (MEAS) {
-    double o[2];
-    block_sum<2>(v, o);
-    if (threadIdx.x == 0) {
-      const int c = MU == 3 ? 2 : 0;
-      double* row = a.meas + 4 * (size_t)L;
-      row[c] = o[0];
-      row[c + 1] = o[1];
+    const double o = block_sum<2>(v);
+    if (threadIdx.x < 2) {
+      const uint32_t c = MU == 3 ? 2 : 0;
+      double* row = a.meas + 4 * (size_t)L + threadIdx.x;
+      row[c] = o;
       row[2 - c] = 0.0;
-      row[3 - c] = 0.0;
     }
   }
   if (KIND == KIND_METROPOLIS && a.accepts && (threadIdx.x & 63) == 0 && acc_wave)

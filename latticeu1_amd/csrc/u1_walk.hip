@@ -156,10 +156,9 @@ __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real
     sg.template rest<KIND == KIND_OVERRELAX>(
         steps, [&] { return first[j1 == wa.len ? lane : threadIdx.x + (uint32_t)wa.width]; });
   if (MEAS) {
-    double o[4];
-    block_sum<4>(v, o);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < 4; ++k) a.meas[4 * ((size_t)(uint32_t)wa.row + (size_t)orbit * (uint32_t)wa.strips + strip) + k] = o[k];
+    const double o = block_sum<4>(v);
+    if (threadIdx.x < 4)
+      a.meas[4 * ((size_t)(uint32_t)wa.row + (size_t)orbit * (uint32_t)wa.strips + strip) + threadIdx.x] = o;
   }
   if (KIND == KIND_METROPOLIS && a.accepts && (threadIdx.x & 63) == 0 && acc)
     atomicAdd(a.accepts, (unsigned long long)acc);
