@@ -85,6 +85,11 @@ struct WalkZT {
   __host__ __device__ __forceinline__ uint32_t tdn(uint32_t x) const { return x == 0 ? Tlast : x - Tb; }
   // lane: in-plane site (below P); diagonal c, first step j
   __host__ __device__ __forceinline__ void init(const RepDesc& r, int32_t parity, uint32_t lane, int32_t c, int32_t j) {
+    init(r, parity, lane, c, j % r.N[2], (c + j) % r.N[3]);
+  }
+  // jz, jt: j modulo Nz, c + j modulo Nt
+  __host__ __device__ __forceinline__ void init(const RepDesc& r, int32_t parity, uint32_t lane, int32_t c, int32_t jz,
+                                                int32_t jt) {
     same = (uint32_t)(parity * r.HV) * S;
     opp = (uint32_t)((1 - parity) * r.HV) * S;
     Pb = (uint32_t)r.sz * S;
@@ -99,8 +104,8 @@ struct WalkZT {
     im[0] = i + (uint32_t)(xodd ? 0 : (xh == 0 ? r.nxh - 1 : -1)) * S;
     ip[1] = i + (uint32_t)((int32_t)y == r.N[1] - 1 ? -(r.N[1] - 1) * r.sy : r.sy) * S;
     im[1] = i + (uint32_t)(y == 0 ? (r.N[1] - 1) * r.sy : -r.sy) * S;
-    t = (c + j) % r.N[3];
-    const int32_t z = (r.N[2] - j % r.N[2]) % r.N[2];
+    t = jt;
+    const int32_t z = jz == 0 ? 0 : r.N[2] - jz;
     zb = (uint32_t)z * Pb;
     tb = (uint32_t)t * Tb;
   }
@@ -223,6 +228,7 @@ struct WalkArgs {
   int32_t gs, go;  // strips and diagonals of a group (rounded up)
   int32_t row;     // first measurement row (batched replicas)
   uint32_t gs_m, gs_s;
+  uint32_t nt_m, nt_s;  // magic division by Nt
 };
 // Batched replicas: workgroup b walks block map[b].y (walk_place, plain order)
 // of replica map[b].x; map[b].x = kWalkNone: empty.
@@ -256,6 +262,9 @@ inline WalkArgs walk_args(const RepDesc& r, int waves, int width, int sg) {
   const MagicDiv m = make_magic((uint32_t)w.gs);
   w.gs_m = m.m;
   w.gs_s = m.s;
+  const MagicDiv t = make_magic((uint32_t)r.N[3]);
+  w.nt_m = t.m;
+  w.nt_s = t.s;
   return w;
 }
 inline int walk_blocks(const WalkArgs& w) { return w.sg == 0 ? w.strips * w.orbits : 8 * w.gs * w.go; }
@@ -266,7 +275,7 @@ inline int walk_rows(const RepDesc& r, int width) {
 // Strip and diagonal of workgroup b; false if it is empty.
 __host__ __device__ __forceinline__ bool walk_place(const WalkArgs& w, uint32_t b, uint32_t* strip, uint32_t* orbit) {
   const uint32_t x = w.sg == 0 ? 0u : b & 7u, k = w.sg == 0 ? b : b >> 3;
-  const uint32_t gx = w.sg == 0 ? 0u : x & (uint32_t)(w.sg - 1), gy = w.sg == 0 ? 0u : x / (uint32_t)w.sg;
+  const uint32_t gx = w.sg == 0 ? 0u : x & (uint32_t)(w.sg - 1), gy = w.sg == 0 ? 0u : x >> __builtin_ctz((uint32_t)w.sg);
   const uint32_t q = mdiv(k, w.gs_m, w.gs_s), s = k - q * (uint32_t)w.gs;
   *strip = gx * (uint32_t)w.gs + s;
   *orbit = gy * (uint32_t)w.go + q;
