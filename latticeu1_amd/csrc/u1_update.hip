@@ -293,16 +293,58 @@ __global__ __launch_bounds__(512) void k_phase(Real* __restrict__ lat_base, Phas
 // PAIR_ANY (batched replicas with planes too large for k_pair_packed) decides
 // per workgroup between the last two; its descriptor is copied into registers
 // (see k_pair_packed).
+// The arguments before a (single lattices) are what the first loads depend on, as
+// many as the dispatcher writes into scalar registers by itself (fourteen, build
+// flag amdgpu-kernarg-preload-count): the kernel's first 0.4 us were the wait for
+// the cold argument lines.  packed: shifts of the four magic divisions by five
+// bits, parity, xcd, tile, ml.  Overrelaxation pair 5.67 -> 5.27 us and Metropolis
+// 8.54 -> 8.06 us at 24^3 x 48, 5.33 -> 4.94 and 7.54 -> 7.10 us at 28 x 20 x 36 x 22.
 enum { PAIR_ONE_STEP = 0, PAIR_SKEW = 1, PAIR_LOOP = 2, PAIR_ANY = 3 };
 template <typename Real, int KIND, int SPT, bool MEAS, bool BATCHED = false, int FORM = PAIR_ANY>
-__global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real* __restrict__ lat_base, PhaseArgs a) {
-  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs)>(blockIdx.x);
+__global__ __launch_bounds__(pair_max_block(sizeof(Real), SPT)) void k_pair(Real* __restrict__ lat_base, uint32_t N1,
+                                                                          uint32_t N2, uint32_t N3, uint32_t nxh,
+                                                                          uint32_t div_nxh_m, uint32_t div_nz_m,
+                                                                          uint32_t div_tile_m, uint32_t div_bz_m,
+                                                                          uint32_t packed, PhaseArgs a) {
+  const uint32_t block = BATCHED ? fetch_args<sizeof(Real*) + 32 + sizeof(PhaseArgs)>(blockIdx.x) : blockIdx.x;
   extern __shared__ __align__(8) unsigned char pair_lds[];
   Real* th0 = reinterpret_cast<Real*>(pair_lds);
-  const uint32_t L = a.xcd ? xcd_remap(block, gridDim.x) : block;
-  RepDesc rep;
-  if constexpr (BATCHED) rep = a.reps[a.blockmap[L]];
-  const RepDesc& r = BATCHED ? rep : a.single;
+  if constexpr (!BATCHED) {
+    a.parity = (int32_t)(packed >> 20 & 1u);
+    a.xcd = packed >> 21 & 1u;
+    a.ml = (int32_t)(packed >> 23 & 7u);
+  }
+  const uint32_t L = a.xcd ? xcd_remap(block, BATCHED ? gridDim.x : N2 * N3) : block;
+  RepDesc r;
+  if constexpr (BATCHED) {
+    r = a.reps[a.blockmap[L]];
+  } else {
+    r = a.single;
+    r.N[1] = (int32_t)N1;
+    r.N[2] = (int32_t)N2;
+    r.N[3] = (int32_t)N3;
+    r.nxh = r.sy = (int32_t)nxh;
+    r.sz = (int32_t)(nxh * N1);
+    r.st = (int32_t)(nxh * N1 * N2);
+    r.HV = (int32_t)(nxh * N1 * N2 * N3);
+    r.V = 2 * r.HV;
+    r.div_nxh_m = div_nxh_m;
+    r.div_nz_m = div_nz_m;
+    r.div_tile_m = div_tile_m;
+    r.div_bz_m = div_bz_m;
+    r.div_nxh_s = packed & 31u;
+    r.div_nz_s = packed >> 5 & 31u;
+    r.div_tile_s = packed >> 10 & 31u;
+    r.div_bz_s = packed >> 15 & 31u;
+    r.tile = packed >> 22 & 1u;
+    r.tile_bz = N2 >> 1;
+    r.tile_bt = N3 >> 2;
+    r.bpp = 1;
+    r.div_bpp_m = 1;  // division by 1
+    r.div_bpp_s = 0;
+    r.blk_begin = 0;
+    r.lat_off = 0;
+  }
   const uint32_t b = L - (uint32_t)r.blk_begin;  // the replica's plane (one chunk per plane)
   const uint32_t P = (uint32_t)r.nxh * (uint32_t)r.N[1];
   const uint32_t step = SPT * blockDim.x;
@@ -566,23 +608,30 @@ hipError_t launch_prec(int kind, int mu, Real* lat, const PhaseArgs& a, int nblo
 
 template <typename Real, int KIND, int SPT, bool MEAS>
 void launch_pair_form(int form, Real* lat, const PhaseArgs& a, int nblocks, int block, size_t lds, hipStream_t s) {
+  const RepDesc& r = a.single;
+  const uint32_t packed = r.div_nxh_s | r.div_nz_s << 5 | r.div_tile_s << 10 | r.div_bz_s << 15 |
+                          (uint32_t)a.parity << 20 | (a.xcd ? 1u : 0u) << 21 | (r.tile ? 1u : 0u) << 22 |
+                          (uint32_t)a.ml << 23;
   if constexpr (SPT <= 3)
     if (form == PAIR_ONE_STEP) {
-      k_pair<Real, KIND, SPT, MEAS, false, PAIR_ONE_STEP><<<nblocks, block, lds, s>>>(lat, a);
+      k_pair<Real, KIND, SPT, MEAS, false, PAIR_ONE_STEP><<<nblocks, block, lds, s>>>(lat, (uint32_t)r.N[1], (uint32_t)r.N[2], (uint32_t)r.N[3],
+                                                                      (uint32_t)r.nxh, r.div_nxh_m, r.div_nz_m, r.div_tile_m, r.div_bz_m, packed, a);
       return;
     }
   if constexpr (SPT == 1)
     if (form == PAIR_SKEW) {
-      k_pair<Real, KIND, SPT, MEAS, false, PAIR_SKEW><<<nblocks, block, lds, s>>>(lat, a);
+      k_pair<Real, KIND, SPT, MEAS, false, PAIR_SKEW><<<nblocks, block, lds, s>>>(lat, (uint32_t)r.N[1], (uint32_t)r.N[2], (uint32_t)r.N[3],
+                                                                      (uint32_t)r.nxh, r.div_nxh_m, r.div_nz_m, r.div_tile_m, r.div_bz_m, packed, a);
       return;
     }
-  k_pair<Real, KIND, SPT, MEAS, false, PAIR_LOOP><<<nblocks, block, lds, s>>>(lat, a);
+  k_pair<Real, KIND, SPT, MEAS, false, PAIR_LOOP><<<nblocks, block, lds, s>>>(lat, (uint32_t)r.N[1], (uint32_t)r.N[2], (uint32_t)r.N[3],
+                                                                      (uint32_t)r.nxh, r.div_nxh_m, r.div_nz_m, r.div_tile_m, r.div_bz_m, packed, a);
 }
 
 template <typename Real, int KIND, int SPT>
 hipError_t launch_pair_meas(Real* lat, const PhaseArgs& a, int nblocks, int block, size_t lds, hipStream_t s) {
   if (a.reps != nullptr) {  // batched replicas: no measuring pairs; the form per workgroup
-    k_pair<Real, KIND, SPT, false, true><<<nblocks, block, lds, s>>>(lat, a);
+    k_pair<Real, KIND, SPT, false, true><<<nblocks, block, lds, s>>>(lat, 0, 0, 0, 0, 0, 0, 0, 0, 0, a);
     return hipGetLastError();
   }
   // a single lattice: its plane and row size fix the form
