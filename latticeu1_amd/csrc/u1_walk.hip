@@ -4,8 +4,6 @@
 // for bit.
 #include "u1_walk.h"
 
-#include <type_traits>
-
 #include "u1_link.h"
 
 namespace u1d {
@@ -92,28 +90,67 @@ enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
 // descriptor, copied into registers before the first store.  64 replicas of
 // 8^4 to 24^3 x 32 (11.7 M sites), binary32: overrelaxation 44 us against
 // 63 us for the two phase launches, Metropolis 82 us against 91 us.
+// The arguments before a (single lattices) are the fourteen words that the
+// dispatcher writes into scalar registers, as for k_pair: what a walk needs before
+// its first load.  packed: shifts of the four magic divisions by five bits, parity,
+// log2 of width and sg, plain order.  Binary32 at 24^3 x 48: overrelaxation 6.07 ->
+// 5.84 us, Metropolis 9.35 -> 9.19; binary64 at 24^3 x 12: overrelaxation 6.3 -> 6.1.
 template <typename Real, int KIND, int MODE, bool UNIFORM, bool BATCHED = false>
-__global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(Real* __restrict__ lat_base, PhaseArgs a,
-                                                                           std::conditional_t<BATCHED, WalkBatch, WalkArgs> w) {
-  const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(w)>(blockIdx.x);
+__global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(
+    Real* __restrict__ lat_base, uint32_t N1, uint32_t N2, uint32_t N3, uint32_t nxh, uint32_t div_nxh_m,
+    uint32_t div_nz_m, uint32_t div_nt_m, uint32_t gs_m, uint32_t orbits, uint32_t len, uint32_t seg_len,
+    uint32_t packed, PhaseArgs a, WalkBatch w) {
+  // binary64 Metropolis is short of scalar registers and reads its other arguments
+  // again and again: all lines at once (8.0 us at 24^3 x 12, 8.6 without)
+  constexpr bool FETCH = BATCHED || (sizeof(Real) == 8 && KIND == KIND_METROPOLIS);
+  const uint32_t block =
+      FETCH ? fetch_args<sizeof(Real*) + 48 + sizeof(PhaseArgs) + sizeof(WalkBatch)>(blockIdx.x) : blockIdx.x;
   using Walk = WalkZT<sizeof(Real), UNIFORM>;
   constexpr int A = Walk::A, B = Walk::B, C = Walk::C, D = Walk::D;
   constexpr bool MEAS = MODE == WALK_MEAS;
   __shared__ Real first[64 * walk_max_waves(sizeof(Real))];
   uint32_t strip, orbit;
-  RepDesc rep;
+  RepDesc r;
   WalkArgs wa;
   if constexpr (BATCHED) {
     const WalkBlock e = w.map[block];
     if (e.x == kWalkNone) return;
-    rep = a.reps[e.x];
+    r = a.reps[e.x];
     wa = w.args[e.x];
     (void)walk_place(wa, e.y, &strip, &orbit);  // never empty in plain order
   } else {
-    wa = w;
+    a.parity = (int32_t)(packed >> 20 & 1u);
+    r = a.single;
+    r.N[1] = (int32_t)N1;
+    r.N[2] = (int32_t)N2;
+    r.N[3] = (int32_t)N3;
+    r.nxh = r.sy = (int32_t)nxh;
+    r.sz = (int32_t)(nxh * N1);
+    r.st = (int32_t)(nxh * N1 * N2);
+    r.HV = (int32_t)(nxh * N1 * N2 * N3);
+    r.V = 2 * r.HV;
+    r.lat_off = 0;
+    r.div_nxh_m = div_nxh_m;
+    r.div_nxh_s = packed & 31u;
+    r.div_nz_m = div_nz_m;
+    r.div_nz_s = packed >> 5 & 31u;
+    const uint32_t wlog = packed >> 21 & 7u, sglog = packed >> 24 & 3u;
+    const bool plain = (packed >> 26 & 1u) != 0;
+    wa.nt_m = div_nt_m;
+    wa.nt_s = packed >> 10 & 31u;
+    wa.gs_m = gs_m;
+    wa.gs_s = packed >> 15 & 31u;
+    wa.orbits = (int32_t)orbits;
+    wa.len = (int32_t)len;
+    wa.seg = (int32_t)seg_len;
+    wa.width = 1 << wlog;
+    wa.strips = (int32_t)(((uint32_t)r.sz + (uint32_t)wa.width - 1u) >> wlog);
+    wa.sg = plain ? 0 : 1 << sglog;
+    wa.gs = plain ? wa.strips : (int32_t)(((uint32_t)wa.strips + (uint32_t)wa.sg - 1u) >> sglog);
+    wa.go = plain ? wa.orbits : (int32_t)((orbits + (8u >> sglog) - 1u) >> (3u - sglog));
+    wa.row = 0;
     if (!walk_place(wa, block, &strip, &orbit)) return;
   }
-  const RepDesc& r = BATCHED ? rep : a.single;
   // segment of this lane, and its place in the strip
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t seg = UNIFORM ? wave : threadIdx.x >> __builtin_ctz((uint32_t)wa.width);
@@ -173,9 +210,9 @@ template <typename Real, int KIND, int MODE>
 hipError_t launch_walk_batch_width(Real* lat, const PhaseArgs& a, const WalkBatch& w, int nblk, int block, int width,
                                    hipStream_t s) {
   if (width == 64)
-    k_walk<Real, KIND, MODE, true, true><<<nblk, block, 0, s>>>(lat, a, w);
+    k_walk<Real, KIND, MODE, true, true><<<nblk, block, 0, s>>>(lat, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, a, w);
   else
-    k_walk<Real, KIND, MODE, false, true><<<nblk, block, 0, s>>>(lat, a, w);
+    k_walk<Real, KIND, MODE, false, true><<<nblk, block, 0, s>>>(lat, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, a, w);
   return hipGetLastError();
 }
 template <typename Real, int KIND>
@@ -193,10 +230,14 @@ hipError_t launch_walk_batch_prec(int kind, Real* lat, const PhaseArgs& a, const
 
 template <typename Real, int KIND, int MODE>
 hipError_t launch_walk_width(Real* lat, const PhaseArgs& a, const WalkArgs& w, int block, hipStream_t s) {
-  if (w.width == 64)
-    k_walk<Real, KIND, MODE, true><<<walk_blocks(w), block, 0, s>>>(lat, a, w);
-  else
-    k_walk<Real, KIND, MODE, false><<<walk_blocks(w), block, 0, s>>>(lat, a, w);
+  const RepDesc& r = a.single;
+  auto* k = w.width == 64 ? k_walk<Real, KIND, MODE, true, false> : k_walk<Real, KIND, MODE, false, false>;
+  const uint32_t packed = r.div_nxh_s | r.div_nz_s << 5 | w.nt_s << 10 | w.gs_s << 15 | (uint32_t)a.parity << 20 |
+                          (uint32_t)__builtin_ctz((uint32_t)w.width) << 21 |
+                          (w.sg ? (uint32_t)__builtin_ctz((uint32_t)w.sg) << 24 : 1u << 26);
+  k<<<walk_blocks(w), block, 0, s>>>(lat, (uint32_t)r.N[1], (uint32_t)r.N[2], (uint32_t)r.N[3], (uint32_t)r.nxh,
+                                     r.div_nxh_m, r.div_nz_m, w.nt_m, w.gs_m, (uint32_t)w.orbits, (uint32_t)w.len,
+                                     (uint32_t)w.seg, packed, a, WalkBatch{});
   return hipGetLastError();
 }
 
