@@ -35,11 +35,12 @@
 // reported, not hung on.
 //
 // Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
-// overrelaxation passes, against the tuned launches: binary64 8^4 75 us against
-// 82, 12^3 x 8 86 against 95; binary32 8^4 39 us against 51, 12^3 x 16 52
-// against 67, 16^3 x 8 52 against 55.  With more sites one XCD's arithmetic
-// takes over (binary64 12^3 x 16: 113 us against 97; binary32 16^4: 84 against
-// 56).
+// overrelaxation passes, against the tuned launches: binary64 8^4 71 us against
+// 81, 12^3 x 8 82 against 95; binary32 8^4 37 us against 50, 12^3 x 16 51
+// against 67, 16^3 x 8 50 against 55.  With more sites one XCD's arithmetic
+// takes over (binary64 12^3 x 16: 115 us against 99; binary32 16^4: 84 against
+// 56).  Level-2 sweeps, every slab by itself: binary32 24^4 59 us against 80,
+// binary64 134 against 167.
 #include "u1_kernels.h"
 #include "u1_link.h"
 
