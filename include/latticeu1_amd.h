@@ -243,7 +243,12 @@ int u1_set_pair_fusion(int32_t mode);
  * decision as "MetropolisChain" / "OverRelaxationChain" entries (block.x 0 =
  * unfused).  A dependency wait that times out (bounded, about 0.1 s) is
  * reported as U1_ERR_HIP by the next call that synchronises the library
- * stream (u1_sync, or any call returning results to the host). */
+ * stream (u1_sync, or any call returning results to the host).
+ * With this mode and the pair fusion both at 1, whole sweeps of small lattices
+ * (Nx Ny Nz Nt <= 2^15), and with a multilevel mask of every slab between frozen
+ * slices, can also run as one launch on one XCD each, where the tuner measures it
+ * faster: the same results, "Sweep<metrop>+<ovrn>[Mask<ml>]" entries, a bounded
+ * wait of several seconds reported in the same way. */
 int u1_set_pass_fusion(int32_t mode);
 /* Multilevel level-2 steps (u1_multilevel): replayed from one captured
  * hipGraph (on = 1, default) or enqueued eagerly (0).  The same kernels read

@@ -48,8 +48,10 @@ namespace u1d {
 
 namespace {
 
-// Polls before a wait gives up: with the poll's round trip about a second.
-constexpr uint32_t kDieSpin = 1u << 22;
+// Polls before a wait gives up: with the poll's round trip several seconds, since
+// other work on the card may hold the CUs that the rest of a barrier's workgroups
+// wait for.
+constexpr uint32_t kDieSpin = 1u << 24;
 
 struct DieSync {
   uint32_t* ctl;  // DIE_WORDS
