@@ -14,7 +14,7 @@
 // XCD, and unless all report the same one, stores and counters go to device
 // scope.
 //
-// Barrier and order.  A phase's workgroup first waits for its stores, then
+// Barrier and order (control words: u1_die_sync.h).  A phase's workgroup first waits for its stores, then
 // counts itself; the next phase's loads of angles that the phase before wrote
 // come after the counter is complete.  All angle loads pass the L1 (device
 // scope; on one XCD the L2 serves them).  Of its eighteen staple angles a phase
@@ -48,70 +48,45 @@ namespace u1d {
 
 namespace {
 
-// Polls before a wait gives up: with the poll's round trip several seconds, since
-// other work on the card may hold the CUs that the rest of a barrier's workgroups
-// wait for.
-constexpr uint32_t kDieSpin = 1u << 24;
-
-struct DieSync {
-  uint32_t* ctl;  // DIE_WORDS
+// The accesses of DieSync: thread 0's relaxed atomics in device memory.
+struct DieMem {
+  // Polls before a wait gives up: with the poll's round trip several seconds, since
+  // other work on the card may hold the CUs that the rest of a barrier's workgroups
+  // wait for.
+  static constexpr uint32_t kSpin = 1u << 24;
+  uint32_t* ctl;  // DIE_CTL words
   uint32_t* err;
-  uint32_t n;       // workgroups
-  uint32_t target;  // arrivals that complete the last barrier
-  bool one;         // all on one XCD
-  bool dead;        // a wait timed out: no more waiting
 
-  __device__ __forceinline__ uint32_t poll(int word) const {
-    return __hip_atomic_load(ctl + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __device__ __forceinline__ void until(int word, uint32_t want) {
-    if (threadIdx.x == 0)
-      for (uint32_t k = 0; !dead && poll(word) < want; ++k) {
-        if (k == kDieSpin) {
-          dead = true;
-          __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
+  __device__ __forceinline__ bool leader() const { return threadIdx.x == 0; }
+  __device__ __forceinline__ void barrier() const {
     __syncthreads();
     asm volatile("" ::: "memory");
   }
-  __device__ __forceinline__ void start() {
-    if (threadIdx.x == 0) {
-      const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11));  // XCC_ID
-      __hip_atomic_fetch_or(ctl + DIE_XCDS, 1u << xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __hip_atomic_fetch_add(ctl + DIE_HERE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    target = 0;
-    one = false;
-    dead = false;
+  __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+  __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
+  __device__ __forceinline__ uint32_t xcd() const { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }  // XCC_ID
+  __device__ __forceinline__ uint32_t uniform(uint32_t v) const { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+  __device__ __forceinline__ uint32_t load(int word) const {
+    return __hip_atomic_load(ctl + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  // before the first store
-  __device__ __forceinline__ void started() {
-    until(DIE_HERE, n);
-    const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)poll(DIE_XCDS));
-    one = (m & (m - 1)) == 0;
+  __device__ __forceinline__ void store(int word, uint32_t v) const {
+    __hip_atomic_store(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  // this workgroup's stores are visible to the others
-  __device__ __forceinline__ void arrive() {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    target += n;
-    if (threadIdx.x == 0) {
-      if (one)
-        __hip_atomic_fetch_add(ctl + DIE_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      else
-        __hip_atomic_fetch_add(ctl + DIE_DONE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+  __device__ __forceinline__ void set_bits(int word, uint32_t v) const {
+    __hip_atomic_fetch_or(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __device__ __forceinline__ void wait() { until(DIE_DONE, target); }
-  // the last workgroup to leave clears the words for the next launch
-  __device__ __forceinline__ void leave() {
-    if (threadIdx.x != 0) return;
-    if (__hip_atomic_fetch_add(ctl + DIE_LEFT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != n) return;
-    for (int w : {DIE_HERE, DIE_XCDS, DIE_DONE, DIE_LEFT})
-      __hip_atomic_store(ctl + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // local: counted and read on one XCD only
+  __device__ __forceinline__ void add(int word, uint32_t v, bool local) const {
+    if (local)
+      __hip_atomic_fetch_add(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+      __hip_atomic_fetch_add(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ uint32_t fetch_add(int word, uint32_t v) const {
+    return __hip_atomic_fetch_add(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ void timed_out() const {
+    __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 };
 
@@ -164,7 +139,7 @@ struct DieSites {
 // One body per MU for all passes and sites: the kernel runs each of them a few
 // times only, and its instructions are cold in every cache when it begins.
 template <typename Real, int MU, bool MEAS>
-__device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArgs& a, const RepDesc& r, DieSync& sync,
+__device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArgs& a, const RepDesc& r, DieSync<DieMem>& sync,
                                           const DieSites& own, uint32_t& acc, double (&v)[4], const DieStep& step) {
   const uint32_t first = own.first, stride = own.stride;
   const uint32_t n = MU == 3 ? own.n3 : own.n, base = MU == 3 ? own.base3 : own.base;
@@ -223,7 +198,7 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
   const uint32_t slab = 8u * row + (block & 7u);
   if (slab >= d.slabs) return;
   Real* lat = lat_base + r.lat_off;
-  DieSync sync{d.ctl + slab * DIE_CTL, d.err, d.groups, 0, false, false};
+  DieSync<DieMem> sync{{d.ctl + slab * DIE_CTL, d.err}, d.groups, 0, false, false};
   sync.start();
   const uint32_t half = (uint32_t)r.st;  // even/odd sites of a slice
   const uint32_t t0 = slab * (uint32_t)a.ml, nt = a.ml ? min((uint32_t)a.ml, (uint32_t)r.N[3] - t0) : (uint32_t)r.N[3];

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "u1_device.h"
+#include "u1_die_sync.h"
 #include "u1_walk.h"
 
 namespace u1d {
@@ -102,7 +103,6 @@ hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseAr
 // zero between launches.  A wait that times out sets *err (host-visible memory).
 // a.meas (no mask): the plaquette of the updated lattice, times scale, to
 // out[4]; a.meas holds 4 doubles per workgroup.
-enum { DIE_HERE = 0, DIE_XCDS = 32, DIE_DONE = 64, DIE_LEFT = 96, DIE_CTL = 128 };
 constexpr int kDieGroups = 32;
 constexpr int die_max_block(int elem_bytes) { return elem_bytes == 8 ? 512 : 1024; }
 struct DieArgs {
