@@ -248,7 +248,9 @@ int u1_set_pair_fusion(int32_t mode);
  * (Nx Ny Nz Nt <= 2^15), and with a multilevel mask of every slab between frozen
  * slices, can also run as one launch on one XCD each, where the tuner measures it
  * faster: the same results, "Sweep<metrop>+<ovrn>[Mask<ml>]" entries, a bounded
- * wait of several seconds reported in the same way. */
+ * wait of several seconds reported in the same way.  Its workgroups must be on the
+ * card together; if other work keeps some of them out for about a millisecond, one
+ * of them does the sweep alone: the same results, at a fraction of the speed. */
 int u1_set_pass_fusion(int32_t mode);
 /* Multilevel level-2 steps (u1_multilevel): replayed from one captured
  * hipGraph (on = 1, default) or enqueued eagerly (0).  The same kernels read
@@ -301,6 +303,15 @@ int u1_bench_updates(const u1_geom* g, int prec, void* lat, int32_t metrop, int3
 int u1_selftest_math(int32_t fn, const double* x, const double* y, double* out, int64_t n);
 /* Philox4x32-10 on the device: ctr[4n], key[2n] -> out[4n] (host arrays). */
 int u1_selftest_philox(const uint32_t* ctr, const uint32_t* key, uint32_t* out, int64_t n);
+/* u1_update (stream U1_STREAM_UPDATE, c3 0) as one launch in workgroups of
+ * `block` threads (64 to 512, binary32 1024, in steps of 64), whatever the tuner
+ * and u1_set_pass_fusion say, and synchronised.  flags 1: the first workgroup to
+ * look does the whole sweep instead of waiting for the others to begin.  accepts
+ * (nullable): as u1_update; plaq (nullable, 4 doubles, mask_ml 0): as
+ * u1_update_plaquette.  U1_ERR_ARG for lattices too large for one launch. */
+int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int32_t ovrn, const u1_metro* m,
+                      uint64_t seed, uint32_t sweep, int32_t mask_ml, int32_t block, int32_t flags, uint64_t* accepts,
+                      double* plaq);
 /* Streaming reference for the roofline (no counterpart in the reference):
  * moves the bytes of one (parity, mu) phase, 36 n (4.5 floats per each of n
  * updated links), with an ideal access pattern and returns the rate in GB/s

@@ -82,6 +82,8 @@ _SIGS = {
                  C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int32),
     "u1_selftest_math": (C.c_int32, C.POINTER(C.c_double), C.POINTER(C.c_double), C.POINTER(C.c_double), C.c_int64),
     "u1_selftest_philox": (C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.c_int64),
+    "u1_selftest_sweep": (C.POINTER(Geom), C.c_int, _P, C.c_int32, C.c_int32, C.POINTER(Metro), C.c_uint64, C.c_uint32,
+                          C.c_int32, C.c_int32, C.c_int32, C.POINTER(C.c_uint64), C.POINTER(C.c_double)),
     "u1_selftest_stream": (C.c_int32, C.c_int64, C.c_int32, C.POINTER(C.c_double)),
     "u1_plaquette": (C.POINTER(Geom), C.c_int, _P, C.POINTER(C.c_double)),
     "u1_plaquette_noalloc": (C.POINTER(Geom), C.c_int, _P, _P),
@@ -460,6 +462,15 @@ def selftest_philox(ctr: np.ndarray, key: np.ndarray) -> np.ndarray:
     call("u1_selftest_philox", ctr.ctypes.data_as(u32), key.ctypes.data_as(u32), out.ctypes.data_as(u32),
          ctr.shape[0])
     return out
+
+
+def selftest_sweep(lat: "Lattice", metrop: int, ovrn: int, m: Metro, seed: int, sweep: int, block: int, flags: int = 0,
+                   mask_ml: int = 0, plaquette: bool = False):
+    """update() as one launch in a given shape (see u1_selftest_sweep): accepts and, without mask, the plaquette."""
+    acc, out = C.c_uint64(0), np.zeros(4)
+    call("u1_selftest_sweep", C.byref(lat.g), lat.prec, lat.buf.ptr, metrop, ovrn, C.byref(m), seed, sweep, mask_ml,
+         block, flags, C.byref(acc), _dp(out) if plaquette else None)
+    return (int(acc.value), out) if plaquette else int(acc.value)
 
 
 def set_verbosity(level: int) -> None:

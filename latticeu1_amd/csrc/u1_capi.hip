@@ -1007,7 +1007,8 @@ int die_prepare() {
   return U1_OK;
 }
 
-int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, const Cfg& c, double* meas_dst) {
+int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, const Cfg& c, double* meas_dst,
+               uint32_t patience = u1d::kDiePatience) {
   RET(die_prepare());
   u1d::DieArgs d{};
   void* err_dev = nullptr;
@@ -1018,6 +1019,7 @@ int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, co
   d.groups = die_groups(a.single, a.ml, c);
   d.metrop = metrop;
   d.ovrn = ovrn;
+  d.patience = patience;
   PhaseArgs b = a;
   b.meas = nullptr;
   if (meas_dst) {
@@ -2864,6 +2866,40 @@ int u1_selftest_math(int32_t fn, const double* x, const double* y, double* out, 
   HIPCHK(u1d::launch_selftest_math(fn, dx.as<double>(), dy.as<double>(), dout.as<double>(), n, G.st));
   HIPCHK(hipMemcpyAsync(out, dout.p, nout * n * sizeof(double), hipMemcpyDeviceToHost, G.st));
   HIPCHK(hipStreamSynchronize(G.st));
+  return U1_OK;
+}
+
+int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int32_t ovrn, const u1_metro* m,
+                      uint64_t seed, uint32_t sweep, int32_t mask_ml, int32_t block, int32_t flags, uint64_t* accepts,
+                      double* plaq) {
+  REQ_INIT();
+  REQ_PTR(lat);
+  RET(check_geom(g));
+  RET(check_prec(prec));
+  RET(check_metro(m));
+  if (metrop < 0 || ovrn < 0 || metrop > 4095 || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
+  if (mask_ml != 0 && mask_ml != 2 && mask_ml != 4) return fail(U1_ERR_ARG, "mask_ml must be 0, 2 or 4");
+  if (flags < 0 || flags > 1 || (plaq && mask_ml != 0)) return fail(U1_ERR_ARG, "bad self-test arguments");
+  PhaseArgs a{};
+  a.single = make_rep(g, seed, 0);
+  a.ml = mask_ml;
+  a.proposal = m->proposal;
+  a.nhit = m->nhit;
+  a.step = m->step;
+  a.stream = U1_STREAM_UPDATE;
+  a.sweep = sweep;
+  if (!die_possible(a.single, mask_ml) || block < 64 || block > u1d::die_max_block((int)elem_size(prec)) || block % 64)
+    return fail(U1_ERR_ARG, "not a one-launch sweep");
+  if (accepts) HIPCHK(u1d::launch_fill_zero(G.counter, sizeof(unsigned long long), G.st));
+  a.accepts = accepts ? G.counter : nullptr;
+  RET(die_launch(prec, lat, a, metrop, ovrn, Cfg{block, 1, 0, 0}, plaq ? G.dres_dev : nullptr,
+                 flags & 1 ? 0u : u1d::kDiePatience));
+  unsigned long long v = 0;
+  if (accepts) HIPCHK(hipMemcpyAsync(&v, G.counter, sizeof(v), hipMemcpyDeviceToHost, G.st));
+  if (plaq) RET(take_results(plaq, 4));
+  HIPCHK(hipStreamSynchronize(G.st));
+  RET(chain_check());
+  if (accepts) *accepts += v;
   return U1_OK;
 }
 

@@ -31,7 +31,8 @@
 // number, and slabs on one XCD share its CUs.
 //
 // All workgroups of a barrier must be resident at once: an XCD is given at most
-// 32, one per CU.  The waits are bounded all the same, and a timeout is
+// 32, one per CU, and if other work keeps some of them out, one does the sweep
+// alone (u1_die_sync.h).  The waits are bounded all the same, and a timeout is
 // reported, not hung on.
 //
 // Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
@@ -50,18 +51,17 @@ namespace {
 
 // The accesses of DieSync: thread 0's relaxed atomics in device memory.
 struct DieMem {
-  // Polls before a wait gives up: with the poll's round trip several seconds, since
-  // other work on the card may hold the CUs that the rest of a barrier's workgroups
-  // wait for.
-  static constexpr uint32_t kSpin = 1u << 24;
+  static constexpr uint32_t kSpin = 1u << 24;  // polls before a wait gives up: several seconds
   uint32_t* ctl;  // DIE_CTL words
   uint32_t* err;
+  uint32_t polls;  // for the others to begin (DieArgs::patience)
 
   __device__ __forceinline__ bool leader() const { return threadIdx.x == 0; }
   __device__ __forceinline__ void barrier() const {
     __syncthreads();
     asm volatile("" ::: "memory");
   }
+  __device__ __forceinline__ uint32_t patience() const { return polls; }
   __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
   __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
   __device__ __forceinline__ uint32_t xcd() const { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }  // XCC_ID
@@ -84,6 +84,11 @@ struct DieMem {
   }
   __device__ __forceinline__ uint32_t fetch_add(int word, uint32_t v) const {
     return __hip_atomic_fetch_add(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ uint32_t cas(int word, uint32_t want, uint32_t v) const {
+    __hip_atomic_compare_exchange_strong(ctl + word, &want, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    return want;  // what was there
   }
   __device__ __forceinline__ void timed_out() const {
     __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -124,7 +129,6 @@ struct DieLoad {
 // What changes from phase to phase, apart from MU.
 struct DieStep {
   int kind;
-  bool begin;  // the sweep's first phase
   bool meas;   // the last pass's parity 1
 };
 
@@ -162,12 +166,7 @@ __device__ __forceinline__ void die_phase(Real* __restrict__ lat, const PhaseArg
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       if (j != LATE) term[j] = staple_term(in, j);
-    if (i == first) {
-      if (step.begin)
-        sync.started();
-      else
-        sync.wait();
-    }
+    if (i == first) sync.wait();
     load.template dir<false, true>(in, LATE);
     term[LATE] = staple_term(in, LATE);
     PlaqPieces<Real> pp = {0, 0, 0, 0};
@@ -198,13 +197,24 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
   const uint32_t slab = 8u * row + (block & 7u);
   if (slab >= d.slabs) return;
   Real* lat = lat_base + r.lat_off;
-  DieSync<DieMem> sync{{d.ctl + slab * DIE_CTL, d.err}, d.groups, 0, false, false};
+  DieSync<DieMem> sync{{d.ctl + slab * DIE_CTL, d.err, d.patience}, d.groups, wg, d.groups, 0, false, false};
   sync.start();
   const uint32_t half = (uint32_t)r.st;  // even/odd sites of a slice
   const uint32_t t0 = slab * (uint32_t)a.ml, nt = a.ml ? min((uint32_t)a.ml, (uint32_t)r.N[3] - t0) : (uint32_t)r.N[3];
   const uint32_t frozen = a.ml ? 1u : 0u;
-  const DieSites own = {(t0 + frozen) * half,          (nt - frozen) * half, t0 * half, nt * half,
-                        ((threadIdx.x >> 6) * d.groups + wg) * 64u + (threadIdx.x & 63u), d.groups * blockDim.x};
+  DieSites own = {(t0 + frozen) * half, (nt - frozen) * half, t0 * half, nt * half,
+                  ((threadIdx.x >> 6) * d.groups + wg) * 64u + (threadIdx.x & 63u), d.groups * blockDim.x};
+  // (in front of the first phase and not, as the other waits, behind its loads: the
+  // choice there cost every phase registers, 102 us at 8^4 instead of 97)
+  sync.started();
+  if (sync.n == 0) {
+    sync.leave();
+    return;
+  }
+  if (sync.n != sync.all) {  // alone: all sites
+    own.first = threadIdx.x;
+    own.stride = blockDim.x;
+  }
   uint32_t acc = 0;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   // (pass, parity) by (pass, parity)
@@ -214,9 +224,8 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
     const bool metro = h < 2 * d.metrop;
     a.pass = (uint32_t)((metro ? h : h - 2 * d.metrop) >> 1);
     a.parity = h & 1;
-    DieStep step = {metro ? KIND_METROPOLIS : KIND_OVERRELAX, h == 0, h == halves - 1};
+    const DieStep step = {metro ? KIND_METROPOLIS : KIND_OVERRELAX, h == halves - 1};
     die_phase<Real, 0, MEAS>(lat, a, r, sync, own, acc, v, step);
-    step.begin = false;
     die_phase<Real, 1, MEAS>(lat, a, r, sync, own, acc, v, step);
     die_phase<Real, 2, MEAS>(lat, a, r, sync, own, acc, v, step);
     die_phase<Real, 3, MEAS>(lat, a, r, sync, own, acc, v, step);
@@ -225,9 +234,9 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
   if (MEAS) {
     // one row per workgroup, folded in their order by the first
     const double o = block_sum<4>(v);
-    if (threadIdx.x < 4) stc(a.meas, 4 * wg + threadIdx.x, o);
+    if (threadIdx.x < 4) stc(a.meas, 4 * sync.wg + threadIdx.x, o);
     sync.arrive();
-    if (wg == 0) {
+    if (sync.wg == 0) {
       sync.wait();
       if (threadIdx.x < 4) {
         double s = 0.0;

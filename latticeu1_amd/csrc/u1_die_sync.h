@@ -14,43 +14,61 @@
 namespace u1d {
 
 // Words of a set of control words, each on a cache line of its own; all zero
-// between launches.
+// between launches.  DIE_HERE: workgroups that have begun, and from bit 16 on one
+// more than the number of the one that goes on alone, if any.
 enum { DIE_HERE = 0, DIE_XCDS = 32, DIE_DONE = 64, DIE_LEFT = 96, DIE_CTL = 128 };
 
+// Progress.  Workgroups may only wait for others that are resident, and other
+// work on the card -- a one-launch sweep of another process, whose workgroups
+// wait too -- may keep some from becoming so.  So the first wait, before the
+// first store, is for all of them to have begun, and one that has waited long
+// enough takes the whole sweep for itself: either the last arrival or its mark
+// comes first on DIE_HERE, and every workgroup, whenever it begins, reads which.
+// Later waits are for workgroups that have begun.
 template <typename Mem>
 struct DieSync {
   Mem mem;
-  uint32_t n;       // workgroups
+  uint32_t all;     // workgroups of the launch
+  uint32_t wg;      // this one
+  uint32_t n;       // workgroups that share the sweep: all, or one
   uint32_t target;  // arrivals that complete the last barrier
   bool one;         // all on one XCD
   bool dead;        // a wait timed out: no more waiting
 
-  __host__ __device__ __forceinline__ void until(int word, uint32_t want) {
-    if (mem.leader())
-      for (uint32_t k = 0; !dead && mem.load(word) < want; ++k) {
-        if (k == Mem::kSpin) {
-          dead = true;
-          mem.timed_out();
-        }
-        mem.pause();
-      }
-    mem.barrier();
-  }
   __host__ __device__ __forceinline__ void start() {
     if (mem.leader()) {
       mem.set_bits(DIE_XCDS, 1u << mem.xcd());
       mem.drain();
       mem.add(DIE_HERE, 1u, false);
     }
+    n = all;
     target = 0;
     one = false;
     dead = false;
   }
-  // before the first store
+  // Before the first store.  n then is all, or 1 if this workgroup goes on alone
+  // (as number 0), or 0 if another one does.
   __host__ __device__ __forceinline__ void started() {
-    until(DIE_HERE, n);
-    const uint32_t m = mem.uniform(mem.load(DIE_XCDS));
+    if (mem.leader()) {
+      uint32_t v = mem.load(DIE_HERE);
+      for (uint32_t k = 0; v < all; ++k) {
+        if (k >= mem.patience()) {
+          const uint32_t mark = v | (wg + 1u) << 16, old = mem.cas(DIE_HERE, v, mark);
+          v = old == v ? mark : old;
+        } else {
+          mem.pause();
+          v = mem.load(DIE_HERE);
+        }
+      }
+    }
+    mem.barrier();
+    const uint32_t v = mem.uniform(mem.load(DIE_HERE)), m = mem.uniform(mem.load(DIE_XCDS));
     one = (m & (m - 1)) == 0;
+    if (v >> 16) {
+      n = v >> 16 == wg + 1u ? 1u : 0u;
+      wg = 0;
+      one = true;
+    }
   }
   // this workgroup's stores are visible to the others
   __host__ __device__ __forceinline__ void arrive() {
@@ -59,7 +77,17 @@ struct DieSync {
     target += n;
     if (mem.leader()) mem.add(DIE_DONE, 1u, one);
   }
-  __host__ __device__ __forceinline__ void wait() { until(DIE_DONE, target); }
+  __host__ __device__ __forceinline__ void wait() {
+    if (mem.leader())
+      for (uint32_t k = 0; !dead && mem.load(DIE_DONE) < target; ++k) {
+        if (k == Mem::kSpin) {
+          dead = true;
+          mem.timed_out();
+        }
+        mem.pause();
+      }
+    mem.barrier();
+  }
   // The last workgroup to leave clears the words for the next launch.  Each
   // counts itself only when its last arrival has completed: one still in flight
   // would land on the cleared word, and the next launch's barriers would all
@@ -67,7 +95,7 @@ struct DieSync {
   __host__ __device__ __forceinline__ void leave() {
     if (!mem.leader()) return;
     mem.drain();
-    if (mem.fetch_add(DIE_LEFT, 1u) + 1 != n) return;
+    if (mem.fetch_add(DIE_LEFT, 1u) + 1 != all) return;
     for (int w : {DIE_HERE, DIE_XCDS, DIE_DONE, DIE_LEFT}) mem.store(w, 0u);
   }
 };

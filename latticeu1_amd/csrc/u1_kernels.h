@@ -101,7 +101,8 @@ hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseAr
 // threads per slab (die_slabs; 1 without mask), slab s on XCD s % 8 and at most
 // kDieGroups workgroups on an XCD; any extents.  ctl: DIE_CTL words per slab,
 // zero between launches.  A wait that times out sets *err (host-visible memory).
-// a.meas (no mask): the plaquette of the updated lattice, times scale, to
+// patience: polls for all of a slab's workgroups to begin, after which one of them
+// does its sweep alone.  a.meas (no mask): the plaquette of the updated lattice, times scale, to
 // out[4]; a.meas holds 4 doubles per workgroup.
 constexpr int kDieGroups = 32;
 constexpr int die_max_block(int elem_bytes) { return elem_bytes == 8 ? 512 : 1024; }
@@ -112,7 +113,10 @@ struct DieArgs {
   double scale;
   int32_t metrop, ovrn;
   uint32_t slabs, groups;
+  uint32_t patience;
 };
+// About a millisecond, what a sweep by one workgroup takes.
+constexpr uint32_t kDiePatience = 1u << 10;
 inline uint32_t die_slabs(int ml, int nt) { return ml ? (uint32_t)((nt + ml - 1) / ml) : 1u; }
 inline uint32_t die_rows(uint32_t slabs) { return (slabs + 7u) / 8u; }  // slabs on an XCD
 hipError_t launch_die(int prec, void* lat, const PhaseArgs& a, const DieArgs& d, int block, hipStream_t s);

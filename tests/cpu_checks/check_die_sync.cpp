@@ -3,7 +3,9 @@
 // every store and addition completed at a random later moment, in any order
 // that the workgroup's drain() calls allow.  Launches follow each other on the
 // same words.  At every barrier a workgroup must find what the others stored in
-// the phase before, and after a launch every word must be zero again.
+// the phase before, and after a launch every word must be zero again.  In some
+// launches only a few of the workgroups can be resident at a time: the sweep must
+// get done all the same, by one of them.
 #include <ucontext.h>
 
 #include <cstdio>
@@ -28,10 +30,11 @@ struct Fiber {
 };
 struct Op {
   int fiber;
-  enum { ADD, OR, STORE, DATA } kind;
+  enum { ADD, OR, CAS, STORE, DATA } kind;
   int word;
   uint32_t v;
-  uint32_t* got;  // where an addition leaves the old value; null: nobody waits for it
+  uint32_t want;  // CAS
+  uint32_t* got;  // where the old value goes; null: nobody waits for it
   bool* landed;
 };
 
@@ -41,7 +44,9 @@ std::vector<Op> flying;
 std::vector<std::unique_ptr<Fiber>> fibers;
 ucontext_t scheduler;
 int current, errors, timeouts;
-bool spread;  // workgroups on two XCDs
+bool spread;   // workgroups on two XCDs
+bool patient;  // waits for the others before a workgroup goes on alone
+int shared, alone;  // workgroups that took part, by verdict
 
 void yield() { swapcontext(&fibers[current]->ctx, &scheduler); }
 
@@ -59,7 +64,10 @@ void land(size_t i) {
   }
   uint32_t& w = ctl[o.word];
   if (o.got) *o.got = w;
-  w = o.kind == Op::ADD ? w + o.v : o.kind == Op::OR ? w | o.v : o.v;
+  if (o.kind == Op::CAS)
+    w = w == o.want ? o.v : w;
+  else
+    w = o.kind == Op::ADD ? w + o.v : o.kind == Op::OR ? w | o.v : o.v;
   if (o.landed) *o.landed = true;
 }
 
@@ -71,9 +79,17 @@ struct CpuMem {
   void pause() const {}
   uint32_t xcd() const { return spread ? (uint32_t)(id & 1) : 3u; }
   uint32_t uniform(uint32_t v) const { return v; }
-  void fly(int kind, int word, uint32_t v, uint32_t* got = nullptr, bool* landed = nullptr) const {
-    flying.push_back(Op{id, (decltype(Op::kind))kind, word, v, got, landed});
+  uint32_t patience() const { return patient ? 300u : 0u; }
+  void fly(int kind, int word, uint32_t v, uint32_t want = 0, uint32_t* got = nullptr, bool* landed = nullptr) const {
+    flying.push_back(Op{id, (decltype(Op::kind))kind, word, v, want, got, landed});
     yield();
+  }
+  uint32_t ask(int kind, int word, uint32_t v, uint32_t want = 0) const {
+    uint32_t got = 0;
+    bool landed = false;
+    fly(kind, word, v, want, &got, &landed);
+    while (!landed) yield();
+    return got;
   }
   void drain() const {
     for (;;) {
@@ -90,13 +106,8 @@ struct CpuMem {
   void store(int word, uint32_t v) const { fly(Op::STORE, word, v); }
   void set_bits(int word, uint32_t v) const { fly(Op::OR, word, v); }
   void add(int word, uint32_t v, bool) const { fly(Op::ADD, word, v); }
-  uint32_t fetch_add(int word, uint32_t v) const {
-    uint32_t got = 0;
-    bool landed = false;
-    fly(Op::ADD, word, v, &got, &landed);
-    while (!landed) yield();
-    return got;
-  }
+  uint32_t fetch_add(int word, uint32_t v) const { return ask(Op::ADD, word, v); }
+  uint32_t cas(int word, uint32_t want, uint32_t v) const { return ask(Op::CAS, word, v, want); }
   void timed_out() const { ++timeouts; }
 };
 
@@ -107,21 +118,21 @@ struct Launch {
 } launch;
 
 void workgroup(int id) {
-  DieSync<CpuMem> sync{{id}, (uint32_t)launch.n, 0, false, false};
+  DieSync<CpuMem> sync{{id}, (uint32_t)launch.n, (uint32_t)id, 0, 0, false, false};
   sync.start();
-  for (int p = 0; p < launch.phases; ++p) {
-    if (p == 0)
-      sync.started();
-    else
-      sync.wait();
+  sync.started();
+  if (sync.n != 0) (sync.n == sync.all ? shared : alone) += 1;
+  for (int p = 0; sync.n != 0 && p < launch.phases; ++p) {
+    sync.wait();
     for (const uint32_t s : slot)
       if (s < launch.base + (uint32_t)p) ++errors;
-    sync.mem.fly(Op::DATA, id, launch.base + (uint32_t)p + 1);
+    for (int i = 0; i < launch.n; ++i)
+      if (i == id || sync.n != sync.all) sync.mem.fly(Op::DATA, i, launch.base + (uint32_t)p + 1);
     sync.arrive();
   }
-  if (launch.meas) {
+  if (launch.meas && sync.n != 0) {
     sync.arrive();
-    if (id == 0) {
+    if (sync.wg == 0) {
       sync.wait();
       for (const uint32_t s : slot)
         if (s < launch.base + (uint32_t)launch.phases) ++errors;
@@ -139,6 +150,7 @@ bool run(const Launch& l, int resident) {
   for (int i = 0; i < l.n; ++i) fibers.push_back(std::make_unique<Fiber>());
   std::vector<int> in;
   int next = 0, left = l.n;
+  shared = alone = 0;
   for (long step = 0; left > 0 || !flying.empty(); ++step) {
     if (step > 40000000) return false;
     while (next < l.n && (int)in.size() < resident) in.push_back(next++);
@@ -172,7 +184,7 @@ bool run(const Launch& l, int resident) {
 }  // namespace
 
 int main() {
-  int bad = 0;
+  int bad = 0, sweeps[2] = {0, 0};
   for (int seed = 0; seed < 400; ++seed) {
     rng.seed((unsigned)seed);
     const int ns[] = {1, 2, 3, 5, 8, 16};
@@ -184,14 +196,21 @@ int main() {
     uint32_t base = 0;
     for (int k = 0; k < 4; ++k) {
       const Launch l = {n, (int)pick(4) + 1, pick(3) == 0, base};
-      const bool ends = run(l, n);
+      patient = pick(4) != 0;
+      const int resident = pick(2) ? n : 1 + (int)pick((uint32_t)n);
+      const bool ends = run(l, resident);
+      // all or one (the only one of a launch counts as all)
+      const bool fair = alone == 0 ? shared == l.n : alone == 1 && shared == 0;
+      ++sweeps[alone];
       bool zero = true;
       for (const uint32_t w : ctl) zero = zero && w == 0;
       base += (uint32_t)l.phases;
       for (const uint32_t s : slot) errors += s != base;
-      if (!ends || !zero || errors || timeouts) {
-        std::printf("seed %d launch %d: %d workgroups, %d phases%s: ended %d, words cleared %d, stale reads %d, timeouts %d\n",
-                    seed, k, l.n, l.phases, l.meas ? ", measured" : "", ends, zero, errors, timeouts);
+      if (!ends || !zero || !fair || errors || timeouts) {
+        std::printf("seed %d launch %d: %d workgroups, %d resident, %d phases%s: ended %d, words cleared %d, %d shared, %d "
+                    "alone, stale reads %d, timeouts %d\n",
+                    seed, k, l.n, resident, l.phases, l.meas ? ", measured" : "", ends, zero, shared, alone, errors,
+                    timeouts);
         ++bad;
         break;
       }
@@ -201,6 +220,10 @@ int main() {
     std::printf("%d of 400 sequences failed\n", bad);
     return 1;
   }
-  std::printf("die sync ok\n");
+  if (sweeps[0] < 100 || sweeps[1] < 100) {
+    std::printf("too few sweeps of a kind: %d shared, %d alone\n", sweeps[0], sweeps[1]);
+    return 1;
+  }
+  std::printf("die sync ok: %d sweeps shared, %d alone\n", sweeps[0], sweeps[1]);
   return 0;
 }
