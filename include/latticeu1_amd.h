@@ -306,7 +306,8 @@ int u1_selftest_philox(const uint32_t* ctr, const uint32_t* key, uint32_t* out, 
 /* u1_update (stream U1_STREAM_UPDATE, c3 0) as one launch in workgroups of
  * `block` threads (64 to 512, binary32 1024, in steps of 64), whatever the tuner
  * and u1_set_pass_fusion say, and synchronised.  flags 1: the first workgroup to
- * look does the whole sweep instead of waiting for the others to begin.  accepts
+ * look does the whole sweep instead of waiting for the others to begin; 2: the
+ * workgroups that share a sweep are on several XCDs instead of one.  accepts
  * (nullable): as u1_update; plaq (nullable, 4 doubles, mask_ml 0): as
  * u1_update_plaquette.  U1_ERR_ARG for lattices too large for one launch. */
 int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int32_t ovrn, const u1_metro* m,

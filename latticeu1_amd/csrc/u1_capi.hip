@@ -1008,7 +1008,7 @@ int die_prepare() {
 }
 
 int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, const Cfg& c, double* meas_dst,
-               uint32_t patience = u1d::kDiePatience) {
+               uint32_t patience = u1d::kDiePatience, bool in_order = false) {
   RET(die_prepare());
   u1d::DieArgs d{};
   void* err_dev = nullptr;
@@ -1020,6 +1020,7 @@ int die_launch(int prec, void* lat, const PhaseArgs& a, int metrop, int ovrn, co
   d.metrop = metrop;
   d.ovrn = ovrn;
   d.patience = patience;
+  d.in_order = in_order ? 1u : 0u;
   PhaseArgs b = a;
   b.meas = nullptr;
   if (meas_dst) {
@@ -2879,7 +2880,7 @@ int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int
   RET(check_metro(m));
   if (metrop < 0 || ovrn < 0 || metrop > 4095 || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
   if (mask_ml != 0 && mask_ml != 2 && mask_ml != 4) return fail(U1_ERR_ARG, "mask_ml must be 0, 2 or 4");
-  if (flags < 0 || flags > 1 || (plaq && mask_ml != 0)) return fail(U1_ERR_ARG, "bad self-test arguments");
+  if (flags < 0 || flags > 3 || (plaq && mask_ml != 0)) return fail(U1_ERR_ARG, "bad self-test arguments");
   PhaseArgs a{};
   a.single = make_rep(g, seed, 0);
   a.ml = mask_ml;
@@ -2893,7 +2894,7 @@ int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int
   if (accepts) HIPCHK(u1d::launch_fill_zero(G.counter, sizeof(unsigned long long), G.st));
   a.accepts = accepts ? G.counter : nullptr;
   RET(die_launch(prec, lat, a, metrop, ovrn, Cfg{block, 1, 0, 0}, plaq ? G.dres_dev : nullptr,
-                 flags & 1 ? 0u : u1d::kDiePatience));
+                 flags & 1 ? 0u : u1d::kDiePatience, (flags & 2) != 0));
   unsigned long long v = 0;
   if (accepts) HIPCHK(hipMemcpyAsync(&v, G.counter, sizeof(v), hipMemcpyDeviceToHost, G.st));
   if (plaq) RET(take_results(plaq, 4));

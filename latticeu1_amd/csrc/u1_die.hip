@@ -193,8 +193,9 @@ template <typename Real, bool MEAS>
 __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __restrict__ lat_base, PhaseArgs a, DieArgs d) {
   const uint32_t block = fetch_args<sizeof(Real*) + sizeof(PhaseArgs) + sizeof(DieArgs)>(blockIdx.x);
   const RepDesc& r = a.single;
-  const uint32_t row = (block >> 3) / d.groups, wg = (block >> 3) - row * d.groups;  // slab row, place in the slab
-  const uint32_t slab = 8u * row + (block & 7u);
+  // place in the slab: by the XCD that the dispatcher hands the workgroup to, or in order
+  const uint32_t k = d.in_order ? block : block >> 3, row = k / d.groups, wg = k - row * d.groups;
+  const uint32_t slab = d.in_order ? row : 8u * row + (block & 7u);
   if (slab >= d.slabs) return;
   Real* lat = lat_base + r.lat_off;
   DieSync<DieMem> sync{{d.ctl + slab * DIE_CTL, d.err, d.patience}, d.groups, wg, d.groups, 0, false, false};

@@ -102,8 +102,9 @@ hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseAr
 // kDieGroups workgroups on an XCD; any extents.  ctl: DIE_CTL words per slab,
 // zero between launches.  A wait that times out sets *err (host-visible memory).
 // patience: polls for all of a slab's workgroups to begin, after which one of them
-// does its sweep alone.  a.meas (no mask): the plaquette of the updated lattice, times scale, to
-// out[4]; a.meas holds 4 doubles per workgroup.
+// does its sweep alone.  in_order: a slab's workgroups are neighbours in the launch
+// and so on several XCDs (for tests).  a.meas (no mask): the plaquette of the updated
+// lattice, times scale, to out[4]; a.meas holds 4 doubles per workgroup.
 constexpr int kDieGroups = 32;
 constexpr int die_max_block(int elem_bytes) { return elem_bytes == 8 ? 512 : 1024; }
 struct DieArgs {
@@ -114,6 +115,7 @@ struct DieArgs {
   int32_t metrop, ovrn;
   uint32_t slabs, groups;
   uint32_t patience;
+  uint32_t in_order;
 };
 // About a millisecond, what a sweep by one workgroup takes.
 constexpr uint32_t kDiePatience = 1u << 10;
