@@ -33,6 +33,7 @@ thread_local std::string g_err;
 constexpr size_t kNoAllocScratchDoubles = 1u << 20;  // 8 MiB
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 constexpr int kMaxDevices = 64;
+constexpr int kMaxHits = 8190;  // Metropolis hits per link and pass
 constexpr int kChainMaxMargin = 1024;  // fused-pass schedule margin accepted from a tune cache
 // A fused pass must take under this fraction of the unfused pass's time:
 // overrelaxation passes save bandwidth and ramps; Metropolis passes, bound by
@@ -175,7 +176,7 @@ int check_metro(const u1_metro* m) {
   if (!m) return fail(U1_ERR_ARG, "null Metropolis settings");
   if (m->proposal != U1_PROPOSAL_INDEPENDENT && m->proposal != U1_PROPOSAL_DELTA)
     return fail(U1_ERR_ARG, "unknown proposal kind");
-  if (m->nhit < 1 || m->nhit > 8190) return fail(U1_ERR_ARG, "nhit must be in [1, 8190]");
+  if (m->nhit < 1 || m->nhit > kMaxHits) return fail(U1_ERR_ARG, "nhit must be in [1, 8190]");
   if (m->proposal == U1_PROPOSAL_DELTA && !(m->step >= 0.0 && m->step <= 3.141592653589793))
     return fail(U1_ERR_ARG, "the delta proposal needs 0 <= step <= pi");
   return U1_OK;
@@ -981,6 +982,8 @@ constexpr int kDieMaxHalfVolume = 1 << 14;
 // With a multilevel mask every slab runs on an XCD by itself: sites of an XCD's
 // slabs up to which the two are compared.
 constexpr int kDieMaxSlabSites = 1 << 16;
+// the accepted hits of a slab's four phases, counted by one wavefront (k_die)
+static_assert(4ull * kDieMaxSlabSites * kMaxHits < 1ull << 32, "more than a 32-bit count holds");
 // A one-launch sweep must take under this fraction of the launches' time.
 constexpr float kDieMinGain = 0.97f;
 

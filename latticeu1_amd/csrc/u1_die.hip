@@ -230,8 +230,11 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
     die_phase<Real, 1, MEAS>(lat, a, r, sync, own, acc, v, step);
     die_phase<Real, 2, MEAS>(lat, a, r, sync, own, acc, v, step);
     die_phase<Real, 3, MEAS>(lat, a, r, sync, own, acc, v, step);
+    // four phases at a time: of at most 2^16 sites and 8190 hits each, acc holds them,
+    // but not those of many passes
+    if (a.accepts && (threadIdx.x & 63) == 0 && acc) atomicAdd(a.accepts, (unsigned long long)acc);
+    acc = 0;
   }
-  if (a.accepts && (threadIdx.x & 63) == 0 && acc) atomicAdd(a.accepts, (unsigned long long)acc);
   if (MEAS) {
     // one row per workgroup, folded in their order by the first
     const double o = block_sum<4>(v);

@@ -65,3 +65,15 @@ def test_selftest_sweep_arguments(u1):
                 lambda: u1.selftest_sweep(big, 1, 1, u1.BENCH_METRO, 1, 0, 64)):
         with pytest.raises(u1.U1Error, match="U1_ERR_ARG"):
             bad()
+
+
+def test_accepts_of_long_sweeps(u1):
+    """More accepted hits per wavefront and sweep than 32 bits hold: 32 workgroups of one
+    wavefront, 512 sites a phase each, 129 passes of 8190 hits are 4.33e9.  At beta = 0 a
+    binary32 hit is refused for accept words that round to 2^32 only, one in 2^25."""
+    dims = (16, 16, 16, 8)
+    lat = u1.Lattice.cold(u1.geom(dims, 0.0), u1.F32)
+    hits = 4 * int(np.prod(dims)) * 129 * 8190
+    say(f"fp32 one-launch sweep of 129 passes of 8190 hits {dims}")
+    got = u1.selftest_sweep(lat, 129, 0, u1.metro(1, 8190, 0.5), 73, 0, 64)
+    assert abs(got / hits - (1.0 - 2.0**-25)) < 1e-8
