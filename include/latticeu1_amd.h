@@ -245,12 +245,13 @@ int u1_set_pair_fusion(int32_t mode);
  * reported as U1_ERR_HIP by the next call that synchronises the library
  * stream (u1_sync, or any call returning results to the host).
  * With this mode and the pair fusion both at 1, whole sweeps of small lattices
- * (Nx Ny Nz Nt <= 2^15), and with a multilevel mask of every slab between frozen
- * slices, can also run as one launch on one XCD each, where the tuner measures it
- * faster: the same results, "Sweep<metrop>+<ovrn>[Mask<ml>]" entries, a bounded
- * wait of several seconds reported in the same way.  Its workgroups must be on the
- * card together; if other work keeps some of them out for about a millisecond, one
- * of them does the sweep alone: the same results, at a fraction of the speed. */
+ * (Nx Ny Nz Nt <= 2^15, up to 2^13 passes), and with a multilevel mask of every
+ * slab between frozen slices, can also run as one launch on one XCD each, where
+ * the tuner measures it faster: the same results, "Sweep<metrop>+<ovrn>[Mask<ml>]"
+ * entries, a bounded wait of several seconds reported in the same way.  Its
+ * workgroups must be on the card together; if other work keeps some of them out
+ * for about a millisecond, one of them does the sweep alone: the same results, at
+ * a fraction of the speed. */
 int u1_set_pass_fusion(int32_t mode);
 /* Multilevel level-2 steps (u1_multilevel): replayed from one captured
  * hipGraph (on = 1, default) or enqueued eagerly (0).  The same kernels read
@@ -309,7 +310,7 @@ int u1_selftest_philox(const uint32_t* ctr, const uint32_t* key, uint32_t* out, 
  * look does the whole sweep instead of waiting for the others to begin; 2: the
  * workgroups that share a sweep are on several XCDs instead of one.  accepts
  * (nullable): as u1_update; plaq (nullable, 4 doubles, mask_ml 0): as
- * u1_update_plaquette.  U1_ERR_ARG for lattices too large for one launch. */
+ * u1_update_plaquette.  U1_ERR_ARG for what is too large for one launch. */
 int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int32_t ovrn, const u1_metro* m,
                       uint64_t seed, uint32_t sweep, int32_t mask_ml, int32_t block, int32_t flags, uint64_t* accepts,
                       double* plaq);

@@ -984,10 +984,15 @@ constexpr int kDieMaxHalfVolume = 1 << 14;
 constexpr int kDieMaxSlabSites = 1 << 16;
 // the accepted hits of a slab's four phases, counted by one wavefront (k_die)
 static_assert(4ull * kDieMaxSlabSites * kMaxHits < 1ull << 32, "more than a 32-bit count holds");
+// Passes of a one-launch sweep: its arrivals are counted in 32 bits, and beyond
+// this many the launch itself is long.
+constexpr int kDieMaxPasses = 1 << 13;
+static_assert(8ull * u1d::kDieGroups * (kDieMaxPasses + 1) < 1ull << 32, "more arrivals than 32 bits count");
 // A one-launch sweep must take under this fraction of the launches' time.
 constexpr float kDieMinGain = 0.97f;
 
-bool die_possible(const RepDesc& r, int ml) {
+bool die_possible(const RepDesc& r, int ml, int metrop, int ovrn) {
+  if ((int64_t)metrop + ovrn > kDieMaxPasses) return false;
   if (ml == 0) return r.HV <= kDieMaxHalfVolume;
   const int64_t rows = u1d::die_rows(u1d::die_slabs(ml, r.N[3]));
   return rows <= u1d::kDieGroups && rows * ml * r.st <= kDieMaxSlabSites;
@@ -1048,7 +1053,7 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
 int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int metrop, int ovrn, const u1_metro* m,
             Cfg* cfg) {
   *cfg = Cfg{0, 1, 0, 0};
-  if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml) || metrop + ovrn == 0) return U1_OK;
+  if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml, metrop, ovrn) || metrop + ovrn == 0) return U1_OK;
   const std::string name = "Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn) +
                            (a.ml ? "Mask" + std::to_string(a.ml) : "");
   const std::string key = tune_key(name.c_str(), g, prec);
@@ -2892,7 +2897,7 @@ int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int
   a.step = m->step;
   a.stream = U1_STREAM_UPDATE;
   a.sweep = sweep;
-  if (!die_possible(a.single, mask_ml) || block < 64 || block > u1d::die_max_block((int)elem_size(prec)) || block % 64)
+  if (!die_possible(a.single, mask_ml, metrop, ovrn) || block < 64 || block > u1d::die_max_block((int)elem_size(prec)) || block % 64)
     return fail(U1_ERR_ARG, "not a one-launch sweep");
   if (accepts) HIPCHK(u1d::launch_fill_zero(G.counter, sizeof(unsigned long long), G.st));
   a.accepts = accepts ? G.counter : nullptr;

@@ -62,6 +62,7 @@ def test_selftest_sweep_arguments(u1):
                 lambda: u1.selftest_sweep(lat, 1, 1, u1.BENCH_METRO, 1, 0, 96),
                 lambda: u1.selftest_sweep(lat, 1, 1, u1.BENCH_METRO, 1, 0, 64, 64),
                 lambda: u1.selftest_sweep(lat, 1, 1, u1.BENCH_METRO, 1, 0, 64, mask_ml=2, plaquette=True),
+                lambda: u1.selftest_sweep(lat, 1, 8192, u1.BENCH_METRO, 1, 0, 64),
                 lambda: u1.selftest_sweep(big, 1, 1, u1.BENCH_METRO, 1, 0, 64)):
         with pytest.raises(u1.U1Error, match="U1_ERR_ARG"):
             bad()
