@@ -33,7 +33,8 @@ thread_local std::string g_err;
 constexpr size_t kNoAllocScratchDoubles = 1u << 20;  // 8 MiB
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 constexpr int kMaxDevices = 64;
-constexpr int kMaxHits = 8190;  // Metropolis hits per link and pass
+constexpr int kMaxHits = 8190;    // Metropolis hits per link and pass
+constexpr int kMaxMetrop = 4095;  // Metropolis passes: 12 bits of Philox counter word 2
 constexpr int kChainMaxMargin = 1024;  // fused-pass schedule margin accepted from a tune cache
 // A fused pass must take under this fraction of the unfused pass's time:
 // overrelaxation passes save bandwidth and ramps; Metropolis passes, bound by
@@ -992,7 +993,7 @@ static_assert(8ull * u1d::kDieGroups * (kDieMaxPasses + 1) < 1ull << 32, "more a
 constexpr float kDieMinGain = 0.97f;
 
 bool die_possible(const RepDesc& r, int ml, int metrop, int ovrn) {
-  if ((int64_t)metrop + ovrn > kDieMaxPasses) return false;
+  if (metrop < 0 || metrop > kMaxMetrop || ovrn < 0 || ovrn > kDieMaxPasses - metrop || metrop + ovrn == 0) return false;
   if (ml == 0) return r.HV <= kDieMaxHalfVolume;
   const int64_t rows = u1d::die_rows(u1d::die_slabs(ml, r.N[3]));
   return rows <= u1d::kDieGroups && rows * ml * r.st <= kDieMaxSlabSites;
@@ -1053,7 +1054,7 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
 int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int metrop, int ovrn, const u1_metro* m,
             Cfg* cfg) {
   *cfg = Cfg{0, 1, 0, 0};
-  if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml, metrop, ovrn) || metrop + ovrn == 0) return U1_OK;
+  if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml, metrop, ovrn)) return U1_OK;
   const std::string name = "Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn) +
                            (a.ml ? "Mask" + std::to_string(a.ml) : "");
   const std::string key = tune_key(name.c_str(), g, prec);
@@ -1131,7 +1132,7 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
                uint32_t stream, uint32_t sweep, uint32_t c3, int ml, unsigned long long* acc_dev,
                double* meas_dst, const uint32_t* sweep_dev, uint32_t sweep_mul, bool one_launch) {
   // the Metropolis pass index takes 12 bits of Philox counter word 2
-  if (metrop < 0 || ovrn < 0 || metrop > 4095) return fail(U1_ERR_ARG, "bad pass counts");
+  if (metrop < 0 || ovrn < 0 || metrop > kMaxMetrop) return fail(U1_ERR_ARG, "bad pass counts");
   PhaseArgs a{};
   a.single = make_rep(g, seed, c3);
   a.reps = nullptr;
@@ -1975,7 +1976,7 @@ int u1_update(const u1_geom* g, int prec, void* lat, int32_t metrop, int32_t ovr
   RET(check_prec(prec));
   RET(check_metro(m));
   if (!lat) return fail(U1_ERR_ARG, "null lattice");
-  if (metrop < 0 || ovrn < 0 || metrop > 4095) return fail(U1_ERR_ARG, "bad pass counts");
+  if (metrop < 0 || ovrn < 0 || metrop > kMaxMetrop) return fail(U1_ERR_ARG, "bad pass counts");
   if (mask_ml != 0 && mask_ml != 2 && mask_ml != 4) return fail(U1_ERR_ARG, "mask_ml must be 0, 2 or 4");
   if (accepts) HIPCHK(u1d::launch_fill_zero(G.counter, sizeof(unsigned long long), G.st));
   RET(run_update(g, prec, lat, metrop, ovrn, m, seed, stream, sweep, c3, mask_ml, accepts ? G.counter : nullptr));
@@ -1996,7 +1997,7 @@ int u1_update_plaquette(const u1_geom* g, int prec, void* lat, int32_t metrop, i
   RET(check_prec(prec));
   RET(check_metro(m));
   if (!lat || !out) return fail(U1_ERR_ARG, "null argument");
-  if (metrop < 0 || ovrn < 0 || metrop > 4095 || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
+  if (metrop < 0 || ovrn < 0 || metrop > kMaxMetrop || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
   RET(run_update(g, prec, lat, metrop, ovrn, m, seed, stream, sweep, c3, 0, nullptr, G.dres_dev));
   return take_results(out, 4);
 }
@@ -2211,7 +2212,7 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     a.step = m->step;
     rc = settle_update_cfgs(prec, g, wl, a, metrop, ovrn);
     a.ml = 2;
-    if (rc == U1_OK) rc = die_cfg(g, prec, wl, a, metrop, ovrn, m, &die);
+    if (rc == U1_OK && k2 > 0) rc = die_cfg(g, prec, wl, a, metrop, ovrn, m, &die);
     if (rc == U1_OK && die.block != 0) rc = die_prepare();
     if (rc != U1_OK) {
       cleanup();
@@ -2386,7 +2387,7 @@ int u1_ensemble_create(u1_ensemble** out, int32_t nrep, const u1_geom* geoms, co
                        const int32_t* hot, int prec, int32_t metrop, int32_t ovrn, const u1_metro* m) {
   REQ_INIT();
   if (!out || !geoms || !seeds || nrep < 1 || nrep > 65535) return fail(U1_ERR_ARG, "bad ensemble arguments");
-  if (metrop < 0 || ovrn < 0 || metrop > 4095 || ovrn > 4095) return fail(U1_ERR_ARG, "bad pass counts");
+  if (metrop < 0 || ovrn < 0 || metrop > kMaxMetrop || ovrn > 4095) return fail(U1_ERR_ARG, "bad pass counts");
   RET(check_prec(prec));
   RET(check_metro(m));
   *out = nullptr;
@@ -2886,7 +2887,7 @@ int u1_selftest_sweep(const u1_geom* g, int prec, void* lat, int32_t metrop, int
   RET(check_geom(g));
   RET(check_prec(prec));
   RET(check_metro(m));
-  if (metrop < 0 || ovrn < 0 || metrop > 4095 || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
+  if (metrop < 0 || ovrn < 0 || metrop > kMaxMetrop || metrop + ovrn == 0) return fail(U1_ERR_ARG, "bad pass counts");
   if (mask_ml != 0 && mask_ml != 2 && mask_ml != 4) return fail(U1_ERR_ARG, "mask_ml must be 0, 2 or 4");
   if (flags < 0 || flags > 3 || (plaq && mask_ml != 0)) return fail(U1_ERR_ARG, "bad self-test arguments");
   PhaseArgs a{};
