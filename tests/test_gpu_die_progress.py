@@ -3,6 +3,8 @@ the others to begin, one workgroup does the whole sweep (of its slab).  Binary64
 bit for bit against the oracle, binary32 against a launch per phase, identical
 accept counts; the plaquette to summation order.  Launches follow each other, so
 that control words left behind by one would show in the next."""
+import time
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,19 @@ def test_accepts_of_long_sweeps(u1):
     say(f"fp32 one-launch sweep of 129 passes of 8190 hits {dims}")
     got = u1.selftest_sweep(lat, 129, 0, u1.metro(1, 8190, 0.5), 73, 0, 64)
     assert abs(got / hits - (1.0 - 2.0**-25)) < 1e-8
+
+
+def test_tuning_time_of_long_sweeps(u1):
+    """Choosing the launches of a sweep does not run that sweep over and over: the first
+    call, tuning included, within ten of the second."""
+    lat = u1.Lattice.cold(u1.geom((4, 4, 6, 4), 1.0), u1.F64)
+    lat.hotstart(3)
+    t = []
+    for s in range(2):
+        u1.sync()
+        t0 = time.perf_counter()
+        lat.update(0, 8000, u1.BENCH_METRO, 3, s)
+        u1.sync()
+        t.append(time.perf_counter() - t0)
+    say(f"fp64 8000 passes: {t[0]:.3f} s with tuning, {t[1]:.3f} s without")
+    assert t[0] < 10 * t[1]
