@@ -248,10 +248,10 @@ int u1_set_pair_fusion(int32_t mode);
  * (Nx Ny Nz Nt <= 2^15, up to 2^13 passes), and with a multilevel mask of every
  * slab between frozen slices, can also run as one launch on one XCD each, where
  * the tuner measures it faster: the same results, "Sweep<metrop>+<ovrn>[Mask<ml>]"
- * entries, a bounded wait of several seconds reported in the same way.  Its
- * workgroups must be on the card together; if other work keeps some of them out
- * for about a millisecond, one of them does the sweep alone: the same results, at
- * a fraction of the speed. */
+ * entries ("...Plaq" for sweeps with their plaquette), a bounded wait of several
+ * seconds reported in the same way.  Its workgroups must be on the card together;
+ * if other work keeps some of them out for about a millisecond, one of them does
+ * the sweep alone: the same results, at a fraction of the speed. */
 int u1_set_pass_fusion(int32_t mode);
 /* Multilevel level-2 steps (u1_multilevel): replayed from one captured
  * hipGraph (on = 1, default) or enqueued eagerly (0).  The same kernels read

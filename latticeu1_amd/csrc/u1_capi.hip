@@ -1050,15 +1050,18 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
 // Workgroup size of the one-launch sweep of these passes, or block = 0: not
 // with forced or forbidden fusion, large lattices or slabs, or where the tuner
 // (on a scratch copy; cached per geometry and pass counts, block.x 0 =
-// launches per phase) measures the launches faster.
+// launches per phase) measures the launches faster.  meas: of the sweep with its
+// plaquette, which costs the one launch about 10 us and the launches less; without
+// tuning, and with no such entry loaded, as the plain sweep.
 int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int metrop, int ovrn, const u1_metro* m,
-            Cfg* cfg) {
+            bool meas, Cfg* cfg) {
   *cfg = Cfg{0, 1, 0, 0};
   if (G.chain != 1 || G.pair != 1 || !die_possible(a.single, a.ml, metrop, ovrn)) return U1_OK;
   const std::string name = "Sweep" + std::to_string(metrop) + "+" + std::to_string(ovrn) +
                            (a.ml ? "Mask" + std::to_string(a.ml) : "");
-  const std::string key = tune_key(name.c_str(), g, prec);
-  const auto it = G.tunecache.find(key);
+  const std::string plain = tune_key(name.c_str(), g, prec), key = meas ? tune_key((name + "Plaq").c_str(), g, prec) : plain;
+  auto it = G.tunecache.find(key);
+  if (it == G.tunecache.end() && meas && !G.tune) it = G.tunecache.find(plain);
   if (it != G.tunecache.end()) {
     *cfg = it->second;
     return U1_OK;
@@ -1067,8 +1070,9 @@ int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int
   HIPCHK(hipStreamIsCapturing(G.st, &cs));
   if (!G.tune || cs != hipStreamCaptureStatusNone) return U1_OK;
   const int64_t bytes = 4 * (int64_t)a.single.V * (int64_t)elem_size(prec);
-  DevBuf scratch;
+  DevBuf scratch, plaq;
   HIPCHK(scratch.alloc(bytes));
+  if (meas) HIPCHK(plaq.alloc(4 * sizeof(double)));
   HIPCHK(hipMemcpyAsync(scratch.p, lat, bytes, hipMemcpyDeviceToDevice, G.st));
   EventSet es;
   hipEvent_t e0, e1;
@@ -1081,9 +1085,9 @@ int die_cfg(const u1_geom* g, int prec, const void* lat, const PhaseArgs& a, int
   // (4^3 x 6, binary64, 8000 passes: 4.5 s of tuning before a sweep of 0.11 s)
   const int mp = std::min(metrop, 4), op = std::min(ovrn, 4);
   auto one = [&](const Cfg& c) -> int {
-    if (c.block != 0) return die_launch(prec, scratch.p, p, mp, op, c, nullptr);
+    if (c.block != 0) return die_launch(prec, scratch.p, p, mp, op, c, plaq.as<double>());
     return run_update(g, prec, scratch.p, mp, op, m, a.single.seed, a.stream, a.sweep, a.single.c3, a.ml,
-                      nullptr, nullptr, nullptr, 0, false);
+                      nullptr, plaq.as<double>(), nullptr, 0, false);
   };
   auto timed = [&](const Cfg& c, float* best) -> int {
     RET(one(c));  // warm-up
@@ -1151,7 +1155,7 @@ int run_update(const u1_geom* g, int prec, void* lat, int metrop, int ovrn, cons
   a.accepts = acc_dev;
   if (one_launch) {
     Cfg die;
-    RET(die_cfg(g, prec, lat, a, metrop, ovrn, m, &die));
+    RET(die_cfg(g, prec, lat, a, metrop, ovrn, m, meas_dst != nullptr, &die));
     if (die.block != 0) return die_launch(prec, lat, a, metrop, ovrn, die, meas_dst);
   }
   Shapes sm, so;
@@ -2215,7 +2219,7 @@ int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32
     a.step = m->step;
     rc = settle_update_cfgs(prec, g, wl, a, metrop, ovrn);
     a.ml = 2;
-    if (rc == U1_OK && k2 > 0) rc = die_cfg(g, prec, wl, a, metrop, ovrn, m, &die);
+    if (rc == U1_OK && k2 > 0) rc = die_cfg(g, prec, wl, a, metrop, ovrn, m, false, &die);
     if (rc == U1_OK && die.block != 0) rc = die_prepare();
     if (rc != U1_OK) {
       cleanup();
