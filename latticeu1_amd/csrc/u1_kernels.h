@@ -46,7 +46,7 @@ hipError_t launch_phase(int prec, int kind, int mu, void* lat_base, const PhaseA
 // Nx/2 * Ny.  Batched replicas (a.reps, a.blockmap): every replica descriptor
 // carries its own set_phase_blocks(r, Nx/2 * Ny) with blk_begin its first
 // workgroup, the block map covers nblocks, plane_sites is the largest plane;
-// no measurement.  spt 1, 2 (both precisions), 3 or 4 (binary32); block a
+// no measurement, spt 1 or 2.  spt 1, 2 (both precisions), 3 or 4 (binary32); block a
 // multiple of 64 up to pair_max_block; plane_sites up to pair_max_plane (the
 // plane's new theta_0 is exchanged through LDS).  a.meas makes phase
 // (parity, 1) measuring.

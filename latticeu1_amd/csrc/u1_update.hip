@@ -631,7 +631,8 @@ void launch_pair_form(int form, Real* lat, const PhaseArgs& a, int nblocks, int 
 template <typename Real, int KIND, int SPT>
 hipError_t launch_pair_meas(Real* lat, const PhaseArgs& a, int nblocks, int block, size_t lds, hipStream_t s) {
   if (a.reps != nullptr) {  // batched replicas: no measuring pairs; the form per workgroup
-    k_pair<Real, KIND, SPT, false, true><<<nblocks, block, lds, s>>>(lat, 0, 0, 0, 0, 0, 0, 0, 0, 0, a);
+    if constexpr (SPT > 2) return hipErrorInvalidValue;  // no ensemble shape has them
+    else k_pair<Real, KIND, SPT, false, true><<<nblocks, block, lds, s>>>(lat, 0, 0, 0, 0, 0, 0, 0, 0, 0, a);
     return hipGetLastError();
   }
   // a single lattice: its plane and row size fix the form
