@@ -64,21 +64,23 @@ PHASES = (1, 1, 1, 2, 2, 2, 4, 4, 4)
 KERNEL_NAMES = ("k_phase<float> Metropolis (parity, mu) phase",
                 "k_phase<float> overrelaxation (parity, mu) phase",
                 "k_phase<float, MEAS> overrelaxation phase summing the plaquette",
-                "k_pair<float> fused Metropolis (parity, 0) + (parity, 1)",
-                "k_pair<float> fused overrelaxation (parity, 0) + (parity, 1)",
-                "k_pair<float, MEAS> fused overrelaxation pair summing the plaquette",
+                "k_pair<float> / k_walk<float> two fused Metropolis phases, (parity, 0) + (parity, 1) / (parity, 2) + (parity, 3)",
+                "k_pair<float> / k_walk<float> two fused overrelaxation phases, (parity, 0) + (parity, 1) / (parity, 2) + "
+                "(parity, 3)",
+                "k_pair<float, MEAS> / k_walk<float, MEAS> two fused overrelaxation phases summing the plaquette",
                 "k_chain<float> fused Metropolis parity pass (phases 0-3)",
                 "k_chain<float> fused overrelaxation parity pass (phases 0-3)",
                 "k_chain<float, MEAS> fused overrelaxation parity pass summing the plaquette")
 # kernel-trace names of each class (template arguments: phase <Real, MU, KIND,
-# BATCHED, SPT, MEAS>, pair <Real, KIND, SPT, MEAS, BATCHED, FORM>, pass <Real,
-# KIND, SPT, MEAS>; KIND 0 Metropolis, 1 overrelaxation)
+# BATCHED, SPT, MEAS>, pair <Real, KIND, SPT, MEAS, BATCHED, FORM>, packed pair
+# <Real, KIND, MEAS>, walk <Real, KIND, MODE, UNIFORM, BATCHED>, pass <Real, KIND,
+# SPT, MEAS>; KIND 0 Metropolis, 1 overrelaxation; MODE 0 plain, 1 measuring)
 TRACE_PATTERNS = (r"k_phase<float, \d, 0, (false|true), \d, false>",
                   r"k_phase<float, \d, 1, (false|true), \d, false>",
                   r"k_phase<float, \d, 1, (false|true), \d, true>",
-                  r"k_pair<float, 0, \d, false(, (false|true)(, \d)?)?>",
-                  r"k_pair<float, 1, \d, false(, (false|true)(, \d)?)?>",
-                  r"k_pair<float, 1, \d, true(, (false|true)(, \d)?)?>",
+                  r"k_(pair<float, 0, \d, false(, (false|true)(, \d)?)?|pair_packed<float, 0, false|walk<float, 0, 0, .*)>",
+                  r"k_(pair<float, 1, \d, false(, (false|true)(, \d)?)?|pair_packed<float, 1, false|walk<float, 1, 0, .*)>",
+                  r"k_(pair<float, 1, \d, true(, (false|true)(, \d)?)?|pair_packed<float, 1, true|walk<float, 1, 1, .*)>",
                   r"k_chain<float, 0, \d, false>",
                   r"k_chain<float, 1, \d, false>",
                   r"k_chain<float, 1, \d, true>")
