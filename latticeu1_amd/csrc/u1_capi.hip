@@ -977,8 +977,8 @@ int settle_update_cfgs(int prec, const u1_geom* g, const void* lat, const PhaseA
 // ------------------------------------------------------- one-launch sweeps
 // Lattices that one XCD's share of the card may still run faster than the whole
 // card does with a launch per one or two phases.  The tuner compares the two up
-// to here: in binary32 16^3 x 8 (2^14 sites per phase) takes 50 us per sweep
-// against 55, 16^4 84 against 56; in binary64 the two meet near 2^13.
+// to here: in binary32 they are level at 16^3 x 8 (2^14 sites per phase, 50 us per
+// sweep), 16^4 takes 84 us against 56; in binary64 they meet near 2^13.
 constexpr int kDieMaxHalfVolume = 1 << 14;
 // With a multilevel mask every slab runs on an XCD by itself: sites of an XCD's
 // slabs up to which the two are compared.

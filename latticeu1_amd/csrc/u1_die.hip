@@ -36,12 +36,12 @@
 // reported, not hung on.
 //
 // Bound by latency: 4^4 takes as long as 8^4.  One Metropolis and three
-// overrelaxation passes, against the tuned launches: binary64 8^4 71 us against
-// 81, 12^3 x 8 82 against 95; binary32 8^4 37 us against 50, 12^3 x 16 51
-// against 67, 16^3 x 8 50 against 55.  With more sites one XCD's arithmetic
-// takes over (binary64 12^3 x 16: 115 us against 99; binary32 16^4: 84 against
-// 56).  Level-2 sweeps, every slab by itself: binary32 24^4 59 us against 80,
-// binary64 134 against 167.
+// overrelaxation passes, against the tuned launches: binary64 8^4 70 us against
+// 79, 12^3 x 8 81 against 91; binary32 8^4 38 us against 52, 12^3 x 16 51
+// against 62, 16^3 x 8 level at 50.  With more sites one XCD's arithmetic
+// takes over (binary64 12^3 x 16: 112 us against 95; binary32 16^4: 84 against
+// 56).  Masked sweeps at 24^4, every slab by itself: level 2 binary32 59 us against
+// 74, binary64 131 against 157; level 4 71 against 81, 162 against 178.
 #include "u1_kernels.h"
 #include "u1_link.h"
 
@@ -65,15 +65,18 @@ struct DieMem {
   __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
   __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
   __device__ __forceinline__ uint32_t xcd() const { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }  // XCC_ID
-  __device__ __forceinline__ uint32_t uniform(uint32_t v) const { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+  // thread 0's v; a barrier
+  __device__ __forceinline__ uint32_t broadcast(uint32_t v) const {
+    __shared__ uint32_t word;
+    if (threadIdx.x == 0) word = v;
+    barrier();
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)word);
+  }
   __device__ __forceinline__ uint32_t load(int word) const {
     return __hip_atomic_load(ctl + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __device__ __forceinline__ void store(int word, uint32_t v) const {
     __hip_atomic_store(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __device__ __forceinline__ void set_bits(int word, uint32_t v) const {
-    __hip_atomic_fetch_or(ctl + word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   // local: counted and read on one XCD only
   __device__ __forceinline__ void add(int word, uint32_t v, bool local) const {
@@ -135,7 +138,7 @@ struct DieStep {
 // The even/odd sites of a workgroup's slab, spatial and temporal phases: n of
 // them from base on, this thread's first + k stride of those.  Wavefronts are
 // dealt to the workgroups in turn, so that a phase with half the sites still
-// uses every CU (binary32 level-2 sweep at 24^4: 70 -> 64 us, level 4 110 -> 86).
+// uses every CU (binary32 level-2 sweep at 24^4: 70 -> 59 us, level 4 110 -> 77).
 struct DieSites {
   uint32_t base, n, base3, n3, first, stride;
 };
@@ -205,8 +208,11 @@ __global__ __launch_bounds__(die_max_block(sizeof(Real))) void k_die(Real* __res
   const uint32_t frozen = a.ml ? 1u : 0u;
   DieSites own = {(t0 + frozen) * half, (nt - frozen) * half, t0 * half, nt * half,
                   ((threadIdx.x >> 6) * d.groups + wg) * 64u + (threadIdx.x & 63u), d.groups * blockDim.x};
-  // (in front of the first phase and not, as the other waits, behind its loads: the
-  // choice there cost every phase registers, 102 us at 8^4 instead of 97)
+  // In front of the first phase and not, as the other waits, behind its loads: the
+  // choice there cost every phase registers (8^4 with plaquette 102 us per call, 97
+  // here).  One addition carries both count and XCDs, and thread 0 hands on what it
+  // polled: with an addition each, and a load by all threads, a sweep took 2 us more
+  // (binary64 8^4 75.7 -> 73.9, binary32 16^3 x 8 55.4 -> 53.4).
   sync.started();
   if (sync.n == 0) {
     sync.leave();

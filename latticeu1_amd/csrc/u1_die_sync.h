@@ -14,9 +14,17 @@
 namespace u1d {
 
 // Words of a set of control words, each on a cache line of its own; all zero
-// between launches.  DIE_HERE: workgroups that have begun, and from bit 16 on one
-// more than the number of the one that goes on alone, if any.
-enum { DIE_HERE = 0, DIE_XCDS = 32, DIE_DONE = 64, DIE_LEFT = 96, DIE_CTL = 128 };
+// between launches.  DIE_HERE, which a workgroup touches once to begin: from bit 0
+// on the workgroups that have begun, from bit 6 on one more than the number of the
+// one that goes on alone, if any, from bit 12 on the sum of their XCDs' numbers
+// and from bit 20 on of the numbers' squares (all on one XCD if and only if the
+// squares' sum times the workgroups is the sum's square).
+enum { DIE_HERE = 0, DIE_DONE = 32, DIE_LEFT = 64, DIE_CTL = 96 };
+constexpr int kDieGroups = 32;  // workgroups at most
+constexpr int kDieXcds = 8;
+static_assert(kDieGroups < 1 << 6 && kDieGroups * (kDieXcds - 1) < 1 << 8 &&
+                  kDieGroups * (kDieXcds - 1) * (kDieXcds - 1) < 1 << 12,
+              "fields of DIE_HERE");
 
 // Progress.  Workgroups may only wait for others that are resident, and other
 // work on the card -- a one-launch sweep of another process, whose workgroups
@@ -37,9 +45,8 @@ struct DieSync {
 
   __host__ __device__ __forceinline__ void start() {
     if (mem.leader()) {
-      mem.set_bits(DIE_XCDS, 1u << mem.xcd());
-      mem.drain();
-      mem.add(DIE_HERE, 1u, false);
+      const uint32_t x = mem.xcd() % kDieXcds;
+      mem.add(DIE_HERE, 1u | x << 12 | x * x << 20, false);
     }
     n = all;
     target = 0;
@@ -49,11 +56,12 @@ struct DieSync {
   // Before the first store.  n then is all, or 1 if this workgroup goes on alone
   // (as number 0), or 0 if another one does.
   __host__ __device__ __forceinline__ void started() {
+    uint32_t v = 0;
     if (mem.leader()) {
-      uint32_t v = mem.load(DIE_HERE);
-      for (uint32_t k = 0; v < all; ++k) {
+      v = mem.load(DIE_HERE);
+      for (uint32_t k = 0; (v & 0xfffu) < all; ++k) {
         if (k >= mem.patience()) {
-          const uint32_t mark = v | (wg + 1u) << 16, old = mem.cas(DIE_HERE, v, mark);
+          const uint32_t mark = v | (wg + 1u) << 6, old = mem.cas(DIE_HERE, v, mark);
           v = old == v ? mark : old;
         } else {
           mem.pause();
@@ -61,11 +69,11 @@ struct DieSync {
         }
       }
     }
-    mem.barrier();
-    const uint32_t v = mem.uniform(mem.load(DIE_HERE)), m = mem.uniform(mem.load(DIE_XCDS));
-    one = (m & (m - 1)) == 0;
-    if (v >> 16) {
-      n = v >> 16 == wg + 1u ? 1u : 0u;
+    v = mem.broadcast(v);
+    const uint32_t mark = v >> 6 & 0x3fu, sum = v >> 12 & 0xffu;
+    one = all * (v >> 20) == sum * sum;
+    if (mark) {
+      n = mark == wg + 1u ? 1u : 0u;
       wg = 0;
       one = true;
     }
@@ -96,7 +104,7 @@ struct DieSync {
     if (!mem.leader()) return;
     mem.drain();
     if (mem.fetch_add(DIE_LEFT, 1u) + 1 != all) return;
-    for (int w : {DIE_HERE, DIE_XCDS, DIE_DONE, DIE_LEFT}) mem.store(w, 0u);
+    for (int w : {DIE_HERE, DIE_DONE, DIE_LEFT}) mem.store(w, 0u);
   }
 };
 

@@ -105,7 +105,6 @@ hipError_t launch_walk_batched(int prec, int kind, void* lat_base, const PhaseAr
 // does its sweep alone.  in_order: a slab's workgroups are neighbours in the launch
 // and so on several XCDs (for tests).  a.meas (no mask): the plaquette of the updated
 // lattice, times scale, to out[4]; a.meas holds 4 doubles per workgroup.
-constexpr int kDieGroups = 32;
 constexpr int die_max_block(int elem_bytes) { return elem_bytes == 8 ? 512 : 1024; }
 struct DieArgs {
   uint32_t* ctl;

@@ -30,7 +30,7 @@ struct Fiber {
 };
 struct Op {
   int fiber;
-  enum { ADD, OR, CAS, STORE, DATA } kind;
+  enum { ADD, CAS, STORE, DATA } kind;
   int word;
   uint32_t v;
   uint32_t want;  // CAS
@@ -67,7 +67,7 @@ void land(size_t i) {
   if (o.kind == Op::CAS)
     w = w == o.want ? o.v : w;
   else
-    w = o.kind == Op::ADD ? w + o.v : o.kind == Op::OR ? w | o.v : o.v;
+    w = o.kind == Op::ADD ? w + o.v : o.v;
   if (o.landed) *o.landed = true;
 }
 
@@ -77,8 +77,8 @@ struct CpuMem {
   bool leader() const { return true; }
   void barrier() const {}
   void pause() const {}
-  uint32_t xcd() const { return spread ? (uint32_t)(id & 1) : 3u; }
-  uint32_t uniform(uint32_t v) const { return v; }
+  uint32_t xcd() const { return spread ? (uint32_t)id % 8u : 3u; }
+  uint32_t broadcast(uint32_t v) const { return v; }
   uint32_t patience() const { return patient ? 300u : 0u; }
   void fly(int kind, int word, uint32_t v, uint32_t want = 0, uint32_t* got = nullptr, bool* landed = nullptr) const {
     flying.push_back(Op{id, (decltype(Op::kind))kind, word, v, want, got, landed});
@@ -104,7 +104,6 @@ struct CpuMem {
     return ctl[word];
   }
   void store(int word, uint32_t v) const { fly(Op::STORE, word, v); }
-  void set_bits(int word, uint32_t v) const { fly(Op::OR, word, v); }
   void add(int word, uint32_t v, bool) const { fly(Op::ADD, word, v); }
   uint32_t fetch_add(int word, uint32_t v) const { return ask(Op::ADD, word, v); }
   uint32_t cas(int word, uint32_t want, uint32_t v) const { return ask(Op::CAS, word, v, want); }
