@@ -161,7 +161,9 @@ int u1_temporal_links(const u1_geom* g, int prec, const void* lat, int32_t mode,
  * Sublattice updates: metrop/ovrn passes with m, Philox streams ML_L4 / ML_L2,
  * c1 = step index, c3 = call_id.  Temporal links: mh_mode (U1_POLY_MULTIHIT as
  * the reference, or U1_POLY_MULTIHIT_STOCHASTIC with mh).  out[2*(Nx/2)];
- * ppspace_dev (nullable): 2*SV*(Nx/2)*3 doubles (MultiLevelField).  Nt % 4 == 0. */
+ * ppspace_dev (nullable): 2*SV*(Nx/2)*3 doubles (MultiLevelField).  Nt % 4 == 0.
+ * The device workspace stays allocated for the next call, up to 1 GiB, until
+ * u1_finalize; a larger one is freed before the call returns. */
 int u1_multilevel(const u1_geom* g, int prec, const void* lat, int32_t n4, int32_t k4, int32_t n2, int32_t k2,
                   int32_t metrop, int32_t ovrn, const u1_metro* m, int32_t mh_mode, const u1_metro* mh,
                   uint64_t seed, uint32_t call_id, double* out, void* ppspace_dev);
@@ -230,7 +232,8 @@ int u1_tune_enable(int32_t on);
  * wavefronts walking along the diagonals e_t - e_z, bit-identical too; entries
  * "MetropolisWalk" / "OverRelaxationWalk" (block.x 0 = two launches).  An
  * ensemble takes both kinds of launch over all its replicas, tuned over whole
- * sweeps (mode 1) or always (mode 2), but for the measuring parity. */
+ * sweeps (mode 1) or always (mode 2); only a pair whose planes are too large to
+ * share workgroups runs as two launches in the measuring parity. */
 int u1_set_pair_fusion(int32_t mode);
 /* Fused parity passes (no reference counterpart): on a single lattice without
  * multilevel mask whose (z, t) planes tile 2 x 4 (Nz even, Nt a multiple of
@@ -263,6 +266,9 @@ int u1_set_graph_capture(int32_t on);
  * its choice on stderr), 2 VERBOSE and 3 DEBUG_VERBOSE (every candidate's
  * time).  Callable before u1_init. */
 int u1_set_verbosity(int32_t level);
+/* Entries of a file replace those held.  A file saved by an older library is
+ * accepted: its choices give the same results, but were made against that
+ * library's launches, and only what it lacks is tuned. */
 int u1_tune_load(const char* path);
 int u1_tune_save(const char* path);
 /* Number of launch-shape entries held (tuned in this process or loaded). */

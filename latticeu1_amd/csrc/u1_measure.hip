@@ -79,7 +79,7 @@ __device__ __forceinline__ void staple_t(const Real* __restrict__ lat, const Rep
 // one wrap step each way (|delta| <= pi); otherwise wrap_d's four.  Bound by
 // its vector instructions: a binary32 hit takes 62 of them (80 before the FMA
 // proposal, the single wrap steps and the sign flips of u1m::sincos_f) and half
-// a Philox draw.  The 100-hit correlator at 24^3 x 48 takes 150 us, 200 us
+// a Philox draw.  The 100-hit correlator at 24^3 x 48 takes 136 us, 200 us
 // before (about 30 us of that from the hits).
 template <typename Real, bool NEAR>
 __device__ __forceinline__ C64 multihit_sum(const RepDesc& r, Real th, Real Sre, Real Sim, uint32_t l, int proposal,

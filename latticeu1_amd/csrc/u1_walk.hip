@@ -94,7 +94,7 @@ enum { WALK_PLAIN = 0, WALK_MEAS = 1, WALK_MASK = 2 };
 // dispatcher writes into scalar registers, as for k_pair: what a walk needs before
 // its first load.  packed: shifts of the four magic divisions by five bits, parity,
 // log2 of width and sg, plain order.  Binary32 at 24^3 x 48: overrelaxation 6.07 ->
-// 5.84 us, Metropolis 9.35 -> 9.19; binary64 at 24^3 x 12: overrelaxation 6.3 -> 6.1.
+// 5.84 us, Metropolis 9.35 -> 9.17; binary64 at 24^3 x 12: overrelaxation 6.3 -> 6.1.
 template <typename Real, int KIND, int MODE, bool UNIFORM, bool BATCHED = false>
 __global__ __launch_bounds__(64 * walk_max_waves(sizeof(Real))) void k_walk(
     Real* __restrict__ lat_base, uint32_t N1, uint32_t N2, uint32_t N3, uint32_t nxh, uint32_t div_nxh_m,
