@@ -48,6 +48,12 @@ constexpr size_t kMlSlotBytes = (size_t)256 << 20;
 constexpr size_t kMlKeepBytes = (size_t)1 << 30;
 // A walk must take under this fraction of the two phases' time.
 constexpr float kWalkMinGain = 0.97f;
+// While tuning, a shape is not timed again whose single launch takes this many times
+// the two phases' time (it counts its event's microseconds), which then falls this
+// far behind them, or this far behind the best shape.
+constexpr float kWalkTooSlow = 3.0f;
+constexpr float kWalkBehind = 1.5f;
+constexpr float kWalkBehindBest = 1.1f;
 double* g_scratch_dev[kMaxDevices] = {};
 
 // Launch shape of an update phase kernel: workgroup size, even/odd sites per
@@ -631,16 +637,17 @@ int walk_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseA
   a.accepts = nullptr;
   a.meas = nullptr;
   Shapes s = sh;
-  auto timed = [&](const Cfg& c, float* best) -> int {
+  // mean time of reps launches after one to warm up
+  auto timed = [&](const Cfg& c, float* best, int reps) -> int {
     s.walk = c;
-    RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));  // warm-up
+    RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));
     HIPCHK(hipEventRecord(e0, G.st));
-    for (int rep = 0; rep < 4; ++rep) RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));
+    for (int rep = 0; rep < reps; ++rep) RET(launch_two_phases(prec, kind, scratch.p, a, s, 2, no_rows));
     HIPCHK(hipEventRecord(e1, G.st));
     HIPCHK(hipEventSynchronize(e1));
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-    *best = std::min(*best, ms);
+    *best = std::min(*best, ms / (float)reps);
     return U1_OK;
   };
   auto shape = [](const Cfg& c) {
@@ -650,32 +657,54 @@ int walk_cfg(int prec, int kind, const u1_geom* g, const void* lat, const PhaseA
     else o << "plain order";
     return o.str();
   };
+  const Cfg none{0, 1, 0, 0};
+  float tsep = 1e30f;
+  for (int round = 0; round < 3; ++round) RET(timed(none, &tsep, 4));
+  const int reps = std::max(1, std::min(4, (int)(0.15f / tsep)));  // a tenth of a millisecond or so
+  // three rounds over the candidates, but not over those that a launch shows to be
+  // far behind the two phases, nor again over those behind the best (with few
+  // diagonals all are, up to fifteen times: a first call at 28 x 20 x 36 x 22,
+  // binary64, took 300 ms, 48 without walks)
   auto search = [&](const std::vector<Cfg>& cands, std::vector<float>& tbest) -> int {
     tbest.assign(cands.size(), 1e30f);
-    for (int round = 0; round < 3; ++round)
-      for (size_t i = 0; i < cands.size(); ++i) RET(timed(cands[i], &tbest[i]));
+    std::vector<char> out(cands.size(), 0);
+    for (size_t i = 0; i < cands.size(); ++i) {
+      RET(timed(cands[i], &tbest[i], 1));
+      out[i] = tbest[i] > kWalkTooSlow * tsep;
+    }
+    for (int round = 0; round < 3; ++round) {
+      for (size_t i = 0; i < cands.size(); ++i)
+        if (!out[i]) RET(timed(cands[i], &tbest[i], reps));
+      const float most = std::min(kWalkBehind * tsep, kWalkBehindBest * *std::min_element(tbest.begin(), tbest.end()));
+      for (size_t i = 0; i < cands.size(); ++i) out[i] = out[i] || tbest[i] > most;
+    }
     if (G.verbosity >= 2)
       for (size_t i = 0; i < cands.size(); ++i)
-        std::fprintf(stderr, "tune %s: %s: %.2f us per walk\n", key.c_str(), shape(cands[i]).c_str(),
-                     1e3 * tbest[i] / 4.0);
+        std::fprintf(stderr, "tune %s: %s: %.2f us per walk\n", key.c_str(), shape(cands[i]).c_str(), 1e3 * tbest[i]);
     return U1_OK;
   };
   std::vector<float> t1, t2;
   RET(search(shapes, t1));
+  if (*std::min_element(t1.begin(), t1.end()) > kWalkBehindBest * tsep) {
+    if (G.verbosity >= 1) std::fprintf(stderr, "tune %s: no walk near two launches %.2f us\n", key.c_str(), 1e3 * tsep);
+    G.tunecache[key] = none;
+    return U1_OK;
+  }
   const std::vector<Cfg> orders = walk_orders(shapes, t1);
   RET(search(orders, t2));
   const Cfg best = orders[(size_t)(std::min_element(t2.begin(), t2.end()) - t2.begin())];
   // both sides timed afresh, alternating (chain_cfg), and a clear win asked for
-  float tb = 1e30f, tsep = 1e30f;
+  float tb = 1e30f;
+  tsep = 1e30f;
   for (int round = 0; round < 5; ++round) {
-    RET(timed(best, &tb));
-    RET(timed(Cfg{0, 1, 0, 0}, &tsep));
+    RET(timed(best, &tb, reps));
+    RET(timed(none, &tsep, reps));
   }
   const bool use = tb < kWalkMinGain * tsep;
   if (G.verbosity >= 1)
-    std::fprintf(stderr, "tune %s: walk %.2f us (%s) vs two launches %.2f us: %s\n", key.c_str(), 1e3 * tb / 4.0,
-                 shape(best).c_str(), 1e3 * tsep / 4.0, use ? "walk" : "separate");
-  *cfg = use ? best : Cfg{0, 1, 0, 0};
+    std::fprintf(stderr, "tune %s: walk %.2f us (%s) vs two launches %.2f us: %s\n", key.c_str(), 1e3 * tb,
+                 shape(best).c_str(), 1e3 * tsep, use ? "walk" : "separate");
+  *cfg = use ? best : none;
   G.tunecache[key] = *cfg;
   return U1_OK;
 }
