@@ -46,7 +46,7 @@ ucontext_t scheduler;
 int current, errors, timeouts;
 bool spread;   // workgroups on two XCDs
 bool patient;  // waits for the others before a workgroup goes on alone
-int shared, alone;  // workgroups that took part, by verdict
+int shared, alone;  // workgroups that took part: in a shared sweep, by themselves
 
 void yield() { swapcontext(&fibers[current]->ctx, &scheduler); }
 
